@@ -44,14 +44,30 @@ struct Coefs {
     EulerCoef<double> eu_d; EulerCoef<float> eu_f;
 };
 
-// One trapezoid launch: tile t stores the points [t*W_out, t*W_out + W_out)
-// (the last tile clipped at nX) after S stages, W_out = 64*PO, from a window
-// of 64*(PO+SB) points; S = 32*SB stages for heat and 16*SB for KS / Euler.
+// One trapezoid launch (Euler): tile t stores the cells [t*W_out, t*W_out +
+// W_out) (the last tile clipped at nX) after 16 stages, W_out = 64*PO, from a
+// window of 64*(PO+SB) cells, SB = 1.
 struct TrapLaunch {
     int eq, bc, PO, SB;
     int64_t n, ntiles, tile_first;
     const void* in;
     void* out;
+};
+
+// One launch of workgroup-wide overlapped tiles (sw1d_wide.hip): `steps` whole
+// time steps of a heat or KS field, plain values in and out.
+struct WideLaunch {
+    int eq, bc, shape, steps;
+    int64_t n;
+    const void* in;
+    void* out;
+};
+// Tile shape and number of launches (of nearly equal steps) for an advance of
+// nsteps on a GPU of `cus` compute units, and the time they should take.
+struct WideChoice {
+    int shape = 0;
+    int64_t launches = 0;
+    double us = 0;
 };
 
 // One problem of a batch.  Periodic heat (c = {Fo, 1-2Fo}) or KS
@@ -96,6 +112,8 @@ inline bool batch_tile_supported(int po) { return po == 2 || po == 4 || po == 8 
 hipError_t launch_trapezoid(const TrapLaunch& L, bool f64, const Coefs& c, hipStream_t s);
 bool trapezoid_supported(int eq, int PO, int SB);
 inline int64_t trapezoid_steps(int eq, int SB) { return eq == EQ_HEAT ? 32 * SB : 8 * SB; }
+hipError_t launch_wide(const WideLaunch& L, bool f64, const Coefs& c, hipStream_t s);
+WideChoice wide_choose(int eq, bool f64, int64_t n, int64_t nsteps, int cus);
 hipError_t launch_swept(const SweptLaunch& L, bool f64, const Coefs& c, hipStream_t s);
 // One classic stage: heat (stage ignored), KS / Euler stage 0 = predictor,
 // 1 = corrector.  State layout as above; heat ping-pongs between in and out,

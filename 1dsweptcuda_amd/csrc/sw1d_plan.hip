@@ -59,6 +59,8 @@ struct sw1d_plan {
     int64_t tile_steps = 0;  // steps advanced by one swept tile launch
     int simds = 0;           // SIMDs of the plan's device (4 per compute unit)
     int64_t cycle_steps = 0; // reference t_fullstep / dt
+    WideChoice wide;         // tile shape and launches of an advance of wide_steps
+    int64_t wide_steps = 0;
     Coefs coef{};
     double consts[9]{};
     int nconsts = 0;
@@ -479,10 +481,10 @@ int hybrid_split_diamond(sw1d_plan* p)
     return SW1D_OK;
 }
 
-// Trapezoid launches in blocks of kTileGraphLaunches replayed from a hipGraph:
-// one graph launch instead of 16 kernel launches.  Small plans (launches of a
-// few microseconds, many plans at once on their own streams) are otherwise
-// bound by the host's launch rate: a loop of 512 such plans runs 1.4x faster.
+// Trapezoid launches (Euler) in blocks of kTileGraphLaunches replayed from a
+// hipGraph: one graph launch instead of 16 kernel launches.  Small plans
+// (launches of a few microseconds, many plans at once on their own streams) are
+// otherwise bound by the host's launch rate.
 // A block is an even number of launches, so it returns to its starting
 // buffer; a graph is kept per starting buffer and both are captured together,
 // so a later call never captures.  The kernels and their order are those of
@@ -519,8 +521,52 @@ int tile_graph_blocks(sw1d_plan* p, int64_t& launches, F&& issue_block)
     return SW1D_OK;
 }
 
+// nsteps steps of a heat or KS field as workgroup-wide overlapped tiles: any
+// number of steps, no remainder.
+int wide_advance(sw1d_plan* p, int64_t nsteps)
+{
+    if (nsteps < 1) return SW1D_OK;
+    if (p->wide_steps != nsteps) {
+        p->wide = wide_choose(p->eq, p->f64, p->n, nsteps, p->simds / 4);
+        p->wide_steps = nsteps;
+    }
+    WideLaunch L;
+    L.eq = p->eq;
+    L.bc = p->bc;
+    L.shape = p->wide.shape;
+    L.n = p->n;
+    const int64_t each = nsteps / p->wide.launches, longer = nsteps % p->wide.launches;
+    for (int64_t i = 0; i < p->wide.launches; ++i) {
+        L.steps = (int)(each + (i < longer));
+        L.in = p->buf[p->cur];
+        L.out = p->buf[p->cur ^ 1];
+        {
+            ProfScope ps(p, KK_DIAMOND);
+            HIP_OR_FAIL(launch_wide(L, p->f64, p->coef, p->stream));
+        }
+        p->cur ^= 1;
+    }
+    return SW1D_OK;
+}
+
+// Whether an advance of a swept plan runs as wide tiles.  The swept rows, one
+// launch each, are kept for Euler (2^20, FP64: 4.4e10 point-updates/s against
+// 3.7e10, wide lanes of Euler cells do not fit the registers), the hybrid,
+// FP32 KS on large fields, and per-kernel profiling, which times the swept
+// kinds.
+bool takes_wide(const sw1d_plan* p)
+{
+    if (p->eq == EQ_EULER || p->profiling) return false;
+    if (p->eq == EQ_HEAT) return p->alg == SW1D_SWEPT;
+    // FP32 KS with two waves per SIMD of 512 points or more: the diamonds (2^20,
+    // 1000 steps: 790 us at W = 512 against 913 us; W = 256 949 us)
+    const int64_t nodes = p->n / p->W;
+    return p->f64 || p->W < 512 || 2 * nodes < 3 * (int64_t)p->simds;
+}
+
 int swept_advance(sw1d_plan* p, int64_t nsteps)
 {
+    if (takes_wide(p)) return wide_advance(p, nsteps);
     const int64_t H = p->tile_steps;
     int64_t rem = nsteps;
     if (nsteps >= H) {
@@ -547,6 +593,9 @@ int swept_advance(sw1d_plan* p, int64_t nsteps)
         if (rc) return rc;
         p->cur ^= 1;
     }
+    // fewer steps than a tile's: classic steps (Euler, profiling), else one wide
+    // launch instead of one or two launches per step
+    if (p->eq != EQ_EULER && !p->profiling) return wide_advance(p, rem);
     for (int64_t s = 0; s < rem; ++s) {
         int rc = classic_step(p);
         if (rc) return rc;
@@ -556,6 +605,7 @@ int swept_advance(sw1d_plan* p, int64_t nsteps)
 
 int trapezoid_advance(sw1d_plan* p, int64_t nsteps)
 {
+    if (p->eq != EQ_EULER) return wide_advance(p, nsteps);
     const int64_t H = p->tile_steps;
     const int64_t launches = nsteps / H;
     TrapLaunch L;

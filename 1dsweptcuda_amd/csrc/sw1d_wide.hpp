@@ -1,0 +1,358 @@
+// Device code of the workgroup-wide overlapped tile, shared by the single-plan
+// kernels (sw1d_wide.hip) and the batched solve (sw1d_batch.hip).
+//
+// A workgroup of NW waves holds a window of consecutive points in VGPRs and
+// advances it by any number of whole time steps; after s steps the points
+// more than R s from the window's ends hold the classic scheme's values (R =
+// points a value travels per step: 1 heat, 4 KS and Euler), and the tile
+// stores those.  The wave is the unit that computes: lane l holds P
+// consecutive points, neighbours cross lanes by DPP, and every lane updates
+// every point it holds, so the steady loop has no mask, no select and no
+// memory access: 12.5 instructions per KS point and stage, 12 of them FP64.
+// Inside the workgroup the waves overlap by HL lanes on each side.  Those halo
+// lanes go stale from the outside, and every K = HL P / R steps a wave takes
+// its neighbours' values for them through LDS: a wave repeats 2 HL / 64 of its
+// neighbours' work, and the workgroup repeats 2 R S / WIN of its neighbours'.
+//
+// Why a workgroup: the redundant share falls with the width of whatever
+// shares its halo.  A wave alone (64 x 18 points) that advances KS by 16 steps
+// repeats 11%, and a row of diamonds idles lanes outside its active set and
+// pays a compare and two selects per point for it; four waves of 18 points
+// per lane advance 48 steps for the same 11%.
+#pragma once
+
+#include "sw1d_internal.hpp"
+#include "sw1d_lanes.hpp"
+
+namespace sw1d {
+namespace wide {
+
+enum Ends : int { ENDS_PERIODIC = 0, ENDS_MIRROR = 1, ENDS_FIXED = 2 };
+
+template <int EQ, int P_, int NW_, int HL_>
+struct Shape {
+    static constexpr int P = P_, NW = NW_, HL = HL_;
+    static constexpr int NC = EQ == EQ_EULER ? 3 : 1;  // values per point between launches
+    static constexpr int RS = EQ == EQ_HEAT ? 1 : 2;   // stencil radius of one stage
+    static constexpr int R = EQ == EQ_HEAT ? 1 : 4;    // reach of one step
+    static constexpr int NT = NW * kWave;
+    static constexpr int STRIDE = (kWave - 2 * HL) * P;      // points a wave owns
+    static constexpr int WIN = NW * STRIDE + 2 * HL * P;     // points of the window
+    static constexpr int K = HL * P / R;                     // steps between exchanges
+    static_assert(K >= 1 && 4 * HL <= kWave, "the halo lanes hold at least one step's reach");
+    // LDS, in values: one component's window image, or the exchanged edges (two
+    // sets used in turn, so one barrier per exchange is enough)
+    static constexpr int EDGE = NW * 2 * HL * NC * P;
+    static constexpr bool DIRECT = P <= 2;  // lanes read and write the field themselves
+    static constexpr int LDS = (!DIRECT && WIN > 2 * EDGE) ? WIN : 2 * EDGE;
+};
+
+// Field index of point g of the window, which may lie outside 0 .. n-1.
+// Periodic: modulo n.  Mirror: reflected at both ends, T[-k] = T[k] (the
+// insulated ends' T[-1] = T[1]); the stencil is symmetric, so the reflected
+// points stay bitwise the mirror image and no end needs a check.  Fixed: the
+// points outside are never used (the ends are pinned), any value will do.
+__device__ __forceinline__ int64_t field_index(int64_t g, int64_t n, int ends, bool near)
+{
+    if (ends == ENDS_PERIODIC) {
+        if (near) return g < 0 ? g + n : (g >= n ? g - n : g);
+        const int32_t m = (int32_t)n;  // a window wider than the field: n is small
+        const int32_t r = (int32_t)g % m;
+        return r < 0 ? r + m : r;
+    }
+    if (ends == ENDS_MIRROR) {
+        if (near) {
+            g = g < 0 ? -g : g;
+            return g >= n ? 2 * (n - 1) - g : g;
+        }
+        const int32_t m = 2 * ((int32_t)n - 1);
+        int32_t r = (int32_t)g % m;
+        r = r < 0 ? -r : r;
+        return r < (int32_t)n ? r : m - r;
+    }
+    return g < 0 ? 0 : (g >= n ? n - 1 : g);
+}
+
+// 16-byte LDS copies of P values (d is 16-byte aligned when P is a multiple of
+// 16 / sizeof(T); else the values go one by one)
+template <typename T, int P>
+__device__ __forceinline__ void put(T* d, const T (&v)[P])
+{
+    constexpr int V = 16 / sizeof(T);
+    typedef T vec __attribute__((ext_vector_type(V)));
+    if constexpr (P % V == 0) {
+#pragma unroll
+        for (int p = 0; p < P; p += V) {
+            vec t;
+#pragma unroll
+            for (int q = 0; q < V; ++q) t[q] = v[p + q];
+            *reinterpret_cast<vec*>(d + p) = t;
+        }
+    } else {
+#pragma unroll
+        for (int p = 0; p < P; ++p) d[p] = v[p];
+    }
+}
+template <typename T, int P>
+__device__ __forceinline__ void take(const T* d, T (&v)[P])
+{
+    constexpr int V = 16 / sizeof(T);
+    typedef T vec __attribute__((ext_vector_type(V)));
+    if constexpr (P % V == 0) {
+#pragma unroll
+        for (int p = 0; p < P; p += V) {
+            const vec t = *reinterpret_cast<const vec*>(d + p);
+#pragma unroll
+            for (int q = 0; q < V; ++q) v[p + q] = t[q];
+        }
+    } else {
+#pragma unroll
+        for (int p = 0; p < P; ++p) v[p] = d[p];
+    }
+}
+
+// One Euler stage over the lane's P cells (Euler:307-389): dst = base + c
+// flux(src), each interface once.  ENDS: this wave holds cell 0 or n-1, which
+// take the Dirichlet states and drop the outermost pressure differences.
+template <typename T, int P, bool ENDS>
+__device__ __forceinline__ void euler_stage(const T (&src)[3][P], T (&dst)[3][P], const T (&base)[3][P],
+                                            T (&hl)[3][2], T (&hr)[3][2], int c0, int cN, T c,
+                                            const EulerCoef<T>& k)
+{
+    T ex[P + 4], ey[P + 4], ez[P + 4];
+    gather_carry<T, P, 2>(src[0], hl[0], hr[0], ex);
+    gather_carry<T, P, 2>(src[1], hl[1], hr[1], ey);
+    gather_carry<T, P, 2>(src[2], hl[2], hr[2], ez);
+    auto cell = [&](int j) { return Q3<T>{ex[j], ey[j], ez[j]}; };
+    T pd[P + 3];
+#pragma unroll
+    for (int j = 0; j < P + 3; ++j) pd[j] = eu_pdiff(cell(j), cell(j + 1));
+    // interface j lies between ext cells j+1 and j+2 (the lane's cell p is ext
+    // cell p+2); c0 / cN: the lane's p of cell 0 / n-1
+    auto iface = [&](int j, Q3<T>& F, Q3<T>& D) {
+        T q0 = pd[j], q2 = pd[j + 2];
+        if (ENDS) {
+            q0 = j - 1 == c0 ? T(0) : q0;
+            q2 = j == cN ? T(0) : q2;
+        }
+        eu_iface(cell(j), cell(j + 1), cell(j + 2), cell(j + 3), q0, pd[j + 1], q2, k, F, D);
+    };
+    Q3<T> FL, DL;
+    iface(0, FL, DL);
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        Q3<T> FR, DR;
+        iface(p + 1, FR, DR);
+        Q3<T> nv = eu_apply(Q3<T>{base[0][p], base[1][p], base[2][p]}, eu_balance(FL, DL, FR, DR), c);
+        if (ENDS) {
+            nv = p == c0 ? k.bl : nv;
+            nv = p == cN ? k.br : nv;
+        }
+        dst[0][p] = nv.x;
+        dst[1][p] = nv.y;
+        dst[2][p] = nv.z;
+        FL = FR;
+        DL = DR;
+    }
+}
+
+template <typename T> struct Coef { T fo, fo2; KsCoef<T> ks; EulerCoef<T> eu; };
+
+// k steps of the wave's points.  The lanes at the window's ends keep the
+// neighbour they last had (carried registers): their points are stale anyway.
+template <typename T, int EQ, class S>
+struct Steps {
+    static constexpr int P = S::P, NC = S::NC, RS = S::RS;
+    T v[NC][P], q[NC][P];
+    T hl[NC][RS], hr[NC][RS], gl[NC][RS], gr[NC][RS];
+
+    __device__ __forceinline__ void start()
+    {
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int i = 0; i < RS; ++i) hl[c][i] = hr[c][i] = gl[c][i] = gr[c][i] = v[c][0];
+    }
+    __device__ __forceinline__ void heat(const T (&s)[P], T (&d)[P], T (&a)[1], T (&b)[1], const Coef<T>& k)
+    {
+        T e[P + 2];
+        gather_carry<T, P, 1>(s, a, b, e);
+#pragma unroll
+        for (int p = 0; p < P; ++p) d[p] = heat_ftcs(e[p], e[p + 1], e[p + 2], k.fo, k.fo2);
+    }
+    template <bool ENDS>
+    __device__ __forceinline__ void run(int steps, const Coef<T>& k, int c0, int cN)
+    {
+        if constexpr (EQ == EQ_HEAT) {
+            if (steps & 1) {
+                heat(v[0], q[0], hl[0], hr[0], k);
+#pragma unroll
+                for (int p = 0; p < P; ++p) v[0][p] = q[0][p];
+            }
+            for (int s = steps >> 1; s > 0; --s) {
+                heat(v[0], q[0], hl[0], hr[0], k);
+                heat(q[0], v[0], gl[0], gr[0], k);
+            }
+        } else if constexpr (EQ == EQ_KS) {
+            for (int s = steps; s > 0; --s) {
+                {
+                    T e[P + 4];
+                    gather_carry<T, P, 2>(v[0], hl[0], hr[0], e);
+#pragma unroll
+                    for (int p = 0; p < P; ++p) q[0][p] = ks_predict(e[p], e[p + 1], e[p + 2], e[p + 3], e[p + 4], k.ks);
+                }
+                {
+                    T e[P + 4];
+                    gather_carry<T, P, 2>(q[0], gl[0], gr[0], e);
+#pragma unroll
+                    for (int p = 0; p < P; ++p)
+                        v[0][p] = ks_correct(v[0][p], e[p], e[p + 1], e[p + 2], e[p + 3], e[p + 4], k.ks);
+                }
+            }
+        } else {
+            const T ca = T(0.25) * k.eu.dtdx, cb = T(0.5) * k.eu.dtdx;
+            for (int s = steps; s > 0; --s) {
+                euler_stage<T, P, ENDS>(v, q, v, hl, hr, c0, cN, ca, k.eu);  // predictor
+                euler_stage<T, P, ENDS>(q, v, v, gl, gr, c0, cN, cb, k.eu);  // corrector
+            }
+        }
+    }
+};
+
+// One tile: out[out0 .. out0 + count) after `steps` steps from the field `in`
+// of n points (component stride cs in both).  The window starts R steps
+// before out0; lds holds Shape::LDS values.
+template <typename T, int EQ, class S>
+__device__ __forceinline__ void tile(T* lds, const T* __restrict__ in, T* __restrict__ out, int64_t n, int64_t cs,
+                                     int64_t out0, int count, int steps, int ends, const Coef<T>& k)
+{
+    constexpr int P = S::P, NW = S::NW, HL = S::HL, NC = S::NC, NT = S::NT, WIN = S::WIN;
+    constexpr int NL = (WIN + NT - 1) / NT;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), w = tid >> 6;
+    const int halo = S::R * steps;
+    const int64_t win = out0 - halo;
+    const int x0 = w * S::STRIDE + lane * P;  // window position of the lane's first point
+    const bool inside = win >= 0 && win + WIN <= n;
+    const bool near = win >= -(n - 1) && win + WIN <= 2 * n - 1;
+    Steps<T, EQ, S> st;
+    if constexpr (S::DIRECT) {
+        if (inside) {
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+#pragma unroll
+                for (int p = 0; p < P; ++p) st.v[c][p] = in[c * cs + win + x0 + p];
+        } else {
+#pragma unroll
+            for (int p = 0; p < P; ++p) {
+                const int64_t g = field_index(win + x0 + p, n, ends, near);
+#pragma unroll
+                for (int c = 0; c < NC; ++c) st.v[c][p] = in[c * cs + g];
+            }
+        }
+    } else {
+        // coalesced through the LDS image, every load of a component in flight
+        // at once (also where the window wraps: one slow tile would hold up
+        // the whole launch)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            T r[NL];
+            if (inside) {
+                const T* a = in + c * cs + win;
+#pragma unroll
+                for (int j = 0; j < NL; ++j)
+                    if (tid + j * NT < WIN) r[j] = a[tid + j * NT];
+            } else {
+#pragma unroll
+                for (int j = 0; j < NL; ++j)
+                    if (tid + j * NT < WIN) r[j] = in[c * cs + field_index(win + tid + j * NT, n, ends, near)];
+            }
+            if (c > 0) __syncthreads();  // the previous component's image has been read
+#pragma unroll
+            for (int j = 0; j < NL; ++j)
+                if (tid + j * NT < WIN) lds[tid + j * NT] = r[j];
+            __syncthreads();
+#pragma unroll
+            for (int p = 0; p < P; ++p) st.v[c][p] = lds[x0 + p];
+        }
+        __syncthreads();
+    }
+    st.start();
+    // Euler's Dirichlet cells 0 and n-1: the lane's p of each where one of its
+    // interfaces touches it (c0 = -1 and cN = P: the neighbour lane's cell)
+    int c0 = -9, cN = -9;
+    bool fixed = false;
+    if constexpr (EQ == EQ_EULER) {
+        const int64_t g = win + x0;
+        if (g <= 1 && g > -P) c0 = (int)-g;
+        if (n - 1 - g >= 0 && n - 1 - g <= P) cN = (int)(n - 1 - g);
+        fixed = __builtin_amdgcn_ballot_w64(c0 != -9 || cN != -9) != 0;
+    }
+
+    const bool left = lane < 2 * HL;
+    const bool wr = (lane >= HL && left) || (lane >= kWave - 2 * HL && lane < kWave - HL);
+    const bool rd = (lane < HL && w > 0) || (lane >= kWave - HL && w < NW - 1);
+    // edge slot (wave, side, lane within the edge): a wave writes its own two
+    // edges and reads the facing ones of its neighbours
+    const int wslot = left ? (2 * w) * HL + lane - HL : (2 * w + 1) * HL + lane - (kWave - 2 * HL);
+    const int rslot = left ? (2 * w - 1) * HL + lane : (2 * w + 2) * HL + lane - (kWave - HL);
+    int todo = steps, set = 0;
+    for (;;) {
+        const int s = NW == 1 || todo < S::K ? todo : S::K;
+        todo -= s;
+        if constexpr (EQ == EQ_EULER) {
+            if (fixed)
+                st.template run<true>(s, k, c0, cN);
+            else
+                st.template run<false>(s, k, c0, cN);
+        } else {
+            st.template run<false>(s, k, c0, cN);
+        }
+        if (todo <= 0) break;
+        T* e = lds + set;
+        set = S::EDGE - set;
+        if (wr) {
+#pragma unroll
+            for (int c = 0; c < NC; ++c) put<T, P>(e + (wslot * NC + c) * P, st.v[c]);
+        }
+        __syncthreads();
+        if (rd) {
+#pragma unroll
+            for (int c = 0; c < NC; ++c) take<T, P>(e + (rslot * NC + c) * P, st.v[c]);
+        }
+    }
+
+    const bool own = (lane >= HL || w == 0) && (lane < kWave - HL || w == NW - 1);
+    if constexpr (S::DIRECT) {
+        if (own) {
+#pragma unroll
+            for (int p = 0; p < P; ++p) {
+                const int i = x0 + p - halo;
+                if (i >= 0 && i < count) {
+#pragma unroll
+                    for (int c = 0; c < NC; ++c) out[c * cs + out0 + i] = st.v[c][p];
+                }
+            }
+        }
+    } else {
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            __syncthreads();  // the last edges, or the previous component, have been read
+            if (own) {
+#pragma unroll
+                for (int p = 0; p < P; ++p) lds[x0 + p] = st.v[c][p];
+            }
+            __syncthreads();
+            T r[NL];
+#pragma unroll
+            for (int j = 0; j < NL; ++j)
+                if (tid + j * NT < count) r[j] = lds[halo + tid + j * NT];
+            T* o = out + c * cs + out0;
+#pragma unroll
+            for (int j = 0; j < NL; ++j)
+                if (tid + j * NT < count) o[tid + j * NT] = r[j];
+        }
+    }
+}
+
+}  // namespace wide
+}  // namespace sw1d

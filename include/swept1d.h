@@ -46,7 +46,11 @@ enum { SW1D_F64 = 0, SW1D_F32 = 1 };
 /* Algorithm = argv[6] of the reference: 0 classic, 1 shared swept,
  * 2 hybrid CPU+GPU swept (heat, Euler) / register swept (KS).
  * 3 (library only, no reference counterpart): overlapped trapezoid tiles —
- * swept up-triangles widened by a redundant halo, any nx, same bits. */
+ * swept up-triangles widened by a redundant halo, any nx, same bits.
+ * Heat and KS advances of 1, 3 and the KS 2 run as overlapped tiles a
+ * workgroup wide wherever those are faster than a row of swept tiles per
+ * launch (all but FP32 KS on large fields); per-kernel profiling runs and
+ * times the swept rows. */
 enum { SW1D_CLASSIC = 0, SW1D_SWEPT = 1, SW1D_ALT = 2, SW1D_TRAPEZOID = 3 };
 /* Boundary conditions.  DEFAULT picks the reference's: heat insulated
  * (mirror, Heat:140-142), KS periodic (KS:199), Euler Dirichlet ghost cells
@@ -131,7 +135,7 @@ int sw1d_advance_noalloc(const sw1d_problem* problem, void* d_state, int64_t nst
 
 /* Plan facts ----------------------------------------------------------------
  * info[0] node width (points per swept node), info[1] steps advanced by one
- * swept tile launch, info[2] values stored per point (2 heat and KS, 6 Euler),
+ * row of swept tiles, info[2] values stored per point (2 heat and KS, 6 Euler),
  * info[3] device bytes held by the plan, info[4] steps per reference cycle
  * (the t_fullstep of sweptWrapper / classicWrapper divided by dt). */
 int sw1d_plan_info(const sw1d_plan* plan, int64_t info[5]);
@@ -143,8 +147,10 @@ int sw1d_plan_constants(const sw1d_plan* plan, double* out, int32_t capacity);
 int sw1d_plan_stream(const sw1d_plan* plan, void** stream);
 
 /* Per-kernel timing: when enabled, every launch of the plan is bracketed by
- * hipEvents on the plan's stream.  kind: 0 classic stage, 1 up-triangle,
- * 2 down-triangle, 3 diamond, 4 split (boundary-straddling) diamond. */
+ * hipEvents on the plan's stream, and SW1D_SWEPT / SW1D_ALT advance by rows of
+ * swept tiles and classic remainder steps.  kind: 0 classic stage,
+ * 1 up-triangle, 2 down-triangle, 3 diamond (SW1D_TRAPEZOID: overlapped tile),
+ * 4 split (boundary-straddling) diamond. */
 int sw1d_set_profiling(sw1d_plan* plan, int32_t enabled);
 int sw1d_kernel_stats(sw1d_plan* plan, int32_t kind, int64_t* launches, double* total_ms);
 
