@@ -7,14 +7,22 @@
 //   L6   64 -> 1 channel    FP32 VALU over BF16 activations
 // output du = L6(...); the integrator adds it to u (residual form).
 //
-// Activations are channel-last [B][X][64] BF16; pre-activations Z are kept in
-// FP32 for the GELU derivative.  A 64->64 layer is a GEMM per 64-position
-// tile: M = positions, N = output channels, K = 5 taps x 64 input channels,
-// staged in LDS in the operand layouts of the MFMA (8 consecutive K values per
-// lane, 16-byte LDS reads).  The weight gradient is a GEMM over positions
-// (K = positions) with both operands staged transposed; each workgroup writes
-// its partial sum and a second kernel adds the partials in a fixed order, so
-// gradients are deterministic.
+// Activations are channel-last [B][X][64] BF16.  A 64->64 layer is a GEMM per
+// tile of 256 (or 64) positions: M = positions, N = output channels, K = 5 taps
+// x 64 input channels, staged in LDS in the operand layouts of the MFMA (8
+// consecutive K values per lane, 16-byte LDS reads).
+//
+// Training (one gradient at batch 64 x 1024: 160 us on the GPU, 480 us before)
+// keeps two more forms of what a layer computes.  The FP32
+// pre-activations Z, for the GELU derivative, are stored in the accumulators'
+// own lane order, since only the lanes that hold the same outputs in the
+// backward pass read them (16 bytes per lane, no gaps).  And the layer inputs
+// and the gradients dZ are stored position-contiguous, [B][64][X], as the
+// accumulators hold them (a lane has four positions of one channel): the weight
+// gradient is a GEMM over positions (K = positions), whose operands are then
+// plain 16-byte loads.  Each workgroup adds its positions' share in registers
+// and LDS and writes one partial sum; a second kernel adds the partials in a
+// fixed order, so gradients are deterministic.
 
 #include <hip/hip_runtime.h>
 
@@ -29,13 +37,16 @@
 namespace sw1dnn {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x2u __attribute__((ext_vector_type(2), aligned(4)));
+typedef __bf16 bf16x4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int C = 64;       // hidden channels
 constexpr int TAPS = 5;     // kernel width
-constexpr int TILE = 64;    // positions per workgroup
+constexpr int TILE = 64;    // positions nx is a multiple of
 constexpr int NT = 256;     // threads per workgroup
-constexpr int ROWP = C + 8; // padded LDS row (bf16 elements)
 
 // ---------------------------------------------------------------- bf16 ---
 // Round to nearest even (NaN kept quiet), the same rule the host oracle uses.
@@ -120,111 +131,77 @@ __global__ void k_mfma_check(int* ok)
     }
 }
 
-// ------------------------------------------------------ L1: 1 -> 64, VALU ---
-// Z1[b][x][c] = b1[c] + sum_t w1[c][t] u[b][x+t-2];  A1 = bf16(gelu(Z1))
-__global__ __launch_bounds__(NT) void k_l1_fwd(const float* __restrict__ u, const float* __restrict__ w1,
-                                               const float* __restrict__ b1, float* __restrict__ Z,
-                                               __bf16* __restrict__ A, int X)
-{
-    const int b = blockIdx.y;
-    const int i = blockIdx.x * NT + threadIdx.x;  // x * C + c within sample b
-    if (i >= X * C) return;
-    const int c = i % C, x = i / C;
-    const float* ub = u + (int64_t)b * X;
-    float z = b1[c];
-    for (int t = 0; t < TAPS; ++t) z = fmaf(w1[c * TAPS + t], ub[wrapx(x + t - 2, X)], z);
-    const int64_t o = (int64_t)b * X * C + i;
-    Z[o] = z;
-    A[o] = f2bf(gelu(z));
-}
-
 // ----------------------------------------------- L2-L5: 64 -> 64, MFMA ---
 // Z[b][x][co] = bias[co] + sum_t sum_ci A[b][x+t-2][ci] W[t][co][ci]
-__global__ __launch_bounds__(NT) void k_mid_fwd(const __bf16* __restrict__ Ain, const __bf16* __restrict__ Wf,
-                                                const float* __restrict__ bias, float* __restrict__ Z,
-                                                __bf16* __restrict__ Aout, int X)
-{
-    __shared__ __attribute__((aligned(16))) __bf16 sA[(TILE + 4) * ROWP];
-    __shared__ __attribute__((aligned(16))) __bf16 sW[TAPS * C * ROWP];
-    const int b = blockIdx.y, x0 = blockIdx.x * TILE;
-    const __bf16* Ab = Ain + (int64_t)b * X * C;
-    // stage rows x0-2 .. x0+TILE+1 (16-byte chunks: 8 channels)
-    for (int q = threadIdx.x; q < (TILE + 4) * (C / 8); q += NT) {
-        const int r = q / (C / 8), ch = (q % (C / 8)) * 8;
-        const int x = wrapx(x0 - 2 + r, X);
-        *reinterpret_cast<uint4*>(&sA[r * ROWP + ch]) =
-            *reinterpret_cast<const uint4*>(&Ab[(int64_t)x * C + ch]);
-    }
-    for (int q = threadIdx.x; q < TAPS * C * (C / 8); q += NT) {
-        const int r = q / (C / 8), ch = (q % (C / 8)) * 8;  // r = t*C + co
-        *reinterpret_cast<uint4*>(&sW[r * ROWP + ch]) = *reinterpret_cast<const uint4*>(&Wf[r * C + ch]);
-    }
-    __syncthreads();
-    const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int m0 = 16 * w, li = l % 16, lk = 8 * (l / 16);
-    f32x4 acc[4];
-    for (int nb = 0; nb < 4; ++nb) acc[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int s = 0; s < TAPS * 2; ++s) {
-        const int t = s >> 1, cb = (s & 1) * 32;
-        const bf16x8 a = *reinterpret_cast<const bf16x8*>(&sA[(m0 + li + t) * ROWP + cb + lk]);
-        for (int nb = 0; nb < 4; ++nb) {
-            const bf16x8 bv = *reinterpret_cast<const bf16x8*>(&sW[(t * C + 16 * nb + li) * ROWP + cb + lk]);
-            acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bv, acc[nb], 0, 0, 0);
-        }
-    }
-    for (int nb = 0; nb < 4; ++nb) {
-        const int co = 16 * nb + li;
-        for (int j = 0; j < 4; ++j) {
-            const int x = x0 + m0 + 4 * (l / 16) + j;
-            const float z = acc[nb][j] + bias[co];
-            const int64_t o = ((int64_t)b * X + x) * C + co;
-            Z[o] = z;
-            Aout[o] = f2bf(gelu(z));
-        }
-    }
-}
-
-// Same product over 256 positions per workgroup of 8 waves: the 40 KB of
-// staged weights serve four times the positions of k_mid_fwd, each wave owns
-// 32 positions x 64 channels (8 accumulator tiles, so four waves fit per SIMD
-// and one workgroup's MFMAs overlap another's GELU epilogue).
+// over TF positions per workgroup of TF/32 waves, 32 positions x 64 channels
+// each (8 accumulator tiles, so four waves fit per SIMD and one workgroup's
+// MFMAs overlap another's GELU epilogue).  TF = 256, for the 40 KB of staged
+// weights to serve many positions, where nx allows; else 64.
 constexpr int TILE_F = 256;
-constexpr int NTW = 512;            // threads of the wide kernels
-constexpr int WROWS = TILE_F / (NTW / 64);  // positions per wave
-constexpr int MB = WROWS / 16;      // 16-row MFMA blocks per wave
-static_assert(NTW >= TILE_F, "the output-layer epilogue maps one thread to one position");
+constexpr int WROWS = 32;       // positions per wave
+constexpr int MB = WROWS / 16;  // 16-row MFMA blocks per wave
+template <int TF> struct Tile {
+    static constexpr int NW = TF / WROWS, NT = NW * 64;
+};
+// Transposed activations [B][64][XT]: position p of a sample at p + 2 of a row
+// of XT = X + 8, which also holds the periodic neighbours -2, -1, X, X + 1, so
+// that the 12 positions around an 8-position operand start 16-byte aligned.
+__host__ __device__ inline int xt(int X) { return X + 8; }
+
 // LDS rows of 64 BF16 (8 chunks of 16 bytes) with chunk c of row r stored at
 // chunk c ^ (r & 7): the 16 rows read together by a fragment load hit 8
 // different chunk slots, so no padding is needed (2 workgroups fit per CU).
 __device__ __forceinline__ int swz(int r, int chunk) { return r * C + ((chunk ^ (r & 7)) << 3); }
 
-// rows x0-2 .. x0+TILE_F+1 of one sample's [X][64] BF16 activation -> sA
-__device__ __forceinline__ void stage_act(__bf16* sA, const __bf16* __restrict__ Ab, int x0, int X)
-{
-    for (int q = threadIdx.x; q < (TILE_F + 4) * (C / 8); q += NTW) {
-        const int r = q / (C / 8), c8 = q % (C / 8);
-        const int x = wrapx(x0 - 2 + r, X);
-        *reinterpret_cast<uint4*>(&sA[swz(r, c8)]) =
-            *reinterpret_cast<const uint4*>(&Ab[(int64_t)x * C + c8 * 8]);
+// 16-byte chunks of rows of 64 BF16 on their way from memory to an LDS tile:
+// every load of a thread is in flight before the first store (one by one they
+// cost a memory latency each, 3 us of a 10 us layer).
+template <int TF, int ROWS>
+struct Staged {
+    static constexpr int NT = Tile<TF>::NT, CHUNKS = ROWS * (C / 8), N = (CHUNKS + NT - 1) / NT;
+    u32x4 v[N];
+    // row r from src(r)
+    template <typename F>
+    __device__ __forceinline__ void load(F&& src)
+    {
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const int q = threadIdx.x + i * NT;
+            if (CHUNKS % NT == 0 || q < CHUNKS)
+                v[i] = *reinterpret_cast<const u32x4*>(src(q / (C / 8)) + q % (C / 8) * 8);
+        }
     }
-}
-// a layer's packed weights [t][co][ci] -> sW (rows t*64 + co)
-__device__ __forceinline__ void stage_w(__bf16* sW, const __bf16* __restrict__ Wf)
-{
-    for (int q = threadIdx.x; q < TAPS * C * (C / 8); q += NTW) {
-        const int r = q / (C / 8), c8 = q % (C / 8);
-        *reinterpret_cast<uint4*>(&sW[swz(r, c8)]) = *reinterpret_cast<const uint4*>(&Wf[r * C + c8 * 8]);
+    __device__ __forceinline__ void store(__bf16* lds) const
+    {
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const int q = threadIdx.x + i * NT;
+            if (CHUNKS % NT == 0 || q < CHUNKS) *reinterpret_cast<u32x4*>(&lds[swz(q / (C / 8), q % (C / 8))]) = v[i];
+        }
     }
+};
+// rows x0-2 .. x0+TF+1 of one sample's [X][64] BF16 activation -> sA, and a
+// layer's packed weights [t][co][ci] -> sW (rows t*64 + co)
+template <int TF>
+__device__ __forceinline__ void stage(__bf16* sA, const __bf16* __restrict__ Ab, int x0, int X, __bf16* sW,
+                                      const __bf16* __restrict__ W)
+{
+    Staged<TF, TF + 4> act;
+    Staged<TF, TAPS * C> wts;
+    act.load([&](int r) { return Ab + (int64_t)wrapx(x0 - 2 + r, X) * C; });
+    wts.load([&](int r) { return W + r * C; });
+    act.store(sA);
+    wts.store(sW);
 }
-// Layer 1 evaluated straight into sA: rows x0-2 .. x0+TILE_F+1 of
-// bf16(gelu(b1 + sum_t w1[c][t] in[x+t-2])), with in = FP32(u) * inv_scale
-// (the same operations and order as k_l1_fwd and k_to_input, so the same bits).
-template <typename TIN>
+// Layer 1 evaluated straight into sA: rows x0-2 .. x0+TF+1 of
+// bf16(gelu(b1 + sum_t w1[c][t] in[x+t-2])), with in = FP32(u) * inv_scale.
+template <int TF, typename TIN>
 __device__ __forceinline__ void stage_l1(__bf16* sA, float* sIn, const TIN* __restrict__ ub, float inv_scale,
                                          const float* __restrict__ w1, const float* __restrict__ b1, int x0,
                                          int X)
 {
-    for (int q = threadIdx.x; q < TILE_F + 8; q += NTW) sIn[q] = (float)ub[wrapx(x0 - 4 + q, X)] * inv_scale;
+    constexpr int NTW = Tile<TF>::NT;
+    for (int q = threadIdx.x; q < TF + 8; q += NTW) sIn[q] = (float)ub[wrapx(x0 - 4 + q, X)] * inv_scale;
     const int c8 = threadIdx.x % (C / 8);  // fixed per thread: NTW is a multiple of 8
     float w[8][TAPS], bb[8];
 #pragma unroll
@@ -234,7 +211,7 @@ __device__ __forceinline__ void stage_l1(__bf16* sA, float* sIn, const TIN* __re
         for (int t = 0; t < TAPS; ++t) w[k][t] = w1[(c8 * 8 + k) * TAPS + t];
     }
     __syncthreads();
-    for (int r = threadIdx.x / (C / 8); r < TILE_F + 4; r += NTW / (C / 8)) {
+    for (int r = threadIdx.x / (C / 8); r < TF + 4; r += NTW / (C / 8)) {
         bf16x8 v;
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
@@ -246,7 +223,9 @@ __device__ __forceinline__ void stage_l1(__bf16* sA, float* sIn, const TIN* __re
         *reinterpret_cast<bf16x8*>(&sA[swz(r, c8)]) = v;
     }
 }
-// acc[mb][nb] = the wave's WROWS positions x 64 channels of sum_t A(x+t-2) W[t]^T
+// acc[mb][nb] = the wave's WROWS positions x 64 channels of
+//   FORWARD: sum_t A(x+t-2) W[t]^T;  else: sum_t dZ(x-t+2) W[t]
+template <bool FORWARD>
 __device__ __forceinline__ void mfma_tile(const __bf16* sA, const __bf16* sW, f32x4 (&acc)[MB][4])
 {
     const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -258,10 +237,10 @@ __device__ __forceinline__ void mfma_tile(const __bf16* sA, const __bf16* sW, f3
 #pragma unroll 2
     for (int s = 0; s < TAPS * 2; ++s) {
         const int t = s >> 1, chunk = (s & 1) * 4 + lq;  // K = channels (s&1)*32 + 8*lq ..
+        const int row = m0 + li + (FORWARD ? t : 4 - t);
         bf16x8 a[MB], bv[4];
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb)
-            a[mb] = *reinterpret_cast<const bf16x8*>(&sA[swz(m0 + 16 * mb + li + t, chunk)]);
+        for (int mb = 0; mb < MB; ++mb) a[mb] = *reinterpret_cast<const bf16x8*>(&sA[swz(row + 16 * mb, chunk)]);
 #pragma unroll
         for (int nb = 0; nb < 4; ++nb)
             bv[nb] = *reinterpret_cast<const bf16x8*>(&sW[swz(t * C + 16 * nb + li, chunk)]);
@@ -272,89 +251,133 @@ __device__ __forceinline__ void mfma_tile(const __bf16* sA, const __bf16* sW, f3
                 acc[mb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mb], bv[nb], acc[mb][nb], 0, 0, 0);
     }
 }
+// Z in the accumulators' order: tile, wave, (mb, nb), lane
+__device__ __forceinline__ int64_t z_index(int64_t tile, int waves, int w, int mb, int nb, int l)
+{
+    return (((tile * waves + w) * MB + mb) * 4 + nb) * 64 + l;
+}
+// four positions x .. x+3 of channel c -> a transposed activation (16 bytes
+// would need the neighbour lane's four), and their periodic copies
+__device__ __forceinline__ void store_t(__bf16* __restrict__ T, int b, int c, int x, int X, const bf16x4& v)
+{
+    __bf16* row = T + ((int64_t)b * C + c) * xt(X);
+    *reinterpret_cast<bf16x4u*>(row + 2 + x) = v;
+    if (x == 0) *reinterpret_cast<bf16x2u*>(row + 2 + X) = bf16x2u{v[0], v[1]};
+    if (x == X - 4) *reinterpret_cast<bf16x2u*>(row) = bf16x2u{v[2], v[3]};
+}
 // bias + GELU of the accumulators, rounded to BF16 into the LDS tile sO (row =
-// position in the tile, swizzled); FP32 pre-activations to Z (rows zrow0 + r)
-// when STORE_Z.  sO may alias sA once every wave has finished mfma_tile.
-template <bool STORE_Z>
+// position in the tile, swizzled).  TRAIN: also the pre-activations to Z (own
+// order) and, where T is given, the activations transposed.  sO may alias sA
+// once every wave has finished mfma_tile.
+template <int TF, bool TRAIN>
 __device__ __forceinline__ void epilogue(const f32x4 (&acc)[MB][4], const float* __restrict__ bias, __bf16* sO,
-                                         float* __restrict__ Z, int64_t zrow0)
+                                         f32x4* __restrict__ Z, __bf16* __restrict__ T, int b, int x0, int X)
 {
     const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int m0 = WROWS * w, li = l % 16, lq = l / 16;
+    const int64_t tile = (int64_t)b * (X / TF) + x0 / TF;
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) {
         const int co = 16 * nb + li;
         const float bc = bias[co];
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb)
+        for (int mb = 0; mb < MB; ++mb) {
+            const int r = m0 + 16 * mb + 4 * lq;
+            f32x4 z;
+            bf16x4 a;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const int r = m0 + 16 * mb + 4 * lq + j;
-                const float z = acc[mb][nb][j] + bc;
-                if (STORE_Z) Z[(zrow0 + r) * C + co] = z;
-                sO[swz(r, co >> 3) + (co & 7)] = f2bf(gelu(z));
+                z[j] = acc[mb][nb][j] + bc;
+                a[j] = f2bf(gelu(z[j]));
+                sO[swz(r + j, co >> 3) + (co & 7)] = a[j];
             }
+            if (TRAIN) {
+                Z[z_index(tile, Tile<TF>::NW, w, mb, nb, l)] = z;
+                if (T) store_t(T, b, co, x0 + r, X, a);
+            }
+        }
     }
 }
-// the LDS tile -> rows x0 .. x0+TILE_F-1 of a [X][64] activation (16-byte stores)
+// the LDS tile -> rows x0 .. x0+TF-1 of a [X][64] activation (16-byte stores)
+template <int TF>
 __device__ __forceinline__ void store_act(const __bf16* sO, __bf16* __restrict__ Ab, int x0)
 {
-    for (int q = threadIdx.x; q < TILE_F * (C / 8); q += NTW) {
+    for (int q = threadIdx.x; q < TF * (C / 8); q += Tile<TF>::NT) {
         const int r = q / (C / 8), c8 = q % (C / 8);
         *reinterpret_cast<uint4*>(&Ab[(int64_t)(x0 + r) * C + c8 * 8]) =
             *reinterpret_cast<const uint4*>(&sO[swz(r, c8)]);
     }
 }
 
-// One 64 -> 64 layer over 256 positions.  STORE_Z keeps the pre-activations
-// for the backward pass (training only).
-template <bool STORE_Z>
-__global__ __launch_bounds__(NTW) void k_mid_fwd_wide(const __bf16* __restrict__ Ain,
-                                                     const __bf16* __restrict__ Wf,
-                                                     const float* __restrict__ bias, float* __restrict__ Z,
-                                                     __bf16* __restrict__ Aout, int X)
+// One 64 -> 64 layer over TF positions.  TRAIN keeps what the backward pass
+// needs (epilogue).
+template <int TF, bool TRAIN>
+__global__ __launch_bounds__(Tile<TF>::NT) void k_mid_fwd(const __bf16* __restrict__ Ain,
+                                                         const __bf16* __restrict__ Wf,
+                                                         const float* __restrict__ bias, f32x4* __restrict__ Z,
+                                                         __bf16* __restrict__ T, __bf16* __restrict__ Aout, int X)
 {
-    __shared__ __attribute__((aligned(16))) __bf16 sA[(TILE_F + 4) * C];
+    __shared__ __attribute__((aligned(16))) __bf16 sA[(TF + 4) * C];
     __shared__ __attribute__((aligned(16))) __bf16 sW[TAPS * C * C];
-    const int b = blockIdx.y, x0 = blockIdx.x * TILE_F;
-    stage_act(sA, Ain + (int64_t)b * X * C, x0, X);
-    stage_w(sW, Wf);
+    const int b = blockIdx.y, x0 = blockIdx.x * TF;
+    stage<TF>(sA, Ain + (int64_t)b * X * C, x0, X, sW, Wf);
     __syncthreads();
     f32x4 acc[MB][4];
-    mfma_tile(sA, sW, acc);
+    mfma_tile<true>(sA, sW, acc);
     __syncthreads();
-    epilogue<STORE_Z>(acc, bias, sA, Z, (int64_t)b * X + x0);
+    epilogue<TF, TRAIN>(acc, bias, sA, Z, T, b, x0, X);
     __syncthreads();
-    store_act(sA, Aout + (int64_t)b * X * C, x0);
+    store_act<TF>(sA, Aout + (int64_t)b * X * C, x0);
 }
 
-// Layers 1 and 2 in one pass (inference): layer 1 is evaluated into the LDS
-// tile from the network input, so its activation never goes to memory.
-template <typename TIN>
-__global__ __launch_bounds__(NTW) void k_l12_fwd(const TIN* __restrict__ in, float inv_scale,
-                                                const float* __restrict__ w1, const float* __restrict__ b1,
-                                                const __bf16* __restrict__ Wf, const float* __restrict__ bias,
-                                                __bf16* __restrict__ Aout, int X)
+// Layers 1 and 2 in one pass: layer 1 is evaluated into the LDS tile from the
+// network input, so its activation goes to memory only where the backward pass
+// wants it (TRAIN: transposed, to T1) and its pre-activation never does (the
+// backward pass evaluates its five terms again).
+template <int TF, typename TIN, bool TRAIN>
+__global__ __launch_bounds__(Tile<TF>::NT) void k_l12_fwd(const TIN* __restrict__ in, float inv_scale,
+                                                         const float* __restrict__ w1,
+                                                         const float* __restrict__ b1,
+                                                         const __bf16* __restrict__ Wf,
+                                                         const float* __restrict__ bias, __bf16* __restrict__ T1,
+                                                         f32x4* __restrict__ Z, __bf16* __restrict__ T,
+                                                         __bf16* __restrict__ Aout, int X)
 {
-    __shared__ __attribute__((aligned(16))) __bf16 sA[(TILE_F + 4) * C];
+    __shared__ __attribute__((aligned(16))) __bf16 sA[(TF + 4) * C];
     __shared__ __attribute__((aligned(16))) __bf16 sW[TAPS * C * C];
-    __shared__ float sIn[TILE_F + 8];
-    const int b = blockIdx.y, x0 = blockIdx.x * TILE_F;
-    stage_w(sW, Wf);
-    stage_l1<TIN>(sA, sIn, in + (int64_t)b * X, inv_scale, w1, b1, x0, X);
+    __shared__ float sIn[TF + 8];
+    const int b = blockIdx.y, x0 = blockIdx.x * TF;
+    Staged<TF, TAPS * C> wts;
+    wts.load([&](int r) { return Wf + r * C; });  // in flight during layer 1
+    stage_l1<TF, TIN>(sA, sIn, in + (int64_t)b * X, inv_scale, w1, b1, x0, X);
+    wts.store(sW);
     __syncthreads();
+    if (TRAIN) {
+#pragma unroll
+        for (int i = 0; i < TF / 4 * C / Tile<TF>::NT; ++i) {
+            // a wave: 16 channels x 16 positions (32 contiguous bytes per channel)
+            const int q = threadIdx.x + i * Tile<TF>::NT, k = q / 64;
+            const int c = 16 * (k % 4) + (q % 64) / 4, r = 16 * (k / 4) + 4 * (q % 4);
+            bf16x4 v;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = sA[swz(r + 2 + j, c >> 3) + (c & 7)];
+            store_t(T1, b, c, x0 + r, X, v);
+        }
+    }
     f32x4 acc[MB][4];
-    mfma_tile(sA, sW, acc);
+    mfma_tile<true>(sA, sW, acc);
     __syncthreads();
-    epilogue<false>(acc, bias, sA, nullptr, 0);
+    epilogue<TF, TRAIN>(acc, bias, sA, Z, T, b, x0, X);
     __syncthreads();
-    store_act(sA, Aout + (int64_t)b * X * C, x0);
+    store_act<TF>(sA, Aout + (int64_t)b * X * C, x0);
 }
 
 // Layer 5 and the output layer (inference): the BF16 layer-5 tile stays in
 // LDS and each thread forms, for its position x, the five tap sums
 //   S[t][b*X + x] = sum_c w6[t][c] A5[x][c],
 // from which du[x] = b6 + sum_t S[t][x+t-2] (k_l6_out).
+constexpr int NTW = Tile<TILE_F>::NT;
+static_assert(NTW >= TILE_F, "the output-layer epilogue maps one thread to one position");
 __global__ __launch_bounds__(NTW) void k_l56_fwd(const __bf16* __restrict__ Ain, const __bf16* __restrict__ Wf,
                                                 const float* __restrict__ bias, const float* __restrict__ w6,
                                                 float* __restrict__ S, int X, int64_t plane)
@@ -363,14 +386,13 @@ __global__ __launch_bounds__(NTW) void k_l56_fwd(const __bf16* __restrict__ Ain,
     __shared__ __attribute__((aligned(16))) __bf16 sW[TAPS * C * C];
     __shared__ float sW6[TAPS * C];
     const int b = blockIdx.y, x0 = blockIdx.x * TILE_F;
-    stage_act(sA, Ain + (int64_t)b * X * C, x0, X);
-    stage_w(sW, Wf);
+    stage<TILE_F>(sA, Ain + (int64_t)b * X * C, x0, X, sW, Wf);
     for (int q = threadIdx.x; q < TAPS * C; q += NTW) sW6[q] = w6[q];
     __syncthreads();
     f32x4 acc[MB][4];
-    mfma_tile(sA, sW, acc);
+    mfma_tile<true>(sA, sW, acc);
     __syncthreads();
-    epilogue<false>(acc, bias, sA, nullptr, 0);
+    epilogue<TILE_F, false>(acc, bias, sA, nullptr, nullptr, b, x0, X);
     __syncthreads();
     const int r = threadIdx.x;
     if (r >= TILE_F) return;
@@ -585,147 +607,42 @@ __global__ __launch_bounds__(NTN) void k_net_fwd(const TIN* in, float inv_scale,
         du[o] = s;
 }
 
-// dA[b][y][ci] = sum_t sum_co dZ[b][y-t+2][co] W[t][co][ci]   (W as Wb[t][ci][co])
-// then dZprev = bf16(dA * gelu'(Zprev)).
-__global__ __launch_bounds__(NT) void k_mid_bwd_data(const __bf16* __restrict__ dZ, const __bf16* __restrict__ Wb,
-                                                     const float* __restrict__ Zprev,
-                                                     __bf16* __restrict__ dZprev, int X)
-{
-    __shared__ __attribute__((aligned(16))) __bf16 sD[(TILE + 4) * ROWP];
-    __shared__ __attribute__((aligned(16))) __bf16 sW[TAPS * C * ROWP];
-    const int b = blockIdx.y, y0 = blockIdx.x * TILE;
-    const __bf16* Db = dZ + (int64_t)b * X * C;
-    for (int q = threadIdx.x; q < (TILE + 4) * (C / 8); q += NT) {
-        const int r = q / (C / 8), ch = (q % (C / 8)) * 8;
-        const int x = wrapx(y0 - 2 + r, X);
-        *reinterpret_cast<uint4*>(&sD[r * ROWP + ch]) =
-            *reinterpret_cast<const uint4*>(&Db[(int64_t)x * C + ch]);
-    }
-    for (int q = threadIdx.x; q < TAPS * C * (C / 8); q += NT) {
-        const int r = q / (C / 8), ch = (q % (C / 8)) * 8;  // r = t*C + ci
-        *reinterpret_cast<uint4*>(&sW[r * ROWP + ch]) = *reinterpret_cast<const uint4*>(&Wb[r * C + ch]);
-    }
-    __syncthreads();
-    const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int m0 = 16 * w, li = l % 16, lk = 8 * (l / 16);
-    f32x4 acc[4];
-    for (int nb = 0; nb < 4; ++nb) acc[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int s = 0; s < TAPS * 2; ++s) {
-        const int t = s >> 1, cb = (s & 1) * 32;
-        // row y = y0+m0+li reads dZ at y-t+2, staged row (y-t+2)-(y0-2)
-        const bf16x8 a = *reinterpret_cast<const bf16x8*>(&sD[(m0 + li - t + 4) * ROWP + cb + lk]);
-        for (int nb = 0; nb < 4; ++nb) {
-            const bf16x8 bv = *reinterpret_cast<const bf16x8*>(&sW[(t * C + 16 * nb + li) * ROWP + cb + lk]);
-            acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bv, acc[nb], 0, 0, 0);
-        }
-    }
-    for (int nb = 0; nb < 4; ++nb) {
-        const int ci = 16 * nb + li;
-        for (int j = 0; j < 4; ++j) {
-            const int y = y0 + m0 + 4 * (l / 16) + j;
-            const int64_t o = ((int64_t)b * X + y) * C + ci;
-            dZprev[o] = f2bf(acc[nb][j] * gelu_d(Zprev[o]));
-        }
-    }
-}
-
-// Partial weight / bias gradients of one 64-position tile:
-// dW[t][co][ci] += sum_x dZ[x][co] A[x+t-2][ci];  db[co] += sum_x dZ[x][co]
-// Both operands are staged transposed (positions contiguous), one shifted
-// copy of A per tap, so every MFMA operand is a 16-byte LDS read.
-__global__ __launch_bounds__(NT) void k_mid_bwd_weight(const __bf16* __restrict__ dZ, const __bf16* __restrict__ Ain,
-                                                       float* __restrict__ part, int X)
-{
-    constexpr int XP = TILE + 8;  // padded position row
-    __shared__ __attribute__((aligned(16))) __bf16 sDT[C * XP];
-    __shared__ __attribute__((aligned(16))) __bf16 sAT[TAPS * C * XP];
-    const int b = blockIdx.y, x0 = blockIdx.x * TILE;
-    const int64_t wg = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
-    const __bf16* Db = dZ + (int64_t)b * X * C;
-    const __bf16* Ab = Ain + (int64_t)b * X * C;
-    for (int q = threadIdx.x; q < TILE * C; q += NT) {
-        const int x = q / C, c = q % C;
-        sDT[c * XP + x] = Db[(int64_t)(x0 + x) * C + c];
-        for (int t = 0; t < TAPS; ++t)
-            sAT[(t * C + c) * XP + x] = Ab[(int64_t)wrapx(x0 + x + t - 2, X) * C + c];
-    }
-    __syncthreads();
-    const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int li = l % 16, lk = 8 * (l / 16);
-    const int co0 = 16 * w;  // wave w: output rows co0..co0+15, all ci, all taps
-    float* pw = part + wg * (TAPS * C * C + C);
-    for (int t = 0; t < TAPS; ++t) {
-        f32x4 acc[4];
-        for (int nb = 0; nb < 4; ++nb) acc[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-        for (int ks = 0; ks < TILE; ks += 32) {
-            const bf16x8 a = *reinterpret_cast<const bf16x8*>(&sDT[(co0 + li) * XP + ks + lk]);
-            for (int nb = 0; nb < 4; ++nb) {
-                const bf16x8 bv =
-                    *reinterpret_cast<const bf16x8*>(&sAT[(t * C + 16 * nb + li) * XP + ks + lk]);
-                acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bv, acc[nb], 0, 0, 0);
-            }
-        }
-        for (int nb = 0; nb < 4; ++nb)
-            for (int j = 0; j < 4; ++j) {
-                const int co = co0 + 4 * (l / 16) + j, ci = 16 * nb + li;
-                pw[(t * C + co) * C + ci] = acc[nb][j];
-            }
-    }
-    if (threadIdx.x < C) {
-        float s = 0.f;
-        for (int x = 0; x < TILE; ++x) s += bf2f(sDT[threadIdx.x * XP + x]);
-        pw[TAPS * C * C + threadIdx.x] = s;
-    }
-}
-
-// out[i] = sum_{w < nparts} part[w][i], fixed order.
-// Sum of nparts partial vectors of length len in two fixed-order passes:
-// group g = blockIdx.y adds partials [g*per, (g+1)*per) into out[g] (first
-// pass, many groups in flight), then one group adds the group sums.
-__global__ __launch_bounds__(NT) void k_reduce_parts(const float* __restrict__ part, int64_t nparts,
-                                                     int64_t len, int64_t per, float* __restrict__ out)
-{
-    const int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x;
-    if (i >= len) return;
-    const int64_t w0 = (int64_t)blockIdx.y * per;
-    const int64_t w1 = w0 + per < nparts ? w0 + per : nparts;
-    float s = 0.f;
-    for (int64_t w = w0; w < w1; ++w) s += part[w * len + i];
-    out[(int64_t)blockIdx.y * len + i] = s;
-}
-
 // ------------------------------------------------------ L6: 64 -> 1, VALU ---
-// du[b][x] = b6 + sum_t sum_ci w6[t][ci] A5[b][x+t-2][ci]
+// du[b][x] = b6 + sum_t sum_ci w6[t][ci] A5[b][x+t-2][ci], one thread per
+// position.  LOSS: against the target, g = d loss / d du = 2 (du - target) / N
+// and the block's sum of (du - target)^2 (loss = their mean over the batch).
+template <bool LOSS>
 __global__ __launch_bounds__(NT) void k_l6_fwd(const __bf16* __restrict__ A, const float* __restrict__ w6,
-                                               const float* __restrict__ b6, float* __restrict__ du, int X)
-{
-    const int b = blockIdx.y, x = blockIdx.x * NT + threadIdx.x;
-    if (x >= X) return;
-    const __bf16* Ab = A + (int64_t)b * X * C;
-    float s = b6[0];
-    for (int t = 0; t < TAPS; ++t) {
-        const bf16x8* row = reinterpret_cast<const bf16x8*>(Ab + (int64_t)wrapx(x + t - 2, X) * C);
-        for (int c8 = 0; c8 < C / 8; ++c8) {
-            const bf16x8 v = row[c8];
-            for (int k = 0; k < 8; ++k) s = fmaf(w6[t * C + c8 * 8 + k], bf2f(v[k]), s);
-        }
-    }
-    du[(int64_t)b * X + x] = s;
-}
-
-// loss = mean (du - target)^2 over the batch (partials per block) and
-// g = d loss / d du = 2 (du - target) / N.
-__global__ __launch_bounds__(NT) void k_mse(const float* __restrict__ du, const float* __restrict__ tgt,
-                                            float* __restrict__ g, float* __restrict__ part, int64_t N)
+                                               const float* __restrict__ b6, float* __restrict__ du,
+                                               const float* __restrict__ tgt, float* __restrict__ g,
+                                               float* __restrict__ part, int X, int64_t N)
 {
     __shared__ float red[NT];
     const int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x;
     float e = 0.f;
     if (i < N) {
-        const float d = du[i] - tgt[i];
-        g[i] = 2.f * d / (float)N;
-        e = d * d;
+        const int x = (int)(i % X);
+        const __bf16* Ab = A + (i - x) * C;
+        float s = b6[0];
+#pragma unroll
+        for (int t = 0; t < TAPS; ++t) {
+            const bf16x8* row = reinterpret_cast<const bf16x8*>(Ab + (int64_t)wrapx(x + t - 2, X) * C);
+#pragma unroll
+            for (int c8 = 0; c8 < C / 8; ++c8) {
+                const bf16x8 v = row[c8];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) s = fmaf(w6[t * C + c8 * 8 + k], bf2f(v[k]), s);
+            }
+        }
+        if (LOSS) {
+            const float d = s - tgt[i];
+            g[i] = 2.f * d / (float)N;
+            e = d * d;
+        } else {
+            du[i] = s;
+        }
     }
+    if (!LOSS) return;
     red[threadIdx.x] = e;
     __syncthreads();
     for (int s = NT / 2; s > 0; s >>= 1) {
@@ -735,59 +652,399 @@ __global__ __launch_bounds__(NT) void k_mse(const float* __restrict__ du, const 
     if (threadIdx.x == 0) part[blockIdx.x] = red[0];
 }
 
-// dA5[b][y][ci] = sum_t g[b][y-t+2] w6[t][ci];  dZ5 = bf16(dA5 * gelu'(Z5))
-__global__ __launch_bounds__(NT) void k_l6_bwd_data(const float* __restrict__ g, const float* __restrict__ w6,
-                                                    const float* __restrict__ Z5, __bf16* __restrict__ dZ5,
-                                                    int X, int B)
+// ------------------------------------------------------------- backward ---
+// A layer's gradient dZ leaves in two forms: row-major (through the LDS tile
+// sD) for the next backward product, and, where T is given, transposed
+// ([B][64][X], no neighbours) for the weight gradient.
+__device__ __forceinline__ void put_dz(__bf16* sD, __bf16* __restrict__ T, int b, int c, int x0, int r, int X,
+                                       const bf16x4& d)
 {
-    const int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x;
-    if (i >= (int64_t)B * X * C) return;
-    const int ci = (int)(i % C);
-    const int64_t bx = i / C;
-    const int y = (int)(bx % X), b = (int)(bx / X);
-    float s = 0.f;
-    for (int t = 0; t < TAPS; ++t) s += g[(int64_t)b * X + wrapx(y - t + 2, X)] * w6[t * C + ci];
-    dZ5[i] = f2bf(s * gelu_d(Z5[i]));
+#pragma unroll
+    for (int j = 0; j < 4; ++j) sD[swz(r + j, c >> 3) + (c & 7)] = d[j];
+    if (T) *reinterpret_cast<bf16x4*>(T + ((int64_t)b * C + c) * X + x0 + r) = d;
 }
 
-// Per-tile partials: dw6[t][ci] = sum_x g[x] A5[x+t-2][ci]; db6 = sum_x g[x]
-__global__ __launch_bounds__(NT) void k_l6_bwd_weight(const float* __restrict__ g, const __bf16* __restrict__ A,
-                                                      float* __restrict__ part, int X)
+// dA5[b][y][ci] = sum_t g[b][y-t+2] w6[t][ci];  dZ5 = bf16(dA5 * gelu'(Z5)),
+// in the lane order of the forward accumulators, which is Z's.
+template <int TF>
+__global__ __launch_bounds__(Tile<TF>::NT) void k_l6_bwd_data(const float* __restrict__ g,
+                                                             const float* __restrict__ w6,
+                                                             const f32x4* __restrict__ Z5, __bf16* __restrict__ T,
+                                                             __bf16* __restrict__ dZ5, int X)
 {
-    const int b = blockIdx.y, x0 = blockIdx.x * TILE;
-    const int64_t wg = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
-    float* pw = part + wg * (TAPS * C + 1);
-    for (int q = threadIdx.x; q < TAPS * C; q += NT) {
-        const int t = q / C, ci = q % C;
-        float s = 0.f;
-        for (int x = x0; x < x0 + TILE; ++x)
-            s += g[(int64_t)b * X + x] * bf2f(A[((int64_t)b * X + wrapx(x + t - 2, X)) * C + ci]);
-        pw[q] = s;
-    }
-    if (threadIdx.x == 0) {
-        float s = 0.f;
-        for (int x = x0; x < x0 + TILE; ++x) s += g[(int64_t)b * X + x];
-        pw[TAPS * C] = s;
-    }
-}
-
-// Per-tile partials: dw1[c][t] = sum_x dZ1[x][c] u[x+t-2]; db1[c] = sum_x dZ1[x][c]
-__global__ __launch_bounds__(NT) void k_l1_bwd_weight(const __bf16* __restrict__ dZ1, const float* __restrict__ u,
-                                                      float* __restrict__ part, int X)
-{
-    const int b = blockIdx.y, x0 = blockIdx.x * TILE;
-    const int64_t wg = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
-    float* pw = part + wg * (C * TAPS + C);
-    for (int q = threadIdx.x; q < C * (TAPS + 1); q += NT) {
-        const int c = q / (TAPS + 1), t = q % (TAPS + 1);
-        float s = 0.f;
-        for (int x = x0; x < x0 + TILE; ++x) {
-            const float d = bf2f(dZ1[((int64_t)b * X + x) * C + c]);
-            s += t < TAPS ? d * u[(int64_t)b * X + wrapx(x + t - 2, X)] : d;
+    __shared__ __attribute__((aligned(16))) __bf16 sD[TF * C];
+    __shared__ float sG[TF + 4];
+    const int b = blockIdx.y, x0 = blockIdx.x * TF;
+    const int l = threadIdx.x & 63, w = threadIdx.x >> 6, li = l % 16, lq = l / 16;
+    for (int q = threadIdx.x; q < TF + 4; q += Tile<TF>::NT) sG[q] = g[(int64_t)b * X + wrapx(x0 - 2 + q, X)];
+    __syncthreads();
+    const int64_t tile = (int64_t)b * (X / TF) + blockIdx.x;
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb) {
+        const int ci = 16 * nb + li;
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) {
+            const int r = WROWS * w + 16 * mb + 4 * lq;
+            const f32x4 z = Z5[z_index(tile, Tile<TF>::NW, w, mb, nb, l)];
+            bf16x4 d;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                float s = 0.f;
+#pragma unroll
+                for (int t = 0; t < TAPS; ++t) s += sG[r + j - t + 4] * w6[t * C + ci];
+                d[j] = f2bf(s * gelu_d(z[j]));
+            }
+            put_dz(sD, T, b, ci, x0, r, X, d);
         }
-        if (t < TAPS) pw[c * TAPS + t] = s;
-        else pw[C * TAPS + c] = s;
     }
+    __syncthreads();
+    store_act<TF>(sD, dZ5 + (int64_t)b * X * C, x0);
+}
+
+// dA[b][y][ci] = sum_t sum_co dZ[b][y-t+2][co] W[t][co][ci]   (W as Wb[t][ci][co])
+// then dZprev = bf16(dA * gelu'(Zprev)).  FIRST: the previous layer is layer 1,
+// whose Z is its five terms of the input again (stage_l1's, in their order).
+template <int TF, bool FIRST>
+__global__ __launch_bounds__(Tile<TF>::NT) void k_mid_bwd_data(const __bf16* __restrict__ dZ,
+                                                              const __bf16* __restrict__ Wb,
+                                                              const f32x4* __restrict__ Zprev,
+                                                              const float* __restrict__ in,
+                                                              const float* __restrict__ w1,
+                                                              const float* __restrict__ b1, __bf16* __restrict__ T,
+                                                              __bf16* __restrict__ dZprev, int X)
+{
+    __shared__ __attribute__((aligned(16))) __bf16 sD[(TF + 4) * C];
+    __shared__ __attribute__((aligned(16))) __bf16 sW[TAPS * C * C];
+    __shared__ float sIn[FIRST ? TF + 4 : 1];
+    const int b = blockIdx.y, y0 = blockIdx.x * TF;
+    const int l = threadIdx.x & 63, w = threadIdx.x >> 6, li = l % 16, lq = l / 16;
+    const int64_t tile = (int64_t)b * (X / TF) + blockIdx.x;
+    if (FIRST)
+        for (int q = threadIdx.x; q < TF + 4; q += Tile<TF>::NT) sIn[q] = in[(int64_t)b * X + wrapx(y0 - 2 + q, X)];
+    stage<TF>(sD, dZ + (int64_t)b * X * C, y0, X, sW, Wb);
+    f32x4 z[MB][4];  // in flight during the product
+    if (!FIRST) {
+#pragma unroll
+        for (int nb = 0; nb < 4; ++nb)
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb) z[mb][nb] = Zprev[z_index(tile, Tile<TF>::NW, w, mb, nb, l)];
+    }
+    __syncthreads();
+    f32x4 acc[MB][4];
+    mfma_tile<false>(sD, sW, acc);
+    __syncthreads();
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb) {
+        const int ci = 16 * nb + li;
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) {
+            const int r = WROWS * w + 16 * mb + 4 * lq;
+            if (FIRST) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    float v = b1[ci];
+#pragma unroll
+                    for (int t = 0; t < TAPS; ++t) v = fmaf(w1[ci * TAPS + t], sIn[r + j + t], v);
+                    z[mb][nb][j] = v;
+                }
+            }
+            bf16x4 d;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) d[j] = f2bf(acc[mb][nb][j] * gelu_d(z[mb][nb][j]));
+            put_dz(sD, T, b, ci, y0, r, X, d);
+        }
+    }
+    __syncthreads();
+    store_act<TF>(sD, dZprev + (int64_t)b * X * C, y0);
+}
+
+// ------------------------------------------------------ weight gradients ---
+// One launch for every layer: blockIdx.y = 0 .. 3 the 64 -> 64 layers, 4 the
+// output layer, 5 layer 1; blockIdx.x = the share of the positions.  Partial
+// sums, one set per share: part[y][x][..] (offsets PART_OFF).
+//   64 -> 64: dW[t][co][ci] = sum_x dZ[x][co] A[x+t-2][ci];  db[co] = sum_x dZ[x][co]
+// Wave w of 8 takes a 32 x 32 quarter of (co, ci) for every tap and every
+// second group of 32 positions: 80 accumulators per lane and two more MFMAs per
+// group for db (B = 1).  A lane loads 8 positions of dZ^T and the 12 positions
+// -2 .. 9 of A^T around them; the five taps' operands are that window shifted,
+// with no LDS.  The two waves of a quarter then add up through LDS (in the
+// accumulators' order, which k_reduce_grad undoes).
+// 256 workgroups of 8 waves at batch 64 x 1024 (one per CU): 21 MB of partials
+// for all layers, where one partial per 64 positions was 84 MB per layer.  All
+// weight gradients and their reduction: 35 us (67 MB of operands, 13 us at the
+// copy rate, then the partials), where a launch per layer with operands
+// transposed through LDS and a two-pass reduction took 340 us.
+constexpr int WG_SHARES = 64;
+constexpr int NTG = 512;
+constexpr int64_t MIDP = TAPS * C * C + C;    // a 64 -> 64 layer's partial
+constexpr int64_t OUTP = TAPS * C + 1;        // the output layer's
+constexpr int64_t FIRSTP = C * TAPS + C;      // layer 1's
+__host__ __device__ inline int64_t part_offset(int y, int shares)
+{
+    return y <= 4 ? y * MIDP * shares : (4 * MIDP + OUTP) * shares;
+}
+struct GradIn {
+    const __bf16* dzt[4];  // dZ of L2..L5, [B][64][X]
+    const __bf16* at[4];   // their inputs A1..A4, [B][64][xt(X)]
+    const float* g;        // d loss / d du, [B][X]
+    const __bf16* a5;      // [B][X][64]
+    const __bf16* dz1;     // [B][X][64]
+    const float* in;       // [B][X]
+};
+
+__device__ __forceinline__ bf16x8 window_tap(const uint32_t (&d)[6], int t)
+{
+    uint32_t r[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+        r[k] = t & 1 ? __builtin_amdgcn_alignbit(d[t / 2 + k + 1], d[t / 2 + k], 16) : d[t / 2 + k];
+    return __builtin_bit_cast(bf16x8, r);
+}
+
+__device__ __forceinline__ void grad_mid(const __bf16* __restrict__ dzt, const __bf16* __restrict__ at,
+                                         float* __restrict__ part, float* lds, int X, int groups, int share,
+                                         int shares)
+{
+    const int l = threadIdx.x & 63, w = threadIdx.x >> 6, li = l % 16, lq = l / 16;
+    const int qco = w & 1, qci = (w >> 1) & 1, pg = w >> 2;
+    const int per = (groups + shares - 1) / shares;
+    const int k0 = share * per, k1 = k0 + per < groups ? k0 + per : groups;
+    const int gx = X / 32;  // groups of 32 positions per sample
+    f32x4 acc[TAPS][2][2], accb[2];
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+        accb[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int t = 0; t < TAPS; ++t)
+#pragma unroll
+            for (int n = 0; n < 2; ++n) acc[t][m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    bf16x8 one;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) one[j] = f2bf(1.f);
+    struct Operands { uint4 a[2]; uint4 b0[2]; uint2 b1[2]; };
+    auto load = [&](int k, Operands& o) {
+        const int b = k / gx, x = (k % gx) * 32 + 8 * lq;
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+            o.a[m] = *reinterpret_cast<const uint4*>(dzt + ((int64_t)b * C + 32 * qco + 16 * m + li) * X + x);
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+            const __bf16* p = at + ((int64_t)b * C + 32 * qci + 16 * n + li) * xt(X) + x;  // position x - 2
+            o.b0[n] = *reinterpret_cast<const uint4*>(p);
+            o.b1[n] = *reinterpret_cast<const uint2*>(p + 8);
+        }
+    };
+    auto product = [&](const Operands& o) {
+        bf16x8 a[2];
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+            a[m] = __builtin_bit_cast(bf16x8, o.a[m]);
+            accb[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], one, accb[m], 0, 0, 0);
+        }
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+            const uint32_t d[6] = {o.b0[n].x, o.b0[n].y, o.b0[n].z, o.b0[n].w, o.b1[n].x, o.b1[n].y};
+#pragma unroll
+            for (int t = 0; t < TAPS; ++t) {
+                const bf16x8 bv = window_tap(d, t);
+#pragma unroll
+                for (int m = 0; m < 2; ++m)
+                    acc[t][m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], bv, acc[t][m][n], 0, 0, 0);
+            }
+        }
+    };
+    // two groups' operands are in flight while one multiplies
+    Operands o0, o1;
+    int k = k0 + pg;
+    if (k < k1) load(k, o0);
+    if (k + 2 < k1) load(k + 2, o1);
+    for (; k < k1; k += 4) {
+        product(o0);
+        if (k + 4 < k1) load(k + 4, o0);
+        if (k + 2 < k1) {
+            product(o1);
+            if (k + 6 < k1) load(k + 6, o1);
+        }
+    }
+    // [quarter][tap, m, n][lane] float4, then [co] bias sums
+    f32x4* sum = reinterpret_cast<f32x4*>(lds) + (w & 3) * (TAPS * 4 * 64) + l;
+    f32x4* out = reinterpret_cast<f32x4*>(part) + (w & 3) * (TAPS * 4 * 64) + l;
+    float* sb = lds + TAPS * C * C;
+    if (pg == 1) {
+#pragma unroll
+        for (int t = 0; t < TAPS; ++t)
+#pragma unroll
+            for (int m = 0; m < 2; ++m)
+#pragma unroll
+                for (int n = 0; n < 2; ++n) sum[((t * 2 + m) * 2 + n) * 64] = acc[t][m][n];
+        if (qci == 0 && li == 0) {
+#pragma unroll
+            for (int m = 0; m < 2; ++m)
+                *reinterpret_cast<f32x4*>(sb + 32 * qco + 16 * m + 4 * lq) = accb[m];
+        }
+    }
+    __syncthreads();
+    if (pg == 0) {
+#pragma unroll
+        for (int t = 0; t < TAPS; ++t)
+#pragma unroll
+            for (int m = 0; m < 2; ++m)
+#pragma unroll
+                for (int n = 0; n < 2; ++n) {
+                    const int f = ((t * 2 + m) * 2 + n) * 64;
+                    out[f] = acc[t][m][n] + sum[f];
+                }
+        if (qci == 0 && li == 0) {
+#pragma unroll
+            for (int m = 0; m < 2; ++m) {
+                const int co = 32 * qco + 16 * m + 4 * lq;
+                *reinterpret_cast<f32x4*>(part + TAPS * C * C + co) = accb[m] + *reinterpret_cast<f32x4*>(sb + co);
+            }
+        }
+    }
+}
+
+// The first and the output layer: rows x of 64 channels (row-major BF16, each
+// loaded once, 16 bytes per lane: lane l takes channels 8 (l & 7) .. + 7 of
+// every eighth row) against five shifted FP32 values, over segments of 64
+// positions, one per wave and round:
+//   OUT:   acc[t] += A[x+t-2] g[x]  (A the rows; g outside the segment is 0)
+//   else:  acc[t] += dZ[x] in[x+t-2], acc[5] += dZ[x]
+template <bool OUT>
+__device__ __forceinline__ void grad_edge(const __bf16* __restrict__ rows, const float* __restrict__ f,
+                                          float* __restrict__ part, float* lds, int X, int groups, int share,
+                                          int shares)
+{
+    constexpr int ROWS = OUT ? 68 : 64, NR = (ROWS + 7) / 8;
+    const int l = threadIdx.x & 63, w = threadIdx.x >> 6, c8 = l & 7, rr = l >> 3;
+    const int segs = groups / 2, per = (segs + shares - 1) / shares;
+    const int s0 = share * per, s1 = s0 + per < segs ? s0 + per : segs;
+    const int sx = X / 64;
+    float* sf = lds + w * 80;  // this wave's f[x0 - 4 .. x0 + 67], then zeros
+    float acc[TAPS + 1][8];
+#pragma unroll
+    for (int t = 0; t <= TAPS; ++t)
+#pragma unroll
+        for (int k = 0; k < 8; ++k) acc[t][k] = 0.f;
+    float sum = 0.f;  // OUT: the lane's share of sum g
+    // the waves of a workgroup run the same number of rounds (barriers)
+    for (int k = 0; k < (per + 7) / 8; ++k) {
+        const int s = s0 + k * 8 + w;
+        const bool live = s < s1;
+        const int b = live ? s / sx : 0, x0 = live ? (s % sx) * 64 : 0;
+        const float* fb = f + (int64_t)b * X;
+        const __bf16* rb = rows + (int64_t)b * X * C + c8 * 8;
+        bf16x8 v[NR];
+#pragma unroll
+        for (int i = 0; i < NR; ++i) {
+            const int r = i * 8 + rr;
+            v[i] = *reinterpret_cast<const bf16x8*>(rb + (int64_t)wrapx(OUT ? x0 - 2 + r : x0 + r, X) * C);
+        }
+        __syncthreads();
+        for (int q = l; q < 80; q += 64) {
+            const int x = x0 - 4 + q;
+            const bool in = live && q < 72 && (!OUT || (x >= x0 && x < x0 + 64));
+            sf[q] = in ? fb[wrapx(x, X)] : 0.f;
+        }
+        __syncthreads();
+        if (!live) continue;
+#pragma unroll
+        for (int i = 0; i < NR; ++i) {
+            // OUT: row x0 - 2 + r meets g[x0 + r - t] (a ninth row past 67 meets
+            // zeros only); else row x0 + r meets in[x0 + r + t - 2]
+            const int r = i * 8 + rr;
+            float e[TAPS];
+#pragma unroll
+            for (int t = 0; t < TAPS; ++t) e[t] = OUT ? sf[r - t + 4] : sf[r + t + 2];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                const float a = bf2f(v[i][q]);
+#pragma unroll
+                for (int t = 0; t < TAPS; ++t) acc[t][q] = fmaf(e[t], a, acc[t][q]);
+                if (!OUT) acc[TAPS][q] += a;
+            }
+        }
+        if (OUT) sum += sf[l + 4];
+    }
+    __syncthreads();
+    // lds: [tap][wave][row lane][channel], then the waves' sums of g
+    constexpr int NA = OUT ? TAPS : TAPS + 1;
+#pragma unroll
+    for (int t = 0; t < NA; ++t)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) lds[((t * 8 + w) * 8 + rr) * C + c8 * 8 + q] = acc[t][q];
+    if (OUT) {
+        for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
+        if (l == 0) lds[NA * 64 * C + w] = sum;
+    }
+    __syncthreads();
+    for (int q = threadIdx.x; q < NA * C; q += NTG) {
+        const int t = q / C, c = q % C;
+        float s = 0.f;
+#pragma unroll 16
+        for (int v = 0; v < 64; ++v) s += lds[(t * 64 + v) * C + c];
+        part[OUT ? q : (t < TAPS ? c * TAPS + t : TAPS * C + c)] = s;
+    }
+    if (OUT && threadIdx.x == 0) {
+        float s = 0.f;
+        for (int v = 0; v < 8; ++v) s += lds[NA * 64 * C + v];
+        part[TAPS * C] = s;
+    }
+}
+
+__global__ __launch_bounds__(NTG) void k_grad_weights(GradIn in, float* __restrict__ part, int X, int groups)
+{
+    // the edge layers' sums, the largest user: 6 taps x 64 lanes of rows x 64 channels
+    constexpr int64_t LDS = 6 * 64 * C > MIDP ? 6 * 64 * C : MIDP;
+    __shared__ __attribute__((aligned(16))) float lds[LDS];
+    const int y = blockIdx.y, share = blockIdx.x, shares = gridDim.x;
+    float* p = part + part_offset(y, shares) + share * (y < 4 ? MIDP : (y == 4 ? OUTP : FIRSTP));
+    if (y < 4)
+        grad_mid(in.dzt[y], in.at[y], p, lds, X, groups, share, shares);
+    else if (y == 4)
+        grad_edge<true>(in.a5, in.g, p, lds, X, groups, share, shares);
+    else
+        grad_edge<false>(in.dz1, in.in, p, lds, X, groups, share, shares);
+}
+
+// g[i] = the sum of the shares' partials in share order, one thread per
+// parameter, in the order the partials are stored in.
+__global__ __launch_bounds__(NT) void k_reduce_grad(const float* __restrict__ part, int shares,
+                                                    float* __restrict__ g)
+{
+    int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x;
+    if (i >= NPARAM) return;
+    int y = 0;
+    int64_t len = MIDP, out;
+    if (i < 4 * MIDP) {
+        y = (int)(i / MIDP);
+        i -= y * MIDP;
+        out = P_MID + y * MID_SZ;
+        if (i < TAPS * C * C) {
+            // [quarter][t, m, n][lane][j] -> [t][co][ci]
+            const int j = i & 3, l = (i >> 2) & 63, f = (int)(i >> 8);
+            const int n = f & 1, m = (f >> 1) & 1, t = (f >> 2) % TAPS, q = f / (4 * TAPS);
+            out += (t * C + 32 * (q & 1) + 16 * m + 4 * (l / 16) + j) * C + 32 * (q >> 1) + 16 * n + l % 16;
+        } else {
+            out += i;
+        }
+    } else if (i < 4 * MIDP + OUTP) {
+        y = 4;
+        i -= 4 * MIDP;
+        len = OUTP;
+        out = P_W6 + i;
+    } else {
+        y = 5;
+        i -= 4 * MIDP + OUTP;
+        len = FIRSTP;
+        out = P_W1 + i;
+    }
+    const float* p = part + part_offset(y, shares) + i;
+    float s = 0.f;
+#pragma unroll 8
+    for (int k = 0; k < shares; ++k) s += p[k * len];
+    g[out] = s;
 }
 
 // -------------------------------------------------------------- optimiser ---
@@ -805,26 +1062,22 @@ __global__ __launch_bounds__(NT) void k_adam(float* __restrict__ p, const float*
     p[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
 }
 
-// BF16 copies of a 64->64 layer's weights in the forward ([t][co][ci]) and
-// backward ([t][ci][co]) layouts.
-__global__ __launch_bounds__(NT) void k_pack_w(const float* __restrict__ w, __bf16* __restrict__ wf,
-                                               __bf16* __restrict__ wb)
+// BF16 copies of the 64->64 layers' weights in the forward ([t][co][ci]) and
+// backward ([t][ci][co]) layouts, one layer per blockIdx.y.
+struct PackOut { __bf16 *wf[4], *wb[4]; };
+__global__ __launch_bounds__(NT) void k_pack_w(const float* __restrict__ p, PackOut o)
 {
     const int i = blockIdx.x * NT + threadIdx.x;
     if (i >= TAPS * C * C) return;
+    const float* w = p + P_MID + blockIdx.y * MID_SZ;
+    __bf16 *wf = o.wf[blockIdx.y], *wb = o.wb[blockIdx.y];
     const int t = i / (C * C), co = (i / C) % C, ci = i % C;
     const __bf16 h = f2bf(w[i]);
     wf[i] = h;
     wb[(t * C + ci) * C + co] = h;
 }
 
-// u (FP64 state) -> normalised FP32 network input; and u += scale * du.
-__global__ __launch_bounds__(NT) void k_to_input(const double* __restrict__ u, float* __restrict__ in,
-                                                 int64_t n, float inv_scale)
-{
-    const int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x;
-    if (i < n) in[i] = (float)u[i] * inv_scale;
-}
+// u += scale * du
 __global__ __launch_bounds__(NT) void k_apply_du(double* __restrict__ u, const float* __restrict__ du,
                                                  int64_t n, double scale)
 {
@@ -927,7 +1180,6 @@ __global__ __launch_bounds__(NT) void k_judge(const double* __restrict__ part, i
 namespace sw1dnn {
 
 inline unsigned nblk(int64_t n) { return (unsigned)((n + NT - 1) / NT); }
-constexpr int64_t RED_GROUPS = 32;  // first-pass groups of the gradient reduction
 
 uint64_t splitmix(uint64_t& s)
 {
@@ -975,13 +1227,13 @@ struct sw1d_nn {
     float* du = nullptr;    // [B][X] output
     float* tgt = nullptr;   // [B][X] target
     float* gdu = nullptr;   // [B][X] d loss / d du
-    float* Z[5] = {};       // [B][X][C] pre-activations of L1..L5
-    __bf16* A[5] = {};      // [B][X][C] activations of L1..L5
-    __bf16 *dZa = nullptr, *dZb = nullptr;  // [B][X][C] gradients
-    float* part = nullptr;  // per-tile partial gradients
-    float* part2 = nullptr; // group sums of the partials
+    f32x4* Z[4] = {};       // pre-activations of L2..L5, accumulator order
+    __bf16* A[2] = {};      // [B][X][C] activations, layers in turn
+    __bf16* AT[4] = {};     // [B][C][xt(X)] activations of L1..L4
+    __bf16* dZ[2] = {};     // [B][X][C] gradients, layers in turn
+    __bf16* dZT[4] = {};    // [B][C][X] gradients of L2..L5
+    float* part = nullptr;  // partial gradients of the weight kernel's shares
     float* lossp = nullptr;
-    int64_t part_len = 0;
     float* taps = nullptr;  // [5][B][X] output-layer tap sums (inference)
     int* keep = nullptr;    // [B] judged-step selection
     double* jacc = nullptr; // [2] judge accumulators over a call: fallbacks, largest error
@@ -996,36 +1248,30 @@ namespace {
 
 int pack_weights(sw1d_nn* N)
 {
+    PackOut o;
     for (int l = 0; l < 4; ++l) {
-        hipLaunchKernelGGL(k_pack_w, dim3(nblk(TAPS * C * C)), dim3(NT), 0, N->stream,
-                           N->p + P_MID + l * MID_SZ, N->wf[l], N->wb[l]);
+        o.wf[l] = N->wf[l];
+        o.wb[l] = N->wb[l];
     }
+    hipLaunchKernelGGL(k_pack_w, dim3(nblk(TAPS * C * C), 4), dim3(NT), 0, N->stream, N->p, o);
     NN_HIP(hipGetLastError());
     return SW1D_OK;
 }
 
-// forward of B samples already in N->x (store_z: keep pre-activations for backward)
-int nn_forward(sw1d_nn* N, int B, bool store_z = true)
+const float* mid_bias(const sw1d_nn* N, int l) { return N->p + P_MID + l * MID_SZ + TAPS * C * C; }
+
+// Layers 1-5 of B samples from `in` (normalised by inv_scale); the layer-5
+// activation ends in N->A[1].  TRAIN keeps what nn_backward needs.
+template <int TF, typename TIN, bool TRAIN>
+int nn_layers(sw1d_nn* N, int B, const TIN* in, float inv_scale)
 {
-    const int X = N->X;
-    hipLaunchKernelGGL(k_l1_fwd, dim3(nblk((int64_t)X * C), B), dim3(NT), 0, N->stream, N->x, N->p + P_W1,
-                       N->p + P_B1, N->Z[0], N->A[0], X);
-    for (int l = 0; l < 4; ++l) {
-        const float* bias = N->p + P_MID + l * MID_SZ + TAPS * C * C;
-        if (X % TILE_F == 0) {
-            if (store_z)
-                hipLaunchKernelGGL(k_mid_fwd_wide<true>, dim3(X / TILE_F, B), dim3(NTW), 0, N->stream, N->A[l],
-                                   N->wf[l], bias, N->Z[l + 1], N->A[l + 1], X);
-            else
-                hipLaunchKernelGGL(k_mid_fwd_wide<false>, dim3(X / TILE_F, B), dim3(NTW), 0, N->stream, N->A[l],
-                                   N->wf[l], bias, N->Z[l + 1], N->A[l + 1], X);
-        } else {
-            hipLaunchKernelGGL(k_mid_fwd, dim3(X / TILE, B), dim3(NT), 0, N->stream, N->A[l], N->wf[l], bias,
-                               N->Z[l + 1], N->A[l + 1], X);
-        }
-    }
-    hipLaunchKernelGGL(k_l6_fwd, dim3(nblk(X), B), dim3(NT), 0, N->stream, N->A[4], N->p + P_W6,
-                       N->p + P_B6, N->du, X);
+    const int X = N->X, NTL = Tile<TF>::NT;
+    const dim3 grid(X / TF, B);
+    hipLaunchKernelGGL((k_l12_fwd<TF, TIN, TRAIN>), grid, dim3(NTL), 0, N->stream, in, inv_scale, N->p + P_W1,
+                       N->p + P_B1, N->wf[0], mid_bias(N, 0), N->AT[0], N->Z[0], N->AT[1], N->A[0], X);
+    for (int l = 1; l < 4; ++l)
+        hipLaunchKernelGGL((k_mid_fwd<TF, TRAIN>), grid, dim3(NTL), 0, N->stream, N->A[(l - 1) & 1], N->wf[l],
+                           mid_bias(N, l), N->Z[l], l < 3 ? N->AT[l + 1] : nullptr, N->A[l & 1], X);
     NN_HIP(hipGetLastError());
     return SW1D_OK;
 }
@@ -1034,8 +1280,8 @@ int nn_forward(sw1d_nn* N, int B, bool store_z = true)
 // in N->du.  Otherwise from the FP64 states u (normalised on the fly by
 // 1/in_scale) to u += out_scale * du.  One launch of the whole-network kernel
 // at nx = 1024; five launches when nx is another multiple of the 256-position
-// tile (or infer_mode = 1); otherwise the training kernels plus the
-// conversions.  All give the same bits.
+// tile (or infer_mode = 1), these two with the same bits; otherwise 64-position
+// tiles and the training's output layer.
 int nn_infer(sw1d_nn* N, int B, double* u)
 {
     const int X = N->X;
@@ -1052,11 +1298,11 @@ int nn_infer(sw1d_nn* N, int B, double* u)
         return SW1D_OK;
     }
     if (X % TILE_F != 0) {
-        if (u)
-            hipLaunchKernelGGL(k_to_input, dim3(nblk(plane)), dim3(NT), 0, N->stream, u, N->x, plane,
-                               (float)(1.0 / N->in_scale));
-        int rc = nn_forward(N, B, false);
+        const int rc = u ? nn_layers<TILE, double, false>(N, B, u, (float)(1.0 / N->in_scale))
+                         : nn_layers<TILE, float, false>(N, B, N->x, 1.0f);
         if (rc) return rc;
+        hipLaunchKernelGGL(k_l6_fwd<false>, dim3(nblk(plane)), dim3(NT), 0, N->stream, N->A[1], N->p + P_W6,
+                           N->p + P_B6, N->du, nullptr, nullptr, nullptr, X, plane);
         if (u)
             hipLaunchKernelGGL(k_apply_du, dim3(nblk(plane)), dim3(NT), 0, N->stream, u, N->du, plane,
                                N->out_scale);
@@ -1065,17 +1311,17 @@ int nn_infer(sw1d_nn* N, int B, double* u)
     }
     const dim3 grid(X / TILE_F, B);
     const float* P = N->p;
-    auto bias = [&](int l) { return P + P_MID + l * MID_SZ + TAPS * C * C; };
     if (u)
-        hipLaunchKernelGGL(k_l12_fwd<double>, grid, dim3(NTW), 0, N->stream, u, (float)(1.0 / N->in_scale),
-                           P + P_W1, P + P_B1, N->wf[0], bias(0), N->A[1], X);
+        hipLaunchKernelGGL((k_l12_fwd<TILE_F, double, false>), grid, dim3(NTW), 0, N->stream, u,
+                           (float)(1.0 / N->in_scale), P + P_W1, P + P_B1, N->wf[0], mid_bias(N, 0), nullptr, nullptr,
+                           nullptr, N->A[0], X);
     else
-        hipLaunchKernelGGL(k_l12_fwd<float>, grid, dim3(NTW), 0, N->stream, N->x, 1.0f, P + P_W1, P + P_B1,
-                           N->wf[0], bias(0), N->A[1], X);
+        hipLaunchKernelGGL((k_l12_fwd<TILE_F, float, false>), grid, dim3(NTW), 0, N->stream, N->x, 1.0f, P + P_W1,
+                           P + P_B1, N->wf[0], mid_bias(N, 0), nullptr, nullptr, nullptr, N->A[0], X);
     for (int l = 1; l <= 2; ++l)
-        hipLaunchKernelGGL(k_mid_fwd_wide<false>, grid, dim3(NTW), 0, N->stream, N->A[l], N->wf[l], bias(l),
-                           nullptr, N->A[l + 1], X);
-    hipLaunchKernelGGL(k_l56_fwd, grid, dim3(NTW), 0, N->stream, N->A[3], N->wf[3], bias(3), P + P_W6, N->taps,
+        hipLaunchKernelGGL((k_mid_fwd<TILE_F, false>), grid, dim3(NTW), 0, N->stream, N->A[(l - 1) & 1], N->wf[l],
+                           mid_bias(N, l), nullptr, nullptr, N->A[l & 1], X);
+    hipLaunchKernelGGL(k_l56_fwd, grid, dim3(NTW), 0, N->stream, N->A[0], N->wf[3], mid_bias(N, 3), P + P_W6, N->taps,
                        X, plane);
     if (u)
         hipLaunchKernelGGL(k_l6_out<true>, dim3(nblk(plane)), dim3(NT), 0, N->stream, N->taps, P + P_B6,
@@ -1087,52 +1333,54 @@ int nn_infer(sw1d_nn* N, int B, double* u)
     return SW1D_OK;
 }
 
-// out[0..len) = sum over the nparts partial vectors in N->part (deterministic)
-void reduce_parts(sw1d_nn* N, int64_t nparts, int64_t len, float* out)
+// loss (mean square against N->tgt) of the samples in N->x and the full
+// gradient into N->g
+template <int TF>
+int nn_gradient(sw1d_nn* N, int B)
 {
-    const int64_t groups = nparts < RED_GROUPS ? nparts : RED_GROUPS;
-    const int64_t per = (nparts + groups - 1) / groups;
-    hipLaunchKernelGGL(k_reduce_parts, dim3(nblk(len), (unsigned)groups), dim3(NT), 0, N->stream, N->part,
-                       nparts, len, per, N->part2);
-    hipLaunchKernelGGL(k_reduce_parts, dim3(nblk(len), 1), dim3(NT), 0, N->stream, N->part2, groups, len,
-                       groups, out);
+    const int X = N->X, NTL = Tile<TF>::NT;
+    const int64_t nout = (int64_t)B * X;
+    const dim3 tiles(X / TF, B);
+    const int rc = nn_layers<TF, float, true>(N, B, N->x, 1.0f);
+    if (rc) return rc;
+    hipLaunchKernelGGL(k_l6_fwd<true>, dim3(nblk(nout)), dim3(NT), 0, N->stream, N->A[1], N->p + P_W6, N->p + P_B6,
+                       nullptr, N->tgt, N->gdu, N->lossp, X, nout);
+    hipLaunchKernelGGL(k_l6_bwd_data<TF>, tiles, dim3(NTL), 0, N->stream, N->gdu, N->p + P_W6, N->Z[3], N->dZT[3],
+                       N->dZ[1], X);
+    for (int l = 3; l >= 1; --l)
+        hipLaunchKernelGGL((k_mid_bwd_data<TF, false>), tiles, dim3(NTL), 0, N->stream, N->dZ[l & 1], N->wb[l],
+                           N->Z[l - 1], nullptr, nullptr, nullptr, N->dZT[l - 1], N->dZ[(l - 1) & 1], X);
+    hipLaunchKernelGGL((k_mid_bwd_data<TF, true>), tiles, dim3(NTL), 0, N->stream, N->dZ[0], N->wb[0], nullptr, N->x,
+                       N->p + P_W1, N->p + P_B1, nullptr, N->dZ[1], X);
+    GradIn in;
+    for (int l = 0; l < 4; ++l) {
+        in.dzt[l] = N->dZT[l];
+        in.at[l] = N->AT[l];
+    }
+    in.g = N->gdu;
+    in.a5 = N->A[1];
+    in.dz1 = N->dZ[1];
+    in.in = N->x;
+    const int groups = (int)(nout / 32);
+    const int shares = groups / 4 < WG_SHARES ? (groups / 4 > 0 ? groups / 4 : 1) : WG_SHARES;
+    hipLaunchKernelGGL(k_grad_weights, dim3(shares, 6), dim3(NTG), 0, N->stream, in, N->part, X, groups);
+    hipLaunchKernelGGL(k_reduce_grad, dim3(nblk(NPARAM)), dim3(NT), 0, N->stream, N->part, shares, N->g);
+    NN_HIP(hipGetLastError());
+    return SW1D_OK;
 }
 
-// loss (mean square against N->tgt) and the full gradient into N->g
-int nn_backward(sw1d_nn* N, int B, double* loss)
+int nn_gradient(sw1d_nn* N, int B, double* loss)
 {
-    const int X = N->X;
-    const int64_t nout = (int64_t)B * X, nfeat = nout * C;
+    const int rc = N->X % TILE_F == 0 ? nn_gradient<TILE_F>(N, B) : nn_gradient<TILE>(N, B);
+    if (rc || !loss) return rc;
+    const int64_t nout = (int64_t)B * N->X;
     const unsigned lb = nblk(nout);
-    hipLaunchKernelGGL(k_mse, dim3(lb), dim3(NT), 0, N->stream, N->du, N->tgt, N->gdu, N->lossp, nout);
-    const dim3 tiles(X / TILE, B);
-    const int64_t ntiles = (int64_t)(X / TILE) * B;
-    // L6
-    hipLaunchKernelGGL(k_l6_bwd_weight, tiles, dim3(NT), 0, N->stream, N->gdu, N->A[4], N->part, X);
-    reduce_parts(N, ntiles, (int64_t)(TAPS * C + 1), N->g + P_W6);
-    hipLaunchKernelGGL(k_l6_bwd_data, dim3(nblk(nfeat)), dim3(NT), 0, N->stream, N->gdu, N->p + P_W6,
-                       N->Z[4], N->dZa, X, B);
-    // L5 .. L2
-    __bf16* dz = N->dZa;
-    __bf16* dzp = N->dZb;
-    for (int l = 3; l >= 0; --l) {
-        hipLaunchKernelGGL(k_mid_bwd_weight, tiles, dim3(NT), 0, N->stream, dz, N->A[l], N->part, X);
-        reduce_parts(N, ntiles, MID_SZ, N->g + P_MID + l * MID_SZ);
-        hipLaunchKernelGGL(k_mid_bwd_data, tiles, dim3(NT), 0, N->stream, dz, N->wb[l], N->Z[l], dzp, X);
-        __bf16* t = dz; dz = dzp; dzp = t;
-    }
-    // L1 (dz now holds dZ1)
-    hipLaunchKernelGGL(k_l1_bwd_weight, tiles, dim3(NT), 0, N->stream, dz, N->x, N->part, X);
-    reduce_parts(N, ntiles, (int64_t)(C * TAPS + C), N->g + P_W1);
-    NN_HIP(hipGetLastError());
-    if (loss) {
-        std::vector<float> lp(lb);
-        NN_HIP(hipMemcpyAsync(lp.data(), N->lossp, lb * sizeof(float), hipMemcpyDeviceToHost, N->stream));
-        NN_HIP(hipStreamSynchronize(N->stream));
-        double s = 0;
-        for (float f : lp) s += f;
-        *loss = s / (double)nout;
-    }
+    std::vector<float> lp(lb);
+    NN_HIP(hipMemcpyAsync(lp.data(), N->lossp, lb * sizeof(float), hipMemcpyDeviceToHost, N->stream));
+    NN_HIP(hipStreamSynchronize(N->stream));
+    double s = 0;
+    for (float f : lp) s += f;
+    *loss = s / (double)nout;
     return SW1D_OK;
 }
 
@@ -1150,13 +1398,18 @@ void nn_release(sw1d_nn* N)
 {
     if (!N) return;
     if (N->stream) (void)hipStreamSynchronize(N->stream);
-    void* ptrs[] = {N->p,   N->g,     N->m,     N->v,    N->x,     N->du,   N->tgt,  N->gdu,  N->dZa,
-                    N->dZb, N->part,  N->part2, N->lossp, N->taps, N->keep, N->jacc, N->usave, N->unn, N->l2p};
+    void* ptrs[] = {N->p,    N->g,    N->m,    N->v,    N->x,     N->du,  N->tgt, N->gdu,
+                    N->part, N->lossp, N->taps, N->keep, N->jacc, N->usave, N->unn, N->l2p};
     for (void* q : ptrs)
         if (q) (void)hipFree(q);
-    for (int l = 0; l < 5; ++l) {
-        if (N->Z[l]) (void)hipFree(N->Z[l]);
+    for (int l = 0; l < 2; ++l) {
         if (N->A[l]) (void)hipFree(N->A[l]);
+        if (N->dZ[l]) (void)hipFree(N->dZ[l]);
+    }
+    for (int l = 0; l < 4; ++l) {
+        if (N->Z[l]) (void)hipFree(N->Z[l]);
+        if (N->AT[l]) (void)hipFree(N->AT[l]);
+        if (N->dZT[l]) (void)hipFree(N->dZT[l]);
     }
     for (int l = 0; l < 4; ++l) {
         if (N->wf[l]) (void)hipFree(N->wf[l]);
@@ -1210,21 +1463,20 @@ int sw1d_nn_create(sw1d_nn** out, int32_t nx, int32_t max_batch, uint64_t seed)
     N->X = nx;
     N->Bmax = max_batch;
     const int64_t nout = (int64_t)nx * max_batch, nfeat = nout * C;
-    const int64_t ntiles = (int64_t)(nx / TILE) * max_batch;
-    N->part_len = ntiles * MID_SZ;
     bool ok = hipStreamCreateWithFlags(&N->stream, hipStreamNonBlocking) == hipSuccess &&
               dalloc(&N->p, NPARAM) == hipSuccess && dalloc(&N->g, NPARAM) == hipSuccess &&
               dalloc(&N->m, NPARAM) == hipSuccess && dalloc(&N->v, NPARAM) == hipSuccess &&
               dalloc(&N->x, nout) == hipSuccess && dalloc(&N->du, nout) == hipSuccess &&
               dalloc(&N->tgt, nout) == hipSuccess && dalloc(&N->gdu, nout) == hipSuccess &&
-              dalloc(&N->dZa, nfeat) == hipSuccess && dalloc(&N->dZb, nfeat) == hipSuccess &&
-              dalloc(&N->part, N->part_len) == hipSuccess &&
-              dalloc(&N->part2, RED_GROUPS * MID_SZ) == hipSuccess &&
+              dalloc(&N->part, WG_SHARES * NPARAM) == hipSuccess &&
               dalloc(&N->lossp, (int64_t)nblk(nout)) == hipSuccess &&
               dalloc(&N->taps, TAPS * nout) == hipSuccess && dalloc(&N->keep, (int64_t)max_batch) == hipSuccess &&
               dalloc(&N->jacc, (int64_t)2) == hipSuccess;
-    for (int l = 0; ok && l < 5; ++l)
-        ok = dalloc(&N->Z[l], nfeat) == hipSuccess && dalloc(&N->A[l], nfeat) == hipSuccess;
+    for (int l = 0; ok && l < 2; ++l)
+        ok = dalloc(&N->A[l], nfeat) == hipSuccess && dalloc(&N->dZ[l], nfeat) == hipSuccess;
+    for (int l = 0; ok && l < 4; ++l)
+        ok = dalloc(&N->Z[l], nfeat / 4) == hipSuccess && dalloc(&N->dZT[l], nfeat) == hipSuccess &&
+             dalloc(&N->AT[l], (int64_t)max_batch * C * xt(nx)) == hipSuccess;
     for (int l = 0; ok && l < 4; ++l)
         ok = dalloc(&N->wf[l], TAPS * C * C) == hipSuccess && dalloc(&N->wb[l], TAPS * C * C) == hipSuccess;
     if (!ok) {
@@ -1322,8 +1574,7 @@ int sw1d_nn_gradient(sw1d_nn* N, const float* x_host, const float* t_host, int32
     const size_t bytes = (size_t)batch * N->X * sizeof(float);
     NN_HIP(hipMemcpyAsync(N->x, x_host, bytes, hipMemcpyHostToDevice, N->stream));
     NN_HIP(hipMemcpyAsync(N->tgt, t_host, bytes, hipMemcpyHostToDevice, N->stream));
-    int rc = nn_forward(N, batch);
-    if (!rc) rc = nn_backward(N, batch, loss);
+    const int rc = nn_gradient(N, batch, loss);
     if (rc) return rc;
     if (grad_host) {
         NN_HIP(hipMemcpyAsync(grad_host, N->g, NPARAM * sizeof(float), hipMemcpyDeviceToHost, N->stream));
@@ -1358,8 +1609,7 @@ int sw1d_nn_train(sw1d_nn* N, const float* d_inputs, const float* d_targets, int
     for (int64_t it = 0; it < iters && !rc; ++it) {
         hipLaunchKernelGGL(k_gather, dim3(nblk(n)), dim3(NT), 0, N->stream, d_inputs, d_targets,
                            didx + it * batch, N->x, N->tgt, N->X, n);
-        rc = nn_forward(N, batch);
-        if (!rc) rc = nn_backward(N, batch, (it == iters - 1 || it % 50 == 0) ? &loss : nullptr);
+        rc = nn_gradient(N, batch, (it == iters - 1 || it % 50 == 0) ? &loss : nullptr);
         if (!rc) rc = adam(N, lr, 0.9f, 0.999f, 1e-8f);
     }
     if (hipStreamSynchronize(N->stream) != hipSuccess && !rc) rc = nn_fail(SW1D_EDEVICE, "training");
