@@ -264,8 +264,8 @@ def program(equation: int, precision: int) -> str:
 
 
 class Batch:
-    """Many independent periodic heat / KS problems advanced by one persistent
-    launch (sw1d_batch_*).  State is the concatenation of the fields."""
+    """Many independent periodic heat / KS problems advanced together
+    (sw1d_batch_*).  State is the concatenation of the fields."""
 
     def __init__(self, equations, nx, dt, dx, *, precision: int = F64, tile_points=None, waves=None):
         L = lib()
@@ -294,8 +294,7 @@ class Batch:
             self.set_workgroup(waves)
 
     def set_workgroup(self, waves: int) -> None:
-        """Waves per workgroup of the persistent launch (2, 4 or 8): the tiles a
-        workgroup works on at once.  Results do not depend on it."""
+        """2, 4 or 8: checked and otherwise unused (sw1d_batch_set_workgroup)."""
         _check(lib().sw1d_batch_set_workgroup(self._h, int(waves)), "sw1d_batch_set_workgroup")
 
     def close(self):

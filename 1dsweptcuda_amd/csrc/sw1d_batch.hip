@@ -1,161 +1,187 @@
-// Batched persistent solve: thousands of independent periodic heat / KS
-// problems of arbitrary sizes advanced by nsteps in one launch.
+// Batched solve: many independent periodic heat / KS problems of arbitrary
+// sizes advanced together, as workgroup-wide overlapped tiles (sw1d_wide.hpp).
 //
-// Each workgroup (NW = 2, 4 or 8 waves: the tiles it works on at once, a
-// batch setting) takes whole problems from a device work queue (an atomic
-// counter over a table sorted largest first), and advances its problem through
-// all the steps itself: trapezoid tiles (sw1d_trap.hpp) over the problem, one
-// wave per tile, ping-ponging between the two packed state arrays with a
-// workgroup barrier between time blocks.  The tiles' arithmetic does not
-// depend on NW, so neither do the results.  Steps that do not fill
-// a time block are taken one stage at a time.  No workgroup ever waits for
-// another, so the launch cannot deadlock, and every wave leaves when the
-// queue is empty.
-//
-// The counter is reset by a one-thread kernel launched just before (no
-// memset), so the pair can be captured in a hipGraph and replayed.
+// A launch advances every problem of a group (one equation, one tile shape) by
+// the same number of steps; its workgroups are the group's tiles, found in a
+// table made on the host, so a large problem spreads over as many compute
+// units as its size asks for.  (A workgroup per problem, stepping it through
+// the whole advance, was bound by the largest one: 512 problems of 2^10 .. 2^16
+// points, 5000 steps, FP64, took 70 ms, 51 ms of them one workgroup's.)  Every
+// group's launches come in an even number, so its result is back in the
+// buffer it started from.
 
-#include "sw1d_trap.hpp"
+#include <algorithm>
+#include <cmath>
+
+#include "sw1d_wide.hpp"
 
 namespace sw1d {
 namespace {
 
-__device__ __forceinline__ int64_t wrap1(int64_t i, int64_t n)
+using namespace wide;
+
+template <typename T, int EQ, class S>
+__global__ __launch_bounds__(S::NT) void k_batch(const BatchTile* __restrict__ tiles,
+                                                 const BatchJob<T>* __restrict__ jobs, const T* __restrict__ in,
+                                                 T* __restrict__ out, int steps)
 {
-    return i < 0 ? i + n : (i >= n ? i - n : i);
+    __shared__ __attribute__((aligned(16))) T lds[S::LDS];
+    const BatchTile t = tiles[blockIdx.x];
+    const BatchJob<T>& J = jobs[t.job];
+    Coef<T> k;
+    k.fo = J.c[0];
+    k.fo2 = J.c[1];
+    k.ks = KsCoef<T>{J.c[0], J.c[1], J.c[2], J.c[3], J.c[4]};
+    tile<T, EQ, S>(lds, in + J.offset, out + J.offset, J.n, 0, t.out0, t.count, steps, ENDS_PERIODIC, k);
 }
 
-template <typename T, int EQ, int PO, int NW>
-__device__ void batch_problem(const BatchJob<T>& J, T* a, T* b, int64_t nsteps, int wave, int lane)
+template <typename T, int EQ, int I = 0>
+hipError_t launch_group(const BatchLaunch& L, hipStream_t s)
 {
-    constexpr int NT = NW * kWave;
-    constexpr int PI = PO + 1, WOUT = kWave * PO, RS = 32;
-    constexpr int S = EQ == EQ_HEAT ? 32 : 16;          // stages per time block
-    constexpr int BLOCK_STEPS = EQ == EQ_HEAT ? 32 : 8;
-    const int64_t n = J.n;
-    const int64_t ntiles = (n + WOUT - 1) / WOUT;
-    const int64_t blocks = nsteps / BLOCK_STEPS;
-    KsCoef<T> k;
-    k.dx4x = J.c[0]; k.dx2 = J.c[1]; k.dx4 = J.c[2]; k.dt = J.c[3]; k.dth = J.c[4];
-    for (int64_t tb = 0; tb < blocks; ++tb) {
-        for (int64_t t = wave; t < ntiles; t += NW) {
-            const int64_t out0 = t * WOUT;
-            const int count = (int)(n - out0 < WOUT ? n - out0 : WOUT);
-            const int64_t win = wrapn(out0 - RS, n);
-            if (EQ == EQ_HEAT)
-                trap_heat<T, PI, S, false>(a, b, n, win, out0, count, lane, J.c[0], J.c[1]);
-            else
-                trap_ks<T, PI, S>(a, b, n, win, out0, count, lane, k);
-        }
-        __syncthreads();
-        T* t = a; a = b; b = t;
+    if constexpr (I < Table<EQ>::count) {
+        if (L.shape != I) return launch_group<T, EQ, I + 1>(L, s);
+        using S = TableShape<EQ, I>;
+        hipLaunchKernelGGL((k_batch<T, EQ, S>), dim3((unsigned)L.ntiles), dim3(S::NT), 0, s, L.tiles,
+                           static_cast<const BatchJob<T>*>(L.jobs), static_cast<const T*>(L.in),
+                           static_cast<T*>(L.out), L.steps);
+        return hipGetLastError();
+    } else {
+        return hipErrorInvalidValue;
     }
-    // remaining steps, one stage per pass (Heat:132-145, KS:189-207)
-    const int64_t rem = nsteps - blocks * BLOCK_STEPS;
-    for (int64_t r = 0; r < rem; ++r) {
-        if (EQ == EQ_HEAT) {
-            for (int64_t i = threadIdx.x; i < n; i += NT)
-                b[i] = heat_ftcs(a[wrap1(i - 1, n)], a[i], a[wrap1(i + 1, n)], J.c[0], J.c[1]);
-            __syncthreads();
-            T* t = a; a = b; b = t;
-        } else {
-            for (int64_t i = threadIdx.x; i < n; i += NT)
-                b[i] = ks_predict(a[wrap1(i - 2, n)], a[wrap1(i - 1, n)], a[i], a[wrap1(i + 1, n)],
-                                  a[wrap1(i + 2, n)], k);
-            __syncthreads();
-            for (int64_t i = threadIdx.x; i < n; i += NT)
-                a[i] = ks_correct(a[i], b[wrap1(i - 2, n)], b[wrap1(i - 1, n)], b[i],
-                                  b[wrap1(i + 1, n)], b[wrap1(i + 2, n)], k);
-            __syncthreads();
-        }
-    }
-}
-
-template <typename T, int NW>
-__global__ __launch_bounds__(NW * kWave) void k_batch(const BatchJob<T>* __restrict__ jobs,
-                                                         int njobs, int* __restrict__ next,
-                                                         T* __restrict__ A, T* __restrict__ B,
-                                                         int64_t nsteps)
-{
-    __shared__ int s_job;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & (kWave - 1);
-    for (;;) {
-        __syncthreads();  // every wave has read the previous s_job
-        if (threadIdx.x == 0) s_job = atomicAdd(next, 1);
-        __syncthreads();
-        const int j = s_job;
-        if (j >= njobs) break;
-        const BatchJob<T> J = jobs[j];
-        T* a = A + J.offset;
-        T* b = B + J.offset;
-        const int blk = J.eq == EQ_HEAT ? 32 : 8;
-        int64_t swaps = nsteps / blk + (J.eq == EQ_HEAT ? nsteps % blk : 0);
-        if (J.eq == EQ_HEAT) {
-            if (J.po == 2) batch_problem<T, EQ_HEAT, 2, NW>(J, a, b, nsteps, wave, lane);
-            else if (J.po == 4) batch_problem<T, EQ_HEAT, 4, NW>(J, a, b, nsteps, wave, lane);
-            else if (J.po == 8) batch_problem<T, EQ_HEAT, 8, NW>(J, a, b, nsteps, wave, lane);
-            else batch_problem<T, EQ_HEAT, 16, NW>(J, a, b, nsteps, wave, lane);
-        } else {
-            if (J.po == 2) batch_problem<T, EQ_KS, 2, NW>(J, a, b, nsteps, wave, lane);
-            else if (J.po == 4) batch_problem<T, EQ_KS, 4, NW>(J, a, b, nsteps, wave, lane);
-            else if (J.po == 8) batch_problem<T, EQ_KS, 8, NW>(J, a, b, nsteps, wave, lane);
-            else batch_problem<T, EQ_KS, 16, NW>(J, a, b, nsteps, wave, lane);
-        }
-        // the result ends in b after an odd number of ping-pongs: copy it home
-        if (swaps & 1) {
-            for (int64_t i = threadIdx.x; i < J.n; i += NW * kWave) a[i] = b[i];
-        }
-    }
-}
-
-__global__ void k_reset_counter(int* c)
-{
-    if (threadIdx.x == 0) *c = 0;
-}
-
-template <typename T, int NW>
-hipError_t batch_launch(const BatchLaunch& L, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_reset_counter, dim3(1), dim3(64), 0, s, L.next);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((k_batch<T, NW>), dim3(L.grid), dim3(NW * kWave), 0, s,
-                       static_cast<const BatchJob<T>*>(L.jobs), L.njobs, L.next,
-                       static_cast<T*>(L.a), static_cast<T*>(L.b), L.nsteps);
-    return hipGetLastError();
 }
 
 template <typename T>
-hipError_t batch_prec(const BatchLaunch& L, hipStream_t s)
+hipError_t launch_prec(const BatchLaunch& L, hipStream_t s)
 {
-    switch (L.waves) {
-    case 2: return batch_launch<T, 2>(L, s);
-    case 8: return batch_launch<T, 8>(L, s);
-    default: return batch_launch<T, 4>(L, s);
-    }
+    return L.eq == EQ_HEAT ? launch_group<T, EQ_HEAT>(L, s) : launch_group<T, EQ_KS>(L, s);
 }
 
-template <typename T, int NW>
-int occupancy()
+// A group's launches and steps per launch (the longer ones), and their time.
+struct Timing { double us = 0; int64_t launches = 0; int steps = 0; };
+
+// Tiles of at most `most` points that the members need (from a sample of large
+// groups: the estimate is made some hundred times per new step count).
+double tiles_of(const std::vector<int64_t>& n, const std::vector<int>& members, double most)
 {
-    int nb = 0;
-    const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_batch<T, NW>, NW * kWave, 0);
-    return e == hipSuccess && nb > 0 ? nb : 1;
+    const size_t stride = (members.size() + 255) / 256;
+    double t = 0;
+    size_t seen = 0;
+    for (size_t j = 0; j < members.size(); j += stride, ++seen) t += std::ceil((double)n[members[j]] / most);
+    return t * (double)members.size() / (double)seen;
+}
+
+// The best steps per launch of a group: the cost model of wide_choose with the
+// group's tiles and an even number of launches.
+Timing time_group(int eq, bool f64, int shape, const std::vector<int64_t>& n, const std::vector<int>& members,
+                  int64_t nsteps, int cus)
+{
+    const Entry& e = entries(eq)[shape];
+    const Cost& c = f64 ? e.f64 : e.f32;
+    const int win = window(e), r = reach(eq);
+    Timing best;
+    for (double f : {.95, .9, .85, .8, .75, .7, .6, .45, .3}) {
+        const double s = std::floor((1 - f) * win / (2 * r));
+        if (s < 1) continue;
+        const double launches = 2 * std::ceil((double)nsteps / (2 * s)), each = std::ceil(nsteps / launches);
+        const double m = std::ceil(tiles_of(n, members, win - 2 * r * each) / cus);
+        const double us = launches * (c.t0 + (m - 1) * c.t2 + each * (c.c1 + (m - 1) * c.c2));
+        if (best.launches == 0 || us < best.us) best = Timing{us, (int64_t)launches, (int)each};
+    }
+    return best;
+}
+
+// A problem's own best shape where every compute unit is busy anyway: the
+// least time per step of its tiles' throughput.
+struct ShapeCost { int shape; double per_tile, us; };  // 1 / (points a tile stores), us per step and tile
+std::vector<ShapeCost> shape_costs(int eq, bool f64, int64_t nsteps)
+{
+    std::vector<ShapeCost> v;
+    for (int i = 0; i < shapes(eq); ++i) {
+        const Entry& e = entries(eq)[i];
+        const Cost& c = f64 ? e.f64 : e.f32;
+        const int win = window(e), r = reach(eq);
+        for (double f : {.95, .9, .85, .8, .7, .6, .45, .3}) {
+            const double s = std::min(std::floor((1 - f) * win / (2 * r)), (double)nsteps);
+            // the launch itself, spread over four tiles per compute unit
+            if (s >= 1) v.push_back({i, 1.0 / (win - 2 * r * s), c.c2 + (c.t2 + c.t0 / 4) / s});
+        }
+    }
+    return v;
+}
+int shape_for(const std::vector<ShapeCost>& costs, int64_t n)
+{
+    int best = 0;
+    double least = 0;
+    for (const ShapeCost& k : costs) {
+        const double us = std::ceil((double)n * k.per_tile) * k.us;
+        if (least == 0 || us < least) {
+            least = us;
+            best = k.shape;
+        }
+    }
+    return best;
 }
 
 }  // namespace
 
 hipError_t launch_batch(const BatchLaunch& L, bool f64, hipStream_t s)
 {
-    return f64 ? batch_prec<double>(L, s) : batch_prec<float>(L, s);
+    return f64 ? launch_prec<double>(L, s) : launch_prec<float>(L, s);
 }
 
-int batch_blocks_per_cu(bool f64, int waves)
+void batch_groups(const std::vector<int32_t>& eq, const std::vector<int64_t>& n, bool f64, int64_t nsteps, int cus,
+                  std::vector<BatchGroup>& groups, std::vector<BatchTile>& tiles)
 {
-    switch (waves) {
-    case 2: return f64 ? occupancy<double, 2>() : occupancy<float, 2>();
-    case 8: return f64 ? occupancy<double, 8>() : occupancy<float, 8>();
-    default: return f64 ? occupancy<double, 4>() : occupancy<float, 4>();
+    groups.clear();
+    tiles.clear();
+    if (cus <= 0) cus = 256;
+    for (int e = EQ_HEAT; e <= EQ_KS; ++e) {
+        std::vector<int> all;
+        for (size_t i = 0; i < n.size(); ++i)
+            if (eq[i] == e) all.push_back((int)i);
+        if (all.empty()) continue;
+        // one shape for every problem (few problems: the chip is not full) ...
+        int shape = 0;
+        Timing best;
+        for (int i = 0; i < shapes(e); ++i) {
+            const Timing t = time_group(e, f64, i, n, all, nsteps, cus);
+            if (t.launches && (best.launches == 0 || t.us < best.us)) {
+                best = t;
+                shape = i;
+            }
+        }
+        // ... or each problem's own
+        std::vector<std::vector<int>> own((size_t)shapes(e));
+        const std::vector<ShapeCost> costs = shape_costs(e, f64, nsteps);
+        for (int i : all) own[(size_t)shape_for(costs, n[i])].push_back(i);
+        std::vector<Timing> each((size_t)shapes(e));
+        double sum = 0;
+        for (int i = 0; i < shapes(e); ++i)
+            if (!own[i].empty()) {
+                each[i] = time_group(e, f64, i, n, own[i], nsteps, cus);
+                sum += each[i].us;
+            }
+        if (sum >= best.us) {
+            for (auto& m : own) m.clear();
+            own[shape] = all;
+            each[shape] = best;
+        }
+        for (int i = 0; i < shapes(e); ++i) {
+            if (own[i].empty()) continue;
+            BatchGroup g;
+            g.eq = e;
+            g.shape = i;
+            g.launches = each[i].launches;
+            g.first = (int64_t)tiles.size();
+            const int64_t most = window(entries(e)[i]) - 2 * (int64_t)reach(e) * each[i].steps;
+            for (int j : own[i]) {
+                const int64_t k = (n[j] + most - 1) / most, w = (n[j] + k - 1) / k;
+                for (int64_t o = 0; o < n[j]; o += w)
+                    tiles.push_back(BatchTile{j, (int32_t)o, (int32_t)std::min(w, n[j] - o)});
+            }
+            g.ntiles = (int64_t)tiles.size() - g.first;
+            groups.push_back(g);
+        }
     }
 }
 

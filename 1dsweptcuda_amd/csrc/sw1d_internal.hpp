@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 #include <cstdint>
+#include <vector>
 
 #include "sw1d_stencil.hpp"
 
@@ -72,22 +73,32 @@ struct WideChoice {
 
 // One problem of a batch.  Periodic heat (c = {Fo, 1-2Fo}) or KS
 // (c = {1/(4dx), 1/dx^2, 1/dx^4, dt, dt/2}), stored at `offset` in the packed
-// state arrays, advanced with trapezoid tiles of 64*po output points.
+// state arrays.
 template <typename T> struct BatchJob {
-    int64_t offset;
-    int32_t n, eq, po, pad;
+    int64_t offset, n;
     T c[5];
 };
 
+// Points [out0, out0 + count) of problem `job`.
+struct BatchTile { int32_t job, out0, count; };
+
+// Problems of one equation advanced with one tile shape: their tiles are
+// tiles[first .. first + ntiles), their launches an even number.
+struct BatchGroup {
+    int eq = 0, shape = 0;
+    int64_t launches = 0, first = 0, ntiles = 0;
+};
+// The groups and tiles of an advance of nsteps.
+void batch_groups(const std::vector<int32_t>& eq, const std::vector<int64_t>& n, bool f64, int64_t nsteps, int cus,
+                  std::vector<BatchGroup>& groups, std::vector<BatchTile>& tiles);
+
 struct BatchLaunch {
-    const void* jobs;  // device BatchJob<T>[njobs], in queue order
-    int32_t njobs;
-    int* next;         // device work-queue counter (set to 0 by the launch)
-    void* a;           // packed state; receives the result
-    void* b;           // packed scratch of the same size
-    int64_t nsteps;
-    int32_t grid;      // persistent workgroups
-    int32_t waves;     // waves (tiles worked on at once) per workgroup: 2, 4 or 8
+    int eq, shape, steps;
+    int64_t ntiles;
+    const BatchTile* tiles;  // on the device
+    const void* jobs;        // device BatchJob<T> per problem
+    const void* in;          // packed states
+    void* out;
 };
 
 }  // namespace sw1d
@@ -106,7 +117,6 @@ bool batch_view(sw1d_batch* b, BatchView& v);
 // Launchers (sw1d_kernels.hip, sw1d_trapezoid.hip, sw1d_batch.hip).  All
 // return a hipError_t.
 hipError_t launch_batch(const BatchLaunch& L, bool f64, hipStream_t s);
-int batch_blocks_per_cu(bool f64, int waves);
 inline bool batch_waves_supported(int w) { return w == 2 || w == 4 || w == 8; }
 inline bool batch_tile_supported(int po) { return po == 2 || po == 4 || po == 8 || po == 16; }
 hipError_t launch_trapezoid(const TrapLaunch& L, bool f64, const Coefs& c, hipStream_t s);

@@ -182,10 +182,10 @@ void fill_coefs(sw1d_plan* p, double* euler_dx)
 
 bool is_pow2(int64_t v) { return v > 0 && (v & (v - 1)) == 0; }
 
-// SW1D_LAUNCH_GRAPHS=0 in the environment: plans and batches launch their
-// kernels one by one instead of replaying hipGraphs (the same kernels in the
-// same order, so the same bits).  For tools that do not follow graph launches,
-// such as hardware-counter collection.
+// SW1D_LAUNCH_GRAPHS=0 in the environment: plans launch their kernels one by
+// one instead of replaying hipGraphs (the same kernels in the same order, so
+// the same bits).  For tools that do not follow graph launches, such as
+// hardware-counter collection.
 bool launch_graphs_enabled()
 {
     static const bool on = [] {
@@ -1194,43 +1194,33 @@ struct sw1d_batch {
     size_t S = 8;
     int64_t count = 0, total = 0;
     std::vector<int64_t> offset, n;
-    std::vector<char> jobs_host;  // BatchJob<T>[count], queue order
+    std::vector<int32_t> eq;
+    std::vector<char> jobs_host;  // BatchJob<T>[count]
     void* jobs = nullptr;
-    int* next = nullptr;
     void* a = nullptr;
     void* b = nullptr;
-    int32_t grid = 0;
-    int32_t waves = 4;  // waves per workgroup (tiles worked on at once)
+    int32_t waves = 4;  // as set by the caller (the tiles have their own)
     int32_t cus = 0;
     hipStream_t stream = nullptr;
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
-    int64_t graph_steps = -1;
+    // launches of an advance of group_steps
+    int64_t group_steps = -1;
+    std::vector<BatchGroup> groups;
+    BatchTile* tiles = nullptr;  // device
+    size_t tiles_cap = 0;
 };
 
 namespace {
 
 template <typename T>
-void build_jobs(sw1d_batch* B, const int32_t* eq, const double* dt, const double* dx,
-                const int32_t* tile_points)
+void build_jobs(sw1d_batch* B, const double* dt, const double* dx)
 {
-    std::vector<int64_t> order((size_t)B->count);
-    for (int64_t i = 0; i < B->count; ++i) order[i] = i;
-    // largest problems first: a greedy longest-processing-time queue
-    std::stable_sort(order.begin(), order.end(),
-                     [&](int64_t x, int64_t y) { return B->n[x] > B->n[y]; });
     B->jobs_host.assign(sizeof(BatchJob<T>) * (size_t)B->count, 0);
     BatchJob<T>* J = reinterpret_cast<BatchJob<T>*>(B->jobs_host.data());
-    for (int64_t k = 0; k < B->count; ++k) {
-        const int64_t i = order[k];
-        BatchJob<T>& j = J[k];
+    for (int64_t i = 0; i < B->count; ++i) {
+        BatchJob<T>& j = J[i];
         j.offset = B->offset[i];
-        j.n = (int32_t)B->n[i];
-        j.eq = eq[i];
-        int tp = tile_points ? tile_points[i] : 0;
-        if (tp <= 0) tp = 512;  // widest tile that won every size class of the tuned workload
-        j.po = tp / 64;
-        if (eq[i] == EQ_HEAT) {
+        j.n = B->n[i];
+        if (B->eq[i] == EQ_HEAT) {
             heat_consts<T>(dt[i], 8.418e-5, dx[i], j.c[0], j.c[1]);
         } else {
             const KsCoef<T> k2 = ks_consts<T>(dt[i], dx[i]);
@@ -1243,10 +1233,8 @@ void batch_release(sw1d_batch* B)
 {
     if (!B) return;
     if (B->stream) (void)hipStreamSynchronize(B->stream);
-    if (B->exec) (void)hipGraphExecDestroy(B->exec);
-    if (B->graph) (void)hipGraphDestroy(B->graph);
     if (B->jobs) (void)hipFree(B->jobs);
-    if (B->next) (void)hipFree(B->next);
+    if (B->tiles) (void)hipFree(B->tiles);
     if (B->a) (void)hipFree(B->a);
     if (B->b) (void)hipFree(B->b);
     if (B->stream) (void)hipStreamDestroy(B->stream);
@@ -1272,6 +1260,7 @@ int sw1d_batch_create(sw1d_batch** out, int32_t precision, int64_t count, const 
     B->count = count;
     B->offset.resize((size_t)count);
     B->n.resize((size_t)count);
+    B->eq.assign(eq, eq + count);
     for (int64_t i = 0; i < count; ++i) {
         if (eq[i] != SW1D_HEAT && eq[i] != SW1D_KS) {
             delete B;
@@ -1291,8 +1280,8 @@ int sw1d_batch_create(sw1d_batch** out, int32_t precision, int64_t count, const 
         B->all_ks = B->all_ks && eq[i] == SW1D_KS;
         B->total += nx[i];
     }
-    if (B->f64) build_jobs<double>(B, eq, dt, dx, tile_points);
-    else build_jobs<float>(B, eq, dt, dx, tile_points);
+    if (B->f64) build_jobs<double>(B, dt, dx);
+    else build_jobs<float>(B, dt, dx);
 
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
@@ -1301,13 +1290,10 @@ int sw1d_batch_create(sw1d_batch** out, int32_t precision, int64_t count, const 
         return fail(SW1D_EDEVICE, "no HIP device");
     }
     B->cus = cus;
-    const int64_t g = (int64_t)cus * batch_blocks_per_cu(B->f64, B->waves);
-    B->grid = (int32_t)std::min<int64_t>(g, count);
     const size_t bytes = (size_t)B->total * B->S;
     if (hipStreamCreateWithFlags(&B->stream, hipStreamNonBlocking) != hipSuccess ||
         hipMalloc(&B->a, bytes) != hipSuccess || hipMalloc(&B->b, bytes) != hipSuccess ||
-        hipMalloc(&B->jobs, B->jobs_host.size()) != hipSuccess ||
-        hipMalloc((void**)&B->next, sizeof(int)) != hipSuccess) {
+        hipMalloc(&B->jobs, B->jobs_host.size()) != hipSuccess) {
         batch_release(B);
         return fail(SW1D_ENOMEM, "batch device allocation of %zu bytes failed", 2 * bytes);
     }
@@ -1347,35 +1333,38 @@ int sw1d_batch_advance(sw1d_batch* B, int64_t nsteps)
     if (!B) return fail(SW1D_EINVAL, "null batch");
     if (nsteps < 0) return fail(SW1D_EINVAL, "nsteps must be >= 0");
     if (nsteps == 0) return SW1D_OK;
-    BatchLaunch L;
-    L.jobs = B->jobs;
-    L.njobs = (int32_t)B->count;
-    L.next = B->next;
-    L.a = B->a;
-    L.b = B->b;
-    L.nsteps = nsteps;
-    L.grid = B->grid;
-    L.waves = B->waves;
-    if (!launch_graphs_enabled()) {
-        HIP_OR_FAIL(launch_batch(L, B->f64, B->stream));
-        return SW1D_OK;
-    }
-    if (B->graph_steps != nsteps) {
-        // the previous graph's launch may still run on the stream: let it
-        // finish before its executable is destroyed
+    if (B->group_steps != nsteps) {
+        std::vector<BatchTile> tiles;
+        batch_groups(B->eq, B->n, B->f64, nsteps, B->cus, B->groups, tiles);
+        // earlier launches may still read the table
         HIP_OR_FAIL(hipStreamSynchronize(B->stream));
-        if (B->exec) { (void)hipGraphExecDestroy(B->exec); B->exec = nullptr; }
-        if (B->graph) { (void)hipGraphDestroy(B->graph); B->graph = nullptr; }
-        B->graph_steps = -1;
-        HIP_OR_FAIL(hipStreamBeginCapture(B->stream, hipStreamCaptureModeThreadLocal));
-        const hipError_t le = launch_batch(L, B->f64, B->stream);
-        const hipError_t ce = hipStreamEndCapture(B->stream, &B->graph);
-        if (le != hipSuccess) return fail(SW1D_EDEVICE, "batch launch capture: %s", hipGetErrorString(le));
-        if (ce != hipSuccess) return fail(SW1D_EDEVICE, "hipStreamEndCapture: %s", hipGetErrorString(ce));
-        HIP_OR_FAIL(hipGraphInstantiate(&B->exec, B->graph, nullptr, nullptr, 0));
-        B->graph_steps = nsteps;
+        B->group_steps = -1;
+        if (tiles.size() > B->tiles_cap) {
+            if (B->tiles) (void)hipFree(B->tiles);
+            B->tiles = nullptr;
+            B->tiles_cap = 0;
+            if (hipMalloc((void**)&B->tiles, tiles.size() * sizeof(BatchTile)) != hipSuccess)
+                return fail(SW1D_ENOMEM, "batch tile table of %zu tiles", tiles.size());
+            B->tiles_cap = tiles.size();
+        }
+        HIP_OR_FAIL(hipMemcpy(B->tiles, tiles.data(), tiles.size() * sizeof(BatchTile), hipMemcpyHostToDevice));
+        B->group_steps = nsteps;
     }
-    HIP_OR_FAIL(hipGraphLaunch(B->exec, B->stream));
+    for (const BatchGroup& g : B->groups) {
+        BatchLaunch L;
+        L.eq = g.eq;
+        L.shape = g.shape;
+        L.ntiles = g.ntiles;
+        L.tiles = B->tiles + g.first;
+        L.jobs = B->jobs;
+        const int64_t each = nsteps / g.launches, longer = nsteps % g.launches;
+        for (int64_t i = 0; i < g.launches; ++i) {
+            L.steps = (int)(each + (i < longer));
+            L.in = i % 2 ? B->b : B->a;
+            L.out = i % 2 ? B->a : B->b;
+            HIP_OR_FAIL(launch_batch(L, B->f64, B->stream));
+        }
+    }
     return SW1D_OK;
 }
 
@@ -1383,14 +1372,7 @@ int sw1d_batch_set_workgroup(sw1d_batch* B, int32_t waves)
 {
     if (!B) return fail(SW1D_EINVAL, "null batch");
     if (!batch_waves_supported(waves)) return fail(SW1D_EINVAL, "waves per workgroup must be 2, 4 or 8");
-    if (waves == B->waves) return SW1D_OK;
-    HIP_OR_FAIL(hipStreamSynchronize(B->stream));
-    if (B->exec) { (void)hipGraphExecDestroy(B->exec); B->exec = nullptr; }
-    if (B->graph) { (void)hipGraphDestroy(B->graph); B->graph = nullptr; }
-    B->graph_steps = -1;
     B->waves = waves;
-    const int64_t g = (int64_t)B->cus * batch_blocks_per_cu(B->f64, waves);
-    B->grid = (int32_t)std::min<int64_t>(g, B->count);
     return SW1D_OK;
 }
 
@@ -1419,7 +1401,7 @@ int sw1d_batch_info(const sw1d_batch* B, int64_t info[4])
 {
     if (!B || !info) return fail(SW1D_EINVAL, "null argument");
     info[0] = B->total;
-    info[1] = B->grid;
+    info[1] = std::min<int64_t>(4 * (int64_t)B->cus, B->count);
     info[2] = B->count;
     info[3] = (int64_t)(2 * (size_t)B->total * B->S + B->jobs_host.size());
     return SW1D_OK;

@@ -1,6 +1,5 @@
-// Device code of the overlapped trapezoid tile (one wave64 per tile), shared
-// by the single-problem kernels (sw1d_trapezoid.hip) and the batched
-// persistent kernel (sw1d_batch.hip).
+// Device code of Euler's overlapped trapezoid tile (one wave64 per tile,
+// sw1d_trapezoid.hip).
 //
 // A tile's window is 64*PI consecutive points (mod n) starting at `win`;
 // lane l holds points l*PI .. l*PI+PI-1 in VGPRs.  After S stages the window
@@ -52,68 +51,6 @@ __device__ __forceinline__ void store_window(T* __restrict__ a, int64_t n, int64
         const int pos = lane * PI + p - RS;
         if (pos >= 0 && pos < count) a[direct ? out0 + pos : wrapn(out0 + pos, n)] = v[p];
     }
-}
-
-// ------------------------------------------------------------------ heat ---
-template <typename T, int PI, int S, bool BND>
-__device__ __forceinline__ void trap_heat(const T* __restrict__ in, T* __restrict__ out, int64_t n,
-                                          int64_t win, int64_t out0, int count, int lane, T fo,
-                                          T fo2)
-{
-    constexpr int RS = S;  // R = 1
-    T v[PI];
-    int64_t g0 = 0;
-    if (BND) g0 = wrapn(win + (int64_t)lane * PI, n);
-    load_window<T, PI>(in, n, win, lane, v);
-    // The window's outer points are discarded, so lane 0 / lane 63 may see
-    // any finite value beyond it: the carried registers keep the first one.
-    T hl[1] = {v[0]}, hr[1] = {v[PI - 1]};
-    for (int s = 0; s < S; ++s) {
-        T e[PI + 2];
-        gather_carry<T, PI, 1>(v, hl, hr, e);
-#pragma unroll
-        for (int p = 0; p < PI; ++p) {
-            T l = e[p], c = e[p + 1], r = e[p + 2];
-            if (BND) {  // insulated ends (Heat:140-142)
-                int64_t g = g0 + p;
-                g = g >= n ? g - n : g;
-                l = g == 0 ? r : l;
-                r = g == n - 1 ? l : r;
-            }
-            v[p] = heat_ftcs(l, c, r, fo, fo2);
-        }
-    }
-    store_window<T, PI>(out, n, out0, count, lane, RS, v);
-}
-
-// -------------------------------------------------------------------- KS ---
-template <typename T, int PI, int S>
-__device__ __forceinline__ void trap_ks(const T* __restrict__ in, T* __restrict__ out, int64_t n,
-                                        int64_t win, int64_t out0, int count, int lane,
-                                        const KsCoef<T>& k)
-{
-    constexpr int RS = 2 * S;
-    T u[PI], uh[PI];
-    load_window<T, PI>(in, n, win, lane, u);
-    // beyond the window (discarded points): the carried registers' values
-    T hl[2] = {u[0], u[0]}, hr[2] = {u[0], u[0]};
-    T hlh[2] = {u[0], u[0]}, hrh[2] = {u[0], u[0]};
-    for (int s = 0; s < S; s += 2) {
-        {
-            T e[PI + 4];
-            gather_carry<T, PI, 2>(u, hl, hr, e);
-#pragma unroll
-            for (int p = 0; p < PI; ++p) uh[p] = ks_predict(e[p], e[p + 1], e[p + 2], e[p + 3], e[p + 4], k);
-        }
-        {
-            T e[PI + 4];
-            gather_carry<T, PI, 2>(uh, hlh, hrh, e);
-#pragma unroll
-            for (int p = 0; p < PI; ++p)
-                u[p] = ks_correct(u[p], e[p], e[p + 1], e[p + 2], e[p + 3], e[p + 4], k);
-        }
-    }
-    store_window<T, PI>(out, n, out0, count, lane, RS, u);
 }
 
 // ----------------------------------------------------------------- Euler ---

@@ -354,5 +354,57 @@ __device__ __forceinline__ void tile(T* lds, const T* __restrict__ in, T* __rest
     }
 }
 
+// ---------------------------------------------------------------- shapes ---
+// A shape and its measured cost, in microseconds: a launch of s steps whose
+// CUs each take m workgroups costs
+//   t0 + (m - 1) t2 + s (c1 + (m - 1) c2)
+// (t0: launch, load, store; c1: one workgroup alone on its CU, bound by issue
+// from about six points per lane and by latency below; c2: each further one).
+struct Cost { float t0, t2, c1, c2; };
+struct Entry { int P, HL; Cost f64, f32; };
+
+inline constexpr int kWaves = 4;  // one wave per SIMD: P sets the window
+// Halo lanes: an exchange every HL P / R steps, 5-9 for KS and 16-42 for heat
+inline constexpr Entry kKs[] = {
+    {2, 10, {2.3f, .06f, .151f, .101f}, {2.1f, .02f, .143f, .085f}},
+    {4, 6, {3.0f, .6f, .248f, .173f}, {2.8f, .35f, .224f, .153f}},
+    {5, 4, {3.2f, .45f, .319f, .217f}, {3.0f, .2f, .301f, .193f}},
+    {6, 4, {3.6f, .4f, .318f, .268f}, {3.3f, .25f, .301f, .226f}},
+    {8, 4, {4.7f, .4f, .383f, .36f}, {3.7f, .2f, .377f, .296f}},
+    {10, 2, {4.8f, .4f, .508f, .46f}, {4.2f, .35f, .469f, .374f}},
+    {12, 2, {5.6f, .6f, .590f, .56f}, {4.9f, .35f, .540f, .43f}},
+    {14, 2, {6.0f, .5f, .634f, .66f}, {5.2f, .35f, .619f, .44f}},
+    {16, 2, {7.0f, .7f, .709f, .75f}, {5.7f, .3f, .698f, .56f}},
+    {19, 2, {8.5f, .9f, .834f, .87f}, {6.4f, .25f, .816f, .68f}},
+};
+inline constexpr Entry kHeat[] = {
+    {2, 8, {2.1f, .18f, .0371f, .0151f}, {2.1f, .08f, .0299f, .0110f}},
+    {3, 8, {2.7f, .38f, .0407f, .0193f}, {2.7f, .15f, .0348f, .0162f}},
+    {4, 6, {3.1f, .5f, .0446f, .0247f}, {2.9f, .2f, .0393f, .0199f}},
+    {5, 4, {3.3f, .4f, .0511f, .0292f}, {3.0f, .17f, .0482f, .0258f}},
+    {7, 4, {3.3f, .45f, .0621f, .0379f}, {3.3f, .25f, .0650f, .0330f}},
+    {9, 4, {4.1f, .5f, .0673f, .0462f}, {3.8f, .3f, .0625f, .0423f}},
+    {12, 2, {4.8f, .6f, .0875f, .0622f}, {4.3f, .37f, .0819f, .0539f}},
+    {15, 2, {5.6f, .7f, .106f, .0770f}, {5.0f, .3f, .0956f, .0623f}},
+    {19, 2, {7.0f, .7f, .1203f, .0970f}, {5.8f, .3f, .1128f, .0811f}},
+    {21, 2, {7.4f, .9f, .1305f, .1066f}, {6.2f, .25f, .1226f, .0892f}},
+};
+
+inline int reach(int eq) { return eq == EQ_HEAT ? 1 : 4; }
+inline int window(const Entry& e) { return kWaves * (kWave - 2 * e.HL) * e.P + 2 * e.HL * e.P; }
+
+template <int EQ> struct Table;
+template <> struct Table<EQ_HEAT> {
+    static constexpr const Entry* e = kHeat;
+    static constexpr int count = sizeof(kHeat) / sizeof(Entry);
+};
+template <> struct Table<EQ_KS> {
+    static constexpr const Entry* e = kKs;
+    static constexpr int count = sizeof(kKs) / sizeof(Entry);
+};
+template <int EQ, int I> using TableShape = Shape<EQ, Table<EQ>::e[I].P, kWaves, Table<EQ>::e[I].HL>;
+inline const Entry* entries(int eq) { return eq == EQ_HEAT ? kHeat : kKs; }
+inline int shapes(int eq) { return eq == EQ_HEAT ? Table<EQ_HEAT>::count : Table<EQ_KS>::count; }
+
 }  // namespace wide
 }  // namespace sw1d

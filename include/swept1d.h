@@ -183,14 +183,16 @@ int sw1d_initial_condition(int32_t kind, int32_t precision, int64_t n, double le
 
 /* Batched solves -------------------------------------------------------------
  * No reference counterpart (the reference solves one problem per process):
- * many independent periodic heat / KS problems of any sizes, advanced together
- * by one persistent kernel launch, replayed from a captured hipGraph.
+ * many independent periodic heat / KS problems of any sizes, advanced together:
+ * one launch steps every problem of an equation and a tile shape, its workgroups
+ * the tiles of all of them.
  * Problem i: equation[i] (SW1D_HEAT periodic or SW1D_KS), nx[i] >= 128 points,
- * time step dt[i], grid spacing dx[i] (heat diffusivity 8.418e-5), tile width
- * tile_points[i] output points per trapezoid tile (128, 256, 512 or 1024;
- * 0 picks 512).  The state is the concatenation of the problems' fields in index
- * order, REAL per the precision.  Every problem's result is bitwise the
- * single-problem result. */
+ * time step dt[i], grid spacing dx[i] (heat diffusivity 8.418e-5).
+ * tile_points[i] (NULL, 0, 128, 256, 512 or 1024) is checked and otherwise
+ * unused: tile shapes and steps per launch come from measured costs.  The state
+ * is the concatenation of the problems' fields in index order, REAL per the
+ * precision.  Every problem's result is bitwise the single-problem result.
+ * The first advance by a new number of steps builds the table of its tiles. */
 typedef struct sw1d_batch sw1d_batch;
 int sw1d_batch_create(sw1d_batch** batch, int32_t precision, int64_t count,
                       const int32_t* equation, const int64_t* nx, const double* dt,
@@ -200,11 +202,10 @@ int sw1d_batch_set_state(sw1d_batch* batch, const void* host);
 int sw1d_batch_get_state(sw1d_batch* batch, void* host);
 int sw1d_batch_advance(sw1d_batch* batch, int64_t nsteps);
 int sw1d_batch_advance_timed(sw1d_batch* batch, int64_t nsteps, double* elapsed_ms);
-/* Waves per workgroup of the persistent launch, the tiles a workgroup works on
- * at once (the diamonds per workgroup of the reference's tuning): 2, 4
- * (default) or 8.  Results do not depend on it. */
+/* The diamonds per workgroup of the reference's tuning: 2, 4 (default) or 8,
+ * checked and otherwise unused (a tile is a workgroup of four waves). */
 int sw1d_batch_set_workgroup(sw1d_batch* batch, int32_t waves);
-/* info[0] total points, info[1] persistent workgroups, info[2] problems,
+/* info[0] total points, info[1] workgroups at work at once, info[2] problems,
  * info[3] device bytes */
 int sw1d_batch_info(const sw1d_batch* batch, int64_t info[4]);
 
