@@ -125,6 +125,9 @@ inline int64_t trapezoid_steps(int eq, int SB) { return eq == EQ_HEAT ? 32 * SB 
 hipError_t launch_wide(const WideLaunch& L, bool f64, const Coefs& c, hipStream_t s);
 WideChoice wide_choose(int eq, bool f64, int64_t n, int64_t nsteps, int cus);
 hipError_t launch_swept(const SweptLaunch& L, bool f64, const Coefs& c, hipStream_t s);
+// the Euler halves of launch_swept and launch_classic (sw1d_euler.hip)
+hipError_t launch_swept_euler(const SweptLaunch& L, bool f64, const Coefs& c, hipStream_t s);
+hipError_t launch_classic_euler(bool f64, int stage, int64_t n, void* buf, const Coefs& c, hipStream_t s);
 // One classic stage: heat (stage ignored), KS / Euler stage 0 = predictor,
 // 1 = corrector.  State layout as above; heat ping-pongs between in and out,
 // KS / Euler keep u and u_half in the same buffer.

@@ -32,76 +32,10 @@
 // Classic kernels — one thread per point, one launch per stage
 //   (classicHeat Heat:132-145, classicKS KS:189-207, classicEuler Euler:400-426).
 
-#include <type_traits>
-#include <utility>
-
-#include "sw1d_internal.hpp"
-#include "sw1d_lanes.hpp"
+#include "sw1d_nodes.hpp"
 
 namespace sw1d {
 namespace {
-
-constexpr int kWavesPerBlock = 4;
-constexpr int kBlock = kWave * kWavesPerBlock;
-constexpr int kClassicBlock = 256;
-
-
-template <typename T, int P>
-__device__ __forceinline__ void load_pts(const T* __restrict__ a, int64_t i0, T (&v)[P])
-{
-#pragma unroll
-    for (int p = 0; p < P; ++p) v[p] = a[i0 + p];
-}
-template <typename T, int P>
-__device__ __forceinline__ void store_pts(T* __restrict__ a, int64_t i0, const T (&v)[P])
-{
-#pragma unroll
-    for (int p = 0; p < P; ++p) a[i0 + p] = v[p];
-}
-
-struct NodeGeom {
-    int64_t base;  // global index of node-local x = 0
-    int64_t lb;    // global index of this lane's first point
-    int lane;
-};
-
-template <int P>
-__device__ __forceinline__ bool node_geom(int64_t n, int64_t nnodes, int64_t node_first,
-                                          int64_t offset, NodeGeom& g)
-{
-    constexpr int W = kWave * P;
-    g.lane = threadIdx.x & (kWave - 1);
-    const int64_t node = node_first + (int64_t)blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6);
-    if (node >= nnodes) return false;
-    int64_t b = node * W + offset;
-    b = b >= n ? b - n : b;
-    g.base = b;
-    int64_t lb = b + (int64_t)g.lane * P;
-    g.lb = lb >= n ? lb - n : lb;
-    return true;
-}
-
-__device__ __forceinline__ int64_t wrap(int64_t i, int64_t n)
-{
-    return i < 0 ? i + n : (i >= n ? i - n : i);
-}
-
-// Calls f(integral_constant<int, i>) for i = 0, 1, .. in order.
-template <typename F, int... I>
-__device__ __forceinline__ void for_each_index(F&& f, std::integer_sequence<int, I...>)
-{
-    (f(std::integral_constant<int, I>{}), ...);
-}
-
-// Calls f(integral_constant<int, j>) for j = A, A + 1, .. B in order (none if A > B).
-template <int A, int B, typename F>
-__device__ __forceinline__ void for_range(F&& f)
-{
-    if constexpr (A <= B) {
-        f(std::integral_constant<int, A>{});
-        for_range<A + 1, B>(f);
-    }
-}
 
 // EXEC-masked stage fmas with a compile-time threshold.  Lane l of a centred
 // region of PC points per lane holds d = |2(l PC + p) - 64 PC + 1| at point
@@ -292,16 +226,6 @@ struct HeatRegion {
     }
 };
 
-// Ring PC of a node (1 <= PC <= P) is the 64 points that the centred region
-// of PC points per lane holds and the region of PC - 1 does not: 32 on each
-// side of the centre.  Lane l takes ring point l, so a ring moves between HBM
-// and the LDS image as two coalesced 256-byte runs per state array.
-template <int W, int PC>
-__device__ __forceinline__ int ring_x(int lane)
-{
-    return lane < 32 ? W / 2 - 32 * PC + lane : W / 2 + 32 * (PC - 1) + (lane - 32);
-}
-
 // A node's HBM traffic ring by ring, for tiles whose levels run on centred
 // regions: NC state arrays of n values, array c at a + c n in HBM and at
 // img + c W in the node's LDS image.  A tile with a down phase issues the
@@ -356,17 +280,6 @@ struct NodeRings {
         for (int c = 0; c < NC; ++c) __builtin_nontemporal_store(img[c * W + x], &a[c * n + gi]);
     }
 };
-
-// Orders a wave's own LDS writes before its own reads of other lanes' data:
-// LDS executes a wave's instructions in order, and the wavefront-scope
-// fences keep the compiler from moving one lane's loads above other lanes'
-// stores.  Each wave of the tile kernels owns its slice of the LDS image.
-__device__ __forceinline__ void wave_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // Swept heat tiles: one wave per node of W = 64*P points.  For P >= 2 the
 // node's image sits in LDS and the diamond's levels run on centred regions of
@@ -778,329 +691,6 @@ __global__ __launch_bounds__(kBlock) void k_ks_swept(const T* __restrict__ in,
     }
 }
 
-// ---------------------------------------------------------- Euler tiles ---
-// Components 0..2 are the conserved values (rho, rho*u, E), 3..5 their
-// predictor.  EulerRegion holds PC cells per lane of the middle 64*PC cells
-// of a node (all of it when PC = P).
-template <typename T, int PC>
-struct EulerRegion {
-    T q[6][PC];
-    T hl[6][2], hr[6][2];
-    int d[PC];
-    bool g0, gN;  // this lane's first / last cell is global cell 0 / n-1
-    // one cell per lane: the lane's cell is global cell 1 / n-2 (with two or
-    // more per lane, cells 0 and 1, and n-2 and n-1, share a lane)
-    bool g1 = false, gNm1 = false;
-
-    // src = 0: predictor from the conserved values (Euler:307-350);
-    // src = 3: corrector from the predictor values (Euler:353-389, :420).
-    // Each interface flux is evaluated once and used by the two cells beside
-    // it (PC+1 interfaces per lane instead of 2 PC).
-    template <int src>
-    __device__ __forceinline__ void stage(int thr, const EulerCoef<T>& k)
-    {
-        constexpr int dst = 3 - src;
-        T ex[PC + 4], ey[PC + 4], ez[PC + 4];
-        gather_carry<T, PC, 2>(q[src + 0], hl[src + 0], hr[src + 0], ex);
-        gather_carry<T, PC, 2>(q[src + 1], hl[src + 1], hr[src + 1], ey);
-        gather_carry<T, PC, 2>(q[src + 2], hl[src + 2], hr[src + 2], ez);
-        auto cell = [&](int j) { return Q3<T>{ex[j], ey[j], ez[j]}; };
-        // pressure differences between ext cells j and j+1
-        T pd[PC + 3];
-#pragma unroll
-        for (int j = 0; j < PC + 3; ++j) pd[j] = eu_pdiff(cell(j), cell(j + 1));
-        // interface j lies between ext cells j+1 and j+2; the interface left
-        // of global cell 1 drops pdiff(-1,0), the one right of cell n-2 drops
-        // pdiff(n-1,n) (the flags of Euler:405, :424).
-        auto iface = [&](int j, Q3<T>& F, Q3<T>& D) {
-            bool drop0 = j == 1 && g0, drop2 = j == PC - 1 && gN;
-            if constexpr (PC == 1) {
-                drop0 = drop0 || (j == 0 && g1);
-                drop2 = drop2 || (j == 1 && gNm1);
-            }
-            const T q0 = drop0 ? T(0) : pd[j];
-            const T q2 = drop2 ? T(0) : pd[j + 2];
-            eu_iface(cell(j), cell(j + 1), cell(j + 2), cell(j + 3), q0, pd[j + 1], q2, k, F, D);
-        };
-        const T c = src == 0 ? T(0.25) * k.dtdx : T(0.5) * k.dtdx;
-        Q3<T> FL, DL;
-        iface(0, FL, DL);
-#pragma unroll
-        for (int p = 0; p < PC; ++p) {
-            Q3<T> FR, DR;
-            iface(p + 1, FR, DR);
-            const Q3<T> f = eu_balance(FL, DL, FR, DR);
-            const Q3<T> base = src == 0 ? cell(p + 2) : Q3<T>{q[0][p], q[1][p], q[2][p]};
-            Q3<T> nv = eu_apply(base, f, c);
-            // ghost cells 0 and n-1 hold the Dirichlet states (Euler:405-425)
-            if (p == 0 && g0) nv = k.bl;
-            if (p == PC - 1 && gN) nv = k.br;
-            const bool act = d[p] <= thr;
-            q[dst + 0][p] = act ? nv.x : q[dst + 0][p];
-            q[dst + 1][p] = act ? nv.y : q[dst + 1][p];
-            q[dst + 2][p] = act ? nv.z : q[dst + 2][p];
-            FL = FR;
-            DL = DR;
-        }
-    }
-    __device__ __forceinline__ void down(int s0, int s1, const EulerCoef<T>& k)
-    {
-        for (int s = s0; s <= s1; s += 2) { stage<0>(4 * s - 1, k); stage<3>(4 * s + 3, k); }
-    }
-    __device__ __forceinline__ void up(int W, int m0, int m1, const EulerCoef<T>& k)
-    {
-        for (int m = m0; m <= m1; m += 2) { stage<0>(W - 1 - 4 * m, k); stage<3>(W - 5 - 4 * m, k); }
-    }
-    __device__ __forceinline__ void place(int W, int x0, int64_t base, int64_t n)
-    {
-#pragma unroll
-        for (int p = 0; p < PC; ++p) d[p] = abs(2 * (x0 + p) - (W - 1));
-        int64_t gi = base + x0;
-        gi = gi >= n ? gi - n : gi;
-        int64_t gl = gi + PC - 1;
-        gl = gl >= n ? gl - n : gl;
-        g0 = gi == 0;
-        gN = gl == n - 1;
-        if (PC == 1) {
-            g1 = gi == 1;
-            gNm1 = gl == n - 2;
-        }
-    }
-    // The region is the middle 64*PC cells of a node of W cells (all of it
-    // when PC = W/64): lane l holds node-local x0 = W/2 - 32 PC + l PC ..
-    // x0 + PC - 1, and the halo is the two cells beyond each end.
-    template <int W>
-    static constexpr int xs() { return W / 2 - 32 * PC; }
-    // every component and the halo from the state arrays (node base `base`)
-    template <int W>
-    __device__ __forceinline__ void load_global(const T* in, int64_t n, int64_t base, int lane)
-    {
-        const int x0 = xs<W>() + lane * PC;
-#pragma unroll
-        for (int c = 0; c < 6; ++c) {
-#pragma unroll
-            for (int p = 0; p < PC; ++p) q[c][p] = in[c * n + wrap(base + x0 + p, n)];
-        }
-        halo_global<W>(in, n, base);
-    }
-    template <int W>
-    __device__ __forceinline__ void halo_global(const T* in, int64_t n, int64_t base)
-    {
-#pragma unroll
-        for (int c = 0; c < 6; ++c) {
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                hl[c][i] = in[c * n + wrap(base + xs<W>() - 1 - i, n)];
-                hr[c][i] = in[c * n + wrap(base + xs<W>() + 64 * PC + i, n)];
-            }
-        }
-    }
-    // Components C0 .. C0+2 to / from a three-component node image (component
-    // c at img + (c - C0) W, node-local cell order).
-    template <int W, int C0>
-    __device__ __forceinline__ void save_half(T* img, int lane) const
-    {
-        const int x0 = xs<W>() + lane * PC;
-#pragma unroll
-        for (int c = C0; c < C0 + 3; ++c)
-#pragma unroll
-            for (int p = 0; p < PC; ++p) img[(c - C0) * W + x0 + p] = q[c][p];
-    }
-    template <int W, int C0>
-    __device__ __forceinline__ void load_half(const T* img, int lane)
-    {
-        const int x0 = xs<W>() + lane * PC;
-#pragma unroll
-        for (int c = C0; c < C0 + 3; ++c)
-#pragma unroll
-            for (int p = 0; p < PC; ++p) q[c][p] = img[(c - C0) * W + x0 + p];
-    }
-    template <int W, int C0>
-    __device__ __forceinline__ void halo_half(const T* img)
-    {
-        static_assert(xs<W>() >= 2 && xs<W>() + 64 * PC + 2 <= W, "halo inside the node");
-#pragma unroll
-        for (int c = C0; c < C0 + 3; ++c) {
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                hl[c][i] = img[(c - C0) * W + xs<W>() - 1 - i];
-                hr[c][i] = img[(c - C0) * W + xs<W>() + 64 * PC + i];
-            }
-        }
-    }
-    // the region's cells to the state arrays
-    template <int W>
-    __device__ __forceinline__ void store_global(T* out, int64_t n, int64_t base, int lane) const
-    {
-        const int x0 = xs<W>() + lane * PC;
-#pragma unroll
-        for (int c = 0; c < 6; ++c)
-#pragma unroll
-            for (int p = 0; p < PC; ++p) out[c * n + wrap(base + x0 + p, n)] = q[c][p];
-    }
-};
-
-// Ring PC's cells of components C0 .. C0+2: from the state arrays into a
-// three-component node image, and from the image to the state arrays.
-template <typename T, int W, int PC, int C0>
-__device__ __forceinline__ void eu_ring_in(T* img, const T* in, int64_t n, int64_t base, int lane)
-{
-    const int x = ring_x<W, PC>(lane);
-#pragma unroll
-    for (int c = C0; c < C0 + 3; ++c) img[(c - C0) * W + x] = in[c * n + wrap(base + x, n)];
-}
-template <typename T, int W, int PC, int C0>
-__device__ __forceinline__ void eu_ring_out(const T* img, T* out, int64_t n, int64_t base, int lane)
-{
-    const int x = ring_x<W, PC>(lane);
-#pragma unroll
-    for (int c = C0; c < C0 + 3; ++c) out[c * n + wrap(base + x, n)] = img[(c - C0) * W + x];
-}
-
-// Smallest region of the phased Euler tiles, in cells per lane.
-constexpr int kEuRegionFirst = 1;
-
-// A phased Euler tile's node: its base in the state arrays and the wave's
-// three-component LDS image (3 W values).
-template <typename T>
-struct EuNode {
-    T* img;
-    const T* in;
-    T* out;
-    int64_t n, base;
-    int lane;
-};
-
-// Region A -> region B = A + 1 cells per lane (B = W/64: the whole node), one
-// half of the state at a time through the image.  The cells of ring B, and
-// the halo of region B, lie outside every region so far, so they still hold
-// the tile's input.
-template <typename T, int W, int A, int B>
-__device__ __forceinline__ void eu_grow(const EulerRegion<T, A>& a, EulerRegion<T, B>& b, const EuNode<T>& d)
-{
-    for_each_index(
-        [&](auto h) {
-            constexpr int C0 = 3 * decltype(h)::value;
-            a.template save_half<W, C0>(d.img, d.lane);
-            eu_ring_in<T, W, B, C0>(d.img, d.in, d.n, d.base, d.lane);
-            wave_sync();
-            b.template load_half<W, C0>(d.img, d.lane);
-            wave_sync();
-        },
-        std::make_integer_sequence<int, 2>{});
-    b.template halo_global<W>(d.in, d.n, d.base);
-    b.place(W, EulerRegion<T, B>::template xs<W>() + d.lane * B, d.base, d.n);
-}
-
-// Region A -> region B = A - 1 cells per lane: ring A is final and goes to
-// the output; region B's halo lies in ring A and comes from the image.
-template <typename T, int W, int A, int B>
-__device__ __forceinline__ void eu_shrink(const EulerRegion<T, A>& a, EulerRegion<T, B>& b, const EuNode<T>& d)
-{
-    for_each_index(
-        [&](auto h) {
-            constexpr int C0 = 3 * decltype(h)::value;
-            a.template save_half<W, C0>(d.img, d.lane);
-            wave_sync();
-            eu_ring_out<T, W, A, C0>(d.img, d.out, d.n, d.base, d.lane);
-            b.template load_half<W, C0>(d.img, d.lane);
-            b.template halo_half<W, C0>(d.img);
-            wave_sync();
-        },
-        std::make_integer_sequence<int, 2>{});
-    b.place(W, EulerRegion<T, B>::template xs<W>() + d.lane * B, d.base, d.n);
-}
-
-// The down phase from region PC (loaded) on: region PC takes down pairs
-// 16 PC - 15 <= s <= 16 PC - 1 (from 1 for the first region), where every
-// threshold is <= 64 PC - 1; the whole node ends it in `full`.
-template <typename T, int P, int PC>
-__device__ __forceinline__ void eu_down(EulerRegion<T, PC>& r, EulerRegion<T, P>& full, const EuNode<T>& d,
-                                        const EulerCoef<T>& k)
-{
-    constexpr int W = kWave * P, H = W / 4;
-    r.down(PC == kEuRegionFirst ? 1 : 16 * PC - 15, 16 * PC - 1, k);
-    if constexpr (PC + 1 < P) {
-        EulerRegion<T, PC + 1> r2;
-        eu_grow<T, W, PC, PC + 1>(r, r2, d);
-        eu_down<T, P, PC + 1>(r2, full, d, k);
-    } else {
-        eu_grow<T, W, PC, P>(r, full, d);
-        full.down(16 * (P - 1) + 1, H - 1, k);
-    }
-}
-
-// The up phase from region PC + 1 (or the whole node, PC + 1 = P) down:
-// region PC takes up pairs 16(P-PC)+1 <= m <= 16(P-PC)+15 (to H-3 for the
-// first region); each ring goes to the output once final, the first region
-// last.
-template <typename T, int P, int PC>
-__device__ __forceinline__ void eu_up(const EulerRegion<T, PC + 1>& a, const EuNode<T>& d, const EulerCoef<T>& k)
-{
-    constexpr int W = kWave * P, H = W / 4;
-    EulerRegion<T, PC> b;
-    eu_shrink<T, W, PC + 1, PC>(a, b, d);
-    if constexpr (PC == kEuRegionFirst) {
-        b.up(W, 16 * (P - PC) + 1, H - 3, k);
-        b.template stage<0>(W - 1 - 4 * (H - 1), k);
-        b.template store_global<W>(d.out, d.n, d.base, d.lane);
-    } else {
-        b.up(W, 16 * (P - PC) + 1, 16 * (P - PC) + 15, k);
-        eu_up<T, P, PC - 1>(b, d, k);
-    }
-}
-
-// Swept Euler tiles: one wave per node of W = 64*P cells.  For P >= 4 the
-// diamond's levels run on the narrowest centred region of 1, 2, .. P cells
-// per lane that holds their active set and the two-cell stencil reach (same
-// operations, same bits), and a change of region moves the lane's cells
-// through an LDS image of three of the six components at a time: 12 KB per
-// wave at W = 512, so that two waves fit on a SIMD (the kernel is held to
-// 256 registers for the same reason).  The node's cells come from the input
-// ring by ring as the regions grow and go to the output ring by ring as they
-// shrink.
-template <typename T, int P, int TILE>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2)))
-void k_euler_swept(const T* __restrict__ in, T* __restrict__ out, int64_t n, int64_t nnodes,
-                   int64_t node_first, int64_t offset, EulerCoef<T> k)
-{
-    constexpr int W = kWave * P, H = W / 4;
-    constexpr bool PHASED = P >= 4;
-    __shared__ T img_all[PHASED ? kWavesPerBlock * 3 * W : 1];
-    NodeGeom g;
-    if (!node_geom<P>(n, nnodes, node_first, offset, g)) return;
-
-    EulerRegion<T, P> full;
-    if constexpr (!PHASED) {
-        full.template load_global<W>(in, n, g.base, g.lane);
-        full.place(W, g.lane * P, g.base, n);
-        if (TILE != TILE_UP) full.down(1, H - 1, k);
-        if (TILE != TILE_DOWN) {
-            full.up(W, 1, H - 3, k);
-            full.template stage<0>(W - 1 - 4 * (H - 1), k);
-        }
-        full.template store_global<W>(out, n, g.base, g.lane);
-    } else {
-        constexpr int F = kEuRegionFirst;
-        const EuNode<T> d{img_all + (threadIdx.x >> 6) * 3 * W, in, out, n, g.base, g.lane};
-        if (TILE != TILE_UP) {
-            EulerRegion<T, F> r;
-            r.template load_global<W>(in, n, g.base, g.lane);
-            r.place(W, EulerRegion<T, F>::template xs<W>() + g.lane * F, g.base, n);
-            eu_down<T, P, F>(r, full, d, k);
-        } else {
-            full.template load_global<W>(in, n, g.base, g.lane);
-            full.place(W, g.lane * P, g.base, n);
-        }
-        if (TILE != TILE_DOWN) {
-            full.up(W, 1, 15, k);
-            eu_up<T, P, P - 1>(full, d, k);
-        } else {
-            full.template store_global<W>(out, n, g.base, g.lane);
-        }
-    }
-}
-
 // ------------------------------------------------------ classic kernels ---
 template <typename T, bool PERIODIC>
 __global__ __launch_bounds__(kClassicBlock) void k_heat_classic(const T* __restrict__ in,
@@ -1170,54 +760,6 @@ __global__ __launch_bounds__(kClassicBlock) void k_ks_classic(T* __restrict__ bu
     }
 }
 
-// Euler classic stage (Euler:391-426) with each interface flux evaluated once:
-// lane l of a wave computes the interface between cells x = 63 w + l - 1 and
-// x + 1, and (l < 63) updates cell x + 1 from it and from lane l + 1's,
-// which a DPP shift brings: 63 cells per wave, and the values the per-cell
-// form computes twice, so the same bits.  Cell indices are clamped at the
-// domain ends as in the per-cell form (the values so read are unused there).
-template <typename T, int STAGE>
-__global__ __launch_bounds__(kClassicBlock) void k_euler_classic(T* __restrict__ buf, int64_t n,
-                                                                 EulerCoef<T> k)
-{
-    constexpr int src = STAGE == 0 ? 0 : 3, dst = 3 - src;
-    const int lane = threadIdx.x & (kWave - 1);
-    const int64_t wave = (int64_t)blockIdx.x * (kClassicBlock / kWave) + (threadIdx.x >> 6);
-    const int64_t x = wave * (kWave - 1) + lane - 1;
-    auto cell = [&](int64_t j) {
-        j = j < 0 ? 0 : (j > n - 1 ? n - 1 : j);
-        return Q3<T>{buf[(src + 0) * n + j], buf[(src + 1) * n + j], buf[(src + 2) * n + j]};
-    };
-    const Q3<T> A = cell(x - 1), B = cell(x), C = cell(x + 1), Dc = cell(x + 2);
-    // the interface right of cell 0 drops pdiff(-1,0), the one left of cell
-    // n-1 drops pdiff(n-1,n) (the flags of Euler:405, :424)
-    const T q0 = x == 0 ? T(0) : eu_pdiff(A, B);
-    const T q1 = eu_pdiff(B, C);
-    const T q2 = x == n - 2 ? T(0) : eu_pdiff(C, Dc);
-    Q3<T> FL, DL;
-    eu_iface(A, B, C, Dc, q0, q1, q2, k, FL, DL);
-    // every lane takes part in the shifts before any leaves
-    const Q3<T> FR{from_right(FL.x, FL.x), from_right(FL.y, FL.y), from_right(FL.z, FL.z)};
-    const Q3<T> DR{from_right(DL.x, DL.x), from_right(DL.y, DL.y), from_right(DL.z, DL.z)};
-    const int64_t i = x + 1;
-    if (lane == kWave - 1 || i >= n) return;
-    Q3<T> nv;
-    if (i == 0) {
-        nv = k.bl;
-    } else if (i == n - 1) {
-        nv = k.br;
-    } else {
-        const Q3<T> f = eu_balance(FL, DL, FR, DR);
-        if (STAGE == 0)
-            nv = eu_apply(C, f, T(0.25) * k.dtdx);
-        else
-            nv = eu_apply(Q3<T>{buf[i], buf[n + i], buf[2 * n + i]}, f, T(0.5) * k.dtdx);
-    }
-    buf[(dst + 0) * n + i] = nv.x;
-    buf[(dst + 1) * n + i] = nv.y;
-    buf[(dst + 2) * n + i] = nv.z;
-}
-
 // ------------------------------------------------------------ lane check ---
 __global__ void k_lane_check(int* ok)
 {
@@ -1246,10 +788,6 @@ template <> float fo2_of<float>(const Coefs& c) { return c.fo2_f; }
 template <typename T> const KsCoef<T>& ks_of(const Coefs& c);
 template <> const KsCoef<double>& ks_of<double>(const Coefs& c) { return c.ks_d; }
 template <> const KsCoef<float>& ks_of<float>(const Coefs& c) { return c.ks_f; }
-template <typename T> const EulerCoef<T>& eu_of(const Coefs& c);
-template <> const EulerCoef<double>& eu_of<double>(const Coefs& c) { return c.eu_d; }
-template <> const EulerCoef<float>& eu_of<float>(const Coefs& c) { return c.eu_f; }
-
 template <typename T, int P, int TILE>
 hipError_t swept_tile(const SweptLaunch& L, const Coefs& c, hipStream_t s)
 {
@@ -1289,11 +827,7 @@ hipError_t swept_tile(const SweptLaunch& L, const Coefs& c, hipStream_t s)
             hipLaunchKernelGGL((k_ks_swept<T, P, TILE, false>), grid, dim3(kBlock), 0, s, in, out, L.n,
                                L.nnodes, L.node_first, L.offset, ks_of<T>(c));
     } else {
-        if constexpr (P <= 8)
-            hipLaunchKernelGGL((k_euler_swept<T, P, TILE>), grid, dim3(kBlock), 0, s, in, out,
-                               L.n, L.nnodes, L.node_first, L.offset, eu_of<T>(c));
-        else
-            return hipErrorInvalidValue;
+        return hipErrorInvalidValue;
     }
     return hipGetLastError();
 }
@@ -1350,13 +884,7 @@ hipError_t classic_prec(int eq, int bc, int stage, int64_t n, const void* in, vo
             hipLaunchKernelGGL((k_ks_classic<T, 1>), g2, dim3(kClassicBlock), 0, s, b, n, ks_of<T>(c));
         }
     } else {
-        T* b = static_cast<T*>(out);
-        const int64_t waves = (n + kWave - 2) / (kWave - 1);  // 63 cells per wave
-        const dim3 ge((unsigned)((waves + kClassicBlock / kWave - 1) / (kClassicBlock / kWave)));
-        if (stage == 0)
-            hipLaunchKernelGGL((k_euler_classic<T, 0>), ge, dim3(kClassicBlock), 0, s, b, n, eu_of<T>(c));
-        else
-            hipLaunchKernelGGL((k_euler_classic<T, 1>), ge, dim3(kClassicBlock), 0, s, b, n, eu_of<T>(c));
+        return hipErrorInvalidValue;
     }
     return hipGetLastError();
 }
@@ -1365,12 +893,14 @@ hipError_t classic_prec(int eq, int bc, int stage, int64_t n, const void* in, vo
 
 hipError_t launch_swept(const SweptLaunch& L, bool f64, const Coefs& c, hipStream_t s)
 {
+    if (L.eq == EQ_EULER) return launch_swept_euler(L, f64, c, s);
     return f64 ? swept_prec<double>(L, c, s) : swept_prec<float>(L, c, s);
 }
 
 hipError_t launch_classic(int eq, int bc, bool f64, int stage, int64_t n, const void* in,
                           void* out, const Coefs& c, hipStream_t s)
 {
+    if (eq == EQ_EULER) return launch_classic_euler(f64, stage, n, out, c, s);
     return f64 ? classic_prec<double>(eq, bc, stage, n, in, out, c, s)
                : classic_prec<float>(eq, bc, stage, n, in, out, c, s);
 }

@@ -40,6 +40,27 @@ __device__ __forceinline__ float from_right(float v, float old)
     return __int_as_float(shl1_i(__float_as_int(v), __float_as_int(old)));
 }
 
+// The neighbour lane's value; 0 in lane 0 / lane 63 (no register to keep, so no
+// copy of one either).
+__device__ __forceinline__ double from_left0(double v)
+{
+    return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x138, 0xf, 0xf, true),
+                            __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x138, 0xf, 0xf, true));
+}
+__device__ __forceinline__ double from_right0(double v)
+{
+    return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x130, 0xf, 0xf, true),
+                            __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x130, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float from_left0(float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float from_right0(float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xf, 0xf, true));
+}
+
 // e[0 .. P+2R-1] = values at node-local x = l*P - R .. l*P + P + R - 1.
 // The point at x = l*P - 1 - i is lane l-1's e[R - 1 - i + P]: its own point
 // P-1-i when i < P, else (a radius wider than a lane, R > P) the value lane

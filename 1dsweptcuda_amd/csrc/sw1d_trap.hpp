@@ -7,6 +7,7 @@
 // are stored to out0 .. out0+count-1 (mod n).
 #pragma once
 
+#include "sw1d_euler.hpp"
 #include "sw1d_internal.hpp"
 #include "sw1d_lanes.hpp"
 
@@ -54,55 +55,33 @@ __device__ __forceinline__ void store_window(T* __restrict__ a, int64_t n, int64
 }
 
 // ----------------------------------------------------------------- Euler ---
+// One stage (eu_lane_stage): dst = base + c flux(src).  The window's outermost
+// cells are discarded, so every stage leaves out their outer interfaces.
 template <typename T, int PI, bool BND>
 __device__ __forceinline__ void eu_trap_stage(const T (&src)[3][PI], T (&dst)[3][PI],
                                               const T (&base)[3][PI], T (&hl)[3][2], T (&hr)[3][2],
                                               int64_t g0, int64_t n, T c, const EulerCoef<T>& k)
 {
-    T ex[PI + 4], ey[PI + 4], ez[PI + 4];
-    gather_carry<T, PI, 2>(src[0], hl[0], hr[0], ex);
-    gather_carry<T, PI, 2>(src[1], hl[1], hr[1], ey);
-    gather_carry<T, PI, 2>(src[2], hl[2], hr[2], ez);
-    auto cell = [&](int j) { return Q3<T>{ex[j], ey[j], ez[j]}; };
-    // global index of ext cell j (lane's point p is ext cell p + 2)
-    auto gidx = [&](int j) {
-        int64_t g = g0 + j - 2;
+    // global index of the lane's cell p, p = -1 .. PI
+    auto gidx = [&](int p) {
+        const int64_t g = g0 + p;
         return g < 0 ? g + n : (g >= n ? g - n : g);
     };
-    T pd[PI + 3];
-#pragma unroll
-    for (int j = 0; j < PI + 3; ++j) pd[j] = eu_pdiff(cell(j), cell(j + 1));
-    // interface j between ext cells j+1 and j+2 (Euler:311-341); the
-    // interface right of cell 0 drops pdiff(-1,0), the one right of cell n-2
-    // drops pdiff(n-1,n) (the flags of Euler:405, :424)
-    auto iface = [&](int j, Q3<T>& F, Q3<T>& D) {
-        T q0 = pd[j], q2 = pd[j + 2];
-        if (BND) {
-            const int64_t gl = gidx(j + 1);
-            q0 = gl == 0 ? T(0) : q0;
-            q2 = gl == n - 2 ? T(0) : q2;
-        }
-        eu_iface(cell(j), cell(j + 1), cell(j + 2), cell(j + 3), q0, pd[j + 1], q2, k, F, D);
-    };
-    Q3<T> FL, DL;
-    iface(0, FL, DL);
-#pragma unroll
-    for (int p = 0; p < PI; ++p) {
-        Q3<T> FR, DR;
-        iface(p + 1, FR, DR);
-        const Q3<T> f = eu_balance(FL, DL, FR, DR);
+    // the interface right of cell 0 drops pdiff(-1,0), the one right of cell
+    // n-2 drops pdiff(n-1,n) (the flags of Euler:405, :424)
+    auto drop0 = [&](int j) { return BND && gidx(j - 1) == 0; };
+    auto drop2 = [&](int j) { return BND && gidx(j - 1) == n - 2; };
+    eu_lane_stage<false, T, PI>(src, hl, hr, k, drop0, drop2, [&](int p, const Q3<T>& f) {
         Q3<T> nv = eu_apply(Q3<T>{base[0][p], base[1][p], base[2][p]}, f, c);
         if (BND) {  // ghost cells hold the Dirichlet states (Euler:407-416)
-            const int64_t g = gidx(p + 2);
+            const int64_t g = gidx(p);
             nv = g == 0 ? k.bl : nv;
             nv = g == n - 1 ? k.br : nv;
         }
         dst[0][p] = nv.x;
         dst[1][p] = nv.y;
         dst[2][p] = nv.z;
-        FL = FR;
-        DL = DR;
-    }
+    });
 }
 
 template <typename T, int PI, int S, bool BND>

@@ -21,6 +21,7 @@
 // per lane advance 48 steps for the same 11%.
 #pragma once
 
+#include "sw1d_euler.hpp"
 #include "sw1d_internal.hpp"
 #include "sw1d_lanes.hpp"
 
@@ -119,31 +120,11 @@ __device__ __forceinline__ void euler_stage(const T (&src)[3][P], T (&dst)[3][P]
                                             T (&hl)[3][2], T (&hr)[3][2], int c0, int cN, T c,
                                             const EulerCoef<T>& k)
 {
-    T ex[P + 4], ey[P + 4], ez[P + 4];
-    gather_carry<T, P, 2>(src[0], hl[0], hr[0], ex);
-    gather_carry<T, P, 2>(src[1], hl[1], hr[1], ey);
-    gather_carry<T, P, 2>(src[2], hl[2], hr[2], ez);
-    auto cell = [&](int j) { return Q3<T>{ex[j], ey[j], ez[j]}; };
-    T pd[P + 3];
-#pragma unroll
-    for (int j = 0; j < P + 3; ++j) pd[j] = eu_pdiff(cell(j), cell(j + 1));
-    // interface j lies between ext cells j+1 and j+2 (the lane's cell p is ext
-    // cell p+2); c0 / cN: the lane's p of cell 0 / n-1
-    auto iface = [&](int j, Q3<T>& F, Q3<T>& D) {
-        T q0 = pd[j], q2 = pd[j + 2];
-        if (ENDS) {
-            q0 = j - 1 == c0 ? T(0) : q0;
-            q2 = j == cN ? T(0) : q2;
-        }
-        eu_iface(cell(j), cell(j + 1), cell(j + 2), cell(j + 3), q0, pd[j + 1], q2, k, F, D);
-    };
-    Q3<T> FL, DL;
-    iface(0, FL, DL);
-#pragma unroll
-    for (int p = 0; p < P; ++p) {
-        Q3<T> FR, DR;
-        iface(p + 1, FR, DR);
-        Q3<T> nv = eu_apply(Q3<T>{base[0][p], base[1][p], base[2][p]}, eu_balance(FL, DL, FR, DR), c);
+    // c0 / cN: the lane's p of cell 0 / n-1
+    auto drop0 = [&](int j) { return ENDS && j - 1 == c0; };
+    auto drop2 = [&](int j) { return ENDS && j == cN; };
+    eu_lane_stage<false, T, P>(src, hl, hr, k, drop0, drop2, [&](int p, const Q3<T>& f) {
+        Q3<T> nv = eu_apply(Q3<T>{base[0][p], base[1][p], base[2][p]}, f, c);
         if (ENDS) {
             nv = p == c0 ? k.bl : nv;
             nv = p == cN ? k.br : nv;
@@ -151,9 +132,7 @@ __device__ __forceinline__ void euler_stage(const T (&src)[3][P], T (&dst)[3][P]
         dst[0][p] = nv.x;
         dst[1][p] = nv.y;
         dst[2][p] = nv.z;
-        FL = FR;
-        DL = DR;
-    }
+    });
 }
 
 template <typename T> struct Coef { T fo, fo2; KsCoef<T> ks; EulerCoef<T> eu; };
