@@ -403,7 +403,7 @@ hipError_t swept_prec(const SweptLaunch& L, const Coefs& c, hipStream_t s)
 }
 
 template <typename T>
-hipError_t classic_prec(int stage, int64_t n, void* buf, const Coefs& c, hipStream_t s)
+hipError_t stage_prec(int stage, int64_t n, void* buf, const Coefs& c, hipStream_t s)
 {
     T* b = static_cast<T*>(buf);
     const int64_t waves = (n + kWave - 2) / (kWave - 1);  // 63 cells per wave
@@ -422,9 +422,9 @@ hipError_t launch_swept_euler(const SweptLaunch& L, bool f64, const Coefs& c, hi
     return f64 ? swept_prec<double>(L, c, s) : swept_prec<float>(L, c, s);
 }
 
-hipError_t launch_classic_euler(bool f64, int stage, int64_t n, void* buf, const Coefs& c, hipStream_t s)
+hipError_t launch_stage_euler(bool f64, int stage, int64_t n, void* buf, const Coefs& c, hipStream_t s)
 {
-    return f64 ? classic_prec<double>(stage, n, buf, c, s) : classic_prec<float>(stage, n, buf, c, s);
+    return f64 ? stage_prec<double>(stage, n, buf, c, s) : stage_prec<float>(stage, n, buf, c, s);
 }
 
 }  // namespace sw1d

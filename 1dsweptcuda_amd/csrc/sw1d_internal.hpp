@@ -125,14 +125,15 @@ inline int64_t trapezoid_steps(int eq, int SB) { return eq == EQ_HEAT ? 32 * SB 
 hipError_t launch_wide(const WideLaunch& L, bool f64, const Coefs& c, hipStream_t s);
 WideChoice wide_choose(int eq, bool f64, int64_t n, int64_t nsteps, int cus);
 hipError_t launch_swept(const SweptLaunch& L, bool f64, const Coefs& c, hipStream_t s);
-// the Euler halves of launch_swept and launch_classic (sw1d_euler.hip)
+// its Euler half (sw1d_euler.hip)
 hipError_t launch_swept_euler(const SweptLaunch& L, bool f64, const Coefs& c, hipStream_t s);
-hipError_t launch_classic_euler(bool f64, int stage, int64_t n, void* buf, const Coefs& c, hipStream_t s);
-// One classic stage: heat (stage ignored), KS / Euler stage 0 = predictor,
-// 1 = corrector.  State layout as above; heat ping-pongs between in and out,
-// KS / Euler keep u and u_half in the same buffer.
-hipError_t launch_classic(int eq, int bc, bool f64, int stage, int64_t n, const void* in,
-                          void* out, const Coefs& c, hipStream_t s);
+// One classic time step from in to out (sw1d_step.hip)
+hipError_t launch_step(int eq, int bc, bool f64, int64_t n, int simds, const void* in, void* out, const Coefs& c,
+                       hipStream_t s);
+// One KS or Euler stage, 0 = predictor, 1 = corrector; the state and the
+// predicted values are the halves of buf.
+hipError_t launch_stage(int eq, bool f64, int stage, int64_t n, void* buf, const Coefs& c, hipStream_t s);
+hipError_t launch_stage_euler(bool f64, int stage, int64_t n, void* buf, const Coefs& c, hipStream_t s);
 // Checks the lane-shift primitive the swept kernels rely on; returns 1 if
 // every lane received its neighbour's value, 0 otherwise, <0 on HIP error.
 int check_lane_shifts();

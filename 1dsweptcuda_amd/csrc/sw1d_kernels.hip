@@ -29,8 +29,9 @@
 //   the domain ends (splitDiamond, Heat:335-408, Euler:666-746).  Boundary
 //   conditions are applied by global index wherever the boundary falls.
 //
-// Classic kernels — one thread per point, one launch per stage
-//   (classicHeat Heat:132-145, classicKS KS:189-207, classicEuler Euler:400-426).
+// Classic stages — one launch per Runge-Kutta stage (classicKS KS:189-207).
+//
+// Heat and KS; Euler's are in sw1d_euler.hip.
 
 #include "sw1d_nodes.hpp"
 
@@ -692,23 +693,8 @@ __global__ __launch_bounds__(kBlock) void k_ks_swept(const T* __restrict__ in,
 }
 
 // ------------------------------------------------------ classic kernels ---
-template <typename T, bool PERIODIC>
-__global__ __launch_bounds__(kClassicBlock) void k_heat_classic(const T* __restrict__ in,
-                                                                T* __restrict__ out, int64_t n,
-                                                                T fo, T fo2)
-{
-    const int64_t i = (int64_t)blockIdx.x * kClassicBlock + threadIdx.x;
-    if (i >= n) return;
-    int64_t l, r;
-    if (PERIODIC) {
-        l = i == 0 ? n - 1 : i - 1;
-        r = i == n - 1 ? 0 : i + 1;
-    } else {
-        l = i == 0 ? 1 : i - 1;
-        r = i == n - 1 ? n - 2 : i + 1;
-    }
-    out[i] = heat_ftcs(in[l], in[i], in[r], fo, fo2);
-}
+// The stages one by one, for per-kernel profiling (a step is one launch
+// otherwise: sw1d_step.hip).
 
 // One KS stage, one point per thread (any n).
 template <typename T, int STAGE>
@@ -857,34 +843,20 @@ hipError_t swept_prec(const SweptLaunch& L, const Coefs& c, hipStream_t s)
 }
 
 template <typename T>
-hipError_t classic_prec(int eq, int bc, int stage, int64_t n, const void* in, void* out,
-                        const Coefs& c, hipStream_t s)
+hipError_t ks_stage(int stage, int64_t n, void* buf, const Coefs& c, hipStream_t s)
 {
+    T* b = static_cast<T*>(buf);
     const dim3 grid((unsigned)((n + kClassicBlock - 1) / kClassicBlock));
-    if (eq == EQ_HEAT) {
-        const T* a = static_cast<const T*>(in);
-        T* b = static_cast<T*>(out);
-        if (bc == BC_PERIODIC)
-            hipLaunchKernelGGL((k_heat_classic<T, true>), grid, dim3(kClassicBlock), 0, s, a, b, n,
-                               fo_of<T>(c), fo2_of<T>(c));
+    const dim3 g2((unsigned)((n / 2 + kClassicBlock - 1) / kClassicBlock));
+    if (n % 2 != 0) {
+        if (stage == 0)
+            hipLaunchKernelGGL((k_ks_classic1<T, 0>), grid, dim3(kClassicBlock), 0, s, b, n, ks_of<T>(c));
         else
-            hipLaunchKernelGGL((k_heat_classic<T, false>), grid, dim3(kClassicBlock), 0, s, a, b, n,
-                               fo_of<T>(c), fo2_of<T>(c));
-    } else if (eq == EQ_KS) {
-        T* b = static_cast<T*>(out);
-        const dim3 g2((unsigned)((n / 2 + kClassicBlock - 1) / kClassicBlock));
-        if (n % 2 != 0) {
-            if (stage == 0)
-                hipLaunchKernelGGL((k_ks_classic1<T, 0>), grid, dim3(kClassicBlock), 0, s, b, n, ks_of<T>(c));
-            else
-                hipLaunchKernelGGL((k_ks_classic1<T, 1>), grid, dim3(kClassicBlock), 0, s, b, n, ks_of<T>(c));
-        } else if (stage == 0) {
-            hipLaunchKernelGGL((k_ks_classic<T, 0>), g2, dim3(kClassicBlock), 0, s, b, n, ks_of<T>(c));
-        } else {
-            hipLaunchKernelGGL((k_ks_classic<T, 1>), g2, dim3(kClassicBlock), 0, s, b, n, ks_of<T>(c));
-        }
+            hipLaunchKernelGGL((k_ks_classic1<T, 1>), grid, dim3(kClassicBlock), 0, s, b, n, ks_of<T>(c));
+    } else if (stage == 0) {
+        hipLaunchKernelGGL((k_ks_classic<T, 0>), g2, dim3(kClassicBlock), 0, s, b, n, ks_of<T>(c));
     } else {
-        return hipErrorInvalidValue;
+        hipLaunchKernelGGL((k_ks_classic<T, 1>), g2, dim3(kClassicBlock), 0, s, b, n, ks_of<T>(c));
     }
     return hipGetLastError();
 }
@@ -897,12 +869,11 @@ hipError_t launch_swept(const SweptLaunch& L, bool f64, const Coefs& c, hipStrea
     return f64 ? swept_prec<double>(L, c, s) : swept_prec<float>(L, c, s);
 }
 
-hipError_t launch_classic(int eq, int bc, bool f64, int stage, int64_t n, const void* in,
-                          void* out, const Coefs& c, hipStream_t s)
+hipError_t launch_stage(int eq, bool f64, int stage, int64_t n, void* buf, const Coefs& c, hipStream_t s)
 {
-    if (eq == EQ_EULER) return launch_classic_euler(f64, stage, n, out, c, s);
-    return f64 ? classic_prec<double>(eq, bc, stage, n, in, out, c, s)
-               : classic_prec<float>(eq, bc, stage, n, in, out, c, s);
+    if (eq == EQ_EULER) return launch_stage_euler(f64, stage, n, buf, c, s);
+    if (eq != EQ_KS) return hipErrorInvalidValue;
+    return f64 ? ks_stage<double>(stage, n, buf, c, s) : ks_stage<float>(stage, n, buf, c, s);
 }
 
 int check_lane_shifts_at(int* d)

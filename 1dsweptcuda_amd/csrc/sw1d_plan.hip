@@ -284,26 +284,29 @@ struct ProfScope {
 };
 
 // --------------------------------------------------------- GPU launches ---
+// A step is one launch; per-kernel profiling times the stages of KS and Euler
+// each on its own.
 int classic_step(sw1d_plan* p)
 {
-    if (p->eq == EQ_HEAT) {
-        ProfScope ps(p, KK_CLASSIC);
-        HIP_OR_FAIL(launch_classic(p->eq, p->bc, p->f64, 0, p->n, p->buf[p->cur],
-                                   p->buf[p->cur ^ 1], p->coef, p->stream));
-        p->cur ^= 1;
-    } else {
+    if (p->profiling && p->eq != EQ_HEAT) {
         for (int st = 0; st < 2; ++st) {
             ProfScope ps(p, KK_CLASSIC);
-            HIP_OR_FAIL(launch_classic(p->eq, p->bc, p->f64, st, p->n, p->buf[p->cur],
-                                       p->buf[p->cur], p->coef, p->stream));
+            HIP_OR_FAIL(launch_stage(p->eq, p->f64, st, p->n, p->buf[p->cur], p->coef, p->stream));
         }
+        return SW1D_OK;
     }
+    {
+        ProfScope ps(p, KK_CLASSIC);
+        HIP_OR_FAIL(launch_step(p->eq, p->bc, p->f64, p->n, p->simds, p->buf[p->cur], p->buf[p->cur ^ 1], p->coef,
+                                p->stream));
+    }
+    p->cur ^= 1;
     return SW1D_OK;
 }
 
 // Classic steps in blocks of kClassicGraphSteps replayed from a hipGraph (one
-// graph launch instead of 64-128 kernel launches; the kernels and their order
-// are the same, so the bits are the same).  Heat alternates its two buffers,
+// graph launch instead of 64 kernel launches; the kernels and their order
+// are the same, so the bits are the same).  The steps alternate the two buffers,
 // so a graph is kept per starting buffer; an even block returns to it.  With
 // per-kernel profiling on, or if capture fails, the steps are launched one by one.
 constexpr int64_t kClassicGraphSteps = 64;
@@ -870,12 +873,10 @@ int sw1d_plan_create(sw1d_plan** out, const sw1d_problem* q)
     }
     if (!launch_graphs_enabled()) p->classic_graph_failed = p->tile_graph_failed = true;
     p->simds = device_simds();
-    if (p->alg != SW1D_CLASSIC) {
-        if (g_lane_check == 0) sw1d_device_check();
-        if (g_lane_check != 1) {
-            delete p;
-            return fail(SW1D_EDEVICE, "DPP lane-shift self check failed on this device");
-        }
+    if (g_lane_check == 0) sw1d_device_check();
+    if (g_lane_check != 1) {
+        delete p;
+        return fail(SW1D_EDEVICE, "DPP lane-shift self check failed on this device");
     }
 
     hipError_t e = hipStreamCreateWithFlags(&p->stream, hipStreamNonBlocking);
@@ -1033,7 +1034,7 @@ int sw1d_advance_noalloc(const sw1d_problem* q, void* d_state, int64_t nsteps, v
         rc = noalloc_device_init(dev, &ws);
         if (rc) return rc;
     }
-    if (p.alg != SW1D_CLASSIC && g_lane_check != 1)
+    if (g_lane_check != 1)
         return fail(SW1D_EDEVICE, "DPP lane-shift self check failed on this device");
     p.buf[0] = ws;
     p.buf[1] = static_cast<unsigned char*>(ws) + half;

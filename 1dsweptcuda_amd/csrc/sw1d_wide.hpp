@@ -126,8 +126,9 @@ __device__ __forceinline__ void euler_stage(const T (&src)[3][P], T (&dst)[3][P]
     eu_lane_stage<false, T, P>(src, hl, hr, k, drop0, drop2, [&](int p, const Q3<T>& f) {
         Q3<T> nv = eu_apply(Q3<T>{base[0][p], base[1][p], base[2][p]}, f, c);
         if (ENDS) {
-            nv = p == c0 ? k.bl : nv;
-            nv = p == cN ? k.br : nv;
+            const bool l = p == c0, r = p == cN;
+            nv = Q3<T>{l ? k.bl.x : nv.x, l ? k.bl.y : nv.y, l ? k.bl.z : nv.z};
+            nv = Q3<T>{r ? k.br.x : nv.x, r ? k.br.y : nv.y, r ? k.br.z : nv.z};
         }
         dst[0][p] = nv.x;
         dst[1][p] = nv.y;
