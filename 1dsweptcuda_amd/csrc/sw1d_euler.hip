@@ -340,7 +340,7 @@ __global__ __launch_bounds__(kClassicBlock) void k_euler_classic(T* __restrict__
     const T q1 = eu_pdiff(B, C);
     const T q2 = x == n - 2 ? T(0) : eu_pdiff(C, Dc);
     Q3<T> FL, DL;
-    eu_iface(A, B, C, Dc, q0, q1, q2, k, FL, DL);
+    eu_iface<Ieee<T>>(A, B, C, Dc, q0, q1, q2, k, FL, DL);
     // every lane takes part in the shifts before any leaves
     const Q3<T> FR{from_right(FL.x, FL.x), from_right(FL.y, FL.y), from_right(FL.z, FL.z)};
     const Q3<T> DR{from_right(DL.x, DL.x), from_right(DL.y, DL.y), from_right(DL.z, DL.z)};

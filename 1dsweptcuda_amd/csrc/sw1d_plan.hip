@@ -413,7 +413,7 @@ void cpu_node_diamond(sw1d_plan* p, T* win)
                 const T q0 = x == xg0 ? T(0) : eu_pdiff(cell(x - 1), cell(x));
                 const T q1 = eu_pdiff(cell(x), cell(x + 1));
                 const T q2 = x == xgN - 1 ? T(0) : eu_pdiff(cell(x + 1), cell(x + 2));
-                eu_iface(cell(x - 1), cell(x), cell(x + 1), cell(x + 2), q0, q1, q2, k, F[x - lo + 1],
+                eu_iface<Ieee<T>>(cell(x - 1), cell(x), cell(x + 1), cell(x + 2), q0, q1, q2, k, F[x - lo + 1],
                          D[x - lo + 1]);
             }
             const T c = st == 0 ? T(0.25) * k.dtdx : T(0.5) * k.dtdx;

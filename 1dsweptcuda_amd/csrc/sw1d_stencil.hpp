@@ -89,12 +89,15 @@ template <typename T> struct Q3 { T x, y, z; };
 
 template <typename T> struct EulerCoef { T gam, mgam, dtdx; Q3<T> bl, br; };
 
-// Euler1D_SweptShared.cu:183-193 (pressure).
-template <typename T>
-SW1D_HD T eu_pressure(const Q3<T>& c, T mgam)
-{
-    return mgam * (c.z - (T(0.5) * c.y * c.y / c.x));
-}
+// The divisions and square roots of a flux.  A divisor is prepared once (over)
+// for all that is divided by it.  Here the operators; sw1d_euler.hpp has the
+// same values in fewer instructions for regular operands.
+template <typename T> struct Ieee {
+    static SW1D_HD T over(T b) { return b; }
+    static SW1D_HD T div(T a, T b) { return a / b; }
+    static SW1D_HD T quot(T a, T b) { return a / b; }  // a is not a negative zero
+    static SW1D_HD T root(T x) { return sqrt(x); }     // of a density
+};
 
 // Euler:222-228 (limitor): cur + 1/2*min(ratio,1)*(other-cur).
 template <typename T>
@@ -105,24 +108,27 @@ SW1D_HD Q3<T> eu_limit(const Q3<T>& cur, const Q3<T>& oth, T ratio)
                  cur.z + m * (oth.z - cur.z)};
 }
 
-// Euler:237-257 (eulerFlux): F(L)+F(R) without the factor 1/2, and
-// Euler:266-292 (eulerSpectral): Roe-averaged (sqrt(gam*p/rho)+|u|)*(L-R).
-template <typename T>
+// Euler:237-257 (eulerFlux): F(L)+F(R) without the factor 1/2, the pressures as
+// Euler:183-193, and Euler:266-292 (eulerSpectral): Roe-averaged
+// (sqrt(gam*p/rho)+|u|)*(L-R).
+template <class M, typename T>
 SW1D_HD void eu_flux_diss(const Q3<T>& L, const Q3<T>& R, const EulerCoef<T>& k,
                           Q3<T>& F, Q3<T>& D)
 {
-    const T uL = L.y / L.x;
-    const T uR = R.y / R.x;
-    const T pL = eu_pressure(L, k.mgam);
-    const T pR = eu_pressure(R, k.mgam);
+    const auto oL = M::over(L.x);
+    const auto oR = M::over(R.x);
+    const T uL = M::div(L.y, oL);
+    const T uR = M::div(R.y, oR);
+    const T pL = k.mgam * (L.z - M::quot(T(0.5) * L.y * L.y, oL));
+    const T pR = k.mgam * (R.z - M::quot(T(0.5) * R.y * R.y, oR));
     F.x = (L.y + R.y);
     F.y = (L.y * uL + R.y * uR + pL + pR);
     F.z = (L.z * uL + R.z * uR + uL * pL + uR * pR);
 
-    const T sl = sqrt(L.x);
-    const T sr = sqrt(R.x);
+    const T sl = M::root(L.x);
+    const T sr = M::root(R.x);
     const T hx = sl * sr;
-    const T den = T(1) / (hx * (sl + sr));
+    const T den = M::quot(T(1), M::over(hx * (sl + sr)));
     const T hy = (sl * R.y + sr * L.y) * den;
     const T hz = (sl * R.z + sr * L.z) * den;
     const T ph = k.mgam * (hz - T(0.5) * hy * hy);  // Euler:202-212 (pressureHalf)
@@ -144,7 +150,7 @@ SW1D_HD T eu_pdiff(const Q3<T>& a, const Q3<T>& b)
 // and the flux / dissipation of Euler:326-332 (left interface of a cell) and
 // Euler:336-341 (right interface): the right interface of cell i and the left
 // interface of cell i+1 are the same expressions on the same operands.
-template <typename T>
+template <class M, typename T>
 SW1D_HD void eu_iface(const Q3<T>& A, const Q3<T>& B, const Q3<T>& C, const Q3<T>& Dc, T q0,
                       T q1, T q2, const EulerCoef<T>& k, Q3<T>& F, Q3<T>& D)
 {
@@ -152,7 +158,7 @@ SW1D_HD void eu_iface(const Q3<T>& A, const Q3<T>& B, const Q3<T>& C, const Q3<T
                    : eu_limit(B, C, (A.x * q1 / (C.x * q0)));
     const Q3<T> tR = (!q1 || !q2 || ((q1 < 0) != (q2 < 0))) ? C
                    : eu_limit(C, B, (Dc.x * q1 / (B.x * q2)));
-    eu_flux_diss(tL, tR, k, F, D);
+    eu_flux_diss<M>(tL, tR, k, F, D);
 }
 
 // Cell balance in the reference's accumulation order (Euler:331-341):
@@ -179,8 +185,8 @@ SW1D_HD Q3<T> eu_net_flux(const Q3<T>& s0, const Q3<T>& s1, const Q3<T>& s2,
     const T pR = eu_pdiff(s2, s3);
     const T pRR = flagR ? T(0) : eu_pdiff(s3, s4);
     Q3<T> FL, DL, FR, DR;
-    eu_iface(s0, s1, s2, s3, pLL, pL, pR, k, FL, DL);
-    eu_iface(s1, s2, s3, s4, pL, pR, pRR, k, FR, DR);
+    eu_iface<Ieee<T>>(s0, s1, s2, s3, pLL, pL, pR, k, FL, DL);
+    eu_iface<Ieee<T>>(s1, s2, s3, s4, pL, pR, pRR, k, FR, DR);
     return eu_balance(FL, DL, FR, DR);
 }
 
