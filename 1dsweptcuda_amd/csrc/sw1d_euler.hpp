@@ -1,5 +1,5 @@
 // One Euler stage over a wave whose lane l holds P consecutive cells, shared by
-// the swept, trapezoid and wide tiles and the classic step.
+// the swept rows, the wide tiles and the classic step.
 //
 // A cell's update needs the fluxes at both its interfaces, an interface is
 // some 300 instructions (seven divisions, three square roots), and two cells

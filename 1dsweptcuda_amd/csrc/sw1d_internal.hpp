@@ -45,18 +45,8 @@ struct Coefs {
     EulerCoef<double> eu_d; EulerCoef<float> eu_f;
 };
 
-// One trapezoid launch (Euler): tile t stores the cells [t*W_out, t*W_out +
-// W_out) (the last tile clipped at nX) after 16 stages, W_out = 64*PO, from a
-// window of 64*(PO+SB) cells, SB = 1.
-struct TrapLaunch {
-    int eq, bc, PO, SB;
-    int64_t n, ntiles, tile_first;
-    const void* in;
-    void* out;
-};
-
 // One launch of workgroup-wide overlapped tiles (sw1d_wide.hip): `steps` whole
-// time steps of a heat or KS field, plain values in and out.
+// time steps, plain values in and out.
 struct WideLaunch {
     int eq, bc, shape, steps;
     int64_t n;
@@ -114,13 +104,17 @@ struct BatchView {
 };
 bool batch_view(sw1d_batch* b, BatchView& v);
 
-// Launchers (sw1d_kernels.hip, sw1d_trapezoid.hip, sw1d_batch.hip).  All
+// Launchers (sw1d_kernels.hip, sw1d_wide.hip, sw1d_step.hip, sw1d_batch.hip).  All
 // return a hipError_t.
 hipError_t launch_batch(const BatchLaunch& L, bool f64, hipStream_t s);
 inline bool batch_waves_supported(int w) { return w == 2 || w == 4 || w == 8; }
 inline bool batch_tile_supported(int po) { return po == 2 || po == 4 || po == 8 || po == 16; }
-hipError_t launch_trapezoid(const TrapLaunch& L, bool f64, const Coefs& c, hipStream_t s);
-bool trapezoid_supported(int eq, int PO, int SB);
+// Tile widths (64 PO points) and depths of SW1D_TRAPEZOID plans.
+inline bool trapezoid_supported(int eq, int PO, int SB)
+{
+    if (eq == EQ_EULER) return SB == 1 && (PO == 2 || PO == 4);
+    return (SB == 1 && (PO == 2 || PO == 4 || PO == 8 || PO == 16)) || (SB == 2 && (PO == 8 || PO == 16));
+}
 inline int64_t trapezoid_steps(int eq, int SB) { return eq == EQ_HEAT ? 32 * SB : 8 * SB; }
 hipError_t launch_wide(const WideLaunch& L, bool f64, const Coefs& c, hipStream_t s);
 WideChoice wide_choose(int eq, bool f64, int64_t n, int64_t nsteps, int cus);

@@ -54,7 +54,6 @@ struct sw1d_plan {
     size_t S = 8;      // sizeof(REAL)
     int nc = 1;        // values per point
     int W = 0, P = 0;  // swept node width, points per lane (0: no swept path)
-    int SB = 0;        // trapezoid: extra points per lane (stages per launch / (32/R))
     int R = 1;         // stage radius
     int64_t tile_steps = 0;  // steps advanced by one swept tile launch
     int simds = 0;           // SIMDs of the plan's device (4 per compute unit)
@@ -71,10 +70,6 @@ struct sw1d_plan {
     // classic algorithm: a hipGraph of kClassicGraphSteps steps per starting buffer
     hipGraphExec_t classic_exec[2]{nullptr, nullptr};
     bool classic_graph_failed = false;
-    // trapezoid launches: a hipGraph of kTileGraphLaunches launches per
-    // starting buffer
-    hipGraphExec_t tile_exec[2]{nullptr, nullptr};
-    bool tile_graph_failed = false;
 
     // hybrid resources
     hipStream_t copy_stream = nullptr;
@@ -484,47 +479,7 @@ int hybrid_split_diamond(sw1d_plan* p)
     return SW1D_OK;
 }
 
-// Trapezoid launches (Euler) in blocks of kTileGraphLaunches replayed from a
-// hipGraph: one graph launch instead of 16 kernel launches.  Small plans
-// (launches of a few microseconds, many plans at once on their own streams) are
-// otherwise bound by the host's launch rate.
-// A block is an even number of launches, so it returns to its starting
-// buffer; a graph is kept per starting buffer and both are captured together,
-// so a later call never captures.  The kernels and their order are those of
-// the launches one by one, so the bits are the same.  With per-kernel
-// profiling on, or if capture fails, the launches go one by one.
-// issue_block launches one block (flipping p->cur).
-constexpr int64_t kTileGraphLaunches = 16;
-
-template <typename F>
-int tile_graph_blocks(sw1d_plan* p, int64_t& launches, F&& issue_block)
-{
-    if (p->profiling || p->tile_graph_failed || launches < kTileGraphLaunches) return SW1D_OK;
-    for (int slot = 0; slot < 2 && !p->tile_graph_failed; ++slot) {
-        if (p->tile_exec[slot]) continue;
-        const int keep = p->cur;
-        p->cur = slot;
-        hipGraph_t g = nullptr;
-        hipError_t e = hipStreamBeginCapture(p->stream, hipStreamCaptureModeThreadLocal);
-        const int rc = e == hipSuccess ? issue_block() : SW1D_OK;
-        const hipError_t e2 = e == hipSuccess ? hipStreamEndCapture(p->stream, &g) : e;
-        if (rc == SW1D_OK && e2 == hipSuccess && g)
-            e = hipGraphInstantiate(&p->tile_exec[slot], g, nullptr, nullptr, 0);
-        if (g) (void)hipGraphDestroy(g);
-        p->cur = keep;  // capture launched nothing
-        if (rc != SW1D_OK || e2 != hipSuccess || e != hipSuccess) {
-            p->tile_exec[slot] = nullptr;
-            p->tile_graph_failed = true;
-            (void)hipGetLastError();
-        }
-    }
-    if (p->tile_graph_failed) return SW1D_OK;
-    for (; launches >= kTileGraphLaunches; launches -= kTileGraphLaunches)
-        HIP_OR_FAIL(hipGraphLaunch(p->tile_exec[p->cur], p->stream));
-    return SW1D_OK;
-}
-
-// nsteps steps of a heat or KS field as workgroup-wide overlapped tiles: any
+// nsteps steps as workgroup-wide overlapped tiles: any
 // number of steps, no remainder.
 int wide_advance(sw1d_plan* p, int64_t nsteps)
 {
@@ -552,15 +507,14 @@ int wide_advance(sw1d_plan* p, int64_t nsteps)
     return SW1D_OK;
 }
 
-// Whether an advance of a swept plan runs as wide tiles.  The swept rows, one
-// launch each, are kept for Euler (2^20, FP64: 4.4e10 point-updates/s against
-// 3.7e10, wide lanes of Euler cells do not fit the registers), the hybrid,
-// FP32 KS on large fields, and per-kernel profiling, which times the swept
-// kinds.
+// Whether an advance of a swept plan runs as wide tiles (both sides' rates for
+// each equation: sw1d_wide.hip).  The swept rows, one launch each, are kept for
+// the hybrid, FP32 KS on large fields, and per-kernel profiling, which times the
+// swept kinds.
 bool takes_wide(const sw1d_plan* p)
 {
-    if (p->eq == EQ_EULER || p->profiling) return false;
-    if (p->eq == EQ_HEAT) return p->alg == SW1D_SWEPT;
+    if (p->profiling) return false;
+    if (p->eq != EQ_KS) return p->alg == SW1D_SWEPT;
     // FP32 KS with two waves per SIMD of 512 points or more: the diamonds (2^20,
     // 1000 steps: 790 us at W = 512 against 913 us; W = 256 949 us)
     const int64_t nodes = p->n / p->W;
@@ -596,53 +550,10 @@ int swept_advance(sw1d_plan* p, int64_t nsteps)
         if (rc) return rc;
         p->cur ^= 1;
     }
-    // fewer steps than a tile's: classic steps (Euler, profiling), else one wide
-    // launch instead of one or two launches per step
-    if (p->eq != EQ_EULER && !p->profiling) return wide_advance(p, rem);
+    // fewer steps than a tile's: one wide launch instead of one per step (two
+    // when each is timed)
+    if (!p->profiling) return wide_advance(p, rem);
     for (int64_t s = 0; s < rem; ++s) {
-        int rc = classic_step(p);
-        if (rc) return rc;
-    }
-    return SW1D_OK;
-}
-
-int trapezoid_advance(sw1d_plan* p, int64_t nsteps)
-{
-    if (p->eq != EQ_EULER) return wide_advance(p, nsteps);
-    const int64_t H = p->tile_steps;
-    const int64_t launches = nsteps / H;
-    TrapLaunch L;
-    L.eq = p->eq;
-    L.bc = p->bc;
-    L.PO = p->P;
-    L.SB = p->SB;
-    L.n = p->n;
-    L.ntiles = (p->n + p->W - 1) / p->W;
-    L.tile_first = 0;
-    auto one = [p, &L]() -> int {
-        L.in = p->buf[p->cur];
-        L.out = p->buf[p->cur ^ 1];
-        {
-            ProfScope ps(p, KK_DIAMOND);
-            HIP_OR_FAIL(launch_trapezoid(L, p->f64, p->coef, p->stream));
-        }
-        p->cur ^= 1;
-        return SW1D_OK;
-    };
-    int64_t left = launches;
-    int rc = tile_graph_blocks(p, left, [&one] {
-        for (int64_t j = 0; j < kTileGraphLaunches; ++j) {
-            const int r = one();
-            if (r) return r;
-        }
-        return (int)SW1D_OK;
-    });
-    if (rc) return rc;
-    for (int64_t i = 0; i < left; ++i) {
-        rc = one();
-        if (rc) return rc;
-    }
-    for (int64_t s = launches * H; s < nsteps; ++s) {
         int rc = classic_step(p);
         if (rc) return rc;
     }
@@ -665,8 +576,6 @@ void release(sw1d_plan* p)
     if (p->ev_out) (void)hipEventDestroy(p->ev_out);
     if (p->copy_stream) (void)hipStreamDestroy(p->copy_stream);
     for (auto x : p->classic_exec)
-        if (x) (void)hipGraphExecDestroy(x);
-    for (auto x : p->tile_exec)
         if (x) (void)hipGraphExecDestroy(x);
     if (p->stream) (void)hipStreamDestroy(p->stream);
     delete p;
@@ -782,7 +691,6 @@ int plan_setup(sw1d_plan* p, const sw1d_problem* q)
         }
         p->W = W;
         p->P = W / 64;
-        p->SB = SB;
         p->tile_steps = trapezoid_steps(p->eq, SB);
     } else if (p->alg != SW1D_CLASSIC) {
         int W = q->node_width > 0 ? q->node_width : tpb;
@@ -871,7 +779,7 @@ int sw1d_plan_create(sw1d_plan** out, const sw1d_problem* q)
         delete p;
         return rc;
     }
-    if (!launch_graphs_enabled()) p->classic_graph_failed = p->tile_graph_failed = true;
+    if (!launch_graphs_enabled()) p->classic_graph_failed = true;
     p->simds = device_simds();
     if (g_lane_check == 0) sw1d_device_check();
     if (g_lane_check != 1) {
@@ -994,7 +902,7 @@ int sw1d_advance(sw1d_plan* p, int64_t nsteps)
     if (p->alg == SW1D_CLASSIC) {
         rc = classic_advance(p, nsteps);
     } else if (p->alg == SW1D_TRAPEZOID) {
-        rc = trapezoid_advance(p, nsteps);
+        rc = wide_advance(p, nsteps);
     } else {
         rc = swept_advance(p, nsteps);
     }
@@ -1042,7 +950,6 @@ int sw1d_advance_noalloc(const sw1d_problem* q, void* d_state, int64_t nsteps, v
     p.simds = device_simds();
     // launches one by one: no launch graph is captured or instantiated
     p.classic_graph_failed = true;
-    p.tile_graph_failed = true;
     rc = copy_state(&p, d_state, nullptr, true, hipMemcpyDeviceToDevice, false);
     if (rc == SW1D_OK) rc = sw1d_advance(&p, nsteps);
     if (rc == SW1D_OK) rc = copy_state(&p, nullptr, d_state, false, hipMemcpyDeviceToDevice, false);

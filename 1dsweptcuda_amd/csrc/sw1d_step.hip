@@ -24,34 +24,6 @@ constexpr int kStepBlock = 256;
 // halo lanes on each side: one step's reach
 template <int EQ, int P> constexpr int kHalo = ((EQ == EQ_HEAT ? 1 : 4) + P - 1) / P;
 
-// P values at any element alignment, in 16-byte accesses where P allows them
-// (a component starts at a multiple of n, which may be odd)
-template <typename T, int P>
-__device__ __forceinline__ void load_pts(const T* a, T (&v)[P])
-{
-    constexpr int V = P * sizeof(T) < 16 ? P : 16 / sizeof(T);
-    typedef T vec __attribute__((ext_vector_type(V), aligned(sizeof(T))));
-#pragma unroll
-    for (int p = 0; p < P; p += V) {
-        const vec t = *reinterpret_cast<const vec*>(a + p);
-#pragma unroll
-        for (int q = 0; q < V; ++q) v[p + q] = t[q];
-    }
-}
-template <typename T, int P>
-__device__ __forceinline__ void store_pts(T* a, const T (&v)[P])
-{
-    constexpr int V = P * sizeof(T) < 16 ? P : 16 / sizeof(T);
-    typedef T vec __attribute__((ext_vector_type(V), aligned(sizeof(T))));
-#pragma unroll
-    for (int p = 0; p < P; p += V) {
-        vec t;
-#pragma unroll
-        for (int q = 0; q < V; ++q) t[q] = v[p + q];
-        *reinterpret_cast<vec*>(a + p) = t;
-    }
-}
-
 template <typename T, int EQ, int P>
 __global__ __launch_bounds__(kStepBlock) void k_step(const T* __restrict__ in, T* __restrict__ out, int64_t n,
                                                      int ends, Coef<T> k)

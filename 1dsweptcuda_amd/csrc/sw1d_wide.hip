@@ -1,5 +1,4 @@
-// Workgroup-wide overlapped tiles (sw1d_wide.hpp) for single heat and KS plans:
-// the kernels, and the choice of a tile shape and of the steps per launch.
+// Workgroup-wide overlapped tiles (sw1d_wide.hpp) for single plans: the kernels, and the choice of a tile shape and of the steps per launch.
 //
 // An advance of N steps is L launches of N/L steps each (any N: no remainder
 // steps), ping-ponging between the plan's two state buffers.  More steps per
@@ -18,11 +17,19 @@
 //          5.10e9    7.9e10    2.28e11   6.4e11    1.08e12   1.18e12   wide
 //   heat   1.02e10   1.58e11   6.2e11    2.23e12   4.95e12   5.1e12    diamonds
 //          2.18e10   3.35e11   1.14e12   3.4e12    7.1e12    8.5e12    wide
+//   Euler  3.5e8     5.5e9     2.1e10    4.3e10    5.5e10    5.8e10    diamonds
+//          7.0e8     1.13e10   2.8e10    4.6e10    5.9e10    6.1e10    wide
+// (Euler before, one wave per tile: 1.3e8, 2.1e9, 8.3e9, 2.3e10, 3.1e10, 3.2e10
+// as trapezoids.)
 // At 2^20 a KS launch of 64 steps takes 62 us: 53 us of FP64 issue at 4.04
 // cycles per instruction (12.7% of it the window's overlap, 6.7% the halo
 // lanes), 3% exchanges, the rest the launch.  FP32 KS at 2^19 and more is the
 // one case the diamonds win (1.32e12 against 1.14e12 at 2^20): FP32
 // instructions of two waves co-issue, and the diamonds evaluate fewer points.
+// An Euler cell's step is some 550 FP64 instructions; at 2^20 a launch of 13
+// steps of 4 cells per lane issues for four fifths of its 232 us, a quarter of
+// it for the overlap and the halo lanes (its 234 registers allow two waves per
+// SIMD, its steps six of the window's 928 cells each).
 
 #include <cmath>
 
@@ -61,20 +68,24 @@ hipError_t launch_prec(const WideLaunch& L, const Coefs& c, hipStream_t s)
 {
     Coef<T> k{};
     if constexpr (sizeof(T) == 8) {
-        k.fo = c.fo_d; k.fo2 = c.fo2_d; k.ks = c.ks_d;
+        k.fo = c.fo_d; k.fo2 = c.fo2_d; k.ks = c.ks_d; k.eu = c.eu_d;
     } else {
-        k.fo = c.fo_f; k.fo2 = c.fo2_f; k.ks = c.ks_f;
+        k.fo = c.fo_f; k.fo2 = c.fo2_f; k.ks = c.ks_f; k.eu = c.eu_f;
     }
     const int win = window(entries(L.eq)[L.shape]);
     const int64_t most = win - 2 * (int64_t)reach(L.eq) * L.steps;  // points a tile can store
     if (most < 1) return hipErrorInvalidValue;
     const int64_t tiles = (L.n + most - 1) / most, wout = (L.n + tiles - 1) / tiles;
     const dim3 grid((unsigned)((L.n + wout - 1) / wout));
-    const int ends = L.bc == BC_MIRROR ? ENDS_MIRROR : ENDS_PERIODIC;
+    const int ends = L.bc == BC_MIRROR ? ENDS_MIRROR : L.bc == BC_DIRICHLET ? ENDS_FIXED : ENDS_PERIODIC;
     const T* in = static_cast<const T*>(L.in);
     T* out = static_cast<T*>(L.out);
-    return L.eq == EQ_HEAT ? launch_shape<T, EQ_HEAT>(L.shape, grid, in, out, L.n, wout, L.steps, ends, k, s)
-                           : launch_shape<T, EQ_KS>(L.shape, grid, in, out, L.n, wout, L.steps, ends, k, s);
+    switch (L.eq) {
+    case EQ_HEAT: return launch_shape<T, EQ_HEAT>(L.shape, grid, in, out, L.n, wout, L.steps, ends, k, s);
+    case EQ_KS: return launch_shape<T, EQ_KS>(L.shape, grid, in, out, L.n, wout, L.steps, ends, k, s);
+    case EQ_EULER: return launch_shape<T, EQ_EULER>(L.shape, grid, in, out, L.n, wout, L.steps, ends, k, s);
+    }
+    return hipErrorInvalidValue;
 }
 
 }  // namespace

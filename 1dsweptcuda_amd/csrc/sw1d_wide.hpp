@@ -13,6 +13,8 @@
 // lanes go stale from the outside, and every K = HL P / R steps a wave takes
 // its neighbours' values for them through LDS: a wave repeats 2 HL / 64 of its
 // neighbours' work, and the workgroup repeats 2 R S / WIN of its neighbours'.
+// An Euler wave updates cells of three values, and the waves that hold cell 0
+// or n-1 run a variant with the Dirichlet ends' checks.
 //
 // Why a workgroup: the redundant share falls with the width of whatever
 // shares its halo.  A wave alone (64 x 18 points) that advances KS by 16 steps
@@ -44,7 +46,10 @@ struct Shape {
     // LDS, in values: one component's window image, or the exchanged edges (two
     // sets used in turn, so one barrier per exchange is enough)
     static constexpr int EDGE = NW * 2 * HL * NC * P;
-    static constexpr bool DIRECT = P <= 2;  // lanes read and write the field themselves
+    // lanes read and write the field themselves, where one component's image
+    // after the other through LDS takes longer (Euler, 4 cells per lane: 8.6 us
+    // for launch, load and store against 4.0)
+    static constexpr bool DIRECT = P <= 2 || EQ == EQ_EULER;
     static constexpr int LDS = (!DIRECT && WIN > 2 * EDGE) ? WIN : 2 * EDGE;
 };
 
@@ -109,6 +114,34 @@ __device__ __forceinline__ void take(const T* d, T (&v)[P])
     } else {
 #pragma unroll
         for (int p = 0; p < P; ++p) v[p] = d[p];
+    }
+}
+
+// P values at any element alignment, in 16-byte accesses where P allows them
+// (a component starts at a multiple of n, which may be odd)
+template <typename T, int P>
+__device__ __forceinline__ void load_pts(const T* a, T (&v)[P])
+{
+    constexpr int V = P % (16 / sizeof(T)) == 0 ? 16 / sizeof(T) : (P % 2 == 0 ? 2 : 1);
+    typedef T vec __attribute__((ext_vector_type(V), aligned(sizeof(T))));
+#pragma unroll
+    for (int p = 0; p < P; p += V) {
+        const vec t = *reinterpret_cast<const vec*>(a + p);
+#pragma unroll
+        for (int q = 0; q < V; ++q) v[p + q] = t[q];
+    }
+}
+template <typename T, int P>
+__device__ __forceinline__ void store_pts(T* a, const T (&v)[P])
+{
+    constexpr int V = P % (16 / sizeof(T)) == 0 ? 16 / sizeof(T) : (P % 2 == 0 ? 2 : 1);
+    typedef T vec __attribute__((ext_vector_type(V), aligned(sizeof(T))));
+#pragma unroll
+    for (int p = 0; p < P; p += V) {
+        vec t;
+#pragma unroll
+        for (int q = 0; q < V; ++q) t[q] = v[p + q];
+        *reinterpret_cast<vec*>(a + p) = t;
     }
 }
 
@@ -218,9 +251,7 @@ __device__ __forceinline__ void tile(T* lds, const T* __restrict__ in, T* __rest
     if constexpr (S::DIRECT) {
         if (inside) {
 #pragma unroll
-            for (int c = 0; c < NC; ++c)
-#pragma unroll
-                for (int p = 0; p < P; ++p) st.v[c][p] = in[c * cs + win + x0 + p];
+            for (int c = 0; c < NC; ++c) load_pts<T, P>(in + c * cs + win + x0, st.v[c]);
         } else {
 #pragma unroll
             for (int p = 0; p < P; ++p) {
@@ -303,13 +334,16 @@ __device__ __forceinline__ void tile(T* lds, const T* __restrict__ in, T* __rest
 
     const bool own = (lane >= HL || w == 0) && (lane < kWave - HL || w == NW - 1);
     if constexpr (S::DIRECT) {
-        if (own) {
+        const int i0 = x0 - halo;
+        if (own && i0 >= 0 && i0 + P <= count) {
+#pragma unroll
+            for (int c = 0; c < NC; ++c) store_pts<T, P>(out + c * cs + out0 + i0, st.v[c]);
+        } else if (own) {
 #pragma unroll
             for (int p = 0; p < P; ++p) {
-                const int i = x0 + p - halo;
-                if (i >= 0 && i < count) {
+                if (i0 + p >= 0 && i0 + p < count) {
 #pragma unroll
-                    for (int c = 0; c < NC; ++c) out[c * cs + out0 + i] = st.v[c][p];
+                    for (int c = 0; c < NC; ++c) out[c * cs + out0 + i0 + p] = st.v[c][p];
                 }
             }
         }
@@ -344,7 +378,8 @@ struct Cost { float t0, t2, c1, c2; };
 struct Entry { int P, HL; Cost f64, f32; };
 
 inline constexpr int kWaves = 4;  // one wave per SIMD: P sets the window
-// Halo lanes: an exchange every HL P / R steps, 5-9 for KS and 16-42 for heat
+// Halo lanes: an exchange every HL P / R steps, 5-9 for KS, 16-42 for heat and 2-5
+// for Euler, whose steps are ten times as long
 inline constexpr Entry kKs[] = {
     {2, 10, {2.3f, .06f, .151f, .101f}, {2.1f, .02f, .143f, .085f}},
     {4, 6, {3.0f, .6f, .248f, .173f}, {2.8f, .35f, .224f, .153f}},
@@ -370,6 +405,17 @@ inline constexpr Entry kHeat[] = {
     {21, 2, {7.4f, .9f, .1305f, .1066f}, {6.2f, .25f, .1226f, .0892f}},
 };
 
+inline constexpr Entry kEuler[] = {
+    {1, 16, {2.2f, .0f, 1.29f, .85f}, {2.0f, .1f, 1.09f, .56f}},
+    {1, 8, {1.75f, .4f, 1.37f, .82f}, {1.8f, .2f, 1.16f, .56f}},
+    {2, 8, {2.3f, .9f, 2.30f, 1.60f}, {2.1f, .15f, 2.00f, 1.13f}},
+    {2, 4, {2.7f, .9f, 2.35f, 1.58f}, {2.4f, .3f, 2.08f, 1.12f}},
+    {3, 4, {4.3f, 1.6f, 3.34f, 2.41f}, {2.7f, .9f, 2.87f, 1.68f}},
+    {4, 4, {5.5f, 2.2f, 4.35f, 3.10f}, {3.7f, .9f, 3.78f, 2.25f}},
+    {5, 4, {9.4f, 2.5f, 5.27f, 5.15f}, {4.2f, 1.5f, 4.64f, 2.82f}},
+    {6, 2, {8.3f, 4.0f, 6.63f, 6.20f}, {3.5f, 2.0f, 5.65f, 3.20f}},
+};
+
 inline int reach(int eq) { return eq == EQ_HEAT ? 1 : 4; }
 inline int window(const Entry& e) { return kWaves * (kWave - 2 * e.HL) * e.P + 2 * e.HL * e.P; }
 
@@ -382,9 +428,16 @@ template <> struct Table<EQ_KS> {
     static constexpr const Entry* e = kKs;
     static constexpr int count = sizeof(kKs) / sizeof(Entry);
 };
+template <> struct Table<EQ_EULER> {
+    static constexpr const Entry* e = kEuler;
+    static constexpr int count = sizeof(kEuler) / sizeof(Entry);
+};
 template <int EQ, int I> using TableShape = Shape<EQ, Table<EQ>::e[I].P, kWaves, Table<EQ>::e[I].HL>;
-inline const Entry* entries(int eq) { return eq == EQ_HEAT ? kHeat : kKs; }
-inline int shapes(int eq) { return eq == EQ_HEAT ? Table<EQ_HEAT>::count : Table<EQ_KS>::count; }
+inline const Entry* entries(int eq) { return eq == EQ_HEAT ? kHeat : eq == EQ_KS ? kKs : kEuler; }
+inline int shapes(int eq)
+{
+    return eq == EQ_HEAT ? Table<EQ_HEAT>::count : eq == EQ_KS ? Table<EQ_KS>::count : Table<EQ_EULER>::count;
+}
 
 }  // namespace wide
 }  // namespace sw1d

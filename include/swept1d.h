@@ -47,10 +47,10 @@ enum { SW1D_F64 = 0, SW1D_F32 = 1 };
  * 2 hybrid CPU+GPU swept (heat, Euler) / register swept (KS).
  * 3 (library only, no reference counterpart): overlapped trapezoid tiles —
  * swept up-triangles widened by a redundant halo, any nx, same bits.
- * Heat and KS advances of 1, 3 and the KS 2 run as overlapped tiles a
- * workgroup wide wherever those are faster than a row of swept tiles per
- * launch (all but FP32 KS on large fields); per-kernel profiling runs and
- * times the swept rows. */
+ * Advances of 1, 3 and the KS 2 run as overlapped tiles a workgroup wide
+ * wherever those are faster than a row of swept tiles per launch (all but FP32
+ * KS on large fields); per-kernel profiling runs and times the swept rows of 1
+ * and 2. */
 enum { SW1D_CLASSIC = 0, SW1D_SWEPT = 1, SW1D_ALT = 2, SW1D_TRAPEZOID = 3 };
 /* Boundary conditions.  DEFAULT picks the reference's: heat insulated
  * (mirror, Heat:140-142), KS periodic (KS:199), Euler Dirichlet ghost cells
