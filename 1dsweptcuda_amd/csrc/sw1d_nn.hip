@@ -30,6 +30,7 @@
 #include <cstdint>
 #include <cstring>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/swept1d.h"
@@ -416,7 +417,7 @@ __global__ __launch_bounds__(NTW) void k_l56_fwd(const __bf16* __restrict__ Ain,
 // to the FP64 state in place of storing du (the operation of k_apply_du).
 template <bool APPLY>
 __global__ __launch_bounds__(NT) void k_l6_out(const float* __restrict__ S, const float* __restrict__ b6,
-                                               float* __restrict__ du, double* __restrict__ u,
+                                               float* __restrict__ du, const double* u, double* out,
                                                double out_scale, int X, int64_t plane)
 {
     const int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x;
@@ -427,7 +428,7 @@ __global__ __launch_bounds__(NT) void k_l6_out(const float* __restrict__ S, cons
 #pragma unroll
     for (int t = 0; t < TAPS; ++t) s += S[t * plane + row + wrapx(x + t - 2, X)];
     if (APPLY)
-        u[i] += out_scale * (double)s;
+        out[i] = u[i] + out_scale * (double)s;
     else
         du[i] = s;
 }
@@ -439,89 +440,84 @@ constexpr int64_t MID_SZ = TAPS * C * C + C;
 constexpr int64_t P_W6 = P_MID + 4 * MID_SZ, P_B6 = P_W6 + TAPS * C;
 constexpr int64_t NPARAM = P_B6 + 1;
 
-// ------------------------------------------ whole network, one sample per WG ---
-// Inference at nx = 1024: one workgroup of 16 waves holds a whole periodic
-// sample's activation (1024 rows x 64 BF16 = 128 KB) in LDS through all six
-// layers, so no activation goes to memory; each wave owns 64 rows (four
-// 16-row MFMA blocks).  The tile keeps copies of rows 1022, 1023 before row 0
-// and of rows 0, 1 after row 1023 (tile row = position + 2, as in the
-// per-layer kernels), refreshed after each layer, so the MFMA operand rows
-// need no wrap.  A layer's weights are staged in two parts (taps 0-2, then
-// 3-4) into a 24 KB buffer, which also holds the network input before layer 1
-// and the output layer's tap sums after layer 5.  Every value goes through
-// the operations of the per-layer kernels in the same order (L1 as stage_l1,
-// the MFMA steps s = 0..9 of mfma_tile, the epilogue, the tap sums of
-// k_l56_fwd and the sum of k_l6_out), so the results are the same bits.
-constexpr int XN = 1024;                   // positions per sample
-constexpr int NTN = 1024;                  // threads of the whole-network kernel
-constexpr int MBN = XN / (NTN / 64) / 16;  // 16-row blocks per wave (4)
-constexpr int WPART = 3;                   // taps per weight part
-static_assert(NTN == XN, "the input and output stages map one thread to one position");
+// -------------------------------------- whole network, a segment of a sample ---
+// Inference at nx = 1024: a workgroup takes SEG positions (a half, a quarter or
+// an eighth) of a periodic sample through all six layers in one launch, its
+// activation (BF16 rows of 64 channels) in LDS, so no activation goes to memory.
+// Tile row q is position p0 - 10 + q: the ten positions on each side that the
+// five 5-tap layers reach are the neighbouring segment's, computed here too
+// (every layer computes rows 2 .. SEG+17, of which its own reach is exact).
+// Each wave owns PB 16-row MFMA blocks, and four waves each take 16 channels of
+// the one block left over.  Every value goes through the operations of the
+// per-layer kernels in the same order (L1 as stage_l1, the MFMA steps s = 0..9
+// of mfma_tile, the epilogue, the tap sums of k_l56_fwd and the sum of
+// k_l6_out), so the results are the same bits.
+//
+// A full chip is bound by issue: 22 us of GELUs (42 cycles per wave and value,
+// half of them the exponential and the reciprocal) and 18 us of MFMAs, which
+// overlap only in part, also between workgroups (16 GELUs and 16 MFMAs of
+// separate waves take 90% of their sum).  A small batch is bound by a
+// workgroup's life, the chain of six layers, and a whole sample per workgroup
+// left the other CUs idle.  So the segments get smaller with the batch; 64
+// samples take 23 us and 8 take 18, where a workgroup per sample took 58 for
+// any batch up to 256, and 256 take 57.  The weights pass through a ring of
+// three steps, the next on its way from memory while one is used; they are the
+// MFMA's row operand, so that a lane holds four channels of a position, one
+// 8-byte store instead of four of 2.
+constexpr int XN = 1024;                 // positions per sample
+constexpr int STEPS = 2 * TAPS;          // MFMA steps of a layer: 32 input channels of a tap each
+constexpr int SLAB = C * 32;             // weights of a step, [co][32 ci]
 
-// taps t0 .. t0+nt-1 of a layer's packed weights [t][co][ci] -> sW rows (t-t0)*64 + co
-__device__ __forceinline__ void stage_w_part(__bf16* sW, const __bf16* __restrict__ Wf, int t0, int nt)
-{
-    for (int q = threadIdx.x; q < nt * C * (C / 8); q += NTN) {
-        *reinterpret_cast<uint4*>(&sW[swz(q / (C / 8), q % (C / 8))]) =
-            *reinterpret_cast<const uint4*>(&Wf[(int64_t)t0 * C * C + q * 8]);
+// One step's weights on their way from memory to a slab in LDS: row co's four
+// 16-byte chunks, swizzled so that 16 rows' reads of a chunk meet no bank twice.
+template <int NTS>
+struct WeightStep {
+    static constexpr int EL = SLAB / NTS;
+    typedef __bf16 vec __attribute__((ext_vector_type(EL)));
+    vec v;
+    __device__ __forceinline__ void load(const __bf16* __restrict__ Wf, int s, int tid)
+    {
+        const int e = tid * EL, co = e / 32;
+        v = *reinterpret_cast<const vec*>(&Wf[((s >> 1) * C + co) * C + (s & 1) * 32 + e % 32]);
     }
-}
-// tile rows 0, 1 <- rows 1024, 1025 and rows 1026, 1027 <- rows 2, 3 (the
-// periodic neighbours of positions 0 and 1023)
-__device__ __forceinline__ void wrap_rows(__bf16* sA)
-{
-    const int q = threadIdx.x;
-    if (q < 4 * (C / 8)) {
-        const int d = q / (C / 8), c8 = q % (C / 8);
-        const int dst = d < 2 ? d : XN + d, src = d < 2 ? XN + d : d;
-        *reinterpret_cast<uint4*>(&sA[swz(dst, c8)]) = *reinterpret_cast<const uint4*>(&sA[swz(src, c8)]);
+    __device__ __forceinline__ void store(__bf16* slab, int tid) const
+    {
+        const int e = tid * EL, co = e / 32, ch = e / 8 % 4;
+        *reinterpret_cast<vec*>(&slab[(co * 4 + (ch ^ (co >> 2 & 3))) * 8 + e % 8]) = v;
     }
-}
-// MFMA steps s = S0 .. S1-1 of mfma_tile over the wave's 64 rows (tile rows
-// row0 .. row0+63 plus the four halo rows); the weights of tap t sit at sW
-// rows (t - S0/2)*64 + co.
-template <int S0, int S1>
-__device__ __forceinline__ void mfma_rows(const __bf16* sA, const __bf16* sW, int row0, f32x4 (&acc)[MBN][4])
-{
-    const int l = threadIdx.x & 63, li = l % 16, lq = l / 16;
-    for (int s = S0; s < S1; ++s) {
-        const int t = s >> 1, chunk = (s & 1) * 4 + lq, tw = t - S0 / 2;
-        const __bf16* pa = &sA[swz(row0 + li + t, chunk)];      // + 16 rows per block
-        const __bf16* pb = &sW[swz(tw * C + li, chunk)];        // + 16 rows per block
-        bf16x8 a[MBN], bv[4];
-#pragma unroll
-        for (int mb = 0; mb < MBN; ++mb) a[mb] = *reinterpret_cast<const bf16x8*>(pa + 16 * mb * C);
-#pragma unroll
-        for (int nb = 0; nb < 4; ++nb) bv[nb] = *reinterpret_cast<const bf16x8*>(pb + 16 * nb * C);
-#pragma unroll
-        for (int mb = 0; mb < MBN; ++mb)
-#pragma unroll
-            for (int nb = 0; nb < 4; ++nb)
-                acc[mb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mb], bv[nb], acc[mb][nb], 0, 0, 0);
-    }
-}
+};
 
 struct MidWeights { const __bf16* w[4]; };  // packed forward weights of L2-L5
 
-// TIN = double: in = FP64 states u (normalised by inv_scale), u += out_scale *
-// du in place (in and u are the same array); TIN = float: in = network
-// inputs x, du written to du.
-template <typename TIN>
-__global__ __launch_bounds__(NTN) void k_net_fwd(const TIN* in, float inv_scale, const float* __restrict__ P,
-                                                MidWeights wf, float* __restrict__ du, double* u,
-                                                double out_scale)
+// TIN = double: in = FP64 states (normalised by inv_scale), out = in + out_scale
+// * du (another array: a neighbouring segment may still have to read in);
+// TIN = float: in = network inputs x, du written to du.
+template <typename TIN, int NSEG, int PB>
+__global__ __launch_bounds__(4 * XN / (NSEG * PB), 4) void k_net_fwd(const TIN* __restrict__ in, float inv_scale,
+                                                          const float* __restrict__ P, MidWeights wf,
+                                                          float* __restrict__ du, double* __restrict__ out,
+                                                          double out_scale)
 {
-    __shared__ __attribute__((aligned(16))) __bf16 sA[(XN + 4) * C];
-    __shared__ __attribute__((aligned(16))) __bf16 sW[WPART * C * C];
-    __shared__ float sW6[TAPS * C];
-    float* sF = reinterpret_cast<float*>(sW);  // network input, later the output-layer tap sums
-    const int b = blockIdx.x, r = threadIdx.x;
-    const int64_t o = (int64_t)b * XN + r;
+    constexpr int SEG = XN / NSEG, NW = SEG / (16 * PB), NTS = 64 * NW, ROWS = SEG + 20;
+    static_assert(NW >= 4 && NTS >= SEG && 3 * SLAB * 2 >= TAPS * (SEG + 4) * 4);
+    __shared__ __attribute__((aligned(16))) __bf16 sA[ROWS * C];
+    __shared__ __attribute__((aligned(16))) __bf16 sW[3 * SLAB];  // ring of three steps' weights
+    __shared__ __attribute__((aligned(16))) float sB[4 * C];      // biases of layers 2-5
+    float* sF = reinterpret_cast<float*>(sW + 2 * SLAB);          // network input (before step 2's weights)
+    float* sS = reinterpret_cast<float*>(sW);                     // output-layer tap sums (after layer 5)
+    const int tid = threadIdx.x, b = blockIdx.x / NSEG, p0 = blockIdx.x % NSEG * SEG;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
-    // layer 1 (stage_l1 over the whole periodic sample) into tile rows 2 .. XN+1
-    sF[r] = (float)in[o] * inv_scale;
+    WeightStep<NTS> w0, w1, ws;
+    w0.load(wf.w[0], 0, tid);
+    w1.load(wf.w[0], 1, tid);
+    ws.load(wf.w[0], 2, tid);
+    // layer 1 (stage_l1) into every tile row
+    for (int i = tid; i < ROWS + 4; i += NTS)
+        sF[i] = (float)in[(int64_t)b * XN + ((p0 - 12 + i) & (XN - 1))] * inv_scale;
+    if (tid < 4 * C) sB[tid] = P[P_MID + (tid / C) * MID_SZ + TAPS * C * C + tid % C];
     {
-        const int c8 = threadIdx.x % (C / 8);
+        const int c8 = tid % (C / 8);
         float w[8][TAPS], bb[8];
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
@@ -529,80 +525,135 @@ __global__ __launch_bounds__(NTN) void k_net_fwd(const TIN* in, float inv_scale,
 #pragma unroll
             for (int t = 0; t < TAPS; ++t) w[k][t] = P[P_W1 + (c8 * 8 + k) * TAPS + t];
         }
+        w0.store(sW, tid);
+        w1.store(sW + SLAB, tid);
         __syncthreads();
-        for (int x = threadIdx.x / (C / 8); x < XN; x += NTN / (C / 8)) {
+        for (int q = tid / (C / 8); q < ROWS; q += NTS / (C / 8)) {
             bf16x8 v;
 #pragma unroll
             for (int k = 0; k < 8; ++k) {
                 float z = bb[k];
 #pragma unroll
-                for (int t = 0; t < TAPS; ++t) z = fmaf(w[k][t], sF[(x + t - 2) & (XN - 1)], z);
+                for (int t = 0; t < TAPS; ++t) z = fmaf(w[k][t], sF[q + t], z);
                 v[k] = f2bf(gelu(z));
             }
-            *reinterpret_cast<bf16x8*>(&sA[swz(x + 2, c8)]) = v;
+            *reinterpret_cast<bf16x8*>(&sA[swz(q, c8)]) = v;
         }
     }
-    for (int q = threadIdx.x; q < TAPS * C; q += NTN) sW6[q] = P[P_W6 + q];
 
-    // layers 2-5
+    // layers 2-5: acc[cb][pb] is channels 16 cb + 4 lq + j of row 16 (4 wave + pb)
+    // + li + 2 (the weights are the MFMA's row operand, so a lane's four values are
+    // 8 bytes of the tile)
+    const bool extra = wave < 4;
     for (int layer = 0; layer < 4; ++layer) {
-        // recomputed per layer rather than kept live across it
-        int lane = threadIdx.x;
-        asm volatile("" : "+v"(lane));
-        const int l = lane & 63, row0 = 64 * (lane >> 6), li = l % 16, lq = l / 16;
-        f32x4 acc[MBN][4];
+        // with 128 registers, addresses recomputed per layer rather than kept
+        // live across it
+        int lane = tid;
+        if constexpr (PB == 4) asm volatile("" : "+v"(lane));
+        const int li = lane % 16, lq = lane / 16 % 4, row0 = 16 * PB * wave + li, rowe = 16 * PB * NW + li;
+        f32x4 acc[4][PB], acce = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int mb = 0; mb < MBN; ++mb)
+        for (int cb = 0; cb < 4; ++cb)
 #pragma unroll
-            for (int nb = 0; nb < 4; ++nb) acc[mb][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-        __syncthreads();  // the layer input is complete; sF / sW are no longer read
-        wrap_rows(sA);
-        stage_w_part(sW, wf.w[layer], 0, WPART);
-        __syncthreads();
-        mfma_rows<0, 2 * WPART>(sA, sW, row0, acc);
-        __syncthreads();
-        stage_w_part(sW, wf.w[layer], WPART, TAPS - WPART);
-        __syncthreads();
-        mfma_rows<2 * WPART, 2 * TAPS>(sA, sW, row0, acc);
-        __syncthreads();  // every wave has read the layer input: overwrite it in place
-        const float* bias = P + P_MID + layer * MID_SZ + TAPS * C * C;
+            for (int pb = 0; pb < PB; ++pb) acc[cb][pb] = f32x4{0.f, 0.f, 0.f, 0.f};
+        int slot = layer % 3;  // of the layer's step 0: 10 layer mod 3
 #pragma unroll
-        for (int nb = 0; nb < 4; ++nb) {
-            const int co = 16 * nb + li;
-            const float bc = bias[co];
+        for (int s = 0; s < STEPS; ++s) {
+            // the input of the layer and this step's weights are complete, and
+            // the previous step's are no longer read
+            __syncthreads();
+            const int free = slot == 0 ? 2 : slot - 1;
+            if (s + 2 < STEPS || layer < 3) ws.store(sW + free * SLAB, tid);
+            if (s + 3 < STEPS)
+                ws.load(wf.w[layer], s + 3, tid);
+            else if (layer < 3)
+                ws.load(wf.w[layer + 1], s + 3 - STEPS, tid);
+            if (s == 0) __builtin_amdgcn_s_setprio(1);
+            const __bf16* slab = sW + slot * SLAB;
+            slot = slot == 2 ? 0 : slot + 1;
+
+            const int t = s >> 1, chunk = (s & 1) * 4 + lq;
+            const __bf16* px = &sA[swz(row0 + t, chunk)];                     // + 16 rows per block
+            const __bf16* pw = slab + (li * 4 + (lq ^ (li >> 2 & 3))) * 8;    // + 16 rows per block
+            bf16x8 w[4], x[PB];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                __bf16* pd = &sA[swz(row0 + 2 + 4 * lq + j, co >> 3) + (co & 7)];  // + 16 rows per block
+            for (int cb = 0; cb < 4; ++cb) w[cb] = *reinterpret_cast<const bf16x8*>(pw + 16 * 32 * cb);
 #pragma unroll
-                for (int mb = 0; mb < MBN; ++mb) pd[16 * mb * C] = f2bf(gelu(acc[mb][nb][j] + bc));
+            for (int pb = 0; pb < PB; ++pb) x[pb] = *reinterpret_cast<const bf16x8*>(px + 16 * pb * C);
+#pragma unroll
+            for (int cb = 0; cb < 4; ++cb)
+#pragma unroll
+                for (int pb = 0; pb < PB; ++pb)
+                    acc[cb][pb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[cb], x[pb], acc[cb][pb], 0, 0, 0);
+            if (extra) {
+                const bf16x8 we = *reinterpret_cast<const bf16x8*>(pw + 16 * 32 * wave);
+                const bf16x8 xe = *reinterpret_cast<const bf16x8*>(&sA[swz(rowe + t, chunk)]);
+                acce = __builtin_amdgcn_mfma_f32_16x16x32_bf16(we, xe, acce, 0, 0, 0);
             }
         }
+        __builtin_amdgcn_s_setprio(0);
+        auto activate = [&](const f32x4& a, int cb) {
+            const f32x4 bc = *reinterpret_cast<const f32x4*>(&sB[layer * C + 16 * cb + 4 * lq]);
+            bf16x4 o;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) o[j] = f2bf(gelu(a[j] + bc[j]));
+            return o;
+        };
+        auto place = [&](int row, int cb, const bf16x4& o) {
+            *reinterpret_cast<bf16x4*>(&sA[swz(row + 2, 2 * cb + (lq >> 1)) + 4 * (lq & 1)]) = o;
+        };
+        bf16x4 o[4][PB], oe;
+#pragma unroll
+        for (int cb = 0; cb < 4; ++cb)
+#pragma unroll
+            for (int pb = 0; pb < PB; ++pb) o[cb][pb] = activate(acc[cb][pb], cb);
+        if (extra) oe = activate(acce, wave);
+        __syncthreads();  // every wave has read the layer input: overwrite it in place
+#pragma unroll
+        for (int cb = 0; cb < 4; ++cb)
+#pragma unroll
+            for (int pb = 0; pb < PB; ++pb) place(row0 + 16 * pb, cb, o[cb][pb]);
+        if (extra) place(rowe, wave, oe);
     }
     __syncthreads();
 
-    // output layer: the five tap sums of position r (k_l56_fwd), then
-    // du = b6 + sum_t S[t][r+t-2] (k_l6_out)
-    {
+    // output layer: the five tap sums S[t][i] of rows 8 + i (k_l56_fwd), i = 0 ..
+    // SEG+3, then du = b6 + sum_t S[t][i+t] (k_l6_out).  The weights of a thread's
+    // own row are scalar operands; 20 threads add one sum of the four rows beyond.
+    const float* __restrict__ w6 = P + P_W6;
+    if (tid < SEG) {
         float sum[TAPS] = {0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int c8 = 0; c8 < C / 8; ++c8) {
-            const bf16x8 v = *reinterpret_cast<const bf16x8*>(&sA[swz(r + 2, c8)]);
+            const bf16x8 v = *reinterpret_cast<const bf16x8*>(&sA[swz(tid + 10, c8)]);
 #pragma unroll
             for (int k = 0; k < 8; ++k) {
                 const float a = bf2f(v[k]);
 #pragma unroll
-                for (int t = 0; t < TAPS; ++t) sum[t] = fmaf(sW6[t * C + c8 * 8 + k], a, sum[t]);
+                for (int t = 0; t < TAPS; ++t) sum[t] = fmaf(w6[t * C + c8 * 8 + k], a, sum[t]);
             }
         }
 #pragma unroll
-        for (int t = 0; t < TAPS; ++t) sF[t * XN + r] = sum[t];
+        for (int t = 0; t < TAPS; ++t) sS[t * (SEG + 4) + tid + 2] = sum[t];
+    }
+    if (tid < 4 * TAPS) {
+        const int t = tid % TAPS, e = tid / TAPS, i = e < 2 ? e : SEG + e;
+        float sum = 0.f;
+        for (int c8 = 0; c8 < C / 8; ++c8) {
+            const bf16x8 v = *reinterpret_cast<const bf16x8*>(&sA[swz(i + 8, c8)]);
+#pragma unroll
+            for (int k = 0; k < 8; ++k) sum = fmaf(w6[t * C + c8 * 8 + k], bf2f(v[k]), sum);
+        }
+        sS[t * (SEG + 4) + i] = sum;
     }
     __syncthreads();
+    if (tid >= SEG) return;
+    const int64_t o = (int64_t)b * XN + p0 + tid;
     float s = P[P_B6];
 #pragma unroll
-    for (int t = 0; t < TAPS; ++t) s += sF[t * XN + ((r + t - 2) & (XN - 1))];
-    if (u)
-        u[o] += out_scale * (double)s;
+    for (int t = 0; t < TAPS; ++t) s += sS[t * (SEG + 4) + tid + t];
+    if (out)
+        out[o] = (double)in[o] + out_scale * (double)s;
     else
         du[o] = s;
 }
@@ -1077,12 +1128,12 @@ __global__ __launch_bounds__(NT) void k_pack_w(const float* __restrict__ p, Pack
     wb[(t * C + ci) * C + co] = h;
 }
 
-// u += scale * du
-__global__ __launch_bounds__(NT) void k_apply_du(double* __restrict__ u, const float* __restrict__ du,
+// out = u + scale * du
+__global__ __launch_bounds__(NT) void k_apply_du(const double* u, const float* __restrict__ du, double* out,
                                                  int64_t n, double scale)
 {
     const int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x;
-    if (i < n) u[i] += scale * (double)du[i];
+    if (i < n) out[i] = u[i] + scale * (double)du[i];
 }
 
 // Judged step: u[p] <- unn[p] for the problems whose network state is kept.
@@ -1217,6 +1268,7 @@ int g_mfma_ok = 0;
 
 struct sw1d_nn {
     int X = 1024, Bmax = 0;
+    int cus = 256;          // compute units of the device
     int infer_mode = 0;     // 0 auto, 1 per-layer launches, 2 whole-network kernel
     double in_scale = 1.0, out_scale = 1.0;
     hipStream_t stream = nullptr;
@@ -1276,24 +1328,59 @@ int nn_layers(sw1d_nn* N, int B, const TIN* in, float inv_scale)
     return SW1D_OK;
 }
 
+// Segments per sample of the whole-network kernel: the fewest microseconds for
+// B samples on `cus` compute units.  A launch lasts as long as the CU with most
+// workgroups; measured with 1 .. cap of them side by side (cap by LDS).
+int net_segments(int64_t B, int cus)
+{
+    struct Split { int segs, cap; float us[6]; };
+    static constexpr Split splits[] = {{8, 5, {0, 18.f, 23.f, 30.f, 38.f, 47.f}}, {4, 3, {0, 23.f, 34.f, 50.f}},
+                                       {2, 2, {0, 37.f, 57.f}}};
+    int best = 2;
+    double least = 0;
+    for (const Split& c : splits) {
+        const int64_t m = (c.segs * B + cus - 1) / cus;
+        const double us = (double)(m / c.cap) * c.us[c.cap] + c.us[m % c.cap];
+        if (least == 0 || us < least) {
+            least = us;
+            best = c.segs;
+        }
+    }
+    return best;
+}
+
+template <typename TIN, int NSEG, int PB>
+void launch_net(sw1d_nn* N, int B, const TIN* in, float inv_scale, double* out)
+{
+    const MidWeights w{{N->wf[0], N->wf[1], N->wf[2], N->wf[3]}};
+    hipLaunchKernelGGL((k_net_fwd<TIN, NSEG, PB>), dim3(B * NSEG), dim3(4 * XN / (NSEG * PB)), 0, N->stream, in,
+                       inv_scale, N->p, w, N->du, out, N->out_scale);
+}
+template <typename TIN>
+void net_forward(sw1d_nn* N, int B, const TIN* in, float inv_scale, double* out)
+{
+    switch (net_segments(B, N->cus)) {
+    case 8: return launch_net<TIN, 8, 2>(N, B, in, inv_scale, out);
+    case 4: return launch_net<TIN, 4, 2>(N, B, in, inv_scale, out);
+    default: return launch_net<TIN, 2, 4>(N, B, in, inv_scale, out);
+    }
+}
+
 // Inference of B samples.  u == nullptr: from the FP32 inputs in N->x to du
 // in N->du.  Otherwise from the FP64 states u (normalised on the fly by
-// 1/in_scale) to u += out_scale * du.  One launch of the whole-network kernel
-// at nx = 1024; five launches when nx is another multiple of the 256-position
-// tile (or infer_mode = 1), these two with the same bits; otherwise 64-position
-// tiles and the training's output layer.
-int nn_infer(sw1d_nn* N, int B, double* u)
+// 1/in_scale) to out = u + out_scale * du, another array.  One launch of the
+// whole-network kernel at nx = 1024; five launches when nx is another multiple
+// of the 256-position tile (or infer_mode = 1), these two with the same bits;
+// otherwise 64-position tiles and the training's output layer.
+int nn_infer(sw1d_nn* N, int B, const double* u, double* out)
 {
     const int X = N->X;
     const int64_t plane = (int64_t)B * X;
     if (X == XN && N->infer_mode != 1) {
-        MidWeights w{{N->wf[0], N->wf[1], N->wf[2], N->wf[3]}};
         if (u)
-            hipLaunchKernelGGL(k_net_fwd<double>, dim3(B), dim3(NTN), 0, N->stream, u,
-                               (float)(1.0 / N->in_scale), N->p, w, nullptr, u, N->out_scale);
+            net_forward<double>(N, B, u, (float)(1.0 / N->in_scale), out);
         else
-            hipLaunchKernelGGL(k_net_fwd<float>, dim3(B), dim3(NTN), 0, N->stream, N->x, 1.0f, N->p, w, N->du,
-                               nullptr, 0.0);
+            net_forward<float>(N, B, N->x, 1.0f, nullptr);
         NN_HIP(hipGetLastError());
         return SW1D_OK;
     }
@@ -1304,7 +1391,7 @@ int nn_infer(sw1d_nn* N, int B, double* u)
         hipLaunchKernelGGL(k_l6_fwd<false>, dim3(nblk(plane)), dim3(NT), 0, N->stream, N->A[1], N->p + P_W6,
                            N->p + P_B6, N->du, nullptr, nullptr, nullptr, X, plane);
         if (u)
-            hipLaunchKernelGGL(k_apply_du, dim3(nblk(plane)), dim3(NT), 0, N->stream, u, N->du, plane,
+            hipLaunchKernelGGL(k_apply_du, dim3(nblk(plane)), dim3(NT), 0, N->stream, u, N->du, out, plane,
                                N->out_scale);
         NN_HIP(hipGetLastError());
         return SW1D_OK;
@@ -1325,10 +1412,10 @@ int nn_infer(sw1d_nn* N, int B, double* u)
                        X, plane);
     if (u)
         hipLaunchKernelGGL(k_l6_out<true>, dim3(nblk(plane)), dim3(NT), 0, N->stream, N->taps, P + P_B6,
-                           nullptr, u, N->out_scale, X, plane);
+                           nullptr, u, out, N->out_scale, X, plane);
     else
         hipLaunchKernelGGL(k_l6_out<false>, dim3(nblk(plane)), dim3(NT), 0, N->stream, N->taps, P + P_B6,
-                           N->du, nullptr, 0.0, X, plane);
+                           N->du, nullptr, nullptr, 0.0, X, plane);
     NN_HIP(hipGetLastError());
     return SW1D_OK;
 }
@@ -1462,6 +1549,10 @@ int sw1d_nn_create(sw1d_nn** out, int32_t nx, int32_t max_batch, uint64_t seed)
     sw1d_nn* N = new sw1d_nn();
     N->X = nx;
     N->Bmax = max_batch;
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) == hipSuccess &&
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0)
+        N->cus = cus;
     const int64_t nout = (int64_t)nx * max_batch, nfeat = nout * C;
     bool ok = hipStreamCreateWithFlags(&N->stream, hipStreamNonBlocking) == hipSuccess &&
               dalloc(&N->p, NPARAM) == hipSuccess && dalloc(&N->g, NPARAM) == hipSuccess &&
@@ -1558,7 +1649,7 @@ int sw1d_nn_forward(sw1d_nn* N, const float* x_host, int32_t batch, float* y_hos
     if (batch < 1 || batch > N->Bmax) return nn_fail(SW1D_EINVAL, "batch out of range");
     const size_t bytes = (size_t)batch * N->X * sizeof(float);
     NN_HIP(hipMemcpyAsync(N->x, x_host, bytes, hipMemcpyHostToDevice, N->stream));
-    int rc = nn_infer(N, batch, nullptr);
+    int rc = nn_infer(N, batch, nullptr, nullptr);
     if (rc) return rc;
     NN_HIP(hipMemcpyAsync(y_host, N->du, bytes, hipMemcpyDeviceToHost, N->stream));
     NN_HIP(hipStreamSynchronize(N->stream));
@@ -1645,7 +1736,10 @@ extern "C" int sw1d_surrogate_advance(sw1d_nn* N, sw1d_batch* batch, int64_t sur
             return nn_fail(SW1D_ENOMEM, "integrator scratch");
         N->int_len = len;
     }
+    // The states alternate between the batch's array u and the scratch array; a
+    // judged step finds its input in u, where the plain solver starts from it.
     double* u = static_cast<double*>(bv.state);
+    double *cur = u, *other = N->usave;
     const size_t bytes = (size_t)len * sizeof(double);
     const int64_t per = (X + NT - 1) / NT;  // l2 blocks per problem (X is a multiple of NT)
     int64_t judged = 0;
@@ -1667,20 +1761,19 @@ extern "C" int sw1d_surrogate_advance(sw1d_nn* N, sw1d_batch* batch, int64_t sur
     hipLaunchKernelGGL(k_zero_f64, dim3(1), dim3(NT), 0, N->stream, N->jacc, (int64_t)2);
     for (int64_t i = 1; i <= surrogate_steps; ++i) {
         const bool judge = judge_every > 0 && i % judge_every == 0;
-        if (judge) NN_HIP(hipMemcpyAsync(N->usave, u, bytes, hipMemcpyDeviceToDevice, N->stream));
-        int rc = nn_infer(N, (int)B, u);
+        int rc = nn_infer(N, (int)B, cur, judge ? N->unn : other);
         if (rc) return rc;
-        if (!judge) continue;
-        // plain solver from the same states: u <- solver^K(usave)
-        NN_HIP(hipMemcpyAsync(N->unn, u, bytes, hipMemcpyDeviceToDevice, N->stream));
-        NN_HIP(hipMemcpyAsync(u, N->usave, bytes, hipMemcpyDeviceToDevice, N->stream));
-        if (judged == 0) {
-            // the batch may capture its graph for k_steps here: start it on idle streams
-            NN_HIP(hipStreamSynchronize(N->stream));
-        } else {
-            NN_HIP(hipEventRecord(ev.a, N->stream));
-            NN_HIP(hipStreamWaitEvent(bv.stream, ev.a, 0));
+        if (!judge) {
+            std::swap(cur, other);
+            continue;
         }
+        // plain solver from the same states: u <- solver^K(u)
+        if (cur != u) {
+            NN_HIP(hipMemcpyAsync(u, cur, bytes, hipMemcpyDeviceToDevice, N->stream));
+            std::swap(cur, other);
+        }
+        NN_HIP(hipEventRecord(ev.a, N->stream));
+        NN_HIP(hipStreamWaitEvent(bv.stream, ev.a, 0));
         ++judged;
         rc = sw1d_batch_advance(batch, k_steps);
         if (rc) return nn_fail(rc, "plain solver step of the judge");
@@ -1691,6 +1784,7 @@ extern "C" int sw1d_surrogate_advance(sw1d_nn* N, sw1d_batch* batch, int64_t sur
         hipLaunchKernelGGL(k_keep_rows, dim3(blocks), dim3(NT), 0, N->stream, u, N->unn, N->keep, (int)X, len);
         NN_HIP(hipGetLastError());
     }
+    if (cur != u) NN_HIP(hipMemcpyAsync(u, cur, bytes, hipMemcpyDeviceToDevice, N->stream));
     double acc[2] = {0.0, 0.0};
     NN_HIP(hipMemcpyAsync(acc, N->jacc, sizeof(acc), hipMemcpyDeviceToHost, N->stream));
     NN_HIP(hipStreamSynchronize(N->stream));
@@ -1862,7 +1956,7 @@ int sw1d_nn_eval(sw1d_nn* N, int64_t first, int64_t count, double* rel_err)
     for (int64_t s = first; s < first + count; s += N->Bmax) {
         const int b = (int)std::min<int64_t>(N->Bmax, first + count - s);
         NN_HIP(hipMemcpyAsync(N->x, D->x + s * row, b * row * sizeof(float), hipMemcpyDeviceToDevice, N->stream));
-        int rc = nn_infer(N, b, nullptr);
+        int rc = nn_infer(N, b, nullptr, nullptr);
         if (rc) return rc;
         y.resize(b * row);
         t.resize(b * row);

@@ -26,10 +26,10 @@
 // lanes), 3% exchanges, the rest the launch.  FP32 KS at 2^19 and more is the
 // one case the diamonds win (1.32e12 against 1.14e12 at 2^20): FP32
 // instructions of two waves co-issue, and the diamonds evaluate fewer points.
-// An Euler cell's step is some 550 FP64 instructions; at 2^20 a launch of 13
-// steps of 4 cells per lane issues for four fifths of its 232 us, a quarter of
-// it for the overlap and the halo lanes (its 234 registers allow two waves per
-// SIMD, its steps six of the window's 928 cells each).
+// An Euler cell's step is some 460 instructions; at 2^20 a launch of 13 steps
+// of 4 cells per lane takes 232 us, nine tenths of it FP64 issue, a quarter of
+// which repeats neighbours' cells: the window's 928 cells lose 8 per step, and
+// 234 registers per lane hold no more than 4 cells beside two waves per SIMD.
 
 #include <cmath>
 
