@@ -34,6 +34,7 @@
 #include <vector>
 
 #include "../../include/swept1d.h"
+#include "sw1d_host.hpp"
 
 namespace sw1dnn {
 
@@ -1272,6 +1273,7 @@ struct sw1d_nn {
     int infer_mode = 0;     // 0 auto, 1 per-layer launches, 2 whole-network kernel
     double in_scale = 1.0, out_scale = 1.0;
     hipStream_t stream = nullptr;
+    sw1d::HostStage stage;  // host copies of inputs and results
     float *p = nullptr, *g = nullptr, *m = nullptr, *v = nullptr;  // NPARAM each
     int64_t adam_t = 0;
     __bf16 *wf[4] = {}, *wb[4] = {};                                // packed mid weights
@@ -1456,18 +1458,21 @@ int nn_gradient(sw1d_nn* N, int B)
     return SW1D_OK;
 }
 
-int nn_gradient(sw1d_nn* N, int B, double* loss)
+// ... and the loss, and the gradient to the host, where asked for
+int nn_gradient(sw1d_nn* N, int B, double* loss, float* grad_host = nullptr)
 {
     const int rc = N->X % TILE_F == 0 ? nn_gradient<TILE_F>(N, B) : nn_gradient<TILE>(N, B);
-    if (rc || !loss) return rc;
+    if (rc || (!loss && !grad_host)) return rc;
     const int64_t nout = (int64_t)B * N->X;
-    const unsigned lb = nblk(nout);
-    std::vector<float> lp(lb);
-    NN_HIP(hipMemcpyAsync(lp.data(), N->lossp, lb * sizeof(float), hipMemcpyDeviceToHost, N->stream));
-    NN_HIP(hipStreamSynchronize(N->stream));
-    double s = 0;
-    for (float f : lp) s += f;
-    *loss = s / (double)nout;
+    std::vector<float> lp(loss ? nblk(nout) : 0);
+    if (loss) NN_HIP(N->stage.down(lp.data(), N->lossp, lp.size() * sizeof(float), N->stream));
+    if (grad_host) NN_HIP(N->stage.down(grad_host, N->g, NPARAM * sizeof(float), N->stream));
+    NN_HIP(N->stage.finish(N->stream));
+    if (loss) {
+        double s = 0;
+        for (float f : lp) s += f;
+        *loss = s / (double)nout;
+    }
     return SW1D_OK;
 }
 
@@ -1554,6 +1559,8 @@ int sw1d_nn_create(sw1d_nn** out, int32_t nx, int32_t max_batch, uint64_t seed)
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0)
         N->cus = cus;
     const int64_t nout = (int64_t)nx * max_batch, nfeat = nout * C;
+    // two inputs, the loss parts and the gradient
+    N->stage.reserve((size_t)(2 * nout + nblk(nout) + NPARAM) * sizeof(float) + 4 * 4096);
     bool ok = hipStreamCreateWithFlags(&N->stream, hipStreamNonBlocking) == hipSuccess &&
               dalloc(&N->p, NPARAM) == hipSuccess && dalloc(&N->g, NPARAM) == hipSuccess &&
               dalloc(&N->m, NPARAM) == hipSuccess && dalloc(&N->v, NPARAM) == hipSuccess &&
@@ -1648,11 +1655,11 @@ int sw1d_nn_forward(sw1d_nn* N, const float* x_host, int32_t batch, float* y_hos
     if (!N || !x_host || !y_host) return nn_fail(SW1D_EINVAL, "null argument");
     if (batch < 1 || batch > N->Bmax) return nn_fail(SW1D_EINVAL, "batch out of range");
     const size_t bytes = (size_t)batch * N->X * sizeof(float);
-    NN_HIP(hipMemcpyAsync(N->x, x_host, bytes, hipMemcpyHostToDevice, N->stream));
+    NN_HIP(N->stage.up(N->x, x_host, bytes, N->stream));
     int rc = nn_infer(N, batch, nullptr, nullptr);
     if (rc) return rc;
-    NN_HIP(hipMemcpyAsync(y_host, N->du, bytes, hipMemcpyDeviceToHost, N->stream));
-    NN_HIP(hipStreamSynchronize(N->stream));
+    NN_HIP(N->stage.down(y_host, N->du, bytes, N->stream));
+    NN_HIP(N->stage.finish(N->stream));
     return SW1D_OK;
 }
 
@@ -1663,15 +1670,9 @@ int sw1d_nn_gradient(sw1d_nn* N, const float* x_host, const float* t_host, int32
     if (!N || !x_host || !t_host || !loss) return nn_fail(SW1D_EINVAL, "null argument");
     if (batch < 1 || batch > N->Bmax) return nn_fail(SW1D_EINVAL, "batch out of range");
     const size_t bytes = (size_t)batch * N->X * sizeof(float);
-    NN_HIP(hipMemcpyAsync(N->x, x_host, bytes, hipMemcpyHostToDevice, N->stream));
-    NN_HIP(hipMemcpyAsync(N->tgt, t_host, bytes, hipMemcpyHostToDevice, N->stream));
-    const int rc = nn_gradient(N, batch, loss);
-    if (rc) return rc;
-    if (grad_host) {
-        NN_HIP(hipMemcpyAsync(grad_host, N->g, NPARAM * sizeof(float), hipMemcpyDeviceToHost, N->stream));
-        NN_HIP(hipStreamSynchronize(N->stream));
-    }
-    return SW1D_OK;
+    NN_HIP(N->stage.up(N->x, x_host, bytes, N->stream));
+    NN_HIP(N->stage.up(N->tgt, t_host, bytes, N->stream));
+    return nn_gradient(N, batch, loss, grad_host);
 }
 
 // Adam on device-resident samples: inputs and targets are [nsamples][nx]

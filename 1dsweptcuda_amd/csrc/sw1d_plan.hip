@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "../../include/swept1d.h"
+#include "sw1d_host.hpp"
 #include "sw1d_internal.hpp"
 #include "sw1d_schedule.hpp"
 
@@ -67,6 +68,7 @@ struct sw1d_plan {
     void* buf[2]{nullptr, nullptr};  // each nc*n REALs, component-major
     int cur = 0;                     // buffer holding the current (flat) state
     hipStream_t stream = nullptr;
+    HostStage stage;  // host copies of the state
     // classic algorithm: a hipGraph of kClassicGraphSteps steps per starting buffer
     hipGraphExec_t classic_exec[2]{nullptr, nullptr};
     bool classic_graph_failed = false;
@@ -793,6 +795,7 @@ int sw1d_plan_create(sw1d_plan** out, const sw1d_problem* q)
         return fail(SW1D_EDEVICE, "hipStreamCreate: %s", hipGetErrorString(e));
     }
     const size_t bytes = (size_t)p->nc * (size_t)p->n * p->S;
+    if (bytes / 2 <= HostStage::kMost) p->stage.reserve(bytes / 2);  // a plain state
     for (int i = 0; i < 2; ++i) {
         e = hipMalloc(&p->buf[i], bytes);
         if (e != hipSuccess) {
@@ -831,67 +834,63 @@ int sw1d_plan_destroy(sw1d_plan* p)
     return SW1D_OK;
 }
 
-// Copies the state in or out of the plan's current buffer on its stream; with
-// sync, waits for the copy.
-static int copy_state(sw1d_plan* p, const void* src, void* dst, bool to_device, hipMemcpyKind kind,
-                      bool sync = true)
+// Copies the state in or out of the plan's current buffer on its stream: host
+// memory through the plan's staging memory, waiting for the copy, device memory
+// with sync.  Only the first value of a point (heat's even row, KS's u, Euler's
+// conserved values) goes in: the second is written before it is read.
+static int copy_state(sw1d_plan* p, const void* src, void* dst, bool to_device, bool host, bool sync = true)
 {
     const size_t S = p->S;
     const int64_t n = p->n;
     char* dev = static_cast<char*>(p->buf[p->cur]);
     if (p->eq != EQ_EULER) {
-        if (to_device) {
-            HIP_OR_FAIL(hipMemcpyAsync(dev, src, n * S, kind, p->stream));
-            // second value (odd row / u_half) starts as a copy; it is written
-            // before it is read
-            HIP_OR_FAIL(hipMemcpyAsync(dev + n * S, dev, n * S, hipMemcpyDeviceToDevice, p->stream));
-        } else {
-            HIP_OR_FAIL(hipMemcpyAsync(dst, dev, n * S, kind, p->stream));
-        }
+        if (host)
+            HIP_OR_FAIL(to_device ? p->stage.up(dev, src, n * S, p->stream) : p->stage.down(dst, dev, n * S, p->stream));
+        else
+            HIP_OR_FAIL(hipMemcpyAsync(to_device ? dev : dst, to_device ? src : dev, n * S, hipMemcpyDeviceToDevice,
+                                       p->stream));
     } else {
         // Host buffers go through the plan's other state buffer (idle between
         // advances, 6n values) in one contiguous copy; device buffers are
         // converted in place of the copy.
-        const bool host = kind != hipMemcpyDeviceToDevice;
         void* scratch = p->buf[p->cur ^ 1];
         if (to_device) {
-            const void* in = src;
-            if (host) {
-                HIP_OR_FAIL(hipMemcpyAsync(scratch, src, 3 * n * S, kind, p->stream));
-                in = scratch;
-            }
-            HIP_OR_FAIL(euler_layout(p, in, dev, true));
+            if (host) HIP_OR_FAIL(p->stage.up(scratch, src, 3 * n * S, p->stream));
+            HIP_OR_FAIL(euler_layout(p, host ? scratch : src, dev, true));
         } else {
             HIP_OR_FAIL(euler_layout(p, dev, host ? scratch : dst, false));
-            if (host) HIP_OR_FAIL(hipMemcpyAsync(dst, scratch, 3 * n * S, kind, p->stream));
+            if (host) HIP_OR_FAIL(p->stage.down(dst, scratch, 3 * n * S, p->stream));
         }
     }
-    if (sync) HIP_OR_FAIL(hipStreamSynchronize(p->stream));
+    if (host)
+        HIP_OR_FAIL(p->stage.finish(p->stream));
+    else if (sync)
+        HIP_OR_FAIL(hipStreamSynchronize(p->stream));
     return SW1D_OK;
 }
 
 int sw1d_set_state(sw1d_plan* p, const void* host)
 {
     if (!p || !host) return fail(SW1D_EINVAL, "null argument");
-    return copy_state(p, host, nullptr, true, hipMemcpyHostToDevice);
+    return copy_state(p, host, nullptr, true, true);
 }
 
 int sw1d_get_state(sw1d_plan* p, void* host)
 {
     if (!p || !host) return fail(SW1D_EINVAL, "null argument");
-    return copy_state(p, nullptr, host, false, hipMemcpyDeviceToHost);
+    return copy_state(p, nullptr, host, false, true);
 }
 
 int sw1d_set_state_device(sw1d_plan* p, const void* dptr)
 {
     if (!p || !dptr) return fail(SW1D_EINVAL, "null argument");
-    return copy_state(p, dptr, nullptr, true, hipMemcpyDeviceToDevice);
+    return copy_state(p, dptr, nullptr, true, false);
 }
 
 int sw1d_get_state_device(sw1d_plan* p, void* dptr)
 {
     if (!p || !dptr) return fail(SW1D_EINVAL, "null argument");
-    return copy_state(p, nullptr, dptr, false, hipMemcpyDeviceToDevice);
+    return copy_state(p, nullptr, dptr, false, false);
 }
 
 int sw1d_advance(sw1d_plan* p, int64_t nsteps)
@@ -950,9 +949,9 @@ int sw1d_advance_noalloc(const sw1d_problem* q, void* d_state, int64_t nsteps, v
     p.simds = device_simds();
     // launches one by one: no launch graph is captured or instantiated
     p.classic_graph_failed = true;
-    rc = copy_state(&p, d_state, nullptr, true, hipMemcpyDeviceToDevice, false);
+    rc = copy_state(&p, d_state, nullptr, true, false, false);
     if (rc == SW1D_OK) rc = sw1d_advance(&p, nsteps);
-    if (rc == SW1D_OK) rc = copy_state(&p, nullptr, d_state, false, hipMemcpyDeviceToDevice, false);
+    if (rc == SW1D_OK) rc = copy_state(&p, nullptr, d_state, false, false, false);
     if (rc == SW1D_OK) {
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) rc = fail(SW1D_EDEVICE, "launch: %s", hipGetErrorString(e));
@@ -1110,6 +1109,7 @@ struct sw1d_batch {
     int32_t waves = 4;  // as set by the caller (the tiles have their own)
     int32_t cus = 0;
     hipStream_t stream = nullptr;
+    HostStage stage;  // host copies of the state
     // launches of an advance of group_steps
     int64_t group_steps = -1;
     std::vector<BatchGroup> groups;
@@ -1199,6 +1199,7 @@ int sw1d_batch_create(sw1d_batch** out, int32_t precision, int64_t count, const 
     }
     B->cus = cus;
     const size_t bytes = (size_t)B->total * B->S;
+    if (bytes <= HostStage::kMost) B->stage.reserve(bytes);
     if (hipStreamCreateWithFlags(&B->stream, hipStreamNonBlocking) != hipSuccess ||
         hipMalloc(&B->a, bytes) != hipSuccess || hipMalloc(&B->b, bytes) != hipSuccess ||
         hipMalloc(&B->jobs, B->jobs_host.size()) != hipSuccess) {
@@ -1223,16 +1224,16 @@ int sw1d_batch_destroy(sw1d_batch* B)
 int sw1d_batch_set_state(sw1d_batch* B, const void* host)
 {
     if (!B || !host) return fail(SW1D_EINVAL, "null argument");
-    HIP_OR_FAIL(hipMemcpyAsync(B->a, host, (size_t)B->total * B->S, hipMemcpyHostToDevice, B->stream));
-    HIP_OR_FAIL(hipStreamSynchronize(B->stream));
+    HIP_OR_FAIL(B->stage.up(B->a, host, (size_t)B->total * B->S, B->stream));
+    HIP_OR_FAIL(B->stage.finish(B->stream));
     return SW1D_OK;
 }
 
 int sw1d_batch_get_state(sw1d_batch* B, void* host)
 {
     if (!B || !host) return fail(SW1D_EINVAL, "null argument");
-    HIP_OR_FAIL(hipMemcpyAsync(host, B->a, (size_t)B->total * B->S, hipMemcpyDeviceToHost, B->stream));
-    HIP_OR_FAIL(hipStreamSynchronize(B->stream));
+    HIP_OR_FAIL(B->stage.down(host, B->a, (size_t)B->total * B->S, B->stream));
+    HIP_OR_FAIL(B->stage.finish(B->stream));
     return SW1D_OK;
 }
 
