@@ -34,19 +34,12 @@ public:
     }
     HostStage(const HostStage&) = delete;
     HostStage& operator=(const HostStage&) = delete;
-    // Allocates for `most` bytes, of all copies between two calls of finish(), or
-    // of those that come first where that is more than kMost.  Called where the
-    // object allocates its device memory: a later allocation could break another
-    // thread's stream capture.
-    void reserve(size_t most)
-    {
-        cap_ = std::min(kMost, round(most));
-        if (cap_ > 0 && hipHostMalloc((void**)&p_, cap_, hipHostMallocDefault) != hipSuccess) {
-            (void)hipGetLastError();
-            p_ = nullptr;
-            cap_ = 0;
-        }
-    }
+    // For `most` bytes, of all copies between two calls of finish(), or of those
+    // that come first where that is more than kMost.  The first copy allocates
+    // (15 to 50 us; states that stay on the GPU need no staging memory).  While
+    // another thread captures a stream in the strictest mode it fails, as the
+    // copy's wait always has.
+    void reserve(size_t most) { cap_ = std::min(kMost, round(most)); }
 
     hipError_t up(void* dev, const void* host, size_t bytes, hipStream_t s)
     {
@@ -92,6 +85,12 @@ private:
     size_t take(size_t bytes)
     {
         if (used_ + bytes > cap_) return kNone;
+        if (!p_ && hipHostMalloc((void**)&p_, cap_, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            p_ = nullptr;
+            cap_ = 0;
+            return kNone;
+        }
         const size_t at = used_;
         used_ = std::min(cap_, at + round(bytes));
         return at;
