@@ -5,7 +5,7 @@ sweep appends a timing line, and the analysis keeps the fastest configuration
 per problem size (pyAnalysisTools/analysis_help.py:31-64, `QualityRuns`).  The
 same idea here, on the device and per size class: problems are grouped by
 floor(log2 nX); for each class a sample batch is timed with every candidate
-tile width (output points per trapezoid tile), and the class gets the fastest.
+`tile_points`, and the class gets the fastest.
 
 `choose` is a pure function of the timing table, so a given set of timings
 always gives the same choice: the minimum time per point-update wins, and
@@ -13,10 +13,12 @@ candidates within `tie` of the minimum resolve to the wider tile (fewer
 redundant halo points).  Classes with no timing take the choice of the
 nearest timed class below, else above.
 
-A second pass tunes the waves per workgroup of the persistent launch (the
-tiles a workgroup works on at once, the reference's "diamonds per block"):
-the whole workload with the chosen tiles is timed at 2, 4 and 8 waves and
+A second pass tunes the waves per workgroup (the reference's "diamonds per
+block"): the whole workload with the chosen tiles is timed at 2, 4 and 8 waves and
 `choose_waves` keeps the fastest, the default 4 when it is within `tie`.
+
+Batches check both settings and run tiles of their own shapes, so neither
+changes a batch's time any more.
 
 A third table serves single plans of the shared swept algorithm: the node
 width (the reference's tpb, the points one diamond spans) per equation,

@@ -1,16 +1,16 @@
 """Runs the library's hot kernels a few launches each, for hardware-counter
 collection.  A counter pass (rocprofv3 --pmc) serialises and instruments every
 dispatch, so this driver keeps the dispatch count small (tens per kernel, a
-few hundred in all) and prints a line after each group.  Plans and batches
-launch directly (SW1D_LAUNCH_GRAPHS=0): counter collection follows kernel
+few hundred in all) and prints a line after each group.  Plans launch
+directly (SW1D_LAUNCH_GRAPHS=0): counter collection follows kernel
 dispatches, not graph launches.
 
 Groups (FP64, the bench's configurations):
-  ks     KS swept, nX = 2^20, node width 1024 (up, diamonds, down)
+  ks     KS swept, nX = 2^20, node width 1024 (wide tiles)
   heat   heat swept, insulated ends, nX = 2^20, node width 512
   euler  Sod swept, nX = 2^20, node width 512
   batch  the batched workload: 4096 heat/KS problems of nX = floor(2^U[10,16]),
-         5000 steps, tuned tiles and waves, FP64 then FP32 (one launch each)
+         5000 steps, FP64 then FP32
   copy   a plain copy kernel of known size (torch.neg over float32), the
          reference for scaling FETCH_SIZE / WRITE_SIZE
 

@@ -35,8 +35,7 @@ def _pkg():
 
 
 def ks_batch(sw, wl, ntraj, seed):
-    """The plain batched solver on `ntraj` seeded trajectories, with the tuned
-    waves per workgroup (the tile width of nX = 1024 is the default 512)."""
+    """The plain batched solver on `ntraj` seeded trajectories."""
     at = importlib.import_module("1dsweptcuda_amd.autotune")
     b = sw.Batch(np.full(ntraj, sw.KS, np.int32), np.full(ntraj, NX, np.int64), np.full(ntraj, DT),
                  np.full(ntraj, DX), waves=at.load_waves())

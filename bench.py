@@ -3,18 +3,19 @@
 Workload (default): Kuramoto-Sivashinsky, FP64, nX = 2^20, dx = 0.5,
 dt = 0.005, IC 2cos(19 pi x/128) + N(0, 1e-3) noise (seed 1), shared swept
 algorithm.  A "step" is one time step of the whole domain (nX point-updates).
-The timed region is --steps steps rounded up to whole swept tile launches (a
-diamond advances W/8 = 128 steps at node width 1024; at least 160 launches),
-with the state already in HBM, bracketed by device synchronisation; "steps"
-in the output is the count actually timed.  Warm-up is rounded the same way.
-The classic algorithm (one launch per RK stage) is timed on the same input
-for the swept/classic ratio.
+The timed region is --steps steps rounded up to whole heights of a swept tile
+(H = W/8 = 128 steps at node width 1024; at least 160 of them), with the state
+already in HBM, bracketed by device synchronisation; "steps" in the output is
+the count actually timed.  Warm-up is rounded the same way.  The classic
+algorithm (one launch per step) is timed on the same input for the
+swept/classic ratio.
 
-The roofline entry is for the dominant kernel (the swept diamond): its
-average duration comes from hipEvents recorded around every launch on the
-plan's stream during a second pass over the same steps; achieved = algorithmic
-FP64 flops per launch (40 flop per KS point-update x nX x W/8 steps) / that
-duration.
+The roofline entry is for the kernel that runs the timed steps, the
+workgroup-wide overlapped tile: its time comes from hipEvents recorded around
+every launch on the stream of a second plan, of the overlapped tiles' own
+algorithm (3), over the same steps, so the same launches.  It is given per H
+steps ("avg_launch_us", "flop_per_launch": 40 flop per KS point-update x nX x
+H) and per kernel launch ("kernel_launches", "avg_kernel_us").
 
 The CPU baseline is the C oracle (the same KS stages) on a bounded sample of
 the same workload (same nX, fewer steps), timed on this host with OpenMP over
@@ -39,21 +40,19 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 KS_FLOP_PER_PU = 40          # stutterStep 20 + finalStep 20 (KS1D_SweptShared.cu:159-171)
-KS_SWEPT_BYTES_PER_PU = 256  # per tile launch: (u, u_half) read + written, 32 B / (W/8 steps) * W
 FP64_PEAK_TFLOPS = 78.6
 HBM_PEAK_GBS = 8000.0
-# HBM bytes per whole-diamond launch (nX, node width) -> bytes, from rocprofv3
-# FETCH_SIZE and WRITE_SIZE per dispatch, each scaled by its reading for a copy
-# kernel of known size (profiles/ks_swept_diamond_nx1048576_hbm_bytes.md).
-DIAMOND_TRAFFIC_BYTES = {(1 << 20, 512): 33.96e6, (1 << 20, 1024): 34.77e6}
+# HBM bytes of H = 128 steps at nX = 2^20, from rocprofv3 FETCH_SIZE and
+# WRITE_SIZE per dispatch, each scaled by its reading for a copy kernel of known
+# size (profiles/ks_wide_nx1048576.md).
+WIDE_TRAFFIC_BYTES = {(1 << 20, 128): 34.6e6}
 METRIC = "point-updates/s on 1 GPU at stated error vs FP64 oracle: swept vs classic/batch/NN"
 # The reference's published figure for the same quantity: KS FP64 shared swept at
 # nX = 2^20, 105.408 us per time step on a Tesla K40c
 # (ResultPlots/ConferencePaper/BestRuns.csv:14).
 REFERENCE_KS_SWEPT_PU_PER_S = (1 << 20) / 105.408e-6
-# Timed and warm-up steps are whole tile launches (a swept advance of fewer
-# steps than one tile runs classic steps instead), at least this many of them:
-# 160 launches of the 2^20-point diamond are ~25 ms of GPU time.
+# Timed and warm-up steps are whole tile heights, at least this many of them:
+# 160 x 128 steps of 2^20 points are ~18 ms of GPU time.
 MIN_TIMED_LAUNCHES = 160
 MIN_WARM_LAUNCHES = 160
 
@@ -77,8 +76,7 @@ def _whole_launches(per, requested, minimum):
 def _warm(plan, steps, minimum=40):
     """Untimed steps before a timed run: at least `steps`, rounded up to whole
     tile launches, and at least `minimum` launches, so the plan's one-time
-    set-up (the launch graphs it captures on its first long advance) stays out
-    of the timed region."""
+    set-up (a classic plan's launch graph) stays out of the timed region."""
     plan.advance(_whole_launches(plan.info()["tile_steps"], steps, minimum))
 
 
@@ -136,20 +134,21 @@ def main():
     secs = _timed(plan, steps)
     value = n * steps / secs
 
-    # per-kernel durations over the same number of steps: hipEvents recorded
-    # around every launch on the plan's stream
-    plan.set_profiling(True)
-    plan.advance(steps)
-    plan.synchronize()
-    dn, dms = plan.kernel_stats(sw.K_DIAMOND)
-    sn, sms = plan.kernel_stats(sw.K_SPLIT)
-    plan.set_profiling(False)
     plan.close()
-    launches = dn + sn
-    if launches == 0 or dms + sms <= 0.0:
-        raise SystemExit(f"bench: the profiled pass of {steps} steps recorded no diamond launch "
-                         f"(tile height {H} steps)")
-    avg_ms = (dms + sms) / launches
+
+    # per-kernel durations over the same number of steps: hipEvents recorded
+    # around every launch on the stream of a plan of the same tiles
+    tplan = sw.Plan(sw.KS, n, dt, algorithm=sw.TRAPEZOID, node_width=128)
+    tplan.set_state(u0)
+    tplan.advance(warm)
+    tplan.set_profiling(True)
+    tplan.advance(steps)
+    tplan.synchronize()
+    launches, kernel_ms = tplan.kernel_stats(sw.K_DIAMOND)
+    tplan.close()
+    if launches == 0 or kernel_ms <= 0.0:
+        raise SystemExit(f"bench: the profiled pass of {steps} steps recorded no tile launch")
+    avg_ms = kernel_ms / (steps // H)
     pu_per_launch = n * H
     flops = KS_FLOP_PER_PU * pu_per_launch
     achieved_tf = flops / (avg_ms * 1e-3) / 1e12
@@ -163,10 +162,9 @@ def main():
     csecs = _timed(cplan, csteps)
     classic_value = n * csteps / csecs
     cplan.close()
-    # HBM roofline of the classic stages over the wall time of the timed steps
-    # (both stage launches and anything between them): predictor reads u and
-    # writes u_half (16 B), corrector reads u_half and u and writes u (24 B).
-    classic_gbs = 40 * n * csteps / csecs / 1e9
+    # HBM roofline of the classic steps over the wall time of the timed steps
+    # (the launches and the gaps between them): a step reads and writes u (16 B).
+    classic_gbs = 16 * n * csteps / csecs / 1e9
     _progress("classic")
 
     out = {
@@ -195,17 +193,19 @@ def main():
         "classic": {"value": classic_value, "steps": csteps, "ms_per_step": csecs / csteps * 1e3,
                     "roofline": {"bound": "hbm", "achieved": classic_gbs, "peak": HBM_PEAK_GBS,
                                  "unit": "GB/s", "frac": classic_gbs / HBM_PEAK_GBS,
-                                 "algorithmic_bytes_per_pu": 40}},
+                                 "algorithmic_bytes_per_pu": 16}},
         "swept_over_classic": value / classic_value,
         "roofline": {"bound": "fp64_valu", "compute": "FP64 vector ALU (no MFMA); peak = MI355X FP64 vector",
-                     "kernel": "k_ks_swept<double,%d,DIAMOND>" % (W // 64),
+                     "kernel": "k_wide<double,KS>: workgroup-wide overlapped tiles, %d steps per launch"
+                               % round(steps / launches),
                      "achieved": achieved_tf, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved_tf / FP64_PEAK_TFLOPS,
-                     "traffic": DIAMOND_TRAFFIC_BYTES.get((n, W)),
-                     "avg_launch_us": avg_ms * 1e3, "launches": launches,
+                     "traffic": WIDE_TRAFFIC_BYTES.get((n, H)),
+                     "avg_launch_us": avg_ms * 1e3, "launches": steps // H,
+                     "kernel_launches": launches, "avg_kernel_us": kernel_ms / launches * 1e3,
                      "wall_us_per_tile_launch": secs / (steps // H) * 1e6,
                      "flop_per_launch": flops,
-                     "algorithmic_bytes_per_launch": 32 * n},
+                     "algorithmic_bytes_per_launch": 16 * n * launches // (steps // H)},
     }
     extras = set() if args.no_extras else set(args.extras.split(",")) - {"none", ""}
     sections = (("trapezoid", lambda: _trapezoid(sw, n, dt, u0, args)),
@@ -361,8 +361,8 @@ def _trapezoid(sw, n, dt, u0, args):
 
 
 def _batched(sw, count=4096, steps=5000, loop_sample=512):
-    """4096 uneven periodic heat/KS problems, 5000 steps, one persistent launch
-    per precision, against a per-problem launch loop (trapezoid plans)."""
+    """4096 uneven periodic heat/KS problems, 5000 steps, all of them in each
+    launch, against a per-problem launch loop (trapezoid plans)."""
     wl = importlib.import_module("1dsweptcuda_amd.workloads")
     at = importlib.import_module("1dsweptcuda_amd.autotune")
     eq, nx, dt, dx = wl.batch_problems(count, seed=2024)
@@ -378,7 +378,7 @@ def _batched(sw, count=4096, steps=5000, loop_sample=512):
     for prec, name in ((sw.F64, "f64"), (sw.F32, "f32")):
         with sw.Batch(eq, nx, dt, dx, precision=prec, tile_points=tps, waves=waves) as b:
             b.set_state(packed)
-            b.advance(steps)  # captures the graph
+            b.advance(steps)  # plans the launches of this step count
             b.set_state(packed)
             t0 = time.perf_counter()
             device_ms = b.advance_timed(steps)  # returns after the launch completes
@@ -392,7 +392,7 @@ def _batched(sw, count=4096, steps=5000, loop_sample=512):
         p = sw.Plan(int(eq[i]), int(nx[i]), float(dt[i]), algorithm=sw.TRAPEZOID, node_width=256,
                     bc=sw.BC_PERIODIC, dx=float(dx[i]))
         p.set_state(ics[i])
-        _warm(p, 0)  # captures the plan's launch graphs outside the timed loop
+        _warm(p, 0)
         p.set_state(ics[i])
         plans.append(p)
     for p in plans:
@@ -499,7 +499,7 @@ def _oracle_check(sw, n, dt, u0, W, steps):
     want = pyoracle.ks_run(u0, steps, pyoracle.ks_consts(dt), max(1, min(16, avail)))
     diff = np.abs(got - want)
     scale = float(np.max(np.abs(want)))
-    return {"steps": steps, "diamond_launches": max(steps // H - 1, 0), "bitwise_equal": bool(np.array_equal(got, want)),
+    return {"steps": steps, "tile_heights": steps // H, "bitwise_equal": bool(np.array_equal(got, want)),
             "max_abs_diff": float(diff.max()), "max_rel_diff": float(diff.max() / scale) if scale else 0.0,
             "tolerance_rel": 1e-12}
 

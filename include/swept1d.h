@@ -68,7 +68,8 @@ typedef struct sw1d_problem {
     double dt;           /* time step, argv[3] */
     double dx;           /* 0: reference value (heat ds 0.001, KS 0.5, Euler 1/(nx-2)) */
     double alpha;        /* heat diffusivity; 0: reference 8.418e-5 (Heat:56) */
-    int32_t tile_depth;  /* SW1D_TRAPEZOID: stages per launch in units of 32/R (0: 1) */
+    int32_t tile_depth;  /* SW1D_TRAPEZOID: 0, 1 or 2; checked and counted in the plan's
+                          * steps per tile (the tiles choose their own depth) */
     int32_t reserved;    /* must be 0 */
 } sw1d_problem;
 
