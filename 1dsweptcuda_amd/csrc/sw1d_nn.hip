@@ -442,9 +442,9 @@ constexpr int64_t P_W6 = P_MID + 4 * MID_SZ, P_B6 = P_W6 + TAPS * C;
 constexpr int64_t NPARAM = P_B6 + 1;
 
 // -------------------------------------- whole network, a segment of a sample ---
-// Inference at nx = 1024: a workgroup takes SEG positions (a half, a quarter or
-// an eighth) of a periodic sample through all six layers in one launch, its
-// activation (BF16 rows of 64 channels) in LDS, so no activation goes to memory.
+// Inference at multiples of 256 positions: a workgroup takes SEG positions of a
+// periodic sample through all six layers in one launch, its activation (BF16
+// rows of 64 channels) in LDS, so no activation goes to memory.
 // Tile row q is position p0 - 10 + q: the ten positions on each side that the
 // five 5-tap layers reach are the neighbouring segment's, computed here too
 // (every layer computes rows 2 .. SEG+17, of which its own reach is exact).
@@ -460,12 +460,11 @@ constexpr int64_t NPARAM = P_B6 + 1;
 // separate waves take 90% of their sum).  A small batch is bound by a
 // workgroup's life, the chain of six layers, and a whole sample per workgroup
 // left the other CUs idle.  So the segments get smaller with the batch; 64
-// samples take 23 us and 8 take 18, where a workgroup per sample took 58 for
-// any batch up to 256, and 256 take 57.  The weights pass through a ring of
+// samples of 1024 positions take 23 us and 8 take 18, where a workgroup per
+// sample took 58 for any batch up to 256, and 256 take 57.  The weights pass through a ring of
 // three steps, the next on its way from memory while one is used; they are the
 // MFMA's row operand, so that a lane holds four channels of a position, one
 // 8-byte store instead of four of 2.
-constexpr int XN = 1024;                 // positions per sample
 constexpr int STEPS = 2 * TAPS;          // MFMA steps of a layer: 32 input channels of a tap each
 constexpr int SLAB = C * 32;             // weights of a step, [co][32 ci]
 
@@ -493,20 +492,21 @@ struct MidWeights { const __bf16* w[4]; };  // packed forward weights of L2-L5
 // TIN = double: in = FP64 states (normalised by inv_scale), out = in + out_scale
 // * du (another array: a neighbouring segment may still have to read in);
 // TIN = float: in = network inputs x, du written to du.
-template <typename TIN, int NSEG, int PB>
-__global__ __launch_bounds__(4 * XN / (NSEG * PB), 4) void k_net_fwd(const TIN* __restrict__ in, float inv_scale,
+template <typename TIN, int SEG, int PB>
+__global__ __launch_bounds__(4 * SEG / PB, 4) void k_net_fwd(const TIN* __restrict__ in, float inv_scale,
                                                           const float* __restrict__ P, MidWeights wf,
                                                           float* __restrict__ du, double* __restrict__ out,
-                                                          double out_scale)
+                                                          double out_scale, int X)
 {
-    constexpr int SEG = XN / NSEG, NW = SEG / (16 * PB), NTS = 64 * NW, ROWS = SEG + 20;
+    constexpr int NW = SEG / (16 * PB), NTS = 64 * NW, ROWS = SEG + 20;
     static_assert(NW >= 4 && NTS >= SEG && 3 * SLAB * 2 >= TAPS * (SEG + 4) * 4);
     __shared__ __attribute__((aligned(16))) __bf16 sA[ROWS * C];
     __shared__ __attribute__((aligned(16))) __bf16 sW[3 * SLAB];  // ring of three steps' weights
     __shared__ __attribute__((aligned(16))) float sB[4 * C];      // biases of layers 2-5
     float* sF = reinterpret_cast<float*>(sW + 2 * SLAB);          // network input (before step 2's weights)
     float* sS = reinterpret_cast<float*>(sW);                     // output-layer tap sums (after layer 5)
-    const int tid = threadIdx.x, b = blockIdx.x / NSEG, p0 = blockIdx.x % NSEG * SEG;
+    const int tid = threadIdx.x, nseg = X / SEG, p0 = (int)(blockIdx.x % nseg) * SEG;
+    const int64_t row = (int64_t)(blockIdx.x / nseg) * X;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
     WeightStep<NTS> w0, w1, ws;
@@ -515,7 +515,7 @@ __global__ __launch_bounds__(4 * XN / (NSEG * PB), 4) void k_net_fwd(const TIN* 
     ws.load(wf.w[0], 2, tid);
     // layer 1 (stage_l1) into every tile row
     for (int i = tid; i < ROWS + 4; i += NTS)
-        sF[i] = (float)in[(int64_t)b * XN + ((p0 - 12 + i) & (XN - 1))] * inv_scale;
+        sF[i] = (float)in[row + wrapx(p0 - 12 + i, X)] * inv_scale;
     if (tid < 4 * C) sB[tid] = P[P_MID + (tid / C) * MID_SZ + TAPS * C * C + tid % C];
     {
         const int c8 = tid % (C / 8);
@@ -649,7 +649,7 @@ __global__ __launch_bounds__(4 * XN / (NSEG * PB), 4) void k_net_fwd(const TIN* 
     }
     __syncthreads();
     if (tid >= SEG) return;
-    const int64_t o = (int64_t)b * XN + p0 + tid;
+    const int64_t o = row + p0 + tid;
     float s = P[P_B6];
 #pragma unroll
     for (int t = 0; t < TAPS; ++t) s += sS[t * (SEG + 4) + tid + t];
@@ -1330,55 +1330,57 @@ int nn_layers(sw1d_nn* N, int B, const TIN* in, float inv_scale)
     return SW1D_OK;
 }
 
-// Segments per sample of the whole-network kernel: the fewest microseconds for
-// B samples on `cus` compute units.  A launch lasts as long as the CU with most
-// workgroups; measured with 1 .. cap of them side by side (cap by LDS).
-int net_segments(int64_t B, int cus)
+// Positions per workgroup of the whole-network kernel: the fewest microseconds
+// for B samples of X positions on `cus` compute units.  A launch lasts as long
+// as the CU with most workgroups; measured with 1 .. cap of them side by side
+// (cap by LDS).
+int net_segment(int64_t B, int64_t X, int cus)
 {
-    struct Split { int segs, cap; float us[6]; };
-    static constexpr Split splits[] = {{8, 5, {0, 18.f, 23.f, 30.f, 38.f, 47.f}}, {4, 3, {0, 23.f, 34.f, 50.f}},
-                                       {2, 2, {0, 37.f, 57.f}}};
-    int best = 2;
+    struct Split { int seg, cap; float us[6]; };
+    static constexpr Split splits[] = {{128, 5, {0, 18.f, 23.f, 30.f, 38.f, 47.f}}, {256, 3, {0, 23.f, 34.f, 50.f}},
+                                       {512, 2, {0, 37.f, 57.f}}};
+    int best = 0;
     double least = 0;
     for (const Split& c : splits) {
-        const int64_t m = (c.segs * B + cus - 1) / cus;
+        if (X % c.seg != 0) continue;
+        const int64_t m = (B * (X / c.seg) + cus - 1) / cus;
         const double us = (double)(m / c.cap) * c.us[c.cap] + c.us[m % c.cap];
-        if (least == 0 || us < least) {
+        if (best == 0 || us < least) {
             least = us;
-            best = c.segs;
+            best = c.seg;
         }
     }
     return best;
 }
 
-template <typename TIN, int NSEG, int PB>
+template <typename TIN, int SEG, int PB>
 void launch_net(sw1d_nn* N, int B, const TIN* in, float inv_scale, double* out)
 {
     const MidWeights w{{N->wf[0], N->wf[1], N->wf[2], N->wf[3]}};
-    hipLaunchKernelGGL((k_net_fwd<TIN, NSEG, PB>), dim3(B * NSEG), dim3(4 * XN / (NSEG * PB)), 0, N->stream, in,
-                       inv_scale, N->p, w, N->du, out, N->out_scale);
+    hipLaunchKernelGGL((k_net_fwd<TIN, SEG, PB>), dim3((unsigned)((int64_t)B * (N->X / SEG))), dim3(4 * SEG / PB), 0,
+                       N->stream, in, inv_scale, N->p, w, N->du, out, N->out_scale, N->X);
 }
 template <typename TIN>
 void net_forward(sw1d_nn* N, int B, const TIN* in, float inv_scale, double* out)
 {
-    switch (net_segments(B, N->cus)) {
-    case 8: return launch_net<TIN, 8, 2>(N, B, in, inv_scale, out);
-    case 4: return launch_net<TIN, 4, 2>(N, B, in, inv_scale, out);
-    default: return launch_net<TIN, 2, 4>(N, B, in, inv_scale, out);
+    switch (net_segment(B, N->X, N->cus)) {
+    case 128: return launch_net<TIN, 128, 2>(N, B, in, inv_scale, out);
+    case 256: return launch_net<TIN, 256, 2>(N, B, in, inv_scale, out);
+    default: return launch_net<TIN, 512, 4>(N, B, in, inv_scale, out);
     }
 }
 
 // Inference of B samples.  u == nullptr: from the FP32 inputs in N->x to du
 // in N->du.  Otherwise from the FP64 states u (normalised on the fly by
 // 1/in_scale) to out = u + out_scale * du, another array.  One launch of the
-// whole-network kernel at nx = 1024; five launches when nx is another multiple
-// of the 256-position tile (or infer_mode = 1), these two with the same bits;
+// whole-network kernel where nx is a multiple of 256 (2048, 128 samples: 60 us
+// against 98; 512, 8 samples: 19 against 33), or five launches (infer_mode = 1), these two with the same bits;
 // otherwise 64-position tiles and the training's output layer.
 int nn_infer(sw1d_nn* N, int B, const double* u, double* out)
 {
     const int X = N->X;
     const int64_t plane = (int64_t)B * X;
-    if (X == XN && N->infer_mode != 1) {
+    if (X % TILE_F == 0 && N->infer_mode != 1) {
         if (u)
             net_forward<double>(N, B, u, (float)(1.0 / N->in_scale), out);
         else
@@ -1624,7 +1626,7 @@ int sw1d_nn_set_scales(sw1d_nn* N, double in_scale, double out_scale)
 int sw1d_nn_set_inference(sw1d_nn* N, int32_t mode)
 {
     if (!N || mode < 0 || mode > 2) return nn_fail(SW1D_EINVAL, "inference mode must be 0, 1 or 2");
-    if (mode == 2 && N->X != XN) return nn_fail(SW1D_EINVAL, "the whole-network kernel needs nx = 1024");
+    if (mode == 2 && N->X != 1024) return nn_fail(SW1D_EINVAL, "the whole-network kernel needs nx = 1024");
     if (mode == 1 && N->X % TILE_F != 0)
         return nn_fail(SW1D_EINVAL, "the per-layer inference kernels need nx to be a multiple of 256");
     N->infer_mode = mode;

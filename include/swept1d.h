@@ -228,8 +228,7 @@ int sw1d_nn_create(sw1d_nn** nn, int32_t nx, int32_t max_batch, uint64_t seed);
 int sw1d_nn_destroy(sw1d_nn* nn);
 int sw1d_nn_set_scales(sw1d_nn* nn, double in_scale, double out_scale);
 /* Inference kernels (forward and surrogate steps): 0 = automatic (one
- * whole-network launch at nx = 1024, per-layer launches for other multiples
- * of 256, the training kernels otherwise), 1 = per-layer launches (nx a
+ * whole-network launch at multiples of 256, the training kernels otherwise), 1 = per-layer launches (nx a
  * multiple of 256), 2 = the whole-network kernel (nx = 1024).  Every choice
  * gives the same bits. */
 int sw1d_nn_set_inference(sw1d_nn* nn, int32_t mode);
