@@ -35,10 +35,11 @@ public:
     HostStage(const HostStage&) = delete;
     HostStage& operator=(const HostStage&) = delete;
     // For `most` bytes, of all copies between two calls of finish(), or of those
-    // that come first where that is more than kMost.  The first copy allocates
-    // (15 to 50 us; states that stay on the GPU need no staging memory).  While
-    // another thread captures a stream in the strictest mode it fails, as the
-    // copy's wait always has.
+    // that come first where that is more than kMost.  The memory is allocated by
+    // the first copy after two rounds (15 to 50 us, and its first touch): an
+    // object whose state goes in and out once is as fast without it, one whose
+    // state stays on the GPU needs none.  While another thread captures a stream
+    // in the strictest mode that fails, as the copy's wait always has.
     void reserve(size_t most) { cap_ = std::min(kMost, round(most)); }
 
     hipError_t up(void* dev, const void* host, size_t bytes, hipStream_t s)
@@ -53,7 +54,7 @@ public:
     {
         const size_t at = count_ < kPending ? take(bytes) : kNone;
         if (at == kNone) {
-            populate(host, bytes);
+            if (bytes >= kPopulate) populate(host, bytes);
             return hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s);
         }
         const hipError_t e = hipMemcpyAsync(p_ + at, dev, bytes, hipMemcpyDeviceToHost, s);
@@ -72,11 +73,12 @@ public:
             memcpy(pending_[i].host, p_ + pending_[i].at, pending_[i].bytes);
         count_ = 0;
         used_ = 0;
+        if (rounds_ < 2) ++rounds_;
         return e;
     }
 
 private:
-    static constexpr size_t kNone = ~(size_t)0;
+    static constexpr size_t kNone = ~(size_t)0, kPopulate = 256u << 10;
     static constexpr int kPending = 4;
     struct Pending { void* host; size_t at, bytes; };
 
@@ -84,7 +86,7 @@ private:
     // offset of `bytes` free bytes; none until finish() where they do not fit
     size_t take(size_t bytes)
     {
-        if (used_ + bytes > cap_) return kNone;
+        if (used_ + bytes > cap_ || (!p_ && rounds_ < 2)) return kNone;
         if (!p_ && hipHostMalloc((void**)&p_, cap_, hipHostMallocDefault) != hipSuccess) {
             (void)hipGetLastError();
             p_ = nullptr;
@@ -113,7 +115,7 @@ private:
     char* p_ = nullptr;
     size_t cap_ = 0, used_ = 0;
     Pending pending_[kPending];
-    int count_ = 0;
+    int count_ = 0, rounds_ = 0;
 };
 
 }  // namespace sw1d

@@ -21,7 +21,7 @@ def test_plan_state_round_trip(sw, eq, prec, n):
     count = n * (3 if eq == 2 else 1)
     want = np.random.default_rng(n).standard_normal(count).astype(dtype)
     with sw.Plan(eq, n, 0.1 / (n - 2) if eq == 2 else 0.001, precision=prec, algorithm=sw.CLASSIC) as p:
-        for off in (0, 8, 4088):  # twice through the same staging memory, and at odd addresses
+        for off in (0, 8, 4088):  # directly, then through the same staging memory; at odd addresses
             src = np.zeros(count * want.itemsize + 8192, np.uint8)[off:off + want.nbytes].view(dtype)
             dst = np.full(count * want.itemsize + 8192, 7, np.uint8)
             src[:] = want + dtype(off)
@@ -36,7 +36,7 @@ def test_batch_state_round_trip(sw, nx):
     print(f"batch host copies nx={nx}", flush=True)
     want = np.random.default_rng(nx).standard_normal(nx)
     with sw.Batch(np.ones(1, np.int32), np.array([nx], np.int64), np.array([0.005]), np.array([0.5])) as b:
-        for k in range(2):
+        for k in range(3):
             b.set_state(want + k)
             assert np.array_equal(b.get_state(), want + k)
 
@@ -56,8 +56,10 @@ def test_gradient_of_a_batch_equals_that_of_its_samples_in_a_larger_network(sw, 
             nn.set_params(params)
             y = nn.forward(x)
             loss, g = nn.gradient(x, t)
-            again = nn.gradient(x, t)
-            assert again[0] == loss and np.array_equal(again[1], g)
+            for _ in range(2):  # directly, then through staging memory
+                again = nn.gradient(x, t)
+                assert again[0] == loss and np.array_equal(again[1], g)
+            assert np.array_equal(nn.forward(x), y)
             got.append((y, loss, g))
     assert np.array_equal(got[0][0], got[1][0]) and got[0][1] == got[1][1] and np.array_equal(got[0][2], got[1][2])
     # the loss of the outputs that forward() returned (float32 sums of 256 squares)
