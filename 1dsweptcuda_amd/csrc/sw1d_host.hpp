@@ -21,8 +21,7 @@
 namespace sw1d {
 
 // One object's staging memory (one thread at a time, like the object).  The
-// caller's memory has been read when up() returns and holds the result when
-// finish() has.
+// caller's memory has been read, and holds the results, when finish() returns.
 class HostStage {
 public:
     static constexpr size_t kMost = 1u << 20;

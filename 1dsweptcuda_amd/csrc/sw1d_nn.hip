@@ -12,7 +12,7 @@
 // x 64 input channels, staged in LDS in the operand layouts of the MFMA (8
 // consecutive K values per lane, 16-byte LDS reads).
 //
-// Training (one gradient at batch 64 x 1024: 160 us on the GPU, 480 us before)
+// Training (one gradient at batch 64 x 1024: 147 us on the GPU, 480 us before)
 // keeps two more forms of what a layer computes.  The FP32
 // pre-activations Z, for the GELU derivative, are stored in the accumulators'
 // own lane order, since only the lanes that hold the same outputs in the
@@ -26,6 +26,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <cstring>
@@ -821,19 +822,23 @@ __global__ __launch_bounds__(Tile<TF>::NT) void k_mid_bwd_data(const __bf16* __r
 // -2 .. 9 of A^T around them; the five taps' operands are that window shifted,
 // with no LDS.  The two waves of a quarter then add up through LDS (in the
 // accumulators' order, which k_reduce_grad undoes).
-// 256 workgroups of 8 waves at batch 64 x 1024 (one per CU): 21 MB of partials
-// for all layers, where one partial per 64 positions was 84 MB per layer.  All
+// At most 256 workgroups of 8 waves, one per CU, so that all run at once: 52 for
+// each 64 -> 64 layer and 24 for each edge layer, whose rounds are shorter (64
+// for each of the six left a second round of edge workgroups: a training
+// iteration of 64 samples 155.7 -> 152.5 us, of 8 103.4 -> 100.1).  17 MB of
+// partials for all layers, where one partial per 64 positions was 84 MB per layer.  All
 // weight gradients and their reduction: 35 us (67 MB of operands, 13 us at the
 // copy rate, then the partials), where a launch per layer with operands
 // transposed through LDS and a two-pass reduction took 340 us.
-constexpr int WG_SHARES = 64;
+constexpr int MID_SHARES = 52, EDGE_SHARES = 24;
+constexpr int WG_SHARES = MID_SHARES;  // partials that the buffer holds for each layer
 constexpr int NTG = 512;
 constexpr int64_t MIDP = TAPS * C * C + C;    // a 64 -> 64 layer's partial
 constexpr int64_t OUTP = TAPS * C + 1;        // the output layer's
 constexpr int64_t FIRSTP = C * TAPS + C;      // layer 1's
-__host__ __device__ inline int64_t part_offset(int y, int shares)
+__host__ __device__ inline int64_t part_offset(int y)
 {
-    return y <= 4 ? y * MIDP * shares : (4 * MIDP + OUTP) * shares;
+    return (y <= 4 ? y * MIDP : 4 * MIDP + OUTP) * WG_SHARES;
 }
 struct GradIn {
     const __bf16* dzt[4];  // dZ of L2..L5, [B][64][X]
@@ -1045,13 +1050,16 @@ __device__ __forceinline__ void grad_edge(const __bf16* __restrict__ rows, const
     }
 }
 
-__global__ __launch_bounds__(NTG) void k_grad_weights(GradIn in, float* __restrict__ part, int X, int groups)
+__global__ __launch_bounds__(NTG) void k_grad_weights(GradIn in, float* __restrict__ part, int X, int groups,
+                                                      int mids, int edges)
 {
     // the edge layers' sums, the largest user: 6 taps x 64 lanes of rows x 64 channels
     constexpr int64_t LDS = 6 * 64 * C > MIDP ? 6 * 64 * C : MIDP;
     __shared__ __attribute__((aligned(16))) float lds[LDS];
-    const int y = blockIdx.y, share = blockIdx.x, shares = gridDim.x;
-    float* p = part + part_offset(y, shares) + share * (y < 4 ? MIDP : (y == 4 ? OUTP : FIRSTP));
+    const bool mid = (int)blockIdx.x < 4 * mids;
+    const int shares = mid ? mids : edges, k = blockIdx.x - (mid ? 0 : 4 * mids);
+    const int y = k / shares + (mid ? 0 : 4), share = k % shares;
+    float* p = part + part_offset(y) + share * (y < 4 ? MIDP : (y == 4 ? OUTP : FIRSTP));
     if (y < 4)
         grad_mid(in.dzt[y], in.at[y], p, lds, X, groups, share, shares);
     else if (y == 4)
@@ -1062,7 +1070,7 @@ __global__ __launch_bounds__(NTG) void k_grad_weights(GradIn in, float* __restri
 
 // g[i] = the sum of the shares' partials in share order, one thread per
 // parameter, in the order the partials are stored in.
-__global__ __launch_bounds__(NT) void k_reduce_grad(const float* __restrict__ part, int shares,
+__global__ __launch_bounds__(NT) void k_reduce_grad(const float* __restrict__ part, int mids, int edges,
                                                     float* __restrict__ g)
 {
     int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x;
@@ -1092,7 +1100,8 @@ __global__ __launch_bounds__(NT) void k_reduce_grad(const float* __restrict__ pa
         len = FIRSTP;
         out = P_W1 + i;
     }
-    const float* p = part + part_offset(y, shares) + i;
+    const float* p = part + part_offset(y) + i;
+    const int shares = y < 4 ? mids : edges;
     float s = 0.f;
 #pragma unroll 8
     for (int k = 0; k < shares; ++k) s += p[k * len];
@@ -1453,9 +1462,11 @@ int nn_gradient(sw1d_nn* N, int B)
     in.dz1 = N->dZ[1];
     in.in = N->x;
     const int groups = (int)(nout / 32);
-    const int shares = groups / 4 < WG_SHARES ? (groups / 4 > 0 ? groups / 4 : 1) : WG_SHARES;
-    hipLaunchKernelGGL(k_grad_weights, dim3(shares, 6), dim3(NTG), 0, N->stream, in, N->part, X, groups);
-    hipLaunchKernelGGL(k_reduce_grad, dim3(nblk(NPARAM)), dim3(NT), 0, N->stream, N->part, shares, N->g);
+    const int most = groups / 4 > 0 ? groups / 4 : 1;
+    const int mids = std::min(MID_SHARES, most), edges = std::min(EDGE_SHARES, most);
+    hipLaunchKernelGGL(k_grad_weights, dim3(4 * mids + 2 * edges), dim3(NTG), 0, N->stream, in, N->part, X, groups, mids,
+                       edges);
+    hipLaunchKernelGGL(k_reduce_grad, dim3(nblk(NPARAM)), dim3(NT), 0, N->stream, N->part, mids, edges, N->g);
     NN_HIP(hipGetLastError());
     return SW1D_OK;
 }
