@@ -25,7 +25,7 @@ __global__ __launch_bounds__(S::NT) void k_batch(const BatchTile* __restrict__ t
                                                  const BatchJob<T>* __restrict__ jobs, const T* __restrict__ in,
                                                  T* __restrict__ out, int steps)
 {
-    __shared__ __attribute__((aligned(16))) T lds[S::LDS];
+    __shared__ __attribute__((aligned(16))) T lds[S::template lds<T>];
     const BatchTile t = tiles[blockIdx.x];
     const BatchJob<T>& J = jobs[t.job];
     Coef<T> k;

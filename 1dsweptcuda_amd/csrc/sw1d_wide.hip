@@ -16,7 +16,7 @@
 //   KS     2.62e9    4.07e10   1.59e11   5.86e11   9.25e11   9.36e11   diamonds
 //          5.10e9    7.9e10    2.28e11   6.4e11    1.08e12   1.18e12   wide
 //   heat   1.02e10   1.58e11   6.2e11    2.23e12   4.95e12   5.1e12    diamonds
-//          2.18e10   3.35e11   1.14e12   3.4e12    7.1e12    8.5e12    wide
+//          2.27e10   3.5e11    1.27e12   3.6e12    7.3e12    8.5e12    wide
 //   Euler  3.5e8     5.5e9     2.1e10    4.3e10    5.5e10    5.8e10    diamonds
 //          7.0e8     1.13e10   2.8e10    4.6e10    5.9e10    6.1e10    wide
 // (Euler before, one wave per tile: 1.3e8, 2.1e9, 8.3e9, 2.3e10, 3.1e10, 3.2e10
@@ -43,7 +43,7 @@ template <typename T, int EQ, class S>
 __global__ __launch_bounds__(S::NT) void k_wide(const T* __restrict__ in, T* __restrict__ out, int64_t n,
                                                 int64_t wout, int steps, int ends, Coef<T> k)
 {
-    __shared__ __attribute__((aligned(16))) T lds[S::LDS];
+    __shared__ __attribute__((aligned(16))) T lds[S::template lds<T>];
     const int64_t out0 = (int64_t)blockIdx.x * wout;
     const int count = (int)(n - out0 < wout ? n - out0 : wout);
     tile<T, EQ, S>(lds, in, out, n, n, out0, count, steps, ends, k);

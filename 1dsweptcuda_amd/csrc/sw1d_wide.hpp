@@ -43,14 +43,20 @@ struct Shape {
     static constexpr int WIN = NW * STRIDE + 2 * HL * P;     // points of the window
     static constexpr int K = HL * P / R;                     // steps between exchanges
     static_assert(K >= 1 && 4 * HL <= kWave, "the halo lanes hold at least one step's reach");
-    // LDS, in values: one component's window image, or the exchanged edges (two
-    // sets used in turn, so one barrier per exchange is enough)
-    static constexpr int EDGE = NW * 2 * HL * NC * P;
-    // lanes read and write the field themselves, where one component's image
-    // after the other through LDS takes longer (Euler, 4 cells per lane: 8.6 us
-    // for launch, load and store against 4.0)
-    static constexpr bool DIRECT = P <= 2 || EQ == EQ_EULER;
-    static constexpr int LDS = (!DIRECT && WIN > 2 * EDGE) ? WIN : 2 * EDGE;
+    static constexpr int EDGE = NW * 2 * HL * NC * P;  // exchanged edges, in values
+    // Lanes read and write the field themselves, 16 bytes at a time, where one
+    // component's image after the other through LDS takes longer: Euler (4 cells
+    // per lane: 8.6 us for launch, load and store against 5.5), heat up to eight
+    // points per lane (5: 3.4 against 2.6 us; a field of 2^18 points, 4000 steps:
+    // 361 -> 292 us in all) and FP32 KS up to five (3.0 against 2.1 us; 2^17, 1000
+    // steps: 321 -> 288 us).  FP64 KS and wider FP32 tiles lose more in their
+    // steps, whose registers the compiler then assigns worse (FP64, 4: 0.269
+    // against 0.245 us per step; FP32, 6: 0.311 against 0.303), than they gain.
+    template <typename T>
+    static constexpr bool direct = P <= 2 || EQ == EQ_EULER || (EQ == EQ_HEAT ? P <= 8 : P <= 5 && sizeof(T) == 4);
+    // LDS, in values: one component's window image, or the edges (two sets used
+    // in turn, so one barrier per exchange is enough)
+    template <typename T> static constexpr int lds = (!direct<T> && WIN > 2 * EDGE) ? WIN : 2 * EDGE;
 };
 
 // Field index of point g of the window, which may lie outside 0 .. n-1.
@@ -234,7 +240,7 @@ struct Steps {
 
 // One tile: out[out0 .. out0 + count) after `steps` steps from the field `in`
 // of n points (component stride cs in both).  The window starts R steps
-// before out0; lds holds Shape::LDS values.
+// before out0; lds holds Shape::lds<T> values.
 template <typename T, int EQ, class S>
 __device__ __forceinline__ void tile(T* lds, const T* __restrict__ in, T* __restrict__ out, int64_t n, int64_t cs,
                                      int64_t out0, int count, int steps, int ends, const Coef<T>& k)
@@ -248,7 +254,7 @@ __device__ __forceinline__ void tile(T* lds, const T* __restrict__ in, T* __rest
     const bool inside = win >= 0 && win + WIN <= n;
     const bool near = win >= -(n - 1) && win + WIN <= 2 * n - 1;
     Steps<T, EQ, S> st;
-    if constexpr (S::DIRECT) {
+    if constexpr (S::template direct<T>) {
         if (inside) {
 #pragma unroll
             for (int c = 0; c < NC; ++c) load_pts<T, P>(in + c * cs + win + x0, st.v[c]);
@@ -333,7 +339,7 @@ __device__ __forceinline__ void tile(T* lds, const T* __restrict__ in, T* __rest
     }
 
     const bool own = (lane >= HL || w == 0) && (lane < kWave - HL || w == NW - 1);
-    if constexpr (S::DIRECT) {
+    if constexpr (S::template direct<T>) {
         const int i0 = x0 - halo;
         if (own && i0 >= 0 && i0 + P <= count) {
 #pragma unroll
@@ -382,8 +388,8 @@ inline constexpr int kWaves = 4;  // one wave per SIMD: P sets the window
 // for Euler, whose steps are ten times as long
 inline constexpr Entry kKs[] = {
     {2, 10, {2.3f, .06f, .151f, .101f}, {2.1f, .02f, .143f, .085f}},
-    {4, 6, {3.0f, .6f, .248f, .173f}, {2.8f, .35f, .224f, .153f}},
-    {5, 4, {3.2f, .45f, .319f, .217f}, {3.0f, .2f, .301f, .193f}},
+    {4, 6, {3.0f, .6f, .248f, .173f}, {2.35f, .3f, .2245f, .1535f}},
+    {5, 4, {3.2f, .45f, .319f, .217f}, {2.15f, .3f, .300f, .188f}},
     {6, 4, {3.6f, .4f, .318f, .268f}, {3.3f, .25f, .301f, .226f}},
     {8, 4, {4.7f, .4f, .383f, .36f}, {3.7f, .2f, .377f, .296f}},
     {10, 2, {4.8f, .4f, .508f, .46f}, {4.2f, .35f, .469f, .374f}},
@@ -393,11 +399,11 @@ inline constexpr Entry kKs[] = {
     {19, 2, {8.5f, .9f, .834f, .87f}, {6.4f, .25f, .816f, .68f}},
 };
 inline constexpr Entry kHeat[] = {
-    {2, 8, {2.1f, .18f, .0371f, .0151f}, {2.1f, .08f, .0299f, .0110f}},
-    {3, 8, {2.7f, .38f, .0407f, .0193f}, {2.7f, .15f, .0348f, .0162f}},
-    {4, 6, {3.1f, .5f, .0446f, .0247f}, {2.9f, .2f, .0393f, .0199f}},
-    {5, 4, {3.3f, .4f, .0511f, .0292f}, {3.0f, .17f, .0482f, .0258f}},
-    {7, 4, {3.3f, .45f, .0621f, .0379f}, {3.3f, .25f, .0650f, .0330f}},
+    {2, 8, {2.1f, .18f, .0350f, .0151f}, {2.1f, .08f, .0299f, .0110f}},
+    {3, 8, {2.2f, .35f, .0420f, .0197f}, {2.35f, .1f, .0358f, .0163f}},
+    {4, 6, {2.35f, .45f, .0432f, .0245f}, {2.2f, .2f, .0410f, .0200f}},
+    {5, 4, {2.6f, .45f, .0503f, .0290f}, {2.35f, .2f, .0447f, .0256f}},
+    {7, 4, {3.0f, .6f, .0610f, .0355f}, {2.7f, .3f, .0542f, .0325f}},
     {9, 4, {4.1f, .5f, .0673f, .0462f}, {3.8f, .3f, .0625f, .0423f}},
     {12, 2, {4.8f, .6f, .0875f, .0622f}, {4.3f, .37f, .0819f, .0539f}},
     {15, 2, {5.6f, .7f, .106f, .0770f}, {5.0f, .3f, .0956f, .0623f}},
