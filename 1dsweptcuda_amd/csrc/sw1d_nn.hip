@@ -1166,14 +1166,17 @@ __global__ __launch_bounds__(NT) void k_gather(const float* __restrict__ sx, con
     t[i] = st[src];
 }
 
-// Relative L2 distance ||a - b|| / ||b|| partial sums per block: (sum (a-b)^2, sum b^2).
-__global__ __launch_bounds__(NT) void k_l2_parts(const double* __restrict__ a, const double* __restrict__ b,
-                                                 int64_t n, double* __restrict__ part)
+// Relative L2 distance ||a - b|| / ||b|| partial sums per block: (sum (a-b)^2, sum
+// b^2).  Block (k, p) adds points k NT .. of problem p, whose last block may be a
+// part of one (X is a multiple of 64).
+__global__ __launch_bounds__(NT) void k_l2_parts(const double* __restrict__ a, const double* __restrict__ b, int X,
+                                                 double* __restrict__ part)
 {
     __shared__ double r0[NT], r1[NT];
-    const int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x;
+    const int x = blockIdx.x * NT + threadIdx.x;
+    const int64_t i = (int64_t)blockIdx.y * X + x;
     double d = 0, s = 0;
-    if (i < n) {
+    if (x < X) {
         d = (a[i] - b[i]) * (a[i] - b[i]);
         s = b[i] * b[i];
     }
@@ -1188,8 +1191,9 @@ __global__ __launch_bounds__(NT) void k_l2_parts(const double* __restrict__ a, c
         __syncthreads();
     }
     if (threadIdx.x == 0) {
-        part[2 * blockIdx.x] = r0[0];
-        part[2 * blockIdx.x + 1] = r1[0];
+        const int64_t k = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
+        part[2 * k] = r0[0];
+        part[2 * k + 1] = r1[0];
     }
 }
 
@@ -1740,13 +1744,14 @@ extern "C" int sw1d_surrogate_advance(sw1d_nn* N, sw1d_batch* batch, int64_t sur
     if (k_steps < 1 || surrogate_steps < 0) return nn_fail(SW1D_EINVAL, "bad step counts");
     const int64_t B = bv.count, X = N->X, len = B * X;
     const unsigned blocks = nblk(len);
+    const int64_t per = (X + NT - 1) / NT;  // l2 blocks per problem
     if (N->int_len < len) {
         if (N->usave) (void)hipFree(N->usave);
         if (N->unn) (void)hipFree(N->unn);
         if (N->l2p) (void)hipFree(N->l2p);
         N->usave = N->unn = N->l2p = nullptr;
         if (dalloc(&N->usave, len) != hipSuccess || dalloc(&N->unn, len) != hipSuccess ||
-            dalloc(&N->l2p, 2 * (int64_t)blocks) != hipSuccess)
+            dalloc(&N->l2p, 2 * per * B) != hipSuccess)
             return nn_fail(SW1D_ENOMEM, "integrator scratch");
         N->int_len = len;
     }
@@ -1755,7 +1760,6 @@ extern "C" int sw1d_surrogate_advance(sw1d_nn* N, sw1d_batch* batch, int64_t sur
     double* u = static_cast<double*>(bv.state);
     double *cur = u, *other = N->usave;
     const size_t bytes = (size_t)len * sizeof(double);
-    const int64_t per = (X + NT - 1) / NT;  // l2 blocks per problem (X is a multiple of NT)
     int64_t judged = 0;
     // The judge runs in stream order: the plain solver on the batch's stream
     // waits for the network step (event a), the decision on the network's
@@ -1793,7 +1797,8 @@ extern "C" int sw1d_surrogate_advance(sw1d_nn* N, sw1d_batch* batch, int64_t sur
         if (rc) return nn_fail(rc, "plain solver step of the judge");
         NN_HIP(hipEventRecord(ev.b, bv.stream));
         NN_HIP(hipStreamWaitEvent(N->stream, ev.b, 0));
-        hipLaunchKernelGGL(k_l2_parts, dim3(blocks), dim3(NT), 0, N->stream, N->unn, u, len, N->l2p);
+        hipLaunchKernelGGL(k_l2_parts, dim3((unsigned)per, (unsigned)B), dim3(NT), 0, N->stream, N->unn, u, (int)X,
+                           N->l2p);
         hipLaunchKernelGGL(k_judge, dim3(1), dim3(NT), 0, N->stream, N->l2p, B, per, tol, N->keep, N->jacc);
         hipLaunchKernelGGL(k_keep_rows, dim3(blocks), dim3(NT), 0, N->stream, u, N->unn, N->keep, (int)X, len);
         NN_HIP(hipGetLastError());
