@@ -1777,13 +1777,13 @@ extern "C" int sw1d_surrogate_advance(sw1d_nn* N, sw1d_batch* batch, int64_t sur
     NN_HIP(hipEventCreateWithFlags(&ev.b, hipEventDisableTiming));
     NN_HIP(hipStreamSynchronize(bv.stream));
     hipLaunchKernelGGL(k_zero_f64, dim3(1), dim3(NT), 0, N->stream, N->jacc, (int64_t)2);
-    for (int64_t i = 1; i <= surrogate_steps; ++i) {
+    auto step = [&](int64_t i) -> int {
         const bool judge = judge_every > 0 && i % judge_every == 0;
         int rc = nn_infer(N, (int)B, cur, judge ? N->unn : other);
         if (rc) return rc;
         if (!judge) {
             std::swap(cur, other);
-            continue;
+            return SW1D_OK;
         }
         // plain solver from the same states: u <- solver^K(u)
         if (cur != u) {
@@ -1802,8 +1802,19 @@ extern "C" int sw1d_surrogate_advance(sw1d_nn* N, sw1d_batch* batch, int64_t sur
         hipLaunchKernelGGL(k_judge, dim3(1), dim3(NT), 0, N->stream, N->l2p, B, per, tol, N->keep, N->jacc);
         hipLaunchKernelGGL(k_keep_rows, dim3(blocks), dim3(NT), 0, N->stream, u, N->unn, N->keep, (int)X, len);
         NN_HIP(hipGetLastError());
+        return SW1D_OK;
+    };
+    int rc = SW1D_OK;
+    for (int64_t i = 1; i <= surrogate_steps && !rc; ++i) rc = step(i);
+    // the batch holds the last step that was taken, also where the next one failed
+    if (cur != u) {
+        const hipError_t e = hipMemcpyAsync(u, cur, bytes, hipMemcpyDeviceToDevice, N->stream);
+        if (e != hipSuccess && !rc) rc = nn_fail(SW1D_EDEVICE, "states into the batch", e);
     }
-    if (cur != u) NN_HIP(hipMemcpyAsync(u, cur, bytes, hipMemcpyDeviceToDevice, N->stream));
+    if (rc) {
+        (void)hipStreamSynchronize(N->stream);
+        return rc;
+    }
     double acc[2] = {0.0, 0.0};
     NN_HIP(hipMemcpyAsync(acc, N->jacc, sizeof(acc), hipMemcpyDeviceToHost, N->stream));
     NN_HIP(hipStreamSynchronize(N->stream));
