@@ -1270,6 +1270,8 @@ int nn_fail(int code, const char* msg, hipError_t e = hipSuccess)
 {
     g_nn_err = msg;
     if (e != hipSuccess) g_nn_err += std::string(": ") + hipGetErrorString(e);
+    // reported here, so not once more by the next call's launches
+    if (code == SW1D_EDEVICE || code == SW1D_ENOMEM) (void)hipGetLastError();
     return code;
 }
 #define NN_HIP(expr)                                          \

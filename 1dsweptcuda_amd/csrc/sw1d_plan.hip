@@ -33,6 +33,8 @@ int fail(int code, const char* fmt, ...)
     vsnprintf(buf, sizeof buf, fmt, ap);
     va_end(ap);
     g_err = buf;
+    // reported here, so not once more by the next call's launches
+    if (code == SW1D_EDEVICE || code == SW1D_ENOMEM) (void)hipGetLastError();
     return code;
 }
 

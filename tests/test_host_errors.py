@@ -64,3 +64,21 @@ with sw.Surrogate(nx, B, seed=0) as nn, sw.Batch(*ks(nx, B)) as b:
     assert np.array_equal(b.get_state(), u0 + 3 + done)
 print("done")
 ''' % done)
+
+
+def test_a_failed_call_does_not_fail_the_next(child):
+    """The runtime's last error, once reported, is not reported by the launches
+    of another object's next call."""
+    child(r'''
+nx = 1024
+with sw.Plan(sw.KS, nx, 0.005, algorithm=sw.CLASSIC) as p, sw.Batch(*ks(nx, 2)) as b, sw.Surrogate(nx, 2) as nn:
+    stub.stub_fail_malloc(C.c_long(0))
+    for f in (lambda: sw.Plan(sw.HEAT, nx, 1e-3), lambda: sw.Batch(*ks(nx, 2)), lambda: sw.Surrogate(nx, 2),
+              lambda: nn.advance(b, 1, 20, judge_every=0)):
+        raises(f, ENOMEM)
+        p.advance(3)
+        p.synchronize()
+        raises(f, ENOMEM)
+        nn.forward(np.zeros((2, nx), np.float32))
+print("done")
+''')
