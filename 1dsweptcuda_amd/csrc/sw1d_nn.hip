@@ -1752,6 +1752,7 @@ extern "C" int sw1d_surrogate_advance(sw1d_nn* N, sw1d_batch* batch, int64_t sur
         if (N->unn) (void)hipFree(N->unn);
         if (N->l2p) (void)hipFree(N->l2p);
         N->usave = N->unn = N->l2p = nullptr;
+        N->int_len = 0;  // also where an allocation fails
         if (dalloc(&N->usave, len) != hipSuccess || dalloc(&N->unn, len) != hipSuccess ||
             dalloc(&N->l2p, 2 * per * B) != hipSuccess)
             return nn_fail(SW1D_ENOMEM, "integrator scratch");

@@ -82,3 +82,24 @@ with sw.Plan(sw.KS, nx, 0.005, algorithm=sw.CLASSIC) as p, sw.Batch(*ks(nx, 2)) 
         nn.forward(np.zeros((2, nx), np.float32))
 print("done")
 ''')
+
+
+@pytest.mark.parametrize("more", [0, 1, 2])
+def test_rollout_after_a_failed_allocation(child, more):
+    """A larger batch whose scratch arrays cannot be allocated is refused; a
+    smaller one afterwards gets arrays of its own."""
+    child(r'''
+nx = 1024
+u0 = np.arange(nx, dtype=float)
+with sw.Surrogate(nx, 4, seed=0) as nn, sw.Batch(*ks(nx, 1)) as one, sw.Batch(*ks(nx, 4)) as four:
+    one.set_state(u0)
+    nn.advance(one, 1, 20, judge_every=0)
+    stub.stub_fail_malloc(C.c_long(%d))
+    raises(lambda: nn.advance(four, 1, 20, judge_every=0), ENOMEM)
+    stub.stub_fail_malloc(C.c_long(-1))
+    nn.advance(one, 2, 20, judge_every=0)
+    assert np.array_equal(one.get_state(), u0 + 3)
+    nn.advance(four, 2, 20, judge_every=0)
+    assert np.array_equal(four.get_state(), np.full(4 * nx, 2.0))
+print("done")
+''' % more)
