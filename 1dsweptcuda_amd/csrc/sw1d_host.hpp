@@ -52,15 +52,12 @@ public:
     hipError_t down(void* host, const void* dev, size_t bytes, hipStream_t s)
     {
         const size_t at = count_ < kPending ? take(bytes) : kNone;
-        if (at == kNone) {
-            if (bytes >= kPopulate) populate(host, bytes);
-            return hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s);
-        }
-        const hipError_t e = hipMemcpyAsync(p_ + at, dev, bytes, hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess)
-            pending_[count_++] = {host, at, bytes};
-        else
+        if (at == kNone && bytes >= kPopulate) populate(host, bytes);
+        const hipError_t e = hipMemcpyAsync(at == kNone ? host : p_ + at, dev, bytes, hipMemcpyDeviceToHost, s);
+        if (e != hipSuccess)
             count_ = 0;  // the call fails: its earlier results are not handed over
+        else if (at != kNone)
+            pending_[count_++] = {host, at, bytes};
         return e;
     }
 

@@ -1484,9 +1484,12 @@ int nn_gradient(sw1d_nn* N, int B, double* loss, float* grad_host = nullptr)
     if (rc || (!loss && !grad_host)) return rc;
     const int64_t nout = (int64_t)B * N->X;
     std::vector<float> lp(loss ? nblk(nout) : 0);
-    if (loss) NN_HIP(N->stage.down(lp.data(), N->lossp, lp.size() * sizeof(float), N->stream));
-    if (grad_host) NN_HIP(N->stage.down(grad_host, N->g, NPARAM * sizeof(float), N->stream));
-    NN_HIP(N->stage.finish(N->stream));
+    hipError_t e = hipSuccess;
+    if (loss) e = N->stage.down(lp.data(), N->lossp, lp.size() * sizeof(float), N->stream);
+    if (grad_host && e == hipSuccess) e = N->stage.down(grad_host, N->g, NPARAM * sizeof(float), N->stream);
+    const hipError_t done = N->stage.finish(N->stream);  // in any case: lp ends here
+    NN_HIP(e);
+    NN_HIP(done);
     if (loss) {
         double s = 0;
         for (float f : lp) s += f;

@@ -23,7 +23,8 @@ std::map<const char*, size_t> sizes;
 struct { Dim grid, block; size_t shared; void* stream; } config;
 char dummy[64];
 long launches, launch_limit = -1, mallocs, malloc_limit = -1, copies, copy_limit = -1, last_error;
-size_t new_limit = ~(size_t)0;
+size_t new_limit = ~(size_t)0, watch;
+void *watched[8], *freed[8];  // live and freed blocks of `watch` bytes (freed ones are kept)
 int fail(long& count, long limit)
 {
     ++count;
@@ -41,11 +42,27 @@ size_t size_of(const void* p)
 void* operator new(size_t n)
 {
     if (n > new_limit) throw std::bad_alloc();
-    if (void* p = malloc(n ? n : 1)) return p;
-    throw std::bad_alloc();
+    void* p = malloc(n ? n : 1);
+    if (!p) throw std::bad_alloc();
+    if (watch && n == watch)
+        for (void*& w : watched)
+            if (!w) {
+                w = p;
+                break;
+            }
+    return p;
 }
-void operator delete(void* p) noexcept { free(p); }
-void operator delete(void* p, size_t) noexcept { free(p); }
+void operator delete(void* p) noexcept
+{
+    if (watch && p)
+        for (int i = 0; i < 8; ++i)
+            if (watched[i] == p && !freed[i]) {
+                freed[i] = memset(p, 0x5a, watch);
+                return;
+            }
+    free(p);
+}
+void operator delete(void* p, size_t) noexcept { operator delete(p); }
 
 extern "C" {
 
@@ -174,4 +191,19 @@ void stub_fail_launch(long more) { launches = 0, launch_limit = more; }
 void stub_fail_malloc(long more) { mallocs = 0, malloc_limit = more; }
 void stub_fail_copy(long more) { copies = 0, copy_limit = more; }
 void stub_fail_new(size_t most) { new_limit = most; }
+// Blocks of `size` bytes from operator new are kept when they are deleted; the
+// number of those that were, and how many of them have been written to since.
+void stub_watch_new(size_t size) { watch = size; }
+int stub_freed() { return (int)(std::end(freed) - std::count(freed, std::end(freed), nullptr) - freed); }
+int stub_freed_written()
+{
+    int n = 0;
+    for (void* p : freed)
+        for (size_t i = 0; p && i < watch; ++i)
+            if (((unsigned char*)p)[i] != 0x5a) {
+                ++n;
+                break;
+            }
+    return n;
+}
 }

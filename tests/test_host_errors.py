@@ -103,3 +103,32 @@ with sw.Surrogate(nx, 4, seed=0) as nn, sw.Batch(*ks(nx, 1)) as one, sw.Batch(*k
     assert np.array_equal(four.get_state(), np.full(4 * nx, 2.0))
 print("done")
 ''' % more)
+
+
+@pytest.mark.parametrize("batch", [7, 100])
+def test_failed_result_copy_leaves_nothing_pending(child, batch):
+    """A gradient whose second result copy fails (through staging memory, or
+    directly where the inputs fill it) writes to the caller's memory neither then
+    nor on a later call, and the next gradient is whole."""
+    child(r'''
+B, nx = %d, 1024
+x = np.ones((B, nx), np.float32)
+with sw.Surrogate(nx, B, seed=0) as nn:
+    def gradient(g):
+        loss = C.c_double(7)
+        rc = sw.lib().sw1d_nn_gradient(nn._h, x.ctypes.data, x.ctypes.data, B, C.byref(loss), g.ctypes.data)
+        return rc, loss.value
+    for _ in range(3):  # the third round allocates the staging memory
+        nn.gradient(x, x)
+    g = np.full(nn.param_count(), 5, np.float32)
+    stub.stub_fail_copy(C.c_long(3))  # two inputs and the loss's sums arrive
+    stub.stub_watch_new(C.c_size_t(4 * B * nx // 256))  # the loss's sums on the host
+    assert gradient(g) == (EDEVICE, 7)
+    assert stub.stub_freed() == 1
+    stub.stub_fail_copy(C.c_long(-1))
+    nn.forward(x)
+    assert stub.stub_freed_written() == 0 and (g == 5).all()
+    stub.stub_watch_new(C.c_size_t(0))
+    assert gradient(g) == (0, 0) and (g == 0).all()
+print("done")
+''' % batch)
