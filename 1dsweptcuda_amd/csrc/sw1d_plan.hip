@@ -69,6 +69,9 @@ struct sw1d_plan {
 
     void* buf[2]{nullptr, nullptr};  // each nc*n REALs, component-major
     int cur = 0;                     // buffer holding the current (flat) state
+    // Once an advance has been captured, the buffer that the caller's graph starts
+    // from on every replay, where every later advance leaves the state too.
+    int home = -1;
     hipStream_t stream = nullptr;
     HostStage stage;  // host copies of the state
     // classic algorithm: a hipGraph of kClassicGraphSteps steps per starting buffer
@@ -307,12 +310,14 @@ int classic_step(sw1d_plan* p)
 // graph launch instead of 64 kernel launches; the kernels and their order
 // are the same, so the bits are the same).  The steps alternate the two buffers,
 // so a graph is kept per starting buffer; an even block returns to it.  With
-// per-kernel profiling on, or if capture fails, the steps are launched one by one.
+// per-kernel profiling on, if capture fails, or while the caller captures the
+// plan's stream (the runtime would run the graph then and there), the steps are
+// launched one by one.
 constexpr int64_t kClassicGraphSteps = 64;
 
-int classic_advance(sw1d_plan* p, int64_t nsteps)
+int classic_advance(sw1d_plan* p, int64_t nsteps, bool captured)
 {
-    if (!p->profiling && !p->classic_graph_failed && nsteps >= kClassicGraphSteps) {
+    if (!captured && !p->profiling && !p->classic_graph_failed && nsteps >= kClassicGraphSteps) {
         const int slot = p->cur;
         if (!p->classic_exec[slot]) {
             hipGraph_t g = nullptr;
@@ -562,6 +567,14 @@ int swept_advance(sw1d_plan* p, int64_t nsteps)
         if (rc) return rc;
     }
     return SW1D_OK;
+}
+
+// captured: the caller is capturing the plan's stream
+int advance(sw1d_plan* p, int64_t nsteps, bool captured)
+{
+    if (p->alg == SW1D_CLASSIC) return classic_advance(p, nsteps, captured);
+    if (p->alg == SW1D_TRAPEZOID) return wide_advance(p, nsteps);
+    return swept_advance(p, nsteps);
 }
 
 void release(sw1d_plan* p)
@@ -899,13 +912,14 @@ int sw1d_advance(sw1d_plan* p, int64_t nsteps)
 {
     if (!p) return fail(SW1D_EINVAL, "null plan");
     if (nsteps < 0) return fail(SW1D_EINVAL, "nsteps must be >= 0");
-    int rc;
-    if (p->alg == SW1D_CLASSIC) {
-        rc = classic_advance(p, nsteps);
-    } else if (p->alg == SW1D_TRAPEZOID) {
-        rc = wide_advance(p, nsteps);
-    } else {
-        rc = swept_advance(p, nsteps);
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    const bool captured = hipStreamIsCapturing(p->stream, &cs) == hipSuccess && cs == hipStreamCaptureStatusActive;
+    if (captured && p->home < 0) p->home = p->cur;
+    const int rc = advance(p, nsteps, captured);
+    if (rc == SW1D_OK && p->home >= 0 && p->cur != p->home) {
+        const size_t bytes = (size_t)(p->nc / 2) * (size_t)p->n * p->S;
+        HIP_OR_FAIL(hipMemcpyAsync(p->buf[p->home], p->buf[p->cur], bytes, hipMemcpyDeviceToDevice, p->stream));
+        p->cur = p->home;
     }
     return rc;
 }
@@ -952,7 +966,7 @@ int sw1d_advance_noalloc(const sw1d_problem* q, void* d_state, int64_t nsteps, v
     // launches one by one: no launch graph is captured or instantiated
     p.classic_graph_failed = true;
     rc = copy_state(&p, d_state, nullptr, true, false, false);
-    if (rc == SW1D_OK) rc = sw1d_advance(&p, nsteps);
+    if (rc == SW1D_OK) rc = advance(&p, nsteps, true);
     if (rc == SW1D_OK) rc = copy_state(&p, nullptr, d_state, false, false, false);
     if (rc == SW1D_OK) {
         const hipError_t e = hipGetLastError();

@@ -104,7 +104,9 @@ int sw1d_get_state_device(sw1d_plan* plan, void* device_ptr);
  * Euler:859-888) and sweptWrapper (Heat:543-682, KS:753-851,
  * Euler:927-1100) between two outputs.  Asynchronous on the plan's stream
  * for the GPU-only algorithms; the hybrid algorithm synchronises once per
- * CPU node.  Results are bitwise the same for every algorithm. */
+ * CPU node.  Results are bitwise the same for every algorithm.  A GPU-only
+ * advance may be captured from the plan's stream into a graph: every replay
+ * advances the state by nsteps more. */
 int sw1d_advance(sw1d_plan* plan, int64_t nsteps);
 int sw1d_synchronize(sw1d_plan* plan);
 /* Advance and return the elapsed device time in milliseconds (hipEvents on
