@@ -8,7 +8,9 @@
 // staging memory's own first touch costs 50 us per MB.  A large result into fresh
 // memory is bound by its pages' first touch (62 MB: 15.9 ms, 3.7 into memory in
 // use), so the pages are made present before the wait for the GPU's work,
-// beside which that costs nothing.
+// beside which that costs nothing.  Memory that the runtime knows (pinned by the
+// caller, or a device's) is copied directly: through staging memory 1 MB of pinned
+// memory took 51 us in and 57 out, directly 28 and 27.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -43,7 +45,7 @@ public:
 
     hipError_t up(void* dev, const void* host, size_t bytes, hipStream_t s)
     {
-        const size_t at = take(bytes);
+        const size_t at = take(host, bytes);
         if (at == kNone) return hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s);
         memcpy(p_ + at, host, bytes);
         return hipMemcpyAsync(dev, p_ + at, bytes, hipMemcpyHostToDevice, s);
@@ -51,8 +53,8 @@ public:
 
     hipError_t down(void* host, const void* dev, size_t bytes, hipStream_t s)
     {
-        const size_t at = count_ < kPending ? take(bytes) : kNone;
-        if (at == kNone && bytes >= kPopulate) populate(host, bytes);
+        const size_t at = count_ < kPending ? take(host, bytes) : kNone;
+        if (at == kNone && bytes >= kPopulate && !known(host)) populate(host, bytes);
         const hipError_t e = hipMemcpyAsync(at == kNone ? host : p_ + at, dev, bytes, hipMemcpyDeviceToHost, s);
         if (e != hipSuccess)
             count_ = 0;  // the call fails: its earlier results are not handed over
@@ -79,10 +81,19 @@ private:
     struct Pending { void* host; size_t at, bytes; };
 
     static size_t round(size_t n) { return (n + 4095) & ~(size_t)4095; }
-    // offset of `bytes` free bytes; none until finish() where they do not fit
-    size_t take(size_t bytes)
+    // 0.1 us
+    static bool known(const void* host)
     {
-        if (used_ + bytes > cap_ || (!p_ && rounds_ < 2)) return kNone;
+        hipPointerAttribute_t a;
+        if (hipPointerGetAttributes(&a, host) == hipSuccess) return a.type != hipMemoryTypeUnregistered;
+        (void)hipGetLastError();
+        return false;
+    }
+    // offset of `bytes` free bytes for a copy to or from `host`; none until finish()
+    // where they do not fit
+    size_t take(const void* host, size_t bytes)
+    {
+        if (used_ + bytes > cap_ || (!p_ && rounds_ < 2) || known(host)) return kNone;
         if (!p_ && hipHostMalloc((void**)&p_, cap_, hipHostMallocDefault) != hipSuccess) {
             (void)hipGetLastError();
             p_ = nullptr;

@@ -22,6 +22,7 @@ std::map<const void*, std::string> names;
 std::map<const char*, size_t> sizes;
 struct { Dim grid, block; size_t shared; void* stream; } config;
 char dummy[64];
+const void *copy_src, *copy_dst;  // of the last asynchronous copy
 long launches, launch_limit = -1, mallocs, malloc_limit = -1, copies, copy_limit = -1, last_error;
 size_t new_limit = ~(size_t)0, watch;
 void *watched[8], *freed[8];  // live and freed blocks of `watch` bytes (freed ones are kept)
@@ -114,10 +115,17 @@ int hipFree(void* p)
     free(p);
     return 0;
 }
-int hipHostMalloc(void** p, size_t n, unsigned) { return (*p = calloc(n, 1)) ? 0 : 2; }
-int hipHostFree(void* p)
+int hipHostMalloc(void** p, size_t n, unsigned)
 {
-    free(p);
+    if (!(*p = calloc(n, 1))) return 2;
+    sizes[(const char*)*p] = n;
+    return 0;
+}
+int hipHostFree(void* p) { return hipFree(p); }
+int hipPointerGetAttributes(int* type, const void* p)  // the first member is the type of memory
+{
+    auto it = sizes.upper_bound((const char*)p);
+    *type = it != sizes.begin() && (--it, (const char*)p < it->first + it->second);
     return 0;
 }
 int hipMemcpy(void* d, const void* s, size_t n, int)
@@ -128,6 +136,8 @@ int hipMemcpy(void* d, const void* s, size_t n, int)
 int hipMemcpyAsync(void* d, const void* s, size_t n, int, void*)
 {
     if (fail(copies, copy_limit)) return 2;
+    copy_src = s;
+    copy_dst = d;
     memcpy(d, s, n);
     return 0;
 }
@@ -191,6 +201,8 @@ void stub_fail_launch(long more) { launches = 0, launch_limit = more; }
 void stub_fail_malloc(long more) { mallocs = 0, malloc_limit = more; }
 void stub_fail_copy(long more) { copies = 0, copy_limit = more; }
 void stub_fail_new(size_t most) { new_limit = most; }
+const void* stub_copy_src() { return copy_src; }
+const void* stub_copy_dst() { return copy_dst; }
 // Blocks of `size` bytes from operator new are kept when they are deleted; the
 // number of those that were, and how many of them have been written to since.
 void stub_watch_new(size_t size) { watch = size; }

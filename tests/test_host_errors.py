@@ -132,3 +132,36 @@ with sw.Surrogate(nx, B, seed=0) as nn:
     assert gradient(g) == (0, 0) and (g == 0).all()
 print("done")
 ''' % batch)
+
+
+@pytest.mark.parametrize("n", [1000, 1 << 17])
+def test_pinned_and_device_memory_is_copied_directly(child, n):
+    """Staging memory serves pageable memory only: a state in memory that the
+    runtime knows (pinned, or a device's) is copied straight from and to it, on
+    every round, at its start and inside it."""
+    child(r'''
+n = %d
+stub.stub_copy_src.restype = stub.stub_copy_dst.restype = C.c_void_p
+u = np.arange(n, dtype=float)
+L = sw.lib()
+pinned = lambda p: stub.hipHostMalloc(p, C.c_size_t(16 * n), 0)
+device = lambda p: stub.hipMalloc(p, C.c_size_t(16 * n))
+for alloc in (pinned, device, None):
+    with sw.Plan(sw.KS, n, 0.005, algorithm=sw.CLASSIC) as p:
+        m = C.c_void_p()
+        if alloc:
+            assert alloc(C.byref(m)) == 0
+        for k in range(5):
+            buf = np.zeros(2 * n)
+            at = (m.value or buf.ctypes.data) + 8 * k
+            want = u + k
+            C.memmove(at, want.ctypes.data, 8 * n)
+            assert L.sw1d_set_state(p._h, C.c_void_p(at)) == 0
+            direct = alloc is not None or k == 0
+            assert (stub.stub_copy_src() == at) == direct, k
+            C.memset(at, 0, 8 * n)
+            assert L.sw1d_get_state(p._h, C.c_void_p(at)) == 0
+            assert (stub.stub_copy_dst() == at) == direct, k
+            assert np.array_equal(np.ctypeslib.as_array(C.cast(at, C.POINTER(C.c_double)), (n,)), want)
+print("done")
+''' % n)
