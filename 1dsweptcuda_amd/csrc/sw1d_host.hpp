@@ -7,8 +7,9 @@
 // directly: 4 MB take 131 us in and 239 out, staged 135 either way, and the
 // staging memory's own first touch costs 50 us per MB.  A large result into fresh
 // memory is bound by its pages' first touch (62 MB: 15.9 ms, 3.7 into memory in
-// use), so the pages are made present before the wait for the GPU's work,
-// beside which that costs nothing.  Memory that the runtime knows (pinned by the
+// use), so the pages of fresh memory are made present before the wait for the
+// GPU's work, beside which that costs nothing.  (For memory in use the walk over
+// its pages alone would cost 10 us of a 2 MB result's 115.)  Memory that the runtime knows (pinned by the
 // caller, or a device's) is copied directly: through staging memory 1 MB of pinned
 // memory took 51 us in and 57 out, directly 28 and 27.
 #pragma once
@@ -105,7 +106,8 @@ private:
         return at;
     }
     // Makes the whole pages of [host, host + bytes) present and writable, their
-    // contents as they are; where the kernel does not know the call, the copy
+    // contents as they are, unless the first, the middle and the last one are
+    // present already (0.5 us); where the kernel does not know the call, the copy
     // faults them in one by one.
     static void populate(void* host, size_t bytes)
     {
@@ -116,7 +118,13 @@ private:
 #endif
         const size_t page = (size_t)sysconf(_SC_PAGESIZE), a = reinterpret_cast<size_t>(host);
         const size_t lo = (a + page - 1) & ~(page - 1), hi = (a + bytes) & ~(page - 1);
-        if (hi > lo) (void)madvise(reinterpret_cast<void*>(lo), hi - lo, advice);
+        if (hi <= lo) return;
+        auto present = [&](size_t at) {
+            unsigned char v = 0;
+            return mincore(reinterpret_cast<void*>(at), page, &v) == 0 && (v & 1);
+        };
+        if (present(lo) && present(lo + (hi - lo) / page / 2 * page) && present(hi - page)) return;
+        (void)madvise(reinterpret_cast<void*>(lo), hi - lo, advice);
     }
 
     char* p_ = nullptr;

@@ -15,6 +15,8 @@
 #include <mutex>
 #include <new>
 #include <string>
+#include <sys/syscall.h>
+#include <unistd.h>
 
 namespace {
 struct Dim { uint32_t x, y, z; };
@@ -23,6 +25,7 @@ std::map<const char*, size_t> sizes;
 struct { Dim grid, block; size_t shared; void* stream; } config;
 char dummy[64];
 const void *copy_src, *copy_dst;  // of the last asynchronous copy
+long populated;  // bytes that madvise was asked to make present
 long launches, launch_limit = -1, mallocs, malloc_limit = -1, copies, copy_limit = -1, last_error;
 size_t new_limit = ~(size_t)0, watch;
 void *watched[8], *freed[8];  // live and freed blocks of `watch` bytes (freed ones are kept)
@@ -201,6 +204,12 @@ void stub_fail_launch(long more) { launches = 0, launch_limit = more; }
 void stub_fail_malloc(long more) { mallocs = 0, malloc_limit = more; }
 void stub_fail_copy(long more) { copies = 0, copy_limit = more; }
 void stub_fail_new(size_t most) { new_limit = most; }
+int madvise(void* p, size_t n, int advice)
+{
+    if (advice == 23) populated += n;  // MADV_POPULATE_WRITE
+    return (int)syscall(SYS_madvise, p, n, advice);
+}
+long stub_populated() { return populated; }
 const void* stub_copy_src() { return copy_src; }
 const void* stub_copy_dst() { return copy_dst; }
 // Blocks of `size` bytes from operator new are kept when they are deleted; the

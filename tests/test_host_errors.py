@@ -165,3 +165,28 @@ for alloc in (pinned, device, None):
             assert np.array_equal(np.ctypeslib.as_array(C.cast(at, C.POINTER(C.c_double)), (n,)), want)
 print("done")
 ''' % n)
+
+
+@pytest.mark.parametrize("touched", ["none", "all", "first", "middle", "last", "but the middle"])
+def test_only_fresh_results_are_made_present(child, touched):
+    """A large result's pages are made present ahead of the copy where they are
+    not (whichever part of the caller's memory has been used), and left alone
+    where they are: walking over them takes time."""
+    child(r'''
+import mmap
+n, touched = 1 << 19, "%s"
+stub.stub_populated.restype = C.c_long
+u = np.arange(n, dtype=float)
+with sw.Plan(sw.KS, n, 0.005, algorithm=sw.CLASSIC) as p, mmap.mmap(-1, 8 * n) as m:
+    p.set_state(u)
+    a = np.frombuffer(m, np.float64)
+    parts = {"none": [], "all": [slice(None)], "first": [slice(0, 9)], "last": [slice(n - 9, n)],
+             "middle": [slice(n // 2, n // 2 + 9)], "but the middle": [slice(0, n // 4), slice(3 * n // 4, n)]}
+    for part in parts[touched]:
+        a[part] = 1
+    assert sw.lib().sw1d_get_state(p._h, C.c_void_p(a.ctypes.data)) == 0
+    assert np.array_equal(a, u)
+    assert stub.stub_populated() == (0 if touched == "all" else 8 * n)
+    del a
+print("done")
+''' % touched)
