@@ -77,14 +77,16 @@ __global__ __launch_bounds__(kStepBlock) void k_step(const T* __restrict__ in, T
 
 // A heat step of a small field: one point per thread, the neighbours loaded
 // too (the three loads are in flight together, nothing follows but the update).
-template <typename T>
+// The kind of ends is a template argument: chosen at run time it became branches,
+// each waiting for an argument load of its own (2^14 points, FP64: 2.02 against
+// 1.99 us per step).
+template <typename T, bool PERIODIC>
 __global__ __launch_bounds__(kStepBlock) void k_heat_point(const T* __restrict__ in, T* __restrict__ out, int64_t n,
-                                                           int ends, T fo, T fo2)
+                                                           T fo, T fo2)
 {
     const int64_t i = (int64_t)blockIdx.x * kStepBlock + threadIdx.x;
     if (i >= n) return;
-    const bool periodic = ends == ENDS_PERIODIC;
-    const int64_t l = i > 0 ? i - 1 : (periodic ? n - 1 : 1), r = i < n - 1 ? i + 1 : (periodic ? 0 : n - 2);
+    const int64_t l = i == 0 ? (PERIODIC ? n - 1 : 1) : i - 1, r = i == n - 1 ? (PERIODIC ? 0 : n - 2) : i + 1;
     out[i] = heat_ftcs(in[l], in[i], in[r], fo, fo2);
 }
 
@@ -100,9 +102,10 @@ hipError_t step_points(int64_t n, int ends, const T* in, T* out, const Coef<T>& 
 // Points per lane.  KS: one while that gives a SIMD no more than one wave (a
 // step is then as long as a wave lives: 2^10 1.9 us against 2.0 in FP64 and
 // 2.1 in FP32), else 16 bytes, the widest load (2^20: 4.1 against 4.7 us in
-// FP64, 3.2 against 3.9 in FP32).  Heat: a point per thread up to two waves
-// per SIMD (2^16, FP64 and FP32: 1.93 and 2.01 us against 2.03 and 2.04), else
-// 16 bytes (2^20: 3.6 against 4.5, 2.7 against 3.3).  Euler: one up to eight
+// FP64, 3.2 against 3.9 in FP32).  Heat: a point per thread up to four waves
+// per SIMD in FP64 (2^18: 2.26 us against 2.29; 400001 points: 2.72 against 2.49)
+// and seven in FP32 (400001: 2.25 against 2.28 to 2.43; 2^19: 2.38 against 2.35),
+// else 16 bytes (2^20: 3.65 against 4.55, 2.75 against 3.38).  Euler: one up to eight
 // waves per SIMD (2^18: 7.9 against 8.7 us), where latency no longer counts
 // two, whose halo repeats 4 of 64 lanes instead of 8 (2^20: 22.4 against 23.9).
 template <typename T>
@@ -119,10 +122,14 @@ hipError_t step_prec(int eq, int bc, int64_t n, int simds, const void* in, void*
     T* b = static_cast<T*>(out);
     const int64_t waves = n / 56;  // of KS and Euler at one point per lane
     if (eq == EQ_HEAT) {
-        const int ends = bc == BC_MIRROR ? ENDS_MIRROR : ENDS_PERIODIC;
-        if (n > 2 * kWave * (int64_t)simds) return step_points<T, EQ_HEAT, V>(n, ends, a, b, k, s);
-        hipLaunchKernelGGL(k_heat_point<T>, dim3((unsigned)((n + kStepBlock - 1) / kStepBlock)), dim3(kStepBlock), 0, s,
-                           a, b, n, ends, k.fo, k.fo2);
+        const bool periodic = bc != BC_MIRROR;
+        if (n > (sizeof(T) == 8 ? 4 : 7) * kWave * (int64_t)simds)
+            return step_points<T, EQ_HEAT, V>(n, periodic ? ENDS_PERIODIC : ENDS_MIRROR, a, b, k, s);
+        const dim3 grid((unsigned)((n + kStepBlock - 1) / kStepBlock));
+        if (periodic)
+            hipLaunchKernelGGL((k_heat_point<T, true>), grid, dim3(kStepBlock), 0, s, a, b, n, k.fo, k.fo2);
+        else
+            hipLaunchKernelGGL((k_heat_point<T, false>), grid, dim3(kStepBlock), 0, s, a, b, n, k.fo, k.fo2);
         return hipGetLastError();
     }
     if (eq == EQ_KS)
