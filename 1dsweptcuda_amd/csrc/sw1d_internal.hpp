@@ -73,14 +73,25 @@ template <typename T> struct BatchJob {
 struct BatchTile { int32_t job, out0, count; };
 
 // Problems of one equation advanced with one tile shape: their tiles are
-// tiles[first .. first + ntiles), their launches an even number.
+// tiles[first .. first + ntiles), a launch of which takes up to `cap` steps.
 struct BatchGroup {
     int eq = 0, shape = 0;
-    int64_t launches = 0, first = 0, ntiles = 0;
+    int64_t cap = 0, first = 0, ntiles = 0;
+    int64_t launches(int64_t nsteps) const;  // for an advance of nsteps: an even number
 };
-// The groups and tiles of an advance of nsteps.
+// The groups and tiles that suit an advance of nsteps best.
 void batch_groups(const std::vector<int32_t>& eq, const std::vector<int64_t>& n, bool f64, int64_t nsteps, int cus,
                   std::vector<BatchGroup>& groups, std::vector<BatchTile>& tiles);
+// The sizes of some problems of equation e, each standing for `weight` of them.
+struct BatchSample {
+    std::vector<int64_t> n;
+    double weight = 1;
+};
+BatchSample batch_sample(const std::vector<int32_t>& eq, const std::vector<int64_t>& n, int e);
+// What an advance of nsteps should take with these groups, and with its own (by the
+// samples of both equations).
+double batch_us(const std::vector<BatchGroup>& groups, bool f64, int64_t nsteps, int cus);
+double batch_least_us(const BatchSample (&s)[2], bool f64, int64_t nsteps, int cus);
 
 struct BatchLaunch {
     int eq, shape, steps;

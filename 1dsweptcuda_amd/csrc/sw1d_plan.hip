@@ -5,6 +5,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -1129,9 +1130,16 @@ struct sw1d_batch {
     int32_t cus = 0;
     hipStream_t stream = nullptr;
     HostStage stage;  // host copies of the state
-    // launches of an advance of group_steps
-    int64_t group_steps = -1;
+    // tiles, made for advances of group_steps (0: none yet) in build_us
+    int64_t group_steps = 0;
+    double build_us = 0;
     std::vector<BatchGroup> groups;
+    // what an advance of other steps loses to tiles of its own, for the last ones
+    // met, and what all since the tiles were made have lost
+    struct Loss { int64_t steps; double us; };
+    std::vector<Loss> losses;
+    double lost_us = 0;
+    BatchSample sample[2];  // of the heat and the KS problems
     BatchTile* tiles = nullptr;  // device
     size_t tiles_cap = 0;
 };
@@ -1168,6 +1176,47 @@ void batch_release(sw1d_batch* B)
     delete B;
 }
 
+// The tiles for advances of nsteps, on the device.
+int batch_build(sw1d_batch* B, int64_t nsteps)
+{
+    const auto start = std::chrono::steady_clock::now();
+    std::vector<BatchTile> tiles;
+    B->group_steps = 0;
+    batch_groups(B->eq, B->n, B->f64, nsteps, B->cus, B->groups, tiles);
+    const auto made = std::chrono::steady_clock::now();
+    // earlier launches may still read the table
+    HIP_OR_FAIL(hipStreamSynchronize(B->stream));
+    const auto waited = std::chrono::steady_clock::now();
+    if (tiles.size() > B->tiles_cap) {
+        if (B->tiles) (void)hipFree(B->tiles);
+        B->tiles = nullptr;
+        B->tiles_cap = 0;
+        if (hipMalloc((void**)&B->tiles, tiles.size() * sizeof(BatchTile)) != hipSuccess)
+            return fail(SW1D_ENOMEM, "batch tile table of %zu tiles", tiles.size());
+        B->tiles_cap = tiles.size();
+    }
+    HIP_OR_FAIL(hipMemcpy(B->tiles, tiles.data(), tiles.size() * sizeof(BatchTile), hipMemcpyHostToDevice));
+    if (B->sample[0].n.empty() && B->sample[1].n.empty())
+        for (int e = EQ_HEAT; e <= EQ_KS; ++e) B->sample[e] = batch_sample(B->eq, B->n, e);
+    B->group_steps = nsteps;
+    B->losses.clear();
+    B->lost_us = 0;
+    const std::chrono::duration<double, std::micro> us = (made - start) + (std::chrono::steady_clock::now() - waited);
+    B->build_us = us.count();
+    return SW1D_OK;
+}
+
+// What an advance of nsteps loses on the tiles that there are.
+double batch_loss(sw1d_batch* B, int64_t nsteps)
+{
+    for (const sw1d_batch::Loss& l : B->losses)
+        if (l.steps == nsteps) return l.us;
+    const double us =
+        batch_us(B->groups, B->f64, nsteps, B->cus) - batch_least_us(B->sample, B->f64, nsteps, B->cus);
+    if (B->losses.size() >= 16) B->losses.erase(B->losses.begin());
+    B->losses.push_back({nsteps, std::max(us, 0.0)});
+    return B->losses.back().us;
+}
 
 }  // namespace
 
@@ -1216,7 +1265,7 @@ int sw1d_batch_create(sw1d_batch** out, int32_t precision, int64_t count, const 
         delete B;
         return fail(SW1D_EDEVICE, "no HIP device");
     }
-    B->cus = cus;
+    B->cus = cus > 0 ? cus : 256;
     const size_t bytes = (size_t)B->total * B->S;
     if (bytes <= HostStage::kMost) B->stage.reserve(bytes);
     if (hipStreamCreateWithFlags(&B->stream, hipStreamNonBlocking) != hipSuccess ||
@@ -1261,22 +1310,16 @@ int sw1d_batch_advance(sw1d_batch* B, int64_t nsteps)
     if (!B) return fail(SW1D_EINVAL, "null batch");
     if (nsteps < 0) return fail(SW1D_EINVAL, "nsteps must be >= 0");
     if (nsteps == 0) return SW1D_OK;
-    if (B->group_steps != nsteps) {
-        std::vector<BatchTile> tiles;
-        batch_groups(B->eq, B->n, B->f64, nsteps, B->cus, B->groups, tiles);
-        // earlier launches may still read the table
-        HIP_OR_FAIL(hipStreamSynchronize(B->stream));
-        B->group_steps = -1;
-        if (tiles.size() > B->tiles_cap) {
-            if (B->tiles) (void)hipFree(B->tiles);
-            B->tiles = nullptr;
-            B->tiles_cap = 0;
-            if (hipMalloc((void**)&B->tiles, tiles.size() * sizeof(BatchTile)) != hipSuccess)
-                return fail(SW1D_ENOMEM, "batch tile table of %zu tiles", tiles.size());
-            B->tiles_cap = tiles.size();
-        }
-        HIP_OR_FAIL(hipMemcpy(B->tiles, tiles.data(), tiles.size() * sizeof(BatchTile), hipMemcpyHostToDevice));
-        B->group_steps = nsteps;
+    // Tiles serve any number of steps, and making them for another one takes time
+    // (20000 problems: 2 ms, where the advance of one step takes 0.2): they are
+    // made anew once that would have paid.
+    if (B->group_steps != nsteps && B->group_steps) {
+        B->lost_us += batch_loss(B, nsteps);
+        if (B->lost_us > B->build_us) B->group_steps = 0;
+    }
+    if (!B->group_steps) {
+        const int rc = batch_build(B, nsteps);
+        if (rc) return rc;
     }
     for (const BatchGroup& g : B->groups) {
         BatchLaunch L;
@@ -1285,8 +1328,8 @@ int sw1d_batch_advance(sw1d_batch* B, int64_t nsteps)
         L.ntiles = g.ntiles;
         L.tiles = B->tiles + g.first;
         L.jobs = B->jobs;
-        const int64_t each = nsteps / g.launches, longer = nsteps % g.launches;
-        for (int64_t i = 0; i < g.launches; ++i) {
+        const int64_t launches = g.launches(nsteps), each = nsteps / launches, longer = nsteps % launches;
+        for (int64_t i = 0; i < launches; ++i) {
             L.steps = (int)(each + (i < longer));
             L.in = i % 2 ? B->b : B->a;
             L.out = i % 2 ? B->a : B->b;

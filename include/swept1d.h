@@ -195,7 +195,9 @@ int sw1d_initial_condition(int32_t kind, int32_t precision, int64_t n, double le
  * unused: tile shapes and steps per launch come from measured costs.  The state
  * is the concatenation of the problems' fields in index order, REAL per the
  * precision.  Every problem's result is bitwise the single-problem result.
- * The first advance by a new number of steps builds the table of its tiles. */
+ * The first advance makes the tables of tiles.  They serve any number of steps,
+ * and are made anew (which waits for the batch's stream and may allocate) once
+ * advances of another number have lost more time on them than that takes. */
 typedef struct sw1d_batch sw1d_batch;
 int sw1d_batch_create(sw1d_batch** batch, int32_t precision, int64_t count,
                       const int32_t* equation, const int64_t* nx, const double* dt,

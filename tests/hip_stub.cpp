@@ -25,6 +25,7 @@ std::map<const char*, size_t> sizes;
 struct { Dim grid, block; size_t shared; void* stream; } config;
 char dummy[64];
 const void *copy_src, *copy_dst;  // of the last asynchronous copy
+long uploads;    // calls of hipMemcpy
 long populated;  // bytes that madvise was asked to make present
 long launches, launch_limit = -1, mallocs, malloc_limit = -1, copies, copy_limit = -1, last_error;
 size_t new_limit = ~(size_t)0, watch;
@@ -133,6 +134,7 @@ int hipPointerGetAttributes(int* type, const void* p)  // the first member is th
 }
 int hipMemcpy(void* d, const void* s, size_t n, int)
 {
+    ++uploads;
     memcpy(d, s, n);
     return 0;
 }
@@ -209,6 +211,7 @@ int madvise(void* p, size_t n, int advice)
     if (advice == 23) populated += n;  // MADV_POPULATE_WRITE
     return (int)syscall(SYS_madvise, p, n, advice);
 }
+long stub_uploads() { return uploads; }
 long stub_populated() { return populated; }
 const void* stub_copy_src() { return copy_src; }
 const void* stub_copy_dst() { return copy_dst; }

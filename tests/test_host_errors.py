@@ -190,3 +190,26 @@ with sw.Plan(sw.KS, n, 0.005, algorithm=sw.CLASSIC) as p, mmap.mmap(-1, 8 * n) a
     del a
 print("done")
 ''' % touched)
+
+
+def test_batch_tiles_serve_other_step_counts(child):
+    """Step counts that change from call to call run on the tiles that there are,
+    until those have lost what new ones cost; much longer advances get tiles of
+    their own at once."""
+    child(r'''
+stub.stub_uploads.restype = C.c_long
+rng = np.random.default_rng(0)
+n = rng.integers(128, 4096, 20000)
+with sw.Batch(rng.integers(0, 2, n.size), n, np.full(n.size, 0.005), np.full(n.size, 0.5)) as b:
+    b.advance(10)
+    before = stub.stub_uploads()
+    for k in range(30):
+        b.advance(9 + k % 3)
+    assert stub.stub_uploads() - before < 10, stub.stub_uploads() - before
+    b.advance(1)
+    before = stub.stub_uploads()
+    for k in range(4):
+        b.advance(100000)
+    assert stub.stub_uploads() - before == 1
+print("done")
+''')
