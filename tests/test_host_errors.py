@@ -213,3 +213,23 @@ with sw.Batch(rng.integers(0, 2, n.size), n, np.full(n.size, 0.005), np.full(n.s
     assert stub.stub_uploads() - before == 1
 print("done")
 ''')
+
+
+def test_batch_advance_without_host_memory(child):
+    """Tiles that the host has no memory for are an error, not the program's end,
+    and the batch goes on afterwards."""
+    child(r'''
+n = np.full(3000, 4096)
+with sw.Batch(np.ones(n.size, np.int32), n, np.full(n.size, 0.005), np.full(n.size, 0.5)) as b:
+    stub.stub_fail_new(C.c_size_t(20000))  # less than the tiles take
+    raises(lambda: b.advance(10), ENOMEM)
+    raises(lambda: b.advance(10), ENOMEM)
+    stub.stub_fail_new(C.c_size_t(-1))
+    b.advance(10)
+    stub.stub_fail_new(C.c_size_t(20000))
+    b.advance(10)
+    raises(lambda: [b.advance(100000) for _ in range(3)], ENOMEM)
+    stub.stub_fail_new(C.c_size_t(-1))
+    b.advance(100000)
+print("done")
+''')
