@@ -15,6 +15,13 @@
 
 namespace sw1d {
 
+// In the operand's own precision.  A plain sqrt or fabs of a float is, on the host,
+// C's function of doubles, and a sum of two of them is rounded once less.
+SW1D_HD double root_of(double x) { return sqrt(x); }
+SW1D_HD float root_of(float x) { return sqrtf(x); }
+SW1D_HD double size_of(double x) { return fabs(x); }
+SW1D_HD float size_of(float x) { return fabsf(x); }
+
 // fused multiply-add, one rounding (FMA instructions on the GPU and the host)
 SW1D_HD double fmadd(double a, double b, double c) { return __builtin_fma(a, b, c); }
 SW1D_HD float fmadd(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
@@ -96,7 +103,7 @@ template <typename T> struct Ieee {
     static SW1D_HD T over(T b) { return b; }
     static SW1D_HD T div(T a, T b) { return a / b; }
     static SW1D_HD T quot(T a, T b) { return a / b; }  // a is not a negative zero
-    static SW1D_HD T root(T x) { return sqrt(x); }     // of a density
+    static SW1D_HD T root(T x) { return root_of(x); }  // of a density
 };
 
 // Euler:222-228 (limitor): cur + 1/2*min(ratio,1)*(other-cur).
@@ -132,7 +139,7 @@ SW1D_HD void eu_flux_diss(const Q3<T>& L, const Q3<T>& R, const EulerCoef<T>& k,
     const T hy = (sl * R.y + sr * L.y) * den;
     const T hz = (sl * R.z + sr * L.z) * den;
     const T ph = k.mgam * (hz - T(0.5) * hy * hy);  // Euler:202-212 (pressureHalf)
-    const T s = (sqrt(ph * k.gam) + fabs(hy));
+    const T s = (root_of(ph * k.gam) + size_of(hy));
     D.x = s * (L.x - R.x);
     D.y = s * (L.y - R.y);
     D.z = s * (L.z - R.z);
