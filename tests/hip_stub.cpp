@@ -14,6 +14,7 @@
 #include <map>
 #include <mutex>
 #include <new>
+#include <set>
 #include <string>
 #include <sys/syscall.h>
 #include <unistd.h>
@@ -22,6 +23,7 @@ namespace {
 struct Dim { uint32_t x, y, z; };
 std::map<const void*, std::string> names;
 std::map<const char*, size_t> sizes;
+std::set<std::string> launched;
 struct { Dim grid, block; size_t shared; void* stream; } config;
 char dummy[64];
 const void *copy_src, *copy_dst;  // of the last asynchronous copy
@@ -94,6 +96,7 @@ int __hipPopCallConfiguration(Dim* grid, Dim* block, size_t* shared, void** stre
 int hipLaunchKernel(const void* f, Dim, Dim, void** args, size_t, void*)
 {
     const std::string& name = names[f];
+    launched.insert(name);
     const bool network = name.find("k_net_fwdId") != std::string::npos;
     if (network && fail(launches, launch_limit)) return 2;
     if (network) {  // (in, 1/in_scale, parameters, weights, du, out, ..)
@@ -181,6 +184,12 @@ int hipEventCreateWithFlags(void** e, unsigned)
 }
 int hipEventDestroy(void*) { return 0; }
 int hipEventRecord(void*, void*) { return 0; }
+int hipEventSynchronize(void*) { return 0; }
+int hipEventElapsedTime(float* ms, void*, void*)
+{
+    *ms = 1;
+    return 0;
+}
 int hipGetDevice(int* d)
 {
     *d = 0;
@@ -213,6 +222,23 @@ int madvise(void* p, size_t n, int advice)
 }
 long stub_uploads() { return uploads; }
 long stub_populated() { return populated; }
+// The names of the library's kernels, and of those launched since the last call, a
+// line each.
+const char* stub_kernels()
+{
+    static std::string lines;
+    lines.clear();
+    for (const auto& k : names) lines += k.second + "\n";
+    return lines.c_str();
+}
+const char* stub_launched()
+{
+    static std::string lines;
+    lines.clear();
+    for (const std::string& k : launched) lines += k + "\n";
+    launched.clear();
+    return lines.c_str();
+}
 const void* stub_copy_src() { return copy_src; }
 const void* stub_copy_dst() { return copy_dst; }
 // Blocks of `size` bytes from operator new are kept when they are deleted; the

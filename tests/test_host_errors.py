@@ -1,47 +1,15 @@
 """What the library's host code does where a runtime call fails: a child process
 loads libswept1d.so with tests/hip_stub.cpp in the HIP runtime's place, which
 fails the calls that a test names.  No GPU."""
-import os
-import subprocess
-import sys
-
 import pytest
 
-from conftest import ROOT
-
-HEAD = r'''
-import ctypes as C, importlib, sys
-import numpy as np
-sys.path.insert(0, sys.argv[1])
-sw = importlib.import_module("1dsweptcuda_amd")
-stub = C.CDLL(None)
-sw.lib()
-def ks(n, count=1):
-    return np.ones(count, np.int32), np.full(count, n, np.int64), np.full(count, 0.005), np.full(count, 0.5)
-def raises(f, code):
-    try:
-        f()
-    except sw.SweptError as e:
-        assert "(%d)" % code in str(e), e
-        return
-    raise AssertionError("no error")
-EINVAL, EDEVICE, ENOMEM = -1, -2, -3
-'''
+import stubbed
 
 
 @pytest.fixture(scope="module")
 def child(tmp_path_factory):
-    so = str(tmp_path_factory.mktemp("stub") / "hip_stub.so")
-    src = os.path.join(os.path.dirname(os.path.abspath(__file__)), "hip_stub.cpp")
-    subprocess.run(["g++", "-O1", "-std=c++17", "-Wall", "-shared", "-fPIC", "-o", so, src], check=True)
-
-    def run(script):
-        preload = " ".join(p for p in (so, os.environ.get("LD_PRELOAD", "")) if p)
-        r = subprocess.run([sys.executable, "-c", HEAD + script, ROOT], env=dict(os.environ, LD_PRELOAD=preload),
-                           capture_output=True, text=True, timeout=120)
-        assert r.returncode == 0 and r.stdout.endswith("done\n"), r.stdout + r.stderr
-
-    return run
+    so = stubbed.build(tmp_path_factory.mktemp("stub"))
+    return lambda script: stubbed.run(so, script)
 
 
 @pytest.mark.parametrize("done", [0, 1, 2, 3])
