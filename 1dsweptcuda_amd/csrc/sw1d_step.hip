@@ -78,8 +78,8 @@ __global__ __launch_bounds__(kStepBlock) void k_step(const T* __restrict__ in, T
 // A heat step of a small field: one point per thread, the neighbours loaded
 // too (the three loads are in flight together, nothing follows but the update).
 // The kind of ends is a template argument: chosen at run time it became branches,
-// each waiting for an argument load of its own (2^14 points, FP64: 2.02 against
-// 1.99 us per step).
+// each waiting for an argument load of its own (2^17 points, FP64: 2.18 against
+// 2.16 us per step).
 template <typename T, bool PERIODIC>
 __global__ __launch_bounds__(kStepBlock) void k_heat_point(const T* __restrict__ in, T* __restrict__ out, int64_t n,
                                                            T fo, T fo2)
@@ -102,10 +102,11 @@ hipError_t step_points(int64_t n, int ends, const T* in, T* out, const Coef<T>& 
 // Points per lane.  KS: one while that gives a SIMD no more than one wave (a
 // step is then as long as a wave lives: 2^10 1.9 us against 2.0 in FP64 and
 // 2.1 in FP32), else 16 bytes, the widest load (2^20: 4.1 against 4.7 us in
-// FP64, 3.2 against 3.9 in FP32).  Heat: a point per thread up to four waves
-// per SIMD in FP64 (2^18: 2.26 us against 2.29; 400001 points: 2.72 against 2.49)
-// and seven in FP32 (400001: 2.25 against 2.28 to 2.43; 2^19: 2.38 against 2.35),
-// else 16 bytes (2^20: 3.65 against 4.55, 2.75 against 3.38).  Euler: one up to eight
+// FP64, 3.2 against 3.9 in FP32).  Heat: a point per thread up to two waves
+// per SIMD in FP64 (150001 points: 2.20 us with 16 bytes against 2.26) and seven in
+// FP32 (2^18: 2.13 against 2.25; 400001: 2.25 against 2.38; 2^19: 2.37 both), else
+// 16 bytes (2^20: 3.65 against 4.55, 2.75 against 3.38); means over plans at 14
+// places in memory, which alone make 5% of a step.  Euler: one up to eight
 // waves per SIMD (2^18: 7.9 against 8.7 us), where latency no longer counts
 // two, whose halo repeats 4 of 64 lanes instead of 8 (2^20: 22.4 against 23.9).
 template <typename T>
@@ -123,7 +124,7 @@ hipError_t step_prec(int eq, int bc, int64_t n, int simds, const void* in, void*
     const int64_t waves = n / 56;  // of KS and Euler at one point per lane
     if (eq == EQ_HEAT) {
         const bool periodic = bc != BC_MIRROR;
-        if (n > (sizeof(T) == 8 ? 4 : 7) * kWave * (int64_t)simds)
+        if (n > (sizeof(T) == 8 ? 2 : 7) * kWave * (int64_t)simds)
             return step_points<T, EQ_HEAT, V>(n, periodic ? ENDS_PERIODIC : ENDS_MIRROR, a, b, k, s);
         const dim3 grid((unsigned)((n + kStepBlock - 1) / kStepBlock));
         if (periodic)

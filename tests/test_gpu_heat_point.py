@@ -1,5 +1,5 @@
 """Classic heat steps around the size where a lane takes 16 bytes instead of one
-point (four waves per SIMD in FP64, seven in FP32), with both kinds of end, against
+point (two waves per SIMD in FP64, seven in FP32), with both kinds of end, against
 the oracle bit for bit."""
 import numpy as np
 import pytest
@@ -8,7 +8,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("bc", [0, 2])
-@pytest.mark.parametrize("prec,n", [(p, s + d) for p, s in ((0, 4 << 16), (1, 7 << 16)) for d in (-1, 0, 1)] +
+@pytest.mark.parametrize("prec,n", [(p, s + d) for p, s in ((0, 2 << 16), (1, 7 << 16)) for d in (-1, 0, 1)] +
                          [(p, n) for p in (0, 1) for n in (8, 255, 256, 257)])
 def test_heat_steps(sw, orc, prec, n, bc):
     dtype = np.float64 if prec == 0 else np.float32
