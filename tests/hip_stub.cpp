@@ -221,6 +221,7 @@ int madvise(void* p, size_t n, int advice)
     return (int)syscall(SYS_madvise, p, n, advice);
 }
 long stub_uploads() { return uploads; }
+long stub_mallocs() { return mallocs; }  // since the last stub_fail_malloc
 long stub_populated() { return populated; }
 // The names of the library's kernels, and of those launched since the last call, a
 // line each.

@@ -201,3 +201,24 @@ with sw.Batch(np.ones(n.size, np.int32), n, np.full(n.size, 0.005), np.full(n.si
     b.advance(100000)
 print("done")
 ''')
+
+
+def test_a_network_is_one_allocation(child):
+    """A network's arrays lie in one allocation, apart and aligned (an allocation
+    and its release take 0.1 ms each), and are refused and released as one."""
+    child(r'''
+stub.stub_mallocs.restype = C.c_long
+nx, B = 320, 5
+sw.Surrogate(nx, B).close()  # the device checks' own
+stub.stub_fail_malloc(C.c_long(-1))
+with sw.Surrogate(nx, B, seed=0) as nn:
+    assert stub.stub_mallocs() == 1
+    want = np.arange(nn.param_count(), dtype=np.float32)
+    nn.set_params(want)
+    nn.forward(np.ones((B, nx), np.float32))
+    nn.gradient(np.ones((B, nx), np.float32), np.ones((B, nx), np.float32))
+    assert np.array_equal(nn.get_params(), want)
+stub.stub_fail_malloc(C.c_long(0))
+raises(lambda: sw.Surrogate(nx, B), ENOMEM)
+print("done")
+''')
