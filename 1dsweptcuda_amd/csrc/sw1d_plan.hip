@@ -523,14 +523,20 @@ int wide_advance(sw1d_plan* p, int64_t nsteps)
 
 // Whether an advance of a swept plan runs as wide tiles (both sides' rates for
 // each equation: sw1d_wide.hip).  The swept rows, one launch each, are kept for
-// the hybrid, FP32 KS on large fields, and per-kernel profiling, which times the
-// swept kinds.
+// the hybrid, FP32 KS with nodes of 512 points or more and at least 1.5 of them
+// per SIMD, and per-kernel profiling, which times the swept kinds.
 bool takes_wide(const sw1d_plan* p)
 {
     if (p->profiling) return false;
     if (p->eq != EQ_KS) return p->alg == SW1D_SWEPT;
-    // FP32 KS with two waves per SIMD of 512 points or more: the diamonds (2^20,
-    // 1000 steps: 790 us at W = 512 against 913 us; W = 256 949 us)
+    // The rows run in rounds of two waves per SIMD, and the masked stages that they
+    // need from 1.5 (swept_tile) issue beside each other.  us per step, rows against
+    // wide tiles, by nodes per SIMD:
+    //             1.5          1.75         2            2.5          3
+    //   W = 512   0.78  0.77   0.78  0.86   0.78  0.94   1.04  1.09   1.04  1.20
+    //   W = 1024  1.38  1.21   1.38  1.28   1.39  1.65   2.33  1.79   2.34  2.21
+    // so W = 512 gains from the line on, W = 1024 around a whole round only; narrower
+    // nodes lose (W = 256 at 2^20: 0.95 against 0.91).
     const int64_t nodes = p->n / p->W;
     return p->f64 || p->W < 512 || 2 * nodes < 3 * (int64_t)p->simds;
 }
@@ -857,7 +863,9 @@ int sw1d_plan_destroy(sw1d_plan* p)
 // Copies the state in or out of the plan's current buffer on its stream: host
 // memory through the plan's staging memory, waiting for the copy, device memory
 // with sync.  Only the first value of a point (heat's even row, KS's u, Euler's
-// conserved values) goes in: the second is written before it is read.
+// conserved values) is the state.  The second is computed before it counts: the
+// swept rows load and carry it, but use it for no point before that (Euler's starts
+// as a copy of the first, heat's and KS's as what the buffer held).
 static int copy_state(sw1d_plan* p, const void* src, void* dst, bool to_device, bool host, bool sync = true)
 {
     const size_t S = p->S;

@@ -12,7 +12,8 @@
 // KS points by the state's way through the caches, a large Euler step by FP64
 // issue.  us per step, FP64, a launch per stage -> this kernel:
 //   KS 2^14 3.92 -> 2.04, 2^20 7.6 -> 4.1, 2^22 26.5 -> 11.6;
-//   Euler 2^14 5.7 -> 3.2, 2^20 37 -> 22 to 26; heat 2^20 4.5 -> 3.6
+//   Euler 2^14 5.7 -> 3.1, 2^20 37 -> 15.7 (Sod) to 20.9 (cells that all differ);
+//   heat 2^20 4.5 -> 3.6
 
 #include "sw1d_wide.hpp"
 
@@ -108,7 +109,8 @@ hipError_t step_points(int64_t n, int ends, const T* in, T* out, const Coef<T>& 
 // 16 bytes (2^20: 3.65 against 4.55, 2.75 against 3.38); means over plans at 14
 // places in memory, which alone make 5% of a step.  Euler: one up to eight
 // waves per SIMD (2^18: 7.9 against 8.7 us), where latency no longer counts
-// two, whose halo repeats 4 of 64 lanes instead of 8 (2^20: 22.4 against 23.9).
+// two, whose halo repeats 4 of 64 lanes instead of 8 (2^20, at the time: 22.4
+// against 23.9).
 template <typename T>
 hipError_t step_prec(int eq, int bc, int64_t n, int simds, const void* in, void* out, const Coefs& c, hipStream_t s)
 {

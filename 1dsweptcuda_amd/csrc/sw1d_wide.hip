@@ -1,4 +1,5 @@
-// Workgroup-wide overlapped tiles (sw1d_wide.hpp) for single plans: the kernels, and the choice of a tile shape and of the steps per launch.
+// Workgroup-wide overlapped tiles (sw1d_wide.hpp) for single plans: the kernels, and
+// the choice of a tile shape and of the steps per launch.
 //
 // An advance of N steps is L launches of N/L steps each (any N: no remainder
 // steps), ping-ponging between the plan's two state buffers.  More steps per
@@ -23,9 +24,10 @@
 // as trapezoids.)
 // At 2^20 a KS launch of 64 steps takes 62 us: 53 us of FP64 issue at 4.04
 // cycles per instruction (12.7% of it the window's overlap, 6.7% the halo
-// lanes), 3% exchanges, the rest the launch.  FP32 KS at 2^19 and more is the
-// one case the diamonds win (1.32e12 against 1.14e12 at 2^20): FP32
-// instructions of two waves co-issue, and the diamonds evaluate fewer points.
+// lanes), 3% exchanges, the rest the launch.  FP32 KS on large fields is the one
+// case the diamonds win (nodes of 512 points at 2^20: 1.33e12 against 1.12e12): FP32
+// instructions of two waves co-issue, and the diamonds evaluate fewer points.  From
+// which size, and at which node widths, takes_wide (sw1d_plan.hip) says.
 // An Euler cell's step is some 460 instructions; at 2^20 a launch of 13 steps
 // of 4 cells per lane takes 232 us, nine tenths of it FP64 issue, a quarter of
 // which repeats neighbours' cells: the window's 928 cells lose 8 per step, and

@@ -84,18 +84,15 @@ def main(argv=None):
             _say(f"euler: {k} launches")
         elif g == "batch":
             wl = importlib.import_module("1dsweptcuda_amd.workloads")
-            at = importlib.import_module("1dsweptcuda_amd.autotune")
             eq, nx, dt, dx = wl.batch_problems(4096, seed=2024)
             packed = np.concatenate(wl.batch_ics(eq, nx, dx))
-            table = at.load()
-            tps = at.tile_points_for(nx, table) if table else None
             _say("batch: initial conditions ready")
             for prec in (sw.F64, sw.F32):
-                with sw.Batch(eq, nx, dt, dx, precision=prec, tile_points=tps, waves=at.load_waves()) as b:
+                with sw.Batch(eq, nx, dt, dx, precision=prec) as b:
                     b.set_state(packed)
                     b.advance(5000)
                     b.get_state()
-                _say(f"batch {'f64' if prec == sw.F64 else 'f32'}: 1 launch, 5000 steps")
+                _say(f"batch {'f64' if prec == sw.F64 else 'f32'}: 5000 steps")
         else:
             raise SystemExit(f"unknown group {g!r}")
 

@@ -15,7 +15,9 @@ workgroup-wide overlapped tile: its time comes from hipEvents recorded around
 every launch on the stream of a second plan, of the overlapped tiles' own
 algorithm (3), over the same steps, so the same launches.  It is given per H
 steps ("avg_launch_us", "flop_per_launch": 40 flop per KS point-update x nX x
-H) and per kernel launch ("kernel_launches", "avg_kernel_us").
+H) and per kernel launch ("kernel_launches", "avg_kernel_us", and in the
+configuration "steps_per_kernel_launch"; its "steps_per_tile_launch" is H, the
+swept tile's height that step counts are rounded to).
 
 The CPU baseline is the C oracle (the same KS stages) on a bounded sample of
 the same workload (same nX, fewer steps), timed on this host with OpenMP over
@@ -189,7 +191,8 @@ def main():
         "config": {"workload": "Kuramoto-Sivashinsky 1D, RK2 + central differences, FP64, periodic, "
                                "shared swept (alg 1)",
                    "nx": n, "dx": 0.5, "dt": dt, "algorithm": "shared swept (alg 1)",
-                   "node_width": W, "steps_per_tile_launch": H},
+                   "node_width": W, "steps_per_tile_launch": H,
+                   "steps_per_kernel_launch": round(steps / launches)},
         "classic": {"value": classic_value, "steps": csteps, "ms_per_step": csecs / csteps * 1e3,
                     "roofline": {"bound": "hbm", "achieved": classic_gbs, "peak": HBM_PEAK_GBS,
                                  "unit": "GB/s", "frac": classic_gbs / HBM_PEAK_GBS,
@@ -344,41 +347,31 @@ def _sizes(sw, seed, steps=20000):
 
 
 def _trapezoid(sw, n, dt, u0, args):
-    """Same workload on the overlapped trapezoid engine (algorithm 3), timed
-    over the same requested steps rounded up to whole tile launches."""
-    res = {}
-    for W, depth in ((512, 2), (1024, 2)):
-        p = sw.Plan(sw.KS, n, dt, algorithm=sw.TRAPEZOID, node_width=W, tile_depth=depth)
-        H = p.info()["tile_steps"]
-        steps = _whole_launches(H, args.steps, MIN_TIMED_LAUNCHES)
-        p.set_state(u0)
-        _warm(p, args.warmup, MIN_WARM_LAUNCHES)
-        secs = _timed(p, steps)
-        p.close()
-        res["W%d_depth%d" % (W, depth)] = n * steps / secs
-    best = max(res, key=res.get)
-    return {"value": res[best], "config": best, "all": res, "unit": "point-updates/s"}
+    """Same workload on the overlapped tiles' own algorithm (3), timed over the
+    same requested steps rounded up to whole tile heights.  The tiles choose their
+    own width and steps per launch, whatever the plan's."""
+    p = sw.Plan(sw.KS, n, dt, algorithm=sw.TRAPEZOID, node_width=1024, tile_depth=2)
+    steps = _whole_launches(p.info()["tile_steps"], args.steps, MIN_TIMED_LAUNCHES)
+    p.set_state(u0)
+    _warm(p, args.warmup, MIN_WARM_LAUNCHES)
+    secs = _timed(p, steps)
+    p.close()
+    return {"value": n * steps / secs, "steps": steps, "unit": "point-updates/s"}
 
 
 def _batched(sw, count=4096, steps=5000, loop_sample=512):
     """4096 uneven periodic heat/KS problems, 5000 steps, all of them in each
     launch, against a per-problem launch loop (trapezoid plans)."""
     wl = importlib.import_module("1dsweptcuda_amd.workloads")
-    at = importlib.import_module("1dsweptcuda_amd.autotune")
     eq, nx, dt, dx = wl.batch_problems(count, seed=2024)
     ics = wl.batch_ics(eq, nx, dx)
-    table = at.load()
-    tps = at.tile_points_for(nx, table) if table else None
-    waves = at.load_waves()
     total = float(nx.sum())
-    res = {"problems": count, "steps": steps, "total_points": int(total),
-           "tile_table": {str(k): v for k, v in table.items()} or "size heuristic",
-           "waves_per_workgroup": waves}
+    res = {"problems": count, "steps": steps, "total_points": int(total)}
     packed = np.concatenate(ics)
     for prec, name in ((sw.F64, "f64"), (sw.F32, "f32")):
-        with sw.Batch(eq, nx, dt, dx, precision=prec, tile_points=tps, waves=waves) as b:
+        with sw.Batch(eq, nx, dt, dx, precision=prec) as b:
             b.set_state(packed)
-            b.advance(steps)  # plans the launches of this step count
+            b.advance(steps)  # makes the tiles
             b.set_state(packed)
             t0 = time.perf_counter()
             device_ms = b.advance_timed(steps)  # returns after the launch completes

@@ -47,10 +47,10 @@ enum { SW1D_F64 = 0, SW1D_F32 = 1 };
  * 2 hybrid CPU+GPU swept (heat, Euler) / register swept (KS).
  * 3 (library only, no reference counterpart): overlapped trapezoid tiles —
  * swept up-triangles widened by a redundant halo, any nx, same bits.
- * Advances of 1, 3 and the KS 2 run as overlapped tiles a workgroup wide
- * wherever those are faster than a row of swept tiles per launch (all but FP32
- * KS on large fields); per-kernel profiling runs and times the swept rows of 1
- * and 2. */
+ * Advances of 1, 3 and the KS 2 run as overlapped tiles a workgroup wide, but for
+ * FP32 KS (1 and 2) on large fields with nodes of 512 points or more, where a row
+ * of swept tiles per launch is faster, and a single step, which is the classic one;
+ * per-kernel profiling runs and times the swept rows of 1 and 2. */
 enum { SW1D_CLASSIC = 0, SW1D_SWEPT = 1, SW1D_ALT = 2, SW1D_TRAPEZOID = 3 };
 /* Boundary conditions.  DEFAULT picks the reference's: heat insulated
  * (mirror, Heat:140-142), KS periodic (KS:199), Euler Dirichlet ghost cells
@@ -210,8 +210,9 @@ int sw1d_batch_advance_timed(sw1d_batch* batch, int64_t nsteps, double* elapsed_
 /* The diamonds per workgroup of the reference's tuning: 2, 4 (default) or 8,
  * checked and otherwise unused (a tile is a workgroup of four waves). */
 int sw1d_batch_set_workgroup(sw1d_batch* batch, int32_t waves);
-/* info[0] total points, info[1] workgroups at work at once, info[2] problems,
- * info[3] device bytes */
+/* info[0] total points, info[1] min(four per compute unit, problems), which says
+ * nothing of the tiles, info[2] problems, info[3] device bytes of the states and
+ * the problems' coefficients */
 int sw1d_batch_info(const sw1d_batch* batch, int64_t info[4]);
 
 /* Learned KS surrogate -------------------------------------------------------
@@ -232,9 +233,10 @@ int sw1d_nn_create(sw1d_nn** nn, int32_t nx, int32_t max_batch, uint64_t seed);
 int sw1d_nn_destroy(sw1d_nn* nn);
 int sw1d_nn_set_scales(sw1d_nn* nn, double in_scale, double out_scale);
 /* Inference kernels (forward and surrogate steps): 0 = automatic (one
- * whole-network launch at multiples of 256, the training kernels otherwise), 1 = per-layer launches (nx a
- * multiple of 256), 2 = the whole-network kernel (nx = 1024).  Every choice
- * gives the same bits. */
+ * whole-network launch at multiples of 256, the training kernels otherwise),
+ * 1 = per-layer launches (nx a multiple of 256), 2 = the whole-network kernel
+ * (accepted for nx = 1024 only; 0 takes it at every multiple of 256).  Every
+ * choice gives the same bits. */
 int sw1d_nn_set_inference(sw1d_nn* nn, int32_t mode);
 int sw1d_nn_get_params(sw1d_nn* nn, float* host);
 int sw1d_nn_set_params(sw1d_nn* nn, const float* host);
