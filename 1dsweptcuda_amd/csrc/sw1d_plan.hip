@@ -1148,6 +1148,7 @@ struct sw1d_batch {
     struct Loss { int64_t steps; double us; };
     std::vector<Loss> losses;
     double lost_us = 0;
+    double scale = 0;       // of the sample's estimates: what they make of group_steps (0: not asked yet)
     BatchSample sample[2];  // of the heat and the KS problems
     BatchTile* tiles = nullptr;  // device
     size_t tiles_cap = 0;
@@ -1209,7 +1210,7 @@ int batch_build(sw1d_batch* B, int64_t nsteps)
         for (int e = EQ_HEAT; e <= EQ_KS; ++e) B->sample[e] = batch_sample(B->eq, B->n, e);
     B->group_steps = nsteps;
     B->losses.clear();
-    B->lost_us = 0;
+    B->lost_us = B->scale = 0;
     const std::chrono::duration<double, std::micro> us = (made - start) + (std::chrono::steady_clock::now() - waited);
     B->build_us = us.count();
     return SW1D_OK;
@@ -1220,8 +1221,9 @@ double batch_loss(sw1d_batch* B, int64_t nsteps)
 {
     for (const sw1d_batch::Loss& l : B->losses)
         if (l.steps == nsteps) return l.us;
-    const double us =
-        batch_us(B->groups, B->f64, nsteps, B->cus) - batch_least_us(B->sample, B->f64, nsteps, B->cus);
+    auto least = [&](int64_t k) { return batch_least_us(B->sample, B->f64, k, B->cus); };
+    if (B->scale == 0) B->scale = batch_us(B->groups, B->f64, B->group_steps, B->cus) / least(B->group_steps);
+    const double us = batch_us(B->groups, B->f64, nsteps, B->cus) - B->scale * least(nsteps);
     if (B->losses.size() >= 16) B->losses.erase(B->losses.begin());
     B->losses.push_back({nsteps, std::max(us, 0.0)});
     return B->losses.back().us;

@@ -179,6 +179,15 @@ with sw.Batch(rng.integers(0, 2, n.size), n, np.full(n.size, 0.005), np.full(n.s
     for k in range(4):
         b.advance(100000)
     assert stub.stub_uploads() - before == 1
+# every 16th problem, of which estimates take a sample, is small: the nearly equal
+# step count still loses nothing
+n = np.where(np.arange(4096) % 16 == 0, 1024, 65536)
+with sw.Batch(np.ones(n.size, np.int32), n, np.full(n.size, 0.005), np.full(n.size, 0.5)) as b:
+    b.advance(1000)
+    before = stub.stub_uploads()
+    for k in range(12):
+        b.advance(1001 + k % 2)
+    assert stub.stub_uploads() - before <= 1, stub.stub_uploads() - before
 print("done")
 ''')
 
