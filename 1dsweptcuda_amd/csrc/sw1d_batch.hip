@@ -58,13 +58,19 @@ hipError_t launch_prec(const BatchLaunch& L, hipStream_t s)
     return L.eq == EQ_HEAT ? launch_group<T, EQ_HEAT>(L, s) : launch_group<T, EQ_KS>(L, s);
 }
 
-// Every `stride`-th of the problems named, for estimates: an advance by a new
-// number of steps makes some hundred of them.
+// One of every `stride` of the problems named, for estimates: an advance by a new
+// number of steps makes some hundred of them.  Which one varies from stride to
+// stride (a generator of its own, so the same every time): sizes in a pattern that
+// repeats would otherwise be sampled at one place of it.
 BatchSample sample_of(const std::vector<int64_t>& n, const std::vector<int>& at)
 {
     BatchSample s;
     const size_t stride = (at.size() + 255) / 256;
-    for (size_t j = 0; j < at.size(); j += stride) s.n.push_back(n[at[j]]);
+    uint32_t pick = 1;
+    for (size_t j = 0; j < at.size(); j += stride) {
+        pick = pick * 1664525u + 1013904223u;  // Numerical Recipes' linear congruential generator
+        s.n.push_back(n[at[j + (pick >> 16) % std::min(stride, at.size() - j)]]);
+    }
     if (!s.n.empty()) s.weight = (double)at.size() / (double)s.n.size();
     return s;
 }

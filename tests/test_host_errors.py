@@ -231,3 +231,22 @@ stub.stub_fail_malloc(C.c_long(0))
 raises(lambda: sw.Surrogate(nx, B), ENOMEM)
 print("done")
 ''')
+
+
+def test_batch_tiles_of_repeating_sizes(child):
+    """Sizes in a pattern that repeats get tiles that suit most of them, whichever
+    problem of the pattern is the first: estimates do not sample one place of it
+    (the large problems here take at least ten points per lane)."""
+    child(r'''
+import re
+stub.stub_launched.restype = C.c_char_p
+for period, count in ((8, 2048), (16, 4096), (3, 700)):
+    n = np.where(np.arange(count) % period == 0, 128, 50000)
+    for shift in range(3):
+        with sw.Batch(np.ones(count, np.int32), np.roll(n, shift), np.full(count, 0.005), np.full(count, 0.5)) as b:
+            stub.stub_launched()
+            b.advance(64)
+            points = [int(p) for p in re.findall(r"ShapeILi1ELi(\d+)E", stub.stub_launched().decode())]
+            assert max(points) >= 10, (period, shift, points)
+print("done")
+''')
