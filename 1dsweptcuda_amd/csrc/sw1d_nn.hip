@@ -1313,6 +1313,10 @@ struct sw1d_nn {
     double* unn = nullptr;
     double* l2p = nullptr;
     int64_t int_len = 0;
+    // training set (sw1d_nn_dataset)
+    float* data_x = nullptr;
+    float* data_t = nullptr;
+    int64_t data_samples = 0;
 };
 
 namespace {
@@ -1514,7 +1518,7 @@ void nn_release(sw1d_nn* N)
 {
     if (!N) return;
     if (N->stream) (void)hipStreamSynchronize(N->stream);
-    for (void* q : {N->arrays, (void*)N->usave, (void*)N->unn, (void*)N->l2p})
+    for (void* q : {N->arrays, (void*)N->usave, (void*)N->unn, (void*)N->l2p, (void*)N->data_x, (void*)N->data_t})
         if (q) (void)hipFree(q);
     if (N->stream) (void)hipStreamDestroy(N->stream);
     delete N;
@@ -1639,11 +1643,8 @@ int sw1d_nn_create(sw1d_nn** out, int32_t nx, int32_t max_batch, uint64_t seed)
     return SW1D_OK;
 }
 
-void sw1d_nn_release_dataset(sw1d_nn* N);
-
 int sw1d_nn_destroy(sw1d_nn* N)
 {
-    if (N) sw1d_nn_release_dataset(N);
     nn_release(N);
     return SW1D_OK;
 }
@@ -1888,33 +1889,6 @@ __global__ __launch_bounds__(NT) void k_sq_parts(const double* __restrict__ a, c
 }
 }  // namespace sw1dnn
 
-struct NnData {
-    float* x = nullptr;
-    float* t = nullptr;
-    int64_t nsamples = 0;
-};
-
-namespace {
-std::vector<std::pair<sw1d_nn*, NnData>> g_data;  // dataset per network
-NnData* data_of(sw1d_nn* N)
-{
-    for (auto& e : g_data)
-        if (e.first == N) return &e.second;
-    g_data.push_back({N, NnData{}});
-    return &g_data.back().second;
-}
-void free_data(sw1d_nn* N)
-{
-    for (size_t i = 0; i < g_data.size(); ++i)
-        if (g_data[i].first == N) {
-            if (g_data[i].second.x) (void)hipFree(g_data[i].second.x);
-            if (g_data[i].second.t) (void)hipFree(g_data[i].second.t);
-            g_data.erase(g_data.begin() + (long)i);
-            return;
-        }
-}
-}  // namespace
-
 extern "C" {
 
 // Build the training set from an FP64 KS batch: advance it nsnap times by
@@ -1956,29 +1930,28 @@ int sw1d_nn_dataset(sw1d_nn* N, sw1d_batch* batch, int32_t nsnap, int32_t k_step
             rc = SW1D_EDEVICE;
         for (size_t k = 0; k < blocks; ++k) { su += parts[2 * k]; sd += parts[2 * k + 1]; }
     }
-    NnData* D = data_of(N);
     if (rc == SW1D_OK) {
         const double cnt = (double)len * nsnap;
         N->in_scale = sqrt(su / cnt);
         N->out_scale = sqrt(sd / cnt);
-        if (D->x) (void)hipFree(D->x);
-        if (D->t) (void)hipFree(D->t);
-        D->x = D->t = nullptr;
-        D->nsamples = (int64_t)nsnap * bv.count;
-        if (hipMalloc((void**)&D->x, (size_t)D->nsamples * N->X * sizeof(float)) != hipSuccess ||
-            hipMalloc((void**)&D->t, (size_t)D->nsamples * N->X * sizeof(float)) != hipSuccess)
+        if (N->data_x) (void)hipFree(N->data_x);
+        if (N->data_t) (void)hipFree(N->data_t);
+        N->data_x = N->data_t = nullptr;
+        N->data_samples = (int64_t)nsnap * bv.count;
+        if (hipMalloc((void**)&N->data_x, (size_t)N->data_samples * N->X * sizeof(float)) != hipSuccess ||
+            hipMalloc((void**)&N->data_t, (size_t)N->data_samples * N->X * sizeof(float)) != hipSuccess)
             rc = SW1D_ENOMEM;
     }
     for (int s = 0; s < nsnap && rc == SW1D_OK; ++s)
         hipLaunchKernelGGL(k_make_pairs, dim3(blocks), dim3(NT), 0, N->stream, raw + (size_t)s * len,
-                           raw + (size_t)(s + 1) * len, D->x + (size_t)s * len, D->t + (size_t)s * len, len,
+                           raw + (size_t)(s + 1) * len, N->data_x + (size_t)s * len, N->data_t + (size_t)s * len, len,
                            1.0 / N->in_scale, 1.0 / N->out_scale);
     if (rc == SW1D_OK && (hipGetLastError() != hipSuccess || hipStreamSynchronize(N->stream) != hipSuccess))
         rc = SW1D_EDEVICE;
     if (dparts) (void)hipFree(dparts);
     (void)hipFree(raw);
     if (rc != SW1D_OK) return nn_fail(rc, "dataset generation failed");
-    if (nsamples) *nsamples = D->nsamples;
+    if (nsamples) *nsamples = N->data_samples;
     if (scales) { scales[0] = N->in_scale; scales[1] = N->out_scale; }
     return SW1D_OK;
 }
@@ -1987,30 +1960,28 @@ int sw1d_nn_dataset(sw1d_nn* N, sw1d_batch* batch, int32_t nsnap, int32_t k_step
 int sw1d_nn_fit(sw1d_nn* N, int64_t nfit, int32_t batch, int64_t iters, float lr, uint64_t seed,
                 double* last_loss)
 {
-    NnData* D = N ? data_of(N) : nullptr;
-    if (!D || !D->x) return nn_fail(SW1D_EINVAL, "no dataset (call sw1d_nn_dataset first)");
-    if (nfit <= 0 || nfit > D->nsamples) nfit = D->nsamples;
-    return sw1d_nn_train(N, D->x, D->t, nfit, batch, iters, lr, seed, last_loss);
+    if (!N || !N->data_x) return nn_fail(SW1D_EINVAL, "no dataset (call sw1d_nn_dataset first)");
+    if (nfit <= 0 || nfit > N->data_samples) nfit = N->data_samples;
+    return sw1d_nn_train(N, N->data_x, N->data_t, nfit, batch, iters, lr, seed, last_loss);
 }
 
 // Relative L2 error of the predicted K-step change over samples [first, first+count).
 int sw1d_nn_eval(sw1d_nn* N, int64_t first, int64_t count, double* rel_err)
 {
-    NnData* D = N ? data_of(N) : nullptr;
-    if (!D || !D->x || !rel_err) return nn_fail(SW1D_EINVAL, "no dataset or null argument");
-    if (first < 0 || count < 1 || first + count > D->nsamples) return nn_fail(SW1D_EINVAL, "range");
+    if (!N || !N->data_x || !rel_err) return nn_fail(SW1D_EINVAL, "no dataset or null argument");
+    if (first < 0 || count < 1 || first + count > N->data_samples) return nn_fail(SW1D_EINVAL, "range");
     const size_t row = (size_t)N->X;
     double se = 0, st = 0;
     std::vector<float> y, t;
     for (int64_t s = first; s < first + count; s += N->Bmax) {
         const int b = (int)std::min<int64_t>(N->Bmax, first + count - s);
-        NN_HIP(hipMemcpyAsync(N->x, D->x + s * row, b * row * sizeof(float), hipMemcpyDeviceToDevice, N->stream));
+        NN_HIP(hipMemcpyAsync(N->x, N->data_x + s * row, b * row * sizeof(float), hipMemcpyDeviceToDevice, N->stream));
         int rc = nn_infer(N, b, nullptr, nullptr);
         if (rc) return rc;
         y.resize(b * row);
         t.resize(b * row);
         NN_HIP(hipMemcpyAsync(y.data(), N->du, b * row * sizeof(float), hipMemcpyDeviceToHost, N->stream));
-        NN_HIP(hipMemcpyAsync(t.data(), D->t + s * row, b * row * sizeof(float), hipMemcpyDeviceToHost, N->stream));
+        NN_HIP(hipMemcpyAsync(t.data(), N->data_t + s * row, b * row * sizeof(float), hipMemcpyDeviceToHost, N->stream));
         NN_HIP(hipStreamSynchronize(N->stream));
         for (size_t k = 0; k < y.size(); ++k) {
             se += (double)(y[k] - t[k]) * (y[k] - t[k]);
@@ -2025,18 +1996,24 @@ int sw1d_nn_eval(sw1d_nn* N, int64_t first, int64_t count, double* rel_err)
 // snapshot s of problem b).  x_host / t_host may be NULL.
 int sw1d_nn_dataset_samples(sw1d_nn* N, int64_t first, int64_t count, float* x_host, float* t_host)
 {
-    NnData* D = N ? data_of(N) : nullptr;
-    if (!D || !D->x) return nn_fail(SW1D_EINVAL, "no dataset (call sw1d_nn_dataset first)");
-    if (first < 0 || count < 1 || first + count > D->nsamples) return nn_fail(SW1D_EINVAL, "range");
+    if (!N || !N->data_x) return nn_fail(SW1D_EINVAL, "no dataset (call sw1d_nn_dataset first)");
+    if (first < 0 || count < 1 || first + count > N->data_samples) return nn_fail(SW1D_EINVAL, "range");
     const size_t row = (size_t)N->X, bytes = (size_t)count * row * sizeof(float);
     if (x_host)
-        NN_HIP(hipMemcpyAsync(x_host, D->x + first * row, bytes, hipMemcpyDeviceToHost, N->stream));
+        NN_HIP(hipMemcpyAsync(x_host, N->data_x + first * row, bytes, hipMemcpyDeviceToHost, N->stream));
     if (t_host)
-        NN_HIP(hipMemcpyAsync(t_host, D->t + first * row, bytes, hipMemcpyDeviceToHost, N->stream));
+        NN_HIP(hipMemcpyAsync(t_host, N->data_t + first * row, bytes, hipMemcpyDeviceToHost, N->stream));
     NN_HIP(hipStreamSynchronize(N->stream));
     return SW1D_OK;
 }
 
-void sw1d_nn_release_dataset(sw1d_nn* N) { free_data(N); }
+void sw1d_nn_release_dataset(sw1d_nn* N)
+{
+    if (!N) return;
+    if (N->data_x) (void)hipFree(N->data_x);
+    if (N->data_t) (void)hipFree(N->data_t);
+    N->data_x = N->data_t = nullptr;
+    N->data_samples = 0;
+}
 
 }  // extern "C"

@@ -24,16 +24,20 @@ struct Dim { uint32_t x, y, z; };
 std::map<const void*, std::string> names;
 std::map<const char*, size_t> sizes;
 std::set<std::string> launched;
-struct { Dim grid, block; size_t shared; void* stream; } config;
+thread_local struct { Dim grid, block; size_t shared; void* stream; } config;
 char dummy[64];
 const void *copy_src, *copy_dst;  // of the last asynchronous copy
 long uploads;    // calls of hipMemcpy
 long populated;  // bytes that madvise was asked to make present
-long launches, launch_limit = -1, mallocs, malloc_limit = -1, copies, copy_limit = -1, last_error;
+long launches, launch_limit = -1, mallocs, malloc_limit = -1, copies, copy_limit = -1;
+thread_local long last_error;
 size_t new_limit = ~(size_t)0, watch;
 void *watched[8], *freed[8];  // live and freed blocks of `watch` bytes (freed ones are kept)
+std::recursive_mutex guard;  // of all the above
+typedef std::lock_guard<std::recursive_mutex> Lock;
 int fail(long& count, long limit)
 {
+    Lock lock(guard);
     ++count;
     if (limit < 0 || count <= limit) return 0;
     last_error = 2;
@@ -41,6 +45,7 @@ int fail(long& count, long limit)
 }
 size_t size_of(const void* p)
 {
+    Lock lock(guard);
     auto it = sizes.find((const char*)p);
     return it == sizes.end() ? 0 : it->second;
 }
@@ -95,6 +100,7 @@ int __hipPopCallConfiguration(Dim* grid, Dim* block, size_t* shared, void** stre
 }
 int hipLaunchKernel(const void* f, Dim, Dim, void** args, size_t, void*)
 {
+    Lock lock(guard);
     const std::string& name = names[f];
     launched.insert(name);
     const bool network = name.find("k_net_fwdId") != std::string::npos;
@@ -113,11 +119,13 @@ int hipMalloc(void** p, size_t n)
     *p = nullptr;
     if (fail(mallocs, malloc_limit)) return 2;
     if (!(*p = calloc(n ? n : 1, 1))) return 2;
+    Lock lock(guard);
     sizes[(const char*)*p] = n;
     return 0;
 }
 int hipFree(void* p)
 {
+    Lock lock(guard);
     sizes.erase((const char*)p);
     free(p);
     return 0;
@@ -125,12 +133,14 @@ int hipFree(void* p)
 int hipHostMalloc(void** p, size_t n, unsigned)
 {
     if (!(*p = calloc(n, 1))) return 2;
+    Lock lock(guard);
     sizes[(const char*)*p] = n;
     return 0;
 }
 int hipHostFree(void* p) { return hipFree(p); }
 int hipPointerGetAttributes(int* type, const void* p)  // the first member is the type of memory
 {
+    Lock lock(guard);
     auto it = sizes.upper_bound((const char*)p);
     *type = it != sizes.begin() && (--it, (const char*)p < it->first + it->second);
     return 0;

@@ -250,3 +250,26 @@ for period, count in ((8, 2048), (16, 4096), (3, 700)):
             assert max(points) >= 10, (period, shift, points)
 print("done")
 ''')
+
+
+def test_networks_of_several_threads(child):
+    """Networks of different threads keep their training sets apart."""
+    child(r'''
+import threading
+nx, failed = 128, []
+def work(t):
+    try:
+        for k in range(200):
+            with sw.Surrogate(nx, 2, seed=t) as nn, sw.Batch(*ks(nx, t + 1)) as b:
+                b.set_state(np.full((t + 1) * nx, t + 1.0))
+                samples = nn.dataset(b, 2, 1)[0]
+                assert samples == 2 * (t + 1), samples
+                assert nn.dataset_samples(0, samples)[0].shape[0] == samples
+    except Exception as e:
+        failed.append(repr(e))
+threads = [threading.Thread(target=work, args=(t,)) for t in range(12)]
+for t in threads: t.start()
+for t in threads: t.join()
+assert not failed, failed
+print("done")
+''')
