@@ -1628,9 +1628,12 @@ int sw1d_nn_create(sw1d_nn** out, int32_t nx, int32_t max_batch, uint64_t seed)
     for (int l = 0; l < 4; ++l)
         for (int64_t i = 0; i < TAPS * C * C; ++i)
             h[P_MID + l * MID_SZ + i] = (float)(normal(s) * sqrt(2.0 / (TAPS * C)));
-    hipError_t e = hipMemcpy(N->p, h.data(), NPARAM * sizeof(float), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemset(N->m, 0, NPARAM * sizeof(float));
-    if (e == hipSuccess) e = hipMemset(N->v, 0, NPARAM * sizeof(float));
+    // on the network's stream, which the null stream does not wait for
+    hipError_t e = hipMemcpyAsync(N->p, h.data(), NPARAM * sizeof(float), hipMemcpyHostToDevice, N->stream);
+    if (e == hipSuccess) e = hipMemsetAsync(N->m, 0, NPARAM * sizeof(float), N->stream);
+    if (e == hipSuccess) e = hipMemsetAsync(N->v, 0, NPARAM * sizeof(float), N->stream);
+    const hipError_t done = hipStreamSynchronize(N->stream);  // h ends here
+    if (e == hipSuccess) e = done;
     if (e != hipSuccess) {
         nn_release(N);
         return nn_fail(SW1D_EDEVICE, "surrogate initialisation", e);
@@ -1908,15 +1911,16 @@ int sw1d_nn_dataset(sw1d_nn* N, sw1d_batch* batch, int32_t nsnap, int32_t k_step
     if (hipMalloc((void**)&raw, bytes * (size_t)(nsnap + 1)) != hipSuccess)
         return nn_fail(SW1D_ENOMEM, "snapshot storage");
     int rc = SW1D_OK;
-    NN_HIP(hipStreamSynchronize(bv.stream));
-    NN_HIP(hipMemcpy(raw, bv.state, bytes, hipMemcpyDeviceToDevice));
-    for (int s = 1; s <= nsnap && rc == SW1D_OK; ++s) {
-        rc = sw1d_batch_advance(batch, k_steps);
-        if (rc == SW1D_OK && hipStreamSynchronize(bv.stream) != hipSuccess) rc = SW1D_EDEVICE;
-        if (rc == SW1D_OK &&
-            hipMemcpy(raw + (size_t)s * len, bv.state, bytes, hipMemcpyDeviceToDevice) != hipSuccess)
+    // Snapshots in the order of the batch's own stream: a plain copy between device
+    // memories returns before it is done, and the null stream that it runs on waits
+    // for no stream of the library's.
+    for (int s = 0; s <= nsnap && rc == SW1D_OK; ++s) {
+        if (s > 0) rc = sw1d_batch_advance(batch, k_steps);
+        if (rc == SW1D_OK && hipMemcpyAsync(raw + (size_t)s * len, bv.state, bytes, hipMemcpyDeviceToDevice,
+                                            bv.stream) != hipSuccess)
             rc = SW1D_EDEVICE;
     }
+    if (hipStreamSynchronize(bv.stream) != hipSuccess && rc == SW1D_OK) rc = SW1D_EDEVICE;
     const unsigned blocks = nblk(len);
     std::vector<double> parts(2 * (size_t)blocks);
     double* dparts = nullptr;

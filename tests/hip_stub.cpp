@@ -28,6 +28,7 @@ thread_local struct { Dim grid, block; size_t shared; void* stream; } config;
 char dummy[64];
 const void *copy_src, *copy_dst;  // of the last asynchronous copy
 long uploads;    // calls of hipMemcpy
+long unordered;  // work on the null stream that its call does not wait for
 long populated;  // bytes that madvise was asked to make present
 long launches, launch_limit = -1, mallocs, malloc_limit = -1, copies, copy_limit = -1;
 thread_local long last_error;
@@ -145,9 +146,10 @@ int hipPointerGetAttributes(int* type, const void* p)  // the first member is th
     *type = it != sizes.begin() && (--it, (const char*)p < it->first + it->second);
     return 0;
 }
-int hipMemcpy(void* d, const void* s, size_t n, int)
+int hipMemcpy(void* d, const void* s, size_t n, int kind)
 {
     ++uploads;
+    if (kind == 3) ++unordered;
     memcpy(d, s, n);
     return 0;
 }
@@ -161,6 +163,7 @@ int hipMemcpyAsync(void* d, const void* s, size_t n, int, void*)
 }
 int hipMemset(void* p, int v, size_t n)
 {
+    ++unordered;
     memset(p, v, n);
     return 0;
 }
@@ -231,6 +234,7 @@ int madvise(void* p, size_t n, int advice)
     return (int)syscall(SYS_madvise, p, n, advice);
 }
 long stub_uploads() { return uploads; }
+long stub_unordered() { return unordered; }
 long stub_mallocs() { return mallocs; }  // since the last stub_fail_malloc
 long stub_populated() { return populated; }
 // The names of the library's kernels, and of those launched since the last call, a
