@@ -1894,6 +1894,15 @@ __global__ __launch_bounds__(NT) void k_sq_parts(const double* __restrict__ a, c
 
 extern "C" {
 
+void sw1d_nn_release_dataset(sw1d_nn* N)
+{
+    if (!N) return;
+    if (N->data_x) (void)hipFree(N->data_x);
+    if (N->data_t) (void)hipFree(N->data_t);
+    N->data_x = N->data_t = nullptr;
+    N->data_samples = 0;
+}
+
 // Build the training set from an FP64 KS batch: advance it nsnap times by
 // k_steps, keep every snapshot, and store the normalised pairs in the network
 // (in_scale = RMS of u, out_scale = RMS of the K-step change).
@@ -1934,29 +1943,31 @@ int sw1d_nn_dataset(sw1d_nn* N, sw1d_batch* batch, int32_t nsnap, int32_t k_step
             rc = SW1D_EDEVICE;
         for (size_t k = 0; k < blocks; ++k) { su += parts[2 * k]; sd += parts[2 * k + 1]; }
     }
-    if (rc == SW1D_OK) {
-        const double cnt = (double)len * nsnap;
-        N->in_scale = sqrt(su / cnt);
-        N->out_scale = sqrt(sd / cnt);
-        if (N->data_x) (void)hipFree(N->data_x);
-        if (N->data_t) (void)hipFree(N->data_t);
-        N->data_x = N->data_t = nullptr;
+    const double cnt = (double)len * nsnap, in_scale = sqrt(su / cnt), out_scale = sqrt(sd / cnt);
+    const bool replaced = rc == SW1D_OK;
+    if (replaced) {
+        sw1d_nn_release_dataset(N);
         N->data_samples = (int64_t)nsnap * bv.count;
-        if (hipMalloc((void**)&N->data_x, (size_t)N->data_samples * N->X * sizeof(float)) != hipSuccess ||
-            hipMalloc((void**)&N->data_t, (size_t)N->data_samples * N->X * sizeof(float)) != hipSuccess)
+        if (dalloc(&N->data_x, (size_t)len * nsnap) != hipSuccess ||
+            dalloc(&N->data_t, (size_t)len * nsnap) != hipSuccess)
             rc = SW1D_ENOMEM;
     }
     for (int s = 0; s < nsnap && rc == SW1D_OK; ++s)
         hipLaunchKernelGGL(k_make_pairs, dim3(blocks), dim3(NT), 0, N->stream, raw + (size_t)s * len,
                            raw + (size_t)(s + 1) * len, N->data_x + (size_t)s * len, N->data_t + (size_t)s * len, len,
-                           1.0 / N->in_scale, 1.0 / N->out_scale);
+                           1.0 / in_scale, 1.0 / out_scale);
     if (rc == SW1D_OK && (hipGetLastError() != hipSuccess || hipStreamSynchronize(N->stream) != hipSuccess))
         rc = SW1D_EDEVICE;
     if (dparts) (void)hipFree(dparts);
     (void)hipFree(raw);
-    if (rc != SW1D_OK) return nn_fail(rc, "dataset generation failed");
+    if (rc != SW1D_OK) {
+        if (replaced) sw1d_nn_release_dataset(N);  // rather than a part of one
+        return nn_fail(rc, "dataset generation failed");
+    }
+    N->in_scale = in_scale;
+    N->out_scale = out_scale;
     if (nsamples) *nsamples = N->data_samples;
-    if (scales) { scales[0] = N->in_scale; scales[1] = N->out_scale; }
+    if (scales) { scales[0] = in_scale; scales[1] = out_scale; }
     return SW1D_OK;
 }
 
@@ -2009,15 +2020,6 @@ int sw1d_nn_dataset_samples(sw1d_nn* N, int64_t first, int64_t count, float* x_h
         NN_HIP(hipMemcpyAsync(t_host, N->data_t + first * row, bytes, hipMemcpyDeviceToHost, N->stream));
     NN_HIP(hipStreamSynchronize(N->stream));
     return SW1D_OK;
-}
-
-void sw1d_nn_release_dataset(sw1d_nn* N)
-{
-    if (!N) return;
-    if (N->data_x) (void)hipFree(N->data_x);
-    if (N->data_t) (void)hipFree(N->data_t);
-    N->data_x = N->data_t = nullptr;
-    N->data_samples = 0;
 }
 
 }  // extern "C"

@@ -293,3 +293,24 @@ with sw.Surrogate(nx, 2, seed=0) as nn, sw.Batch(*ks(nx, 2)) as b, sw.Plan(sw.EU
 assert stub.stub_unordered() == 0, stub.stub_unordered()
 print("done")
 ''')
+
+
+@pytest.mark.parametrize("more", [0, 1, 2, 3])
+def test_a_training_set_without_memory_is_none(child, more):
+    """A training set of which one array cannot be allocated is refused, and there is
+    none to train on then: not a part of one, and not the earlier one's arrays."""
+    child(r'''
+nx = 128
+with sw.Surrogate(nx, 2, seed=0) as nn, sw.Batch(*ks(nx, 2)) as b:
+    b.set_state(np.ones(2 * nx))
+    assert nn.dataset(b, 3, 5)[0] == 6
+    stub.stub_fail_malloc(C.c_long(%d))  # the snapshots, their sums, the inputs, the targets
+    raises(lambda: nn.dataset(b, 4, 5), ENOMEM)
+    stub.stub_fail_malloc(C.c_long(-1))
+    kept = %d < 2  # refused before anything was replaced
+    for f in (lambda: nn.fit(2, batch=2, lr=1e-3, seed=0), lambda: nn.eval(0, 2), lambda: nn.dataset_samples(0, 2)):
+        f() if kept else raises(f, EINVAL)
+    assert nn.dataset(b, 2, 5)[0] == 4
+    nn.fit(2, batch=2, lr=1e-3, seed=0)
+print("done")
+''' % (more, more))
