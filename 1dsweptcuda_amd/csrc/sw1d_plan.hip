@@ -1186,6 +1186,16 @@ void batch_release(sw1d_batch* B)
     delete B;
 }
 
+// A table that the batch's kernels read, in the order of their stream.  (A plain copy
+// of up to some 16 KB returns before it has arrived, and the null stream that it
+// runs on is not waited for by the batch's.)  The host's memory has been read.
+hipError_t batch_upload(sw1d_batch* B, void* dev, const void* host, size_t bytes)
+{
+    const hipError_t e = hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, B->stream);
+    const hipError_t done = hipStreamSynchronize(B->stream);
+    return e != hipSuccess ? e : done;
+}
+
 // The tiles for advances of nsteps, on the device.
 int batch_build(sw1d_batch* B, int64_t nsteps)
 {
@@ -1205,7 +1215,7 @@ int batch_build(sw1d_batch* B, int64_t nsteps)
             return fail(SW1D_ENOMEM, "batch tile table of %zu tiles", tiles.size());
         B->tiles_cap = tiles.size();
     }
-    HIP_OR_FAIL(hipMemcpy(B->tiles, tiles.data(), tiles.size() * sizeof(BatchTile), hipMemcpyHostToDevice));
+    HIP_OR_FAIL(batch_upload(B, B->tiles, tiles.data(), tiles.size() * sizeof(BatchTile)));
     if (B->sample[0].n.empty() && B->sample[1].n.empty())
         for (int e = EQ_HEAT; e <= EQ_KS; ++e) B->sample[e] = batch_sample(B->eq, B->n, e);
     B->group_steps = nsteps;
@@ -1285,7 +1295,7 @@ int sw1d_batch_create(sw1d_batch** out, int32_t precision, int64_t count, const 
         batch_release(B);
         return fail(SW1D_ENOMEM, "batch device allocation of %zu bytes failed", 2 * bytes);
     }
-    hipError_t e = hipMemcpy(B->jobs, B->jobs_host.data(), B->jobs_host.size(), hipMemcpyHostToDevice);
+    hipError_t e = batch_upload(B, B->jobs, B->jobs_host.data(), B->jobs_host.size());
     if (e != hipSuccess) {
         batch_release(B);
         return fail(SW1D_EDEVICE, "job table upload: %s", hipGetErrorString(e));

@@ -27,7 +27,7 @@ std::set<std::string> launched;
 thread_local struct { Dim grid, block; size_t shared; void* stream; } config;
 char dummy[64];
 const void *copy_src, *copy_dst;  // of the last asynchronous copy
-long uploads;    // calls of hipMemcpy
+long uploads;    // copies from the host to the device
 long unordered;  // work on the null stream that its call does not wait for
 long populated;  // bytes that madvise was asked to make present
 long launches, launch_limit = -1, mallocs, malloc_limit = -1, copies, copy_limit = -1;
@@ -148,13 +148,14 @@ int hipPointerGetAttributes(int* type, const void* p)  // the first member is th
 }
 int hipMemcpy(void* d, const void* s, size_t n, int kind)
 {
-    ++uploads;
-    if (kind == 3) ++unordered;
+    uploads += kind == 1;
+    unordered += kind == 1 || kind == 3;
     memcpy(d, s, n);
     return 0;
 }
-int hipMemcpyAsync(void* d, const void* s, size_t n, int, void*)
+int hipMemcpyAsync(void* d, const void* s, size_t n, int kind, void*)
 {
+    uploads += kind == 1;
     if (fail(copies, copy_limit)) return 2;
     copy_src = s;
     copy_dst = d;

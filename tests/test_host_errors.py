@@ -276,13 +276,17 @@ print("done")
 
 
 def test_no_work_on_the_null_stream_is_left_behind(child):
-    """Copies between device memories and fills return before they are done.  None
-    runs on the null stream, for which the library's streams do not wait: a
-    network's first optimiser state and a training set's snapshots are in the order
-    of the stream that uses them."""
+    """Copies between device memories, small ones to the device and fills return
+    before they are done.  None runs on the null stream, for which the library's
+    streams do not wait (but for the device checks', whose kernels run there too): a
+    batch's tables, a network's first optimiser state and a training set's snapshots
+    are in the order of the stream that uses them."""
     child(r'''
 stub.stub_unordered.restype = C.c_long
 nx = 128
+sw.Plan(sw.KS, 1024, 0.005).close()  # the device checks
+sw.Surrogate(nx, 2).close()
+checks = stub.stub_unordered()
 with sw.Surrogate(nx, 2, seed=0) as nn, sw.Batch(*ks(nx, 2)) as b, sw.Plan(sw.EULER, 1024, 1e-5) as p:
     b.set_state(np.ones(2 * nx))
     nn.dataset(b, 3, 5)
@@ -290,7 +294,7 @@ with sw.Surrogate(nx, 2, seed=0) as nn, sw.Batch(*ks(nx, 2)) as b, sw.Plan(sw.EU
     nn.advance(b, 3, 5, judge_every=2, tol=1.0)
     p.advance(9)
     p.get_state()
-assert stub.stub_unordered() == 0, stub.stub_unordered()
+assert stub.stub_unordered() == checks, (stub.stub_unordered(), checks)
 print("done")
 ''')
 
