@@ -979,7 +979,7 @@ int sw1d_advance_noalloc(const sw1d_problem* q, void* d_state, int64_t nsteps, v
     // launches one by one: no launch graph is captured or instantiated
     p.classic_graph_failed = true;
     rc = copy_state(&p, d_state, nullptr, true, false, false);
-    if (rc == SW1D_OK) rc = advance(&p, nsteps, true);
+    if (rc == SW1D_OK) rc = advance(&p, nsteps, false);
     if (rc == SW1D_OK) rc = copy_state(&p, nullptr, d_state, false, false, false);
     if (rc == SW1D_OK) {
         const hipError_t e = hipGetLastError();
