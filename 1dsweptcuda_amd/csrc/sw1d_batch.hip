@@ -30,10 +30,11 @@ __global__ __launch_bounds__(S::NT) void k_batch(const BatchTile* __restrict__ t
     __shared__ __attribute__((aligned(16))) T lds[S::template lds<T>];
     const BatchTile t = tiles[blockIdx.x];
     const BatchJob<T>& J = jobs[t.job];
-    Coef<T> k;
-    k.fo = J.c[0];
-    k.fo2 = J.c[1];
-    k.ks = KsCoef<T>{J.c[0], J.c[1], J.c[2], J.c[3], J.c[4]};
+    Coef<T, EQ> k;
+    if constexpr (EQ == EQ_HEAT)
+        k = {J.c[0], J.c[1]};
+    else
+        k = {KsCoef<T>{J.c[0], J.c[1], J.c[2], J.c[3], J.c[4]}};
     tile<T, EQ, S>(lds, in + J.offset, out + J.offset, J.n, 0, t.out0, t.count, steps, ENDS_PERIODIC, k);
 }
 

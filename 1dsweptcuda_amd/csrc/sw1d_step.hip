@@ -27,7 +27,7 @@ template <int EQ, int P> constexpr int kHalo = ((EQ == EQ_HEAT ? 1 : 4) + P - 1)
 
 template <typename T, int EQ, int P>
 __global__ __launch_bounds__(kStepBlock) void k_step(const T* __restrict__ in, T* __restrict__ out, int64_t n,
-                                                     int ends, Coef<T> k)
+                                                     int ends, Coef<T, EQ> k)
 {
     constexpr int HL = kHalo<EQ, P>;
     using S = Shape<EQ, P, 1, HL>;
@@ -92,11 +92,11 @@ __global__ __launch_bounds__(kStepBlock) void k_heat_point(const T* __restrict__
 }
 
 template <typename T, int EQ, int P>
-hipError_t step_points(int64_t n, int ends, const T* in, T* out, const Coef<T>& k, hipStream_t s)
+hipError_t step_points(int64_t n, int ends, const T* in, T* out, const Coefs& c, hipStream_t s)
 {
     constexpr int64_t own = (kWave - 2 * kHalo<EQ, P>) * P * (kStepBlock / kWave);
     hipLaunchKernelGGL((k_step<T, EQ, P>), dim3((unsigned)((n + own - 1) / own)), dim3(kStepBlock), 0, s, in, out, n,
-                       ends, k);
+                       ends, (coef_of<T, EQ>(c)));
     return hipGetLastError();
 }
 
@@ -114,12 +114,6 @@ hipError_t step_points(int64_t n, int ends, const T* in, T* out, const Coef<T>& 
 template <typename T>
 hipError_t step_prec(int eq, int bc, int64_t n, int simds, const void* in, void* out, const Coefs& c, hipStream_t s)
 {
-    Coef<T> k{};
-    if constexpr (sizeof(T) == 8) {
-        k.fo = c.fo_d; k.fo2 = c.fo2_d; k.ks = c.ks_d; k.eu = c.eu_d;
-    } else {
-        k.fo = c.fo_f; k.fo2 = c.fo2_f; k.ks = c.ks_f; k.eu = c.eu_f;
-    }
     constexpr int V = 16 / sizeof(T);
     const T* a = static_cast<const T*>(in);
     T* b = static_cast<T*>(out);
@@ -127,8 +121,9 @@ hipError_t step_prec(int eq, int bc, int64_t n, int simds, const void* in, void*
     if (eq == EQ_HEAT) {
         const bool periodic = bc != BC_MIRROR;
         if (n > (sizeof(T) == 8 ? 2 : 7) * kWave * (int64_t)simds)
-            return step_points<T, EQ_HEAT, V>(n, periodic ? ENDS_PERIODIC : ENDS_MIRROR, a, b, k, s);
+            return step_points<T, EQ_HEAT, V>(n, periodic ? ENDS_PERIODIC : ENDS_MIRROR, a, b, c, s);
         const dim3 grid((unsigned)((n + kStepBlock - 1) / kStepBlock));
+        const Coef<T, EQ_HEAT> k = coef_of<T, EQ_HEAT>(c);
         if (periodic)
             hipLaunchKernelGGL((k_heat_point<T, true>), grid, dim3(kStepBlock), 0, s, a, b, n, k.fo, k.fo2);
         else
@@ -136,11 +131,11 @@ hipError_t step_prec(int eq, int bc, int64_t n, int simds, const void* in, void*
         return hipGetLastError();
     }
     if (eq == EQ_KS)
-        return waves <= simds ? step_points<T, EQ_KS, 1>(n, ENDS_PERIODIC, a, b, k, s)
-                              : step_points<T, EQ_KS, V>(n, ENDS_PERIODIC, a, b, k, s);
+        return waves <= simds ? step_points<T, EQ_KS, 1>(n, ENDS_PERIODIC, a, b, c, s)
+                              : step_points<T, EQ_KS, V>(n, ENDS_PERIODIC, a, b, c, s);
     if (eq == EQ_EULER)
-        return waves <= 8 * (int64_t)simds ? step_points<T, EQ_EULER, 1>(n, ENDS_FIXED, a, b, k, s)
-                                           : step_points<T, EQ_EULER, 2>(n, ENDS_FIXED, a, b, k, s);
+        return waves <= 8 * (int64_t)simds ? step_points<T, EQ_EULER, 1>(n, ENDS_FIXED, a, b, c, s)
+                                           : step_points<T, EQ_EULER, 2>(n, ENDS_FIXED, a, b, c, s);
     return hipErrorInvalidValue;
 }
 

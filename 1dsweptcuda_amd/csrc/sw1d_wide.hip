@@ -43,7 +43,7 @@ namespace {
 
 template <typename T, int EQ, class S>
 __global__ __launch_bounds__(S::NT) void k_wide(const T* __restrict__ in, T* __restrict__ out, int64_t n,
-                                                int64_t wout, int steps, int ends, Coef<T> k)
+                                                int64_t wout, int steps, int ends, Coef<T, EQ> k)
 {
     __shared__ __attribute__((aligned(16))) T lds[S::template lds<T>];
     const int64_t out0 = (int64_t)blockIdx.x * wout;
@@ -53,12 +53,13 @@ __global__ __launch_bounds__(S::NT) void k_wide(const T* __restrict__ in, T* __r
 
 template <typename T, int EQ, int I = 0>
 hipError_t launch_shape(int shape, dim3 grid, const T* in, T* out, int64_t n, int64_t wout, int steps, int ends,
-                        const Coef<T>& k, hipStream_t s)
+                        const Coefs& c, hipStream_t s)
 {
     if constexpr (I < Table<EQ>::count) {
-        if (shape != I) return launch_shape<T, EQ, I + 1>(shape, grid, in, out, n, wout, steps, ends, k, s);
+        if (shape != I) return launch_shape<T, EQ, I + 1>(shape, grid, in, out, n, wout, steps, ends, c, s);
         using S = TableShape<EQ, I>;
-        hipLaunchKernelGGL((k_wide<T, EQ, S>), grid, dim3(S::NT), 0, s, in, out, n, wout, steps, ends, k);
+        hipLaunchKernelGGL((k_wide<T, EQ, S>), grid, dim3(S::NT), 0, s, in, out, n, wout, steps, ends,
+                           (coef_of<T, EQ>(c)));
         return hipGetLastError();
     } else {
         return hipErrorInvalidValue;
@@ -68,12 +69,6 @@ hipError_t launch_shape(int shape, dim3 grid, const T* in, T* out, int64_t n, in
 template <typename T>
 hipError_t launch_prec(const WideLaunch& L, const Coefs& c, hipStream_t s)
 {
-    Coef<T> k{};
-    if constexpr (sizeof(T) == 8) {
-        k.fo = c.fo_d; k.fo2 = c.fo2_d; k.ks = c.ks_d; k.eu = c.eu_d;
-    } else {
-        k.fo = c.fo_f; k.fo2 = c.fo2_f; k.ks = c.ks_f; k.eu = c.eu_f;
-    }
     const int win = window(entries(L.eq)[L.shape]);
     const int64_t most = win - 2 * (int64_t)reach(L.eq) * L.steps;  // points a tile can store
     if (most < 1) return hipErrorInvalidValue;
@@ -83,9 +78,9 @@ hipError_t launch_prec(const WideLaunch& L, const Coefs& c, hipStream_t s)
     const T* in = static_cast<const T*>(L.in);
     T* out = static_cast<T*>(L.out);
     switch (L.eq) {
-    case EQ_HEAT: return launch_shape<T, EQ_HEAT>(L.shape, grid, in, out, L.n, wout, L.steps, ends, k, s);
-    case EQ_KS: return launch_shape<T, EQ_KS>(L.shape, grid, in, out, L.n, wout, L.steps, ends, k, s);
-    case EQ_EULER: return launch_shape<T, EQ_EULER>(L.shape, grid, in, out, L.n, wout, L.steps, ends, k, s);
+    case EQ_HEAT: return launch_shape<T, EQ_HEAT>(L.shape, grid, in, out, L.n, wout, L.steps, ends, c, s);
+    case EQ_KS: return launch_shape<T, EQ_KS>(L.shape, grid, in, out, L.n, wout, L.steps, ends, c, s);
+    case EQ_EULER: return launch_shape<T, EQ_EULER>(L.shape, grid, in, out, L.n, wout, L.steps, ends, c, s);
     }
     return hipErrorInvalidValue;
 }

@@ -175,7 +175,29 @@ __device__ __forceinline__ void euler_stage(const T (&src)[3][P], T (&dst)[3][P]
     });
 }
 
-template <typename T> struct Coef { T fo, fo2; KsCoef<T> ks; EulerCoef<T> eu; };
+// An equation's own coefficients, a kernel argument: a launch takes longer with more
+// bytes of arguments. With those of all three equations (more than 100 B in FP64) a plain
+// launch took KS 2^10 4.3-4.9 us, heat 2^18 4.2-4.9 and heat 2^20 4.7-4.9; with its own
+// 3.6-3.8, 3.4-3.8 and 4.1. FP64 Euler (104 B of its own) is as before, FP32 too.
+template <typename T, int EQ> struct Coef;
+template <typename T> struct Coef<T, EQ_HEAT> { T fo, fo2; };
+template <typename T> struct Coef<T, EQ_KS> { KsCoef<T> ks; };
+template <typename T> struct Coef<T, EQ_EULER> { EulerCoef<T> eu; };
+template <typename T, int EQ>
+inline Coef<T, EQ> coef_of(const Coefs& c)
+{
+    constexpr bool f64 = sizeof(T) == 8;
+    if constexpr (EQ == EQ_HEAT) {
+        if constexpr (f64) return {c.fo_d, c.fo2_d};
+        else return {c.fo_f, c.fo2_f};
+    } else if constexpr (EQ == EQ_KS) {
+        if constexpr (f64) return {c.ks_d};
+        else return {c.ks_f};
+    } else {
+        if constexpr (f64) return {c.eu_d};
+        else return {c.eu_f};
+    }
+}
 
 // k steps of the wave's points.  The lanes at the window's ends keep the
 // neighbour they last had (carried registers): their points are stale anyway.
@@ -192,7 +214,7 @@ struct Steps {
 #pragma unroll
             for (int i = 0; i < RS; ++i) hl[c][i] = hr[c][i] = gl[c][i] = gr[c][i] = v[c][0];
     }
-    __device__ __forceinline__ void heat(const T (&s)[P], T (&d)[P], T (&a)[1], T (&b)[1], const Coef<T>& k)
+    __device__ __forceinline__ void heat(const T (&s)[P], T (&d)[P], T (&a)[1], T (&b)[1], const Coef<T, EQ>& k)
     {
         T e[P + 2];
         gather_carry<T, P, 1>(s, a, b, e);
@@ -200,7 +222,7 @@ struct Steps {
         for (int p = 0; p < P; ++p) d[p] = heat_ftcs(e[p], e[p + 1], e[p + 2], k.fo, k.fo2);
     }
     template <bool ENDS>
-    __device__ __forceinline__ void run(int steps, const Coef<T>& k, int c0, int cN)
+    __device__ __forceinline__ void run(int steps, const Coef<T, EQ>& k, int c0, int cN)
     {
         if constexpr (EQ == EQ_HEAT) {
             if (steps & 1) {
@@ -218,7 +240,8 @@ struct Steps {
                     T e[P + 4];
                     gather_carry<T, P, 2>(v[0], hl[0], hr[0], e);
 #pragma unroll
-                    for (int p = 0; p < P; ++p) q[0][p] = ks_predict(e[p], e[p + 1], e[p + 2], e[p + 3], e[p + 4], k.ks);
+                    for (int p = 0; p < P; ++p)
+                        q[0][p] = ks_predict(e[p], e[p + 1], e[p + 2], e[p + 3], e[p + 4], k.ks);
                 }
                 {
                     T e[P + 4];
@@ -243,7 +266,8 @@ struct Steps {
 // before out0; lds holds Shape::lds<T> values.
 template <typename T, int EQ, class S>
 __device__ __forceinline__ void tile(T* lds, const T* __restrict__ in, T* __restrict__ out, int64_t n, int64_t cs,
-                                     int64_t out0, int count, int steps, int ends, const Coef<T>& k)
+                                     int64_t out0, int count, int steps, int ends,
+                                     const Coef<T, EQ>& k)
 {
     constexpr int P = S::P, NW = S::NW, HL = S::HL, NC = S::NC, NT = S::NT, WIN = S::WIN;
     constexpr int NL = (WIN + NT - 1) / NT;
